@@ -21,12 +21,13 @@
 //                   `if (c) for x: A else for x: B`;
 //   drop_barriers   barriers between regions that share no written array go.
 //
-// Three rewrites work on the whole program because they change a launch:
+// Four rewrites work on the whole program because they change a launch:
 //   GatherTranspose column gathers X[d, c] over an innermost sequential d read a
 //                   transposed copy made by a tiled kernel in front of the launch;
+//   RaggedSum       sums whose bounds are data (a CSR row): teams of lanes take
+//                   the rows, whole workgroups the very long ones;
 //   LaneSplit       eight adjacent lanes share one iteration's sequential sum
-//                   (constant bounds: 16-byte pieces of each line; bounds that
-//                   are data, as in a CSR row: one element each, stride 8);
+//                   over constant bounds, 16-byte pieces of each line each;
 //   Coarsen         a large element-wise launch with one element per thread is
 //                   cut to a quarter so that vectorize gives each thread four.
 //
@@ -36,14 +37,15 @@
 // defined by concern in hipopt_control.cpp (constants, short loops, guards,
 // branches, aliases), hipopt_prefetch.cpp, hipopt_lds.cpp, hipopt_vector.cpp,
 // hipopt_regs.cpp (budget, hoisting, register caching), hipopt_keep.cpp and
-// hipopt_alias.cpp; the whole-program rewrites are in hipopt_launch.cpp and
-// hipopt_persist.cpp.
+// hipopt_alias.cpp; the whole-program rewrites are in hipopt_launch.cpp,
+// hipopt_ragged.cpp and hipopt_persist.cpp.
 #include "hipopt_pass.hpp"
 
 namespace parpy {
 
 void hip_optimize(Program& p, const Options& opts, NameGen& gen) {
   if (opts.opt_gather_transpose) hipopt::gather_transpose(p, opts, gen);
+  if (opts.opt_lane_split) hipopt::ragged_sum(p, opts, gen);
   if (opts.opt_lane_split && !opts.opt_mfma_sddmm) hipopt::lane_split(p, opts, gen);
   if (opts.opt_vectorize) hipopt::coarsen(p, opts, gen);
   for (auto& k : p.kernels) {

@@ -1,0 +1,522 @@
+// gfx950 memory passes, rewrites that change a launch: sums whose bounds are data (rows of a sparse matrix).
+#include <algorithm>
+#include <functional>
+
+#include "hipopt_pass.hpp"
+
+namespace parpy {
+namespace hipopt {
+
+namespace {
+
+// ================================================================ teams of lanes for sums of uneven length
+// `for row: for i in rows[row] .. rows[row + 1]: y[row] += f(i)` and the same with a column loop around the sum
+// (`C[row, j] += f(i, j)`): how long a row is stands in memory, a few rows may hold a thousand times the average,
+// and each element costs two dependent loads (its column, then what the column selects).  Two things bound such a
+// kernel when a fixed group of lanes walks each row one element at a time: the round trips of the longest row, and
+// one element in flight per lane.
+//
+//   * A row belongs to a team of T = L * P adjacent lanes of a wavefront: L lanes lie along the columns (16 bytes
+//     each where the columns allow it), P subteams take every P-th element of the row.
+//   * A subteam issues U elements at a time: index loads first, then what they select.  The last batch is clamped to
+//     the row's last element instead of branching, so that its loads are issued together as well.
+//   * A row longer than `longest` elements is left to the workgroup: its teams queue such rows in LDS, and after a
+//     barrier all waves share each of them.
+//
+// Measured (100 000 rows of 50 non-zeros on average, the longest 15 800, float64): eight lanes per row, one element in
+// flight 547 us, in teams 39 us.  Five million 8-byte gathers out of L2 are then what bounds it: 128 lines per
+// nanosecond, the rate at which random lines come out of L2 on this part.  20 000 rows of 24 on average (longest 3400)
+// times a 128-column matrix: one workgroup per row with the sum read and written back in LDS per element 840 us, in
+// teams 42 us: the workgroups that share the longest rows pull 1.7 MB each through one compute unit.
+struct RaggedSum {
+  Program& p;
+  const Options& opts;
+  NameGen& gen;
+  ElemSize isz;
+  Type ity;
+  Type bty = Type::scalar(ElemSize::Bool);
+
+  RaggedSum(Program& prog, const Options& o, NameGen& g) : p(prog), opts(o), gen(g), isz(o.int_size()), ity(Type::scalar(o.int_size())) {}
+
+  // a launch of this shape, taken apart
+  struct Rows {
+    Name row;
+    int64_t n = 0;            // rows
+    bool has_col = false;
+    Name col;
+    int64_t cols = 1;
+    Stmts pre;                // definitions of the row in front of the sum
+    S loop;                   // the sum loop
+    Stmts defs;               // definitions inside it
+    E acc, term, start;       // accumulator, summand, value the sum starts from
+    Stmts post;               // statements after the sum
+    int64_t elements = 0;     // length of the array that the loop variable walks, 0 when there is none
+    int64_t tpb = 0;          // threads per workgroup
+    bool one_group = false;   // the launch was a single workgroup
+  };
+
+  E iint(int64_t v) { return mk_int(v, isz); }
+  E add(E a, E b) { return mk_binop(BinOp::Add, a, b, a->ty); }
+
+  // `acc = acc + term` with definitions in front of it, bounds that are not both constants
+  bool sum_loop(const S& s, Rows& r) {
+    if (!(s->k == Stmt::For && s->map.k == GpuMap::None && !s->unroll && s->step == 1 && !s->body.empty() && !s->par.reduction)) return false;
+    if (s->lo->k == Expr::Int && s->hi->k == Expr::Int) return false;
+    std::set<Name> inner;
+    for (size_t q = 0; q + 1 < s->body.size(); ++q) {
+      const S& d = s->body[q];
+      if (d->k != Stmt::Def || !d->ty.is_scalar()) return false;
+      inner.insert(d->id);
+    }
+    const S& a = s->body.back();
+    if (a->k != Stmt::Assign) return false;
+    const E& acc = a->dst;
+    bool scalar_acc = acc->k == Expr::Var && acc->ty.is_scalar() && !inner.count(acc->name);
+    bool elem_acc = acc->k == Expr::Index && acc->args[0]->k == Expr::Var && !mentions(acc->args[1], s->id) && !has_load(acc->args[1]);
+    if (!(scalar_acc || elem_acc) || !(acc->ty.sz == ElemSize::F32 || acc->ty.sz == ElemSize::F64)) return false;
+    if (elem_acc)
+      for (auto& n : inner) if (mentions(acc->args[1], n)) return false;
+    if (!(a->expr->k == Expr::BinOpE && a->expr->bop == BinOp::Add)) return false;
+    const E &l = a->expr->args[0], &rr = a->expr->args[1];
+    E term = expr_eq(l, acc) ? rr : expr_eq(rr, acc) ? l : E();
+    if (!term) return false;
+    const Name& acc_name = scalar_acc ? acc->name : acc->args[0]->name;
+    bool ok = !mentions(term, acc_name) && !mentions(s->lo, acc_name) && !mentions(s->hi, acc_name);
+    int loads = 0;
+    auto scan = [&](const E& e) {
+      visit_exprs(e, [&](const E& x) {
+        if (x->k == Expr::Call || x->k == Expr::AddrOf || x->k == Expr::Raw || x->k == Expr::RegElem) ok = false;
+        if (x->k != Expr::Index) return;
+        ++loads;
+        E rest;
+        if (x->dim_shape.size() == 1 && affine_unit(x->args[1], s->id, &rest) && rest->k == Expr::Int)
+          r.elements = std::max(r.elements, x->dim_shape[0]);
+      });
+    };
+    scan(term);
+    for (size_t q = 0; q + 1 < s->body.size(); ++q) {
+      scan(s->body[q]->expr);
+      if (mentions(s->body[q]->expr, acc_name)) ok = false;
+    }
+    if (!ok || loads < 1) return false;
+    r.loop = s;
+    r.acc = acc;
+    r.term = term;
+    r.defs = Stmts(s->body.begin(), s->body.end() - 1);
+    return true;
+  }
+
+  // statements of one row (or of one row and column): definitions, the sum, what is done with it
+  bool row_body(const Stmts& body, Rows& r) {
+    int pos = -1;
+    for (size_t q = 0; q < body.size(); ++q) {
+      const S& st = body[q];
+      if (st->k == Stmt::For) {
+        if (pos >= 0 || !sum_loop(st, r)) return false;
+        pos = (int)q;
+        continue;
+      }
+      bool simple = (st->k == Stmt::Def && st->ty.is_scalar()) ||
+                    (st->k == Stmt::Assign && (st->dst->k == Expr::Index || (st->dst->k == Expr::Var && st->dst->ty.is_scalar())));
+      if (!simple) return false;
+      bool raw = false;
+      auto scan = [&](const E& e) { visit_exprs(e, [&](const E& x) { if (x->k == Expr::Call || x->k == Expr::AddrOf || x->k == Expr::Raw) raw = true; }); };
+      scan(st->expr);
+      scan(st->dst);
+      if (raw) return false;
+    }
+    if (pos < 0) return false;
+    const bool elem = r.acc->k == Expr::Index;
+    const Name& acc_name = elem ? r.acc->args[0]->name : r.acc->name;
+    for (int q = 0; q < (int)body.size(); ++q) {
+      if (q == pos) continue;
+      const S& st = body[q];
+      if (q < pos) {
+        // what the sum starts from: the last store to the element, or the definition of the scalar
+        bool init = elem ? st->k == Stmt::Assign && expr_eq(st->dst, r.acc) : st->k == Stmt::Def && st->id == acc_name;
+        if (init && !r.start && !mentions(st->expr, acc_name)) { r.start = st->expr; continue; }
+        if (st->k == Stmt::Assign && st->dst->k == Expr::Index) return false;
+        if (mentions(st->expr, acc_name) || (st->dst && mentions(st->dst, acc_name))) return false;
+        if (r.start && st->k == Stmt::Assign && mentions(r.start, st->dst->name)) return false;   // (the start value is evaluated behind the sum)
+        r.pre.push_back(st);
+      } else {
+        if (elem && (mentions(st->expr, acc_name) || (st->dst && mentions(st->dst, acc_name)))) return false;
+        if (st->k == Stmt::Assign && st->dst->k == Expr::Index && st->dst->args[0]->k != Expr::Var) return false;
+        r.post.push_back(st);
+      }
+    }
+    if (!r.start) {
+      if (!elem) return false;
+      r.start = r.acc;
+    }
+    // a store behind the sum to an array that the start value reads would be reordered with it only across rows; inside
+    // the row the start value is read first, as written
+    return true;
+  }
+
+  bool match(const Kernel& k, Rows& r) {
+    if (k.body.size() != 1 || k.block.y != 1 || k.block.z != 1) return false;
+    const S& root = k.body[0];
+    if (!(root->k == Stmt::For && root->step == 1 && root->lo->k == Expr::Int && root->lo->iv == 0 && root->hi->k == Expr::Int)) return false;
+    r.row = root->id;
+    r.n = root->hi->iv;
+    if (r.n < 64) return false;   // (less than a wavefront of rows)
+    const bool one_group = root->map.k == GpuMap::Thread && k.grid.x == 1;
+    if ((root->map.k == GpuMap::ThreadBlock || one_group) && root->map.dim == 0) {
+      // one thread per row
+      if (k.grid.y != 1 || k.grid.z != 1 || (one_group && r.n > root->map.n)) return false;
+      r.tpb = one_group ? 256 : root->map.tpb;
+      r.one_group = one_group;
+      return row_body(root->body, r);
+    }
+    if (root->map.k == GpuMap::Block && k.grid.x * k.grid.y * k.grid.z == r.n && root->map.n == r.n) {
+      // one workgroup per row, its threads along the columns
+      S inner;
+      Stmts before;
+      for (auto& st : root->body) {
+        if (st->k == Stmt::Sync) continue;
+        if (st->k == Stmt::Def && st->ty.is_scalar() && !inner) { before.push_back(st); continue; }
+        if (inner || !thread_mapped(st)) return false;
+        inner = st;
+      }
+      if (!inner || inner->step != 1 || inner->lo->k != Expr::Int || inner->lo->iv != 0 || inner->hi->k != Expr::Int || inner->par.reduction) return false;
+      r.has_col = true;
+      r.col = inner->id;
+      r.cols = inner->hi->iv;
+      r.tpb = 1024;   // the threads that share a long row (3000 rows of 60 times 256 columns: 256 / 512 / 1024 threads 107 / 67 / 57 us)
+      if (r.cols < 1 || !row_body(inner->body, r)) return false;
+      // everything in front of the sum belongs to the row; its bounds are the same for all columns
+      for (auto& st : r.pre)
+        if (st->k != Stmt::Def || mentions(st->expr, r.col)) return false;
+      if (mentions(r.loop->lo, r.col) || mentions(r.loop->hi, r.col)) return false;
+      if (r.acc->k == Expr::Index && !mentions(r.acc->args[1], r.col)) return false;
+      before.insert(before.end(), r.pre.begin(), r.pre.end());
+      r.pre = before;
+      return true;
+    }
+    return false;
+  }
+
+  // columns a lane takes side by side: 16 bytes when every access along the columns is unit-stride through an
+  // aligned parameter and rows are whole vectors
+  int64_t column_vector(const Kernel& k, const Rows& r) {
+    if (!r.has_col || !opts.assume_aligned) return 1;
+    int64_t v = 0;
+    bool ok = true;
+    std::set<Name> params;
+    for (auto& q : k.params) if (q.ty.is_pointer()) params.insert(q.id);
+    auto scan = [&](const E& e) {
+      visit_exprs(e, [&](const E& x) {
+        if (x->k != Expr::Index || !mentions(x->args[1], r.col)) return;
+        E rest;
+        if (!affine_unit(x->args[1], r.col, &rest) || x->args[0]->k != Expr::Var || !params.count(x->args[0]->name)) { ok = false; return; }
+        int64_t w = 16 / elem_bytes(x->ty.sz);
+        if (w != 4 && w != 2) { ok = false; return; }
+        v = v == 0 ? w : std::min(v, w);
+      });
+    };
+    scan(r.term);
+    scan(r.acc);
+    for (auto& d : r.defs) scan(d->expr);
+    return ok && v > 0 && r.cols % v == 0 ? v : 1;
+  }
+
+  static int64_t pow2_at_least(int64_t n) { int64_t q = 1; while (q < n) q *= 2; return q; }
+
+  bool apply(Kernel& k, const StmtP& launch) {
+    Rows r;
+    if (!match(k, r)) return false;
+    const int64_t V = column_vector(k, r);
+    const int64_t slots = r.cols / V;                       // vectors along the columns
+    const int64_t L = std::min<int64_t>(WAVE_SIZE, pow2_at_least(slots));
+    const int64_t chunks = (slots + L - 1) / L;
+    const int64_t K = chunks * V;                           // sums a lane holds
+    const int64_t words = elem_bytes(r.acc->ty.sz) / 4;
+    if (K * words > 16) return false;
+    // elements in flight per lane: up to sixteen registers of what they select
+    const int64_t U = r.has_col ? std::max<int64_t>(2, std::min<int64_t>(8, 16 / (K * words))) : 4;
+    const int64_t avg = r.elements > 0 ? std::max<int64_t>(1, r.elements / r.n) : 32;
+    // Subteams: two elements of an average row per lane, at least four lanes so that they share cache lines.  (100 000
+    // rows of 50 non-zeros, float64: 4 / 8 / 16 / 32 / 64 lanes 53 / 47 / 40 / 38 / 45 us; 300 000 rows of 16: 41.7 us
+    // on four lanes, 36.0 on eight and sixteen; 50 000 rows of 200: 110 us on 16, 94 on 64; 50 000 rows of 8 times 32
+    // columns: 22.4 / 17.7 / 17.4 / 20.9 us for 1 / 2 / 4 / 8 subteams.)  Rows that were the threads of one workgroup
+    // are too few to fill the chip in any case: 10.3 us on 16 lanes, 11.0 on eight.
+    const int64_t P = r.one_group ? 8 : std::min<int64_t>(WAVE_SIZE / L, std::max<int64_t>(pow2_at_least((avg + 1) / 2), r.has_col ? 1 : 4));
+    const int64_t T = L * P, tpb = r.tpb;
+    if (tpb % WAVE_SIZE != 0 || tpb < L * V || r.n * T > (int64_t(1) << 30)) return false;
+    const int64_t teams = tpb / T, waves = tpb / WAVE_SIZE;
+    if (r.has_col && (tpb < r.cols || waves * L * K * elem_bytes(r.acc->ty.sz) > 64 * 1024)) return false;
+    // Rows longer than this are shared by the workgroup.  A shared row costs two barriers and a round trip of its own,
+    // and the waves that have no such row wait for it: 256 elements for single sums (128 costs 5 to 20 %), fewer when
+    // every element moves a row of columns (64 against 256 elements: 17.4 and 20.1 us for the 32-column product above).
+    const int64_t longest = r.has_col ? std::max<int64_t>(64, 2 * avg) : std::max<int64_t>(256, 4 * avg);
+    // element numbers in 32 bits when the array they walk is known to be small enough
+    const bool small = r.elements > 0 && r.elements < (int64_t(1) << 29);
+    const ElemSize esz = small && isz == ElemSize::I64 ? ElemSize::I32 : isz;
+    const Type ety = Type::scalar(esz);
+    auto eint = [&](int64_t v) { return mk_int(v, esz); };
+    auto narrow = [&](const E& e) { return e->ty.sz == esz ? e : mk_convert(e, esz); };
+    auto widen = [&](const E& e) { return e->ty.sz == isz ? e : mk_convert(e, isz); };
+
+    const Name reg = gen.fresh(r.acc->k == Expr::Var ? r.acc->name.s + "_part" : "part");
+    const Type sty = Type::scalar(r.acc->ty.sz);
+    auto part = [&](const E& c) {
+      auto e = std::make_shared<Expr>();
+      e->k = Expr::RegElem;
+      e->ty = sty;
+      e->name = reg;
+      e->args = {c};
+      return E(e);
+    };
+    // for (c = 0; c < K; ++c) unrolled around the statements that f makes for slot c
+    auto per_slot = [&](std::function<Stmts(const E&)> f) {
+      Name c = gen.fresh("c");
+      auto loop = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(
+          mk_for(c, iint(0), iint(K), 1, f(mk_var(c, ity)), LoopPar())));
+      loop->unroll = true;
+      return S(loop);
+    };
+    // the column of slot c of lane l; `inside`: the last vector of columns instead of one past it
+    auto column = [&](const E& c, const E& l, bool inside) {
+      E chunk = mk_binop(BinOp::FloorDiv, c, iint(V), ity), v = mk_binop(BinOp::Rem, c, iint(V), ity);
+      E base = chunks == 1 ? l : add(mk_binop(BinOp::Mul, chunk, iint(L), ity), l);
+      if (inside && L * chunks != slots) base = mk_binop(BinOp::Min, base, iint(slots - 1), ity);
+      return V == 1 ? base : add(mk_binop(BinOp::Mul, base, iint(V), ity), v);
+    };
+    const bool partial = L * K != r.cols;   // lanes or slots past the last column exist
+    // statements that add the elements first, first + stride, ... of the row to the lane's sums
+    auto walk = [&](Stmts& out, const E& lo, const E& hi, const E& first, int64_t stride, const E& l) {
+      out.push_back([&] {
+        auto d = std::make_shared<Stmt>();
+        d->k = Stmt::RegDecl;
+        d->id = reg;
+        d->ty = sty;
+        d->iv = K;
+        return S(d);
+      }());
+      out.push_back(per_slot([&](const E& c) { return Stmts{mk_assign(part(c), mk_float(0.0, sty.sz))}; }));
+      Name b = gen.fresh(r.loop->id.s + "_b"), at = gen.fresh(r.loop->id.s + "_at");
+      E bv = mk_var(b, ety), iv = mk_var(r.loop->id, ety), atv = mk_var(at, ety);
+      Stmts batch;
+      batch.push_back(mk_def(at, ety, mk_binop(BinOp::Min, iv, mk_binop(BinOp::Sub, hi, eint(1), ety), ety), r.loop->i));
+      std::map<Name, E> to_clamped{{r.loop->id, widen(atv)}};
+      // loaded values that select other elements get a name: an index is in bounds by contract, and a named one takes
+      // part in 32-bit address arithmetic
+      std::vector<std::pair<E, Name>> named;
+      auto bind = [&](const E& e0, Stmts& to) {
+        E e = subst_vars(e0, to_clamped);
+        std::function<E(const E&, bool)> go = [&](const E& x, bool inside) -> E {
+          if (!x) return x;
+          E y = map_children(x, [&](const E& ch) { return go(ch, inside || x->k == Expr::Index); });
+          if (!(inside && y->k == Expr::Index && is_int(y->ty.sz))) return y;
+          for (auto& nv : named) if (expr_eq(nv.first, y)) return mk_var(nv.second, y->ty);
+          Name nm = gen.fresh("sel");
+          named.push_back({y, nm});
+          to.push_back(mk_def(nm, y->ty, y, r.loop->i));
+          return mk_var(nm, y->ty);
+        };
+        return go(e, false);
+      };
+      auto summand = [&](const E& c) {
+        Stmts ss;
+        named.clear();
+        if (r.has_col) {
+          ss.push_back(mk_def(r.col, ity, fold_expr(column(c, l, true)), r.loop->i));
+        }
+        for (auto& d : r.defs) { E e = bind(d->expr, ss); ss.push_back(mk_def(d->id, d->ty, e, d->i)); }
+        Name tv = gen.fresh("term");
+        E te = bind(r.term, ss);
+        ss.push_back(mk_def(tv, sty, te, r.loop->i));
+        E masked = mk_ifexpr(mk_binop(BinOp::Lt, iv, hi, bty), mk_var(tv, sty), mk_float(0.0, sty.sz), sty);
+        ss.push_back(mk_assign(part(c), mk_binop(BinOp::Add, part(c), masked, sty), r.loop->i));
+        return ss;
+      };
+      batch.push_back(per_slot(summand));
+      auto inner = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(
+          mk_for(r.loop->id, bv, mk_binop(BinOp::Add, bv, eint(U * stride), ety), stride, batch, LoopPar(), r.loop->i)));
+      inner->unroll = true;
+      out.push_back(mk_for(b, mk_binop(BinOp::Add, lo, first, ety), hi, U * stride, {S(inner)}, LoopPar(), r.loop->i));
+    };
+    auto team_sum = [&](const std::string& fn) {
+      return per_slot([&](const E& c) {
+        auto call = std::make_shared<Expr>();
+        call->k = Expr::Call;
+        call->ty = sty;
+        call->sval = fn;
+        call->args = {part(c)};
+        return Stmts{mk_assign(part(c), call)};
+      });
+    };
+    // what is done with a finished sum
+    auto finish = [&](const E& sum) {
+      Stmts ss;
+      E whole = r.start->k == Expr::Float && r.start->fv == 0.0 ? sum : mk_binop(BinOp::Add, r.start, sum, sty);
+      if (r.acc->k == Expr::Index) ss.push_back(mk_assign(r.acc, whole, r.loop->i));
+      else ss.push_back(mk_def(r.acc->name, sty, whole, r.loop->i));
+      ss.insert(ss.end(), r.post.begin(), r.post.end());
+      return ss;
+    };
+    auto finish_slots = [&](const E& l) {
+      if (!r.has_col) return finish(part(iint(0)));
+      return Stmts{per_slot([&](const E& c) {
+        Stmts ss{mk_def(r.col, ity, fold_expr(column(c, l, false)), r.loop->i)};
+        Stmts f = finish(part(c));
+        if (partial) ss.push_back(mk_if(mk_binop(BinOp::Lt, mk_var(r.col, ity), iint(r.cols), bty), f, {}));
+        else ss.insert(ss.end(), f.begin(), f.end());
+        return ss;
+      })};
+    };
+    auto bounds = [&](Stmts& ss, E* lo, E* hi) {
+      for (auto& st : r.pre) ss.push_back(st);
+      Name ln = gen.fresh("first"), hn = gen.fresh("end");
+      ss.push_back(mk_def(ln, ety, narrow(r.loop->lo), r.loop->i));
+      ss.push_back(mk_def(hn, ety, narrow(r.loop->hi), r.loop->i));
+      *lo = mk_var(ln, ety);
+      *hi = mk_var(hn, ety);
+    };
+
+    Name queue = gen.fresh("long_rows"), count = gen.fresh("long_count");
+    Stmts top;
+    {
+      auto d = std::make_shared<Stmt>();
+      d->k = Stmt::LdsDecl;
+      d->id = queue;
+      d->ty = Type::scalar(ElemSize::I32);
+      d->iv = teams;
+      top.push_back(d);
+      auto e = std::make_shared<Stmt>(*d);
+      e->id = count;
+      e->iv = 1;
+      top.push_back(e);
+    }
+    top.push_back(mk_rawstmt("if (threadIdx.x == 0) " + count.str() + "[0] = 0;"));
+    top.push_back(mk_sync());
+
+    // every team its row
+    Name lane = gen.fresh(r.row.s + "_lane"), q = gen.fresh("g");
+    E lv = mk_var(lane, ity), qv = mk_var(q, ity);
+    {
+      Stmts body;
+      body.push_back(mk_def(r.row, ity, mk_binop(BinOp::FloorDiv, lv, iint(T), ity), r.loop->i));
+      body.push_back(mk_def(q, ity, mk_binop(BinOp::Rem, lv, iint(T), ity), r.loop->i));
+      E lo, hi;
+      bounds(body, &lo, &hi);
+      Stmts own;
+      E l = L == 1 ? iint(0) : mk_binop(BinOp::Rem, qv, iint(L), ity), sub = L == 1 ? qv : mk_binop(BinOp::FloorDiv, qv, iint(L), ity);
+      if (r.has_col && L > 1) {
+        Name ln = gen.fresh("l");
+        own.push_back(mk_def(ln, ity, l));
+        l = mk_var(ln, ity);
+      }
+      walk(own, lo, hi, narrow(sub), P, l);
+      if (P > 1) own.push_back(team_sum(L == 1 && P == 8 ? "parpy_sum8" : "parpy_team_sum<" + std::to_string(L) + ", " + std::to_string(T) + ">"));
+      Stmts f = finish_slots(l);
+      if (P > 1) own.push_back(mk_if(mk_binop(BinOp::Lt, qv, iint(L), bty), f, {}));
+      else own.insert(own.end(), f.begin(), f.end());
+      Stmts defer{mk_if(mk_binop(BinOp::Eq, qv, iint(0), bty),
+                        {mk_rawstmt(queue.str() + "[atomicAdd(&" + count.str() + "[0], 1)] = (int)" + r.row.str() + ";")}, {})};
+      body.push_back(mk_if(mk_binop(BinOp::Leq, mk_binop(BinOp::Sub, hi, lo, ety), eint(longest), bty), own, defer));
+      auto nr = clone(k.body[0]);
+      nr->id = lane;
+      nr->hi = iint(r.n * T);
+      nr->body = body;
+      nr->els.clear();
+      nr->map = GpuMap();
+      nr->map.k = GpuMap::ThreadBlock;
+      nr->map.tpb = tpb;
+      nr->map.n = (r.n * T + WAVE_SIZE - 1) / WAVE_SIZE * WAVE_SIZE;
+      top.push_back(nr);
+    }
+    top.push_back(mk_sync());
+
+    // long rows, one after the other, by all threads of the workgroup
+    {
+      Name h = gen.fresh("h"), tid = gen.fresh("tid");
+      E tv = mk_var(tid, ity);
+      auto tx = std::make_shared<Expr>();
+      tx->k = Expr::ThreadIdx;
+      tx->ty = ity;
+      tx->iv = 0;
+      Stmts body;
+      body.push_back(mk_def(r.row, ity, mk_raw("((int64_t)" + queue.str() + "[" + h.str() + "])", ity), r.loop->i));
+      body.push_back(mk_def(tid, ity, tx));
+      E lo, hi;
+      bounds(body, &lo, &hi);
+      E l = L == 1 ? iint(0) : mk_binop(BinOp::Rem, tv, iint(L), ity), sub = L == 1 ? tv : mk_binop(BinOp::FloorDiv, tv, iint(L), ity);
+      walk(body, lo, hi, narrow(sub), tpb / L, l);
+      if (!r.has_col) {
+        Name w = gen.fresh("whole");
+        body.push_back(mk_def(w, sty, part(iint(0))));
+        auto red = std::make_shared<Stmt>();
+        red->k = Stmt::WaveReduce;
+        red->id = w;
+        red->ty = sty;
+        red->bop = BinOp::Add;
+        red->iv = tpb;
+        red->unroll = true;   // the slots are used again for the next row
+        body.push_back(red);
+        body.push_back(mk_if(mk_binop(BinOp::Eq, tv, iint(0), bty), finish(mk_var(w, sty)), {}));
+      } else {
+        if (L < WAVE_SIZE) body.push_back(team_sum("parpy_team_sum<" + std::to_string(L) + ", " + std::to_string(WAVE_SIZE) + ">"));
+        Name shared = gen.fresh("long_sums");
+        auto d = std::make_shared<Stmt>();
+        d->k = Stmt::LdsDecl;
+        d->id = shared;
+        d->ty = sty;
+        d->iv = waves * L * K;
+        top.push_back(d);
+        E base = mk_var(shared, Type::pointer(sty.sz, Mem::LDS));
+        E wave = mk_binop(BinOp::FloorDiv, tv, iint(WAVE_SIZE), ity);
+        Stmts put{per_slot([&](const E& c) {
+          E at = add(mk_binop(BinOp::Mul, wave, iint(L * K), ity), column(c, l, false));
+          return Stmts{mk_assign(mk_index(base, fold_expr(at), sty), part(c))};
+        })};
+        body.push_back(mk_if(mk_binop(BinOp::Lt, mk_binop(BinOp::Rem, tv, iint(WAVE_SIZE), ity), iint(L), bty), put, {}));
+        body.push_back(mk_sync());
+        Name s = gen.fresh("whole"), w = gen.fresh("w");
+        Stmts sum{mk_def(r.col, ity, tv), mk_def(s, sty, mk_float(0.0, sty.sz))};
+        auto over = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(mk_for(
+            w, iint(0), iint(waves), 1,
+            {mk_assign(mk_var(s, sty), mk_binop(BinOp::Add, mk_var(s, sty),
+                                                mk_index(base, add(mk_binop(BinOp::Mul, mk_var(w, ity), iint(L * K), ity), tv), sty), sty))},
+            LoopPar())));
+        over->unroll = true;
+        sum.push_back(over);
+        Stmts f = finish(mk_var(s, sty));
+        sum.insert(sum.end(), f.begin(), f.end());
+        body.push_back(mk_if(mk_binop(BinOp::Lt, tv, iint(r.cols), bty), sum, {}));
+        body.push_back(mk_sync());
+        k.lds_bytes += waves * L * K * elem_bytes(sty.sz);
+      }
+      top.push_back(mk_for(h, iint(0), mk_raw("((int64_t)" + count.str() + "[0])", ity), 1, body, LoopPar()));
+    }
+    k.lds_bytes += (teams + 1) * 4;
+    k.body = top;
+    k.block = Dim3{tpb, 1, 1};
+    k.grid = Dim3{(r.n + teams - 1) / teams, 1, 1};
+    launch->grid = k.grid;
+    launch->block = k.block;
+    return true;
+  }
+
+  void run() {
+    Stmts host;
+    for (auto& s : p.host) {
+      if (s->k != Stmt::Launch) { host.push_back(s); continue; }
+      Kernel* k = nullptr;
+      for (auto& kk : p.kernels)
+        if (kk.name == s->fname) k = &kk;
+      auto ns = std::make_shared<Stmt>(*s);
+      if (k && !k->opaque_body) apply(*k, ns);
+      host.push_back(ns);
+    }
+    p.host = host;
+  }
+};
+
+}  // namespace
+
+void ragged_sum(Program& p, const Options& opts, NameGen& gen) { RaggedSum(p, opts, gen).run(); }
+
+}  // namespace hipopt
+}  // namespace parpy

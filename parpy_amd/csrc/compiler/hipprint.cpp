@@ -175,6 +175,30 @@ template <class T> __device__ __forceinline__ T parpy_sum8(T v) {
   v = v + parpy_dpp<0x141>(v);  // the other quad of the 8-lane half row
   return v;
 }
+// the value of lane ^ S, S a power of two
+template <int S, class T> __device__ __forceinline__ T parpy_xor_lane(T v) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "");
+  if constexpr (S == 1) return parpy_dpp<0xB1>(v);
+  else if constexpr (S == 2) return parpy_dpp<0x4E>(v);
+  else {
+    auto move = [](int x) {
+      if constexpr (S < 32) return __builtin_amdgcn_ds_swizzle(x, (S << 10) | 0x1F);
+      else return __builtin_amdgcn_ds_bpermute((((int)threadIdx.x & 63) ^ 32) << 2, x);
+    };
+    if constexpr (sizeof(T) == 8) {
+      const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+      const unsigned lo = (unsigned)move((int)(unsigned)x), hi = (unsigned)move((int)(unsigned)(x >> 32));
+      return __builtin_bit_cast(T, ((unsigned long long)hi << 32) | lo);
+    } else {
+      return __builtin_bit_cast(T, move(__builtin_bit_cast(int, v)));
+    }
+  }
+}
+// sum over the lanes of an aligned team of TEAM lanes that agree modulo L; every one of them receives it
+template <int L, int TEAM, class T> __device__ __forceinline__ T parpy_team_sum(T v) {
+  if constexpr (L < TEAM) return parpy_team_sum<2 * L, TEAM>(v + parpy_xor_lane<L>(v));
+  else return v;
+}
 // Barrier over all workgroups of a launch whose whole grid is resident on the device.  The kernels that use it
 // load and store what they exchange at device scope, so no cache has to be written back or emptied here: every
 // wave waits until its own memory operations have completed, the workgroup's first thread counts the workgroup in
@@ -1155,6 +1179,13 @@ struct DevicePrinter {
     packs.clear();
     os.str("");
     find_reassigned(k.body, reassigned);
+    {
+      Interval r;
+      r.known = true;
+      r.lo = 0;
+      r.hi = k.block.x - 1;
+      ranges[Name{"threadIdx.x", -1}] = r;
+    }
     stream_out.clear();
     if (opts.opt_nontemporal && !k.cached_stores) {
       // parameters that are stored to (directly, never through an alias) and never read in this kernel

@@ -1,0 +1,110 @@
+"""Sums over rows of uneven length (bounds that are data): teams of lanes per row, very long rows shared by a workgroup,
+with and without columns; row counts, row lengths and column counts at the edges of what a team, a batch, a wavefront
+and the queue of long rows hold.  The expectation is NumPy in float64."""
+import numpy as np
+import pytest
+
+import parpy_amd as parpy
+from parpy_amd.compile import hiprtc_compile
+from parpy_amd.operators import float32
+
+HIP = parpy.CompileBackend.Hip
+
+
+def weighted(A, x, y, z):
+    parpy.label('row')
+    for row in range(A["nrows"]):
+        y[row] = z[row]
+        parpy.label('i')
+        for i in range(A["rows"][row], A["rows"][row + 1]):
+            col = A["cols"][i]
+            y[row] += A["values"][i] * x[col]
+
+
+def columns(A, B, C, z):
+    parpy.label('i')
+    for i in range(A["nrows"]):
+        parpy.label('j')
+        for j in range(B["ncols"]):
+            t = z[i] * 0.5
+            parpy.label('k')
+            for k in range(A["rows"][i], A["rows"][i + 1]):
+                t = t + A["values"][k] * B["values"][A["cols"][k], j]
+            C[i, j] = t * z[i] + 1.0
+
+
+def fixed_length(x, out, N, M):
+    parpy.label('i')
+    for i in range(N):
+        t = float32(3.0)
+        for d in range(M):
+            t = t + x[i, d]
+        out[i] = t
+
+
+def matrix(n, m, dtype, seed):
+    """Row lengths: empty, one, around a team, around the longest row a team keeps, and one that dwarfs the rest."""
+    rng = np.random.default_rng(seed)
+    lens = rng.choice([0, 1, 2, 7, 8, 9, 31, 32, 33], size=n)
+    edge = [63, 64, 65, 127, 128, 129, 255, 256, 257, 1023, 1025, 5000]
+    lens[rng.choice(n, size=len(edge), replace=False)] = edge
+    rows = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    cols = rng.integers(0, m, rows[-1]).astype(np.int64)
+    values = rng.standard_normal(rows[-1]).astype(dtype)
+    return {"values": values, "rows": rows, "cols": cols, "nrows": n}
+
+
+def row_sums(A, terms):
+    """float64 sums of `terms` (one row of columns per non-zero) over the rows of A."""
+    total = np.concatenate([np.zeros((1,) + terms.shape[1:]), np.cumsum(terms.astype(np.float64), axis=0)])
+    return total[A["rows"][1:]] - total[A["rows"][:-1]]
+
+
+def opts_for(p):
+    o = parpy.par(p)
+    o.backend = HIP
+    return o
+
+
+def test_long_rows_are_queued_for_the_workgroup():
+    A = matrix(5000, 300, np.float32, 1)
+    v = np.zeros(5000, dtype=np.float32)
+    s = parpy.print_compiled(weighted, [A, np.zeros(300, dtype=np.float32), v, v.copy()], opts_for({"row": parpy.threads(5000)}))
+    hiprtc_compile(s[:s.index("// host side")], opts_for({}))
+    assert "atomicAdd(&long_count" in s and "parpy_block_reduce<parpy_op_add, 16>" in s
+    B = {"values": np.zeros((300, 64), dtype=np.float32), "ncols": 64}
+    s = parpy.print_compiled(columns, [A, B, np.zeros((5000, 64), dtype=np.float32), v], opts_for({"i": parpy.threads(5000), "j": parpy.threads(64)}))
+    hiprtc_compile(s[:s.index("// host side")], opts_for({}))
+    assert "parpy_team_sum<16, 64>" in s and "long_sums" in s
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=lambda d: np.dtype(d).name)
+@pytest.mark.parametrize("n", [64, 65, 1000, 1025, 20001])
+def test_sums_of_uneven_rows(n, dtype):
+    A = matrix(n, 300, dtype, n)
+    rng = np.random.default_rng(n + 1)
+    x, z, y = rng.standard_normal(300).astype(dtype), rng.standard_normal(n).astype(dtype), np.full(n, np.nan, dtype=dtype)
+    parpy.jit(weighted)(A, x, y, z, opts=opts_for({"row": parpy.threads(n)}))
+    want = z + row_sums(A, A["values"].astype(np.float64) * x[A["cols"]])
+    assert np.allclose(y, want, atol=1e-3 if dtype == np.float32 else 1e-9)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=lambda d: np.dtype(d).name)
+@pytest.mark.parametrize("n,cols", [(64, 1), (65, 3), (100, 32), (1000, 100), (300, 101), (129, 256), (200, 258), (70, 513), (64, 1024)])
+def test_sums_of_uneven_rows_with_columns(n, cols, dtype):
+    A = matrix(n, 50, dtype, n)
+    rng = np.random.default_rng(cols)
+    B, z, C = rng.standard_normal((50, cols)).astype(dtype), rng.standard_normal(n).astype(dtype), np.full((n, cols), np.nan, dtype=dtype)
+    parpy.jit(columns)(A, {"values": B, "ncols": cols}, C, z, opts=opts_for({"i": parpy.threads(n), "j": parpy.threads(cols)}))
+    want = (0.5 * z[:, None] + row_sums(A, A["values"].astype(np.float64)[:, None] * B[A["cols"]])) * z[:, None] + 1.0
+    assert np.allclose(C, want, atol=2e-3 if dtype == np.float32 else 1e-9)
+
+
+@pytest.mark.gpu
+def test_start_value_of_a_shared_sum_counts_once():
+    x = np.random.default_rng(3).standard_normal((300, 132)).astype(np.float32)
+    out = np.zeros(300, dtype=np.float32)
+    parpy.jit(fixed_length)(x, out, 300, 132, opts=opts_for({'i': parpy.threads(300)}))
+    assert np.allclose(out, 3.0 + x.astype(np.float64).sum(1), atol=1e-4)
