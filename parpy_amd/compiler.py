@@ -23,7 +23,7 @@ LIB_PATH = pathlib.Path(__file__).parent / "libparpy_hipc.so"
 SOURCES = ["ast.cpp", "front.cpp", "constfold.cpp", "specialize.cpp", "lower.cpp",
            "gpu.cpp", "hipopt.cpp", "hipopt_util.cpp", "hipopt_control.cpp", "hipopt_prefetch.cpp", "hipopt_lds.cpp",
            "hipopt_vector.cpp", "hipopt_regs.cpp", "hipopt_keep.cpp", "hipopt_alias.cpp", "hipopt_launch.cpp",
-           "hipopt_ragged.cpp", "hipopt_persist.cpp", "hipprint.cpp", "capi.cpp"]
+           "hipopt_ragged.cpp", "hipopt_timetile.cpp", "hipopt_persist.cpp", "hipprint.cpp", "capi.cpp"]
 
 _lib = None
 
@@ -222,7 +222,7 @@ def describe_opts(opts):
     if opts.force_float_size is not None:
         parts.append(f"(force_float_size {opts.force_float_size.value})")
     for name in ("opt_vectorize", "opt_lds_rows", "opt_reg_cache", "opt_hoist_invariant",
-                 "opt_narrow_index", "opt_mfma_sddmm", "opt_unswitch", "opt_gather_transpose", "opt_nontemporal", "opt_lane_split", "opt_drop_barriers", "opt_unswitch_uniform", "opt_offset32", "opt_if_convert", "opt_noalias_scopes", "opt_expand_short_loops", "opt_guard_bounds", "opt_prefetch_steps", "opt_pack_accesses", "opt_share_iterations", "opt_fence_iterations", "opt_keep_stored", "opt_keep_own", "assume_aligned"):
+                 "opt_narrow_index", "opt_mfma_sddmm", "opt_unswitch", "opt_gather_transpose", "opt_nontemporal", "opt_lane_split", "opt_drop_barriers", "opt_unswitch_uniform", "opt_offset32", "opt_if_convert", "opt_noalias_scopes", "opt_expand_short_loops", "opt_guard_bounds", "opt_prefetch_steps", "opt_pack_accesses", "opt_share_iterations", "opt_fence_iterations", "opt_keep_stored", "opt_keep_own", "opt_tile_steps", "assume_aligned"):
         v = getattr(opts, name, None)
         if v is not None:
             parts.append(f"({name} {1 if v else 0})")

@@ -406,6 +406,7 @@ struct Options {  // src/option.rs:14-108
   bool opt_keep_own = false;     // ... and across steps when source and destination swap every step (own elements never re-read from LDS)
   bool opt_keep_stored = true;   // values a thread stores and reads back itself later in the same step stay in registers
   bool opt_fence_iterations = true;   // the unrolled iterations of a thread that read and write LDS are scheduled one after the other
+  bool opt_tile_steps = true;         // several steps of a host loop of element-wise launches run in one launch
   bool opt_expand_short_loops = true; // counted loops of <= 8 iterations inside a parallel iteration are expanded in place
   int64_t reg_budget = 0;     // 32-bit registers per thread the caching passes may claim (0 = by block size)
   int64_t reg_budget_scale = 100;   // percent of the by-block-size budget (the driver lowers it when a code object spills)

@@ -21,7 +21,9 @@
 //                   `if (c) for x: A else for x: B`;
 //   drop_barriers   barriers between regions that share no written array go.
 //
-// Four rewrites work on the whole program because they change a launch:
+// Five rewrites work on the whole program because they change a launch:
+//   TimeTile        several steps of a host loop of element-wise launches over
+//                   shifted elements run in one launch;
 //   GatherTranspose column gathers X[d, c] over an innermost sequential d read a
 //                   transposed copy made by a tiled kernel in front of the launch;
 //   RaggedSum       sums whose bounds are data (a CSR row): teams of lanes take
@@ -38,13 +40,14 @@
 // branches, aliases), hipopt_prefetch.cpp, hipopt_lds.cpp, hipopt_vector.cpp,
 // hipopt_regs.cpp (budget, hoisting, register caching), hipopt_keep.cpp and
 // hipopt_alias.cpp; the whole-program rewrites are in hipopt_launch.cpp,
-// hipopt_ragged.cpp and hipopt_persist.cpp.
+// hipopt_ragged.cpp, hipopt_timetile.cpp and hipopt_persist.cpp.
 #include "hipopt_pass.hpp"
 
 namespace parpy {
 
 void hip_optimize(Program& p, const Options& opts, NameGen& gen) {
   if (opts.opt_gather_transpose) hipopt::gather_transpose(p, opts, gen);
+  if (opts.opt_tile_steps && !opts.persistent_loops) hipopt::time_tile(p, opts, gen);
   if (opts.opt_lane_split) hipopt::ragged_sum(p, opts, gen);
   if (opts.opt_lane_split && !opts.opt_mfma_sddmm) hipopt::lane_split(p, opts, gen);
   if (opts.opt_vectorize) hipopt::coarsen(p, opts, gen);

@@ -1,0 +1,401 @@
+// gfx950 memory passes, rewrites that change a launch: several steps of a host-side time loop in one pass over memory.
+#include <algorithm>
+#include <functional>
+
+#include "hipopt_pass.hpp"
+
+namespace parpy {
+namespace hipopt {
+
+namespace {
+
+// ================================================================ time loops over stencils, several steps per launch
+// `for t: B[1:-1] = f(A[:-2], A[1:-1], A[2:]); A[1:-1] = f(B[:-2], ...)` runs as one launch per statement and step:
+// each launch reads and writes whole arrays and waits for the one before it, a few microseconds for some tens of
+// nanoseconds of work per compute unit.  When every launch of the loop updates arrays element by element from
+// elements a fixed distance away, a stretch of the arrays can be carried through several steps on its own, provided it
+// starts with a margin of (steps x distance) elements on either side that is computed along and thrown away.
+//
+//   * A wavefront owns a stretch of 64 * E elements, E neighbouring ones per lane, in registers: own elements and
+//     those of the neighbouring lanes (DPP wave shifts by one lane) are all a step needs, so the steps take neither
+//     LDS nor barriers.
+//   * Stretches overlap, so a launch must not overwrite what its neighbours still read: it writes to a second set of
+//     arrays, and the next launch brings the values back.  The number of launches is even; their steps differ by at
+//     most one.
+//   * The arithmetic of an element is that of the statement as written: same operations, same order.
+//
+// A three-point average back and forth over 10^6 float64 elements, 98 updates: 447 us as launches of 4.5 us each, 51 us
+// in two launches of 25 steps; the vector ALU is then what bounds it (two additions and a division in four
+// instructions per element and update, a quarter of them in the margins).
+struct TimeTile {
+  Program& p;
+  const Options& opts;
+  NameGen& gen;
+  ElemSize isz;
+  Type ity;
+  Type bty = Type::scalar(ElemSize::Bool);
+
+  TimeTile(Program& prog, const Options& o, NameGen& g) : p(prog), opts(o), gen(g), isz(o.int_size()), ity(Type::scalar(o.int_size())) {}
+
+  struct Arr { Name host; ElemSize sz = ElemSize::F32; int64_t n = 0; bool written = false; int64_t left = 0, right = 0; };
+  struct Update {                 // one launch of the loop
+    int64_t lo = 0, hi = 0;       // elements it writes, in array coordinates
+    int64_t c = 0;                // array coordinate = iteration + c
+    Name id;
+    Stmts body;
+    std::map<Name, Name> host;    // parameter -> host variable
+    int64_t radius = 0;
+  };
+
+  static constexpr int64_t SCRATCH_BYTES = int64_t(16) << 20;   // PARPY_HIP_SCRATCH_BYTES of the runtime
+
+  E iint(int64_t v) { return mk_int(v, isz); }
+  E add(E a, E b) { return mk_binop(BinOp::Add, a, b, ity); }
+  static int64_t pow2_at_least(int64_t n) { int64_t q = 1; while (q < n) q *= 2; return q; }
+
+  bool update_of(const Kernel& k, const S& launch, Update& u, std::vector<Arr>& arrays) {
+    if (k.opaque_body || k.body.size() != 1 || k.grid.y != 1 || k.grid.z != 1 || k.block.y != 1 || k.block.z != 1) return false;
+    const S& root = k.body[0];
+    if (!(root->k == Stmt::For && root->step == 1 && root->lo->k == Expr::Int && root->hi->k == Expr::Int && root->hi->iv > root->lo->iv && root->els.empty()))
+      return false;
+    if (!(root->map.dim == 0 && (root->map.k == GpuMap::ThreadBlock || (root->map.k == GpuMap::Thread && k.grid.x == 1)))) return false;
+    for (size_t q = 0; q < k.params.size(); ++q) {
+      if (!k.params[q].ty.is_pointer() && !k.params[q].ty.is_array()) return false;
+      const E& a = launch->args[q];
+      if (a->k != Expr::Var) return false;
+      for (auto& kv : u.host) if (kv.second == a->name) return false;
+      u.host[k.params[q].id] = a->name;
+    }
+    auto arr = [&](const Name& host) -> Arr& {
+      for (auto& a : arrays) if (a.host == host) return a;
+      arrays.push_back(Arr());
+      arrays.back().host = host;
+      return arrays.back();
+    };
+    u.id = root->id;
+    u.body = root->body;
+    bool first = true;
+    std::set<Name> written;
+    for (auto& st : root->body) {
+      if (st->k == Stmt::Def && st->ty.is_scalar()) continue;
+      if (st->k != Stmt::Assign || st->dst->k != Expr::Index || st->dst->args[0]->k != Expr::Var || !u.host.count(st->dst->args[0]->name)) return false;
+      E rest;
+      if (st->dst->dim_shape.size() != 1 || !affine_unit(st->dst->args[1], root->id, &rest) || rest->k != Expr::Int) return false;
+      if (!first && rest->iv != u.c) return false;
+      u.c = rest->iv;
+      first = false;
+      written.insert(u.host[st->dst->args[0]->name]);
+    }
+    if (first) return false;
+    u.lo = root->lo->iv + u.c;
+    u.hi = root->hi->iv + u.c;
+    bool ok = true;
+    auto access = [&](const E& x, bool store) {
+      if (x->k == Expr::Call || x->k == Expr::Raw || x->k == Expr::AddrOf || x->k == Expr::RegElem) { ok = false; return; }
+      if (x->k != Expr::Index) return;
+      if (x->args[0]->k != Expr::Var || !u.host.count(x->args[0]->name) || x->dim_shape.size() != 1) { ok = false; return; }
+      Arr& a = arr(u.host[x->args[0]->name]);
+      const int bytes = elem_bytes(x->ty.sz);
+      if ((a.n != 0 && (a.n != x->dim_shape[0] || a.sz != x->ty.sz)) || (bytes != 4 && bytes != 8)) { ok = false; return; }
+      a.n = x->dim_shape[0];
+      a.sz = x->ty.sz;
+      E rest;
+      if (!affine_unit(x->args[1], root->id, &rest) || rest->k != Expr::Int) { ok = false; return; }
+      const int64_t d = rest->iv - u.c;
+      if (d != 0 && written.count(a.host)) ok = false;   // reads what other iterations of the same launch write
+      if (store) a.written = true;
+      a.left = std::max(a.left, -d);
+      a.right = std::max(a.right, d);
+      u.radius = std::max(u.radius, std::abs(d));
+    };
+    for (auto& st : root->body) {
+      visit_exprs(st->expr, [&](const E& x) { access(x, false); });
+      if (st->dst) access(st->dst, true);
+    }
+    return ok;
+  }
+
+  S tile(const S& loop) {
+    if (!(loop->k == Stmt::For && loop->map.k == GpuMap::None && loop->step == 1 && loop->lo->k == Expr::Int && loop->hi->k == Expr::Int && !loop->body.empty()))
+      return S();
+    const int64_t steps = loop->hi->iv - loop->lo->iv;
+    std::vector<Arr> arrays;
+    std::vector<Update> ups;
+    for (auto& l : loop->body) {
+      if (l->k != Stmt::Launch) return S();
+      const Kernel* k = nullptr;
+      for (auto& kk : p.kernels) if (kk.name == l->fname) k = &kk;
+      for (auto& a : l->args) if (mentions(a, loop->id)) return S();
+      Update u;
+      if (!k || !update_of(*k, l, u, arrays)) return S();
+      ups.push_back(u);
+    }
+    int64_t per_step = 0, reach = 0, n = 0, words = 0, second_set = 0, lo = 0, hi = INT64_MAX;
+    for (auto& u : ups) {
+      per_step += u.radius;
+      lo = std::max(lo, u.lo);
+      hi = std::min(hi, u.hi);
+      if (u.lo < 0) return S();
+    }
+    for (auto& a : arrays) {
+      reach = std::max(reach, std::max(a.left, a.right));
+      n = std::max(n, a.n);
+      hi = std::min(hi, a.n);
+      words += elem_bytes(a.sz) / 4;
+      if (a.written) second_set += (a.n * elem_bytes(a.sz) + 255) / 256 * 256;
+      for (auto& u : ups) if (u.hi > a.n) { bool w = false; for (auto& st : u.body) if (st->dst && st->dst->k == Expr::Index && u.host[st->dst->args[0]->name] == a.host) w = true; if (w) return S(); }
+    }
+    if (n < 512 || n > (int64_t(1) << 30) || steps * (int64_t)ups.size() < 4 || steps < 2) return S();
+    // Elements per lane: eight where that leaves every SIMD a wavefront or two, four for smaller arrays, where the
+    // latency of a step is what counts (98 updates of a three-point average, float64: 10^6 elements 153 / 73 / 56 / 51 /
+    // 68 us for 1 / 2 / 4 / 8 / 16 elements per lane, 6 * 10^5: 35 on four, 38 on eight, 10^5: 15 and 24).
+    int64_t Es = n >= 800000 ? 8 : 4;
+    while (Es * words > 64 && Es > 1) Es /= 2;
+    Es = std::max(Es, pow2_at_least(std::max<int64_t>(1, reach)));
+    if (Es * words > 64 || per_step > 8 * Es) return S();
+    // Steps per launch: a margin of up to a quarter of the stretch on either side.  Launches cost more than the margins
+    // (10^5 elements: margins of 1/16, 1/8 and 1/4 of the stretch 32, 22 and 15 us; 10^6 elements: 60, 52, 51).
+    const int64_t most = per_step > 0 ? 16 * Es / per_step : steps;
+    const int64_t pairs = (steps + 2 * most - 1) / (2 * most), launches = 2 * pairs;
+    const int64_t base_steps = steps / launches, extra = steps % launches;
+    const int64_t margin = ((base_steps + (extra > 0)) * per_step + Es - 1) / Es * Es;
+    const int64_t width = WAVE_SIZE * Es, useful = width - 2 * margin;
+    if (useful < width / 4) return S();
+    const int64_t tpb = 256;
+
+    // ---- the kernel
+    Kernel f;
+    f.name = p.name + "_steps_" + std::to_string(gen.next++);
+    f.block.x = tpb;
+    f.grid.x = ((n + useful - 1) / useful + tpb / WAVE_SIZE - 1) / (tpb / WAVE_SIZE);
+    f.cached_stores = true;
+    f.aligned_params = opts.assume_aligned;
+    std::map<Name, Name> reg, dst;
+    for (auto& a : arrays) {
+      KernelParam q;
+      q.id = a.host;
+      q.ty = Type::pointer(a.sz);
+      f.params.push_back(q);
+      reg[a.host] = gen.fresh(a.host.s + "_r");
+    }
+    for (auto& a : arrays)
+      if (a.written) {
+        KernelParam q;
+        q.id = dst[a.host] = gen.fresh(a.host.s + "_to");
+        q.ty = Type::pointer(a.sz);
+        f.params.push_back(q);
+      }
+    KernelParam count;
+    count.id = gen.fresh("steps");
+    count.ty = Type::scalar(ElemSize::I32);
+    f.params.push_back(count);
+    auto slot = [&](const Arr& a, int64_t e) {
+      auto x = std::make_shared<Expr>();
+      x->k = Expr::RegElem;
+      x->ty = Type::scalar(a.sz);
+      x->name = reg[a.host];
+      x->args = {iint(e)};
+      return E(x);
+    };
+    auto arr_of = [&](const Name& host) -> const Arr& {
+      for (auto& a : arrays) if (a.host == host) return a;
+      return arrays[0];
+    };
+    Name lane = gen.fresh("lane"), wave = gen.fresh("wave"), at = gen.fresh("at");
+    E lv = mk_var(lane, ity), wv = mk_var(wave, ity), av = mk_var(at, ity);
+    auto index_reg = [&](Expr::Kind kk) {
+      auto x = std::make_shared<Expr>();
+      x->k = kk;
+      x->ty = ity;
+      x->iv = 0;
+      return E(x);
+    };
+    Stmts top;
+    top.push_back(mk_def(lane, ity, mk_binop(BinOp::Rem, index_reg(Expr::ThreadIdx), iint(WAVE_SIZE), ity)));
+    top.push_back(mk_def(wave, ity, add(mk_binop(BinOp::Mul, index_reg(Expr::BlockIdx), iint(tpb / WAVE_SIZE), ity),
+                                        mk_binop(BinOp::FloorDiv, index_reg(Expr::ThreadIdx), iint(WAVE_SIZE), ity))));
+    E start = mk_binop(BinOp::Sub, mk_binop(BinOp::Mul, wv, iint(useful), ity), iint(margin), ity);
+    top.push_back(mk_def(at, ity, add(start, mk_binop(BinOp::Mul, lv, iint(Es), ity))));
+    for (auto& a : arrays) {
+      auto d = std::make_shared<Stmt>();
+      d->k = Stmt::RegDecl;
+      d->id = reg[a.host];
+      d->ty = Type::scalar(a.sz);
+      d->iv = Es;
+      top.push_back(d);
+    }
+    auto elem = [&](const Name& array, const Arr& a, int64_t e) {
+      auto x = std::make_shared<Expr>(*mk_index(mk_var(array, Type::pointer(a.sz)), fold_expr(add(av, iint(e))), Type::scalar(a.sz)));
+      return E(x);
+    };
+    auto lt = [&](E a, E b) { return mk_binop(BinOp::Lt, a, b, bty); };
+    auto le = [&](E a, E b) { return mk_binop(BinOp::Leq, a, b, bty); };
+    auto both = [&](E a, E b) { return mk_binop(BinOp::And, a, b, bty); };
+    auto within = [&](int64_t e, int64_t from, int64_t to) {   // from <= at + e < to
+      E g = fold_expr(add(av, iint(e)));
+      return both(le(iint(from), g), lt(g, iint(to)));
+    };
+
+    // the path of a stretch: `edge` tests every element against the bounds of the arrays and of the updates
+    auto path = [&](bool edge) {
+      Stmts ss;
+      for (auto& a : arrays)
+        for (int64_t e = 0; e < Es; ++e) {
+          S ld = mk_assign(slot(a, e), elem(a.host, a, e));
+          ss.push_back(edge ? mk_if(within(e, 0, a.n), {ld}, {mk_assign(slot(a, e), is_float(a.sz) ? mk_float(0.0, a.sz) : mk_int(0, a.sz))}) : ld);
+        }
+      Stmts step;
+      for (auto& u : ups) {
+        // what the neighbouring lanes hold
+        std::map<std::pair<Name, int64_t>, E> from;
+        std::map<Name, std::pair<int64_t, int64_t>> need;
+        for (auto& st : u.body)
+          visit_exprs(st->expr, [&](const E& x) {
+            if (x->k != Expr::Index) return;
+            E rest;
+            affine_unit(x->args[1], u.id, &rest);
+            int64_t d = rest->iv - u.c;
+            auto& nd = need[u.host[x->args[0]->name]];
+            nd.first = std::max(nd.first, -d);
+            nd.second = std::max(nd.second, d);
+          });
+        for (auto& kv : need) {
+          const Arr& a = arr_of(kv.first);
+          auto fetch = [&](int64_t pos, int64_t own, const char* fn) {
+            Name nm = gen.fresh(a.host.s + (pos < 0 ? "_left" : "_right"));
+            auto call = std::make_shared<Expr>();
+            call->k = Expr::Call;
+            call->ty = Type::scalar(a.sz);
+            call->sval = fn;
+            call->args = {slot(a, own)};
+            step.push_back(mk_def(nm, Type::scalar(a.sz), call));
+            from[{a.host, pos}] = mk_var(nm, Type::scalar(a.sz));
+          };
+          for (int64_t q = 1; q <= kv.second.first; ++q) fetch(-q, Es - q, "parpy_lane_before");
+          for (int64_t q = 0; q < kv.second.second; ++q) fetch(Es + q, q, "parpy_lane_after");
+        }
+        for (int64_t e = 0; e < Es; ++e) {
+          std::map<Name, E> names{{u.id, fold_expr(add(av, iint(e - u.c)))}};
+          auto value = [&](const E& x0) {
+            E x1 = rewrite_expr(x0, [&](const E& x) -> E {
+              if (x->k != Expr::Index) return x;
+              E rest;
+              affine_unit(x->args[1], u.id, &rest);
+              const int64_t pos = e + rest->iv - u.c;
+              const Arr& a = arr_of(u.host[x->args[0]->name]);
+              return pos >= 0 && pos < Es ? slot(a, pos) : from.at({a.host, pos});
+            });
+            return subst_vars(x1, names);
+          };
+          Stmts one;
+          for (auto& st : u.body) {
+            E v = value(st->expr);
+            if (st->k == Stmt::Def) {
+              Name nm = gen.fresh(st->id.s);
+              one.push_back(mk_def(nm, st->ty, v, st->i));
+              names[st->id] = mk_var(nm, st->ty);
+            } else {
+              E to = slot(arr_of(u.host[st->dst->args[0]->name]), e);
+              // (computed for every element and kept where the update covers it: no branches between the elements)
+              one.push_back(mk_assign(to, edge ? mk_ifexpr(within(e, u.lo, u.hi), v, to, to->ty) : v, st->i));
+            }
+          }
+          step.insert(step.end(), one.begin(), one.end());
+        }
+      }
+      Name s = gen.fresh("s");
+      ss.push_back(mk_for(s, mk_int(0, ElemSize::I32), mk_var(count.id, Type::scalar(ElemSize::I32)), 1, step, LoopPar()));
+      Stmts put;
+      for (auto& a : arrays)
+        if (a.written)
+          for (int64_t e = 0; e < Es; ++e) {
+            S stt = mk_assign(elem(dst[a.host], a, e), slot(a, e));
+            put.push_back(edge ? mk_if(within(e, 0, a.n), {stt}, {}) : stt);
+          }
+      const int64_t outer = margin / Es;
+      ss.push_back(mk_if(both(le(iint(outer), lv), lt(lv, iint(WAVE_SIZE - outer))), put, {}));
+      return ss;
+    };
+    // A stretch that lies inside all bounds takes the plain path.  Values next to the bounds of a stretch are wrong (its
+    // outermost lanes have no neighbour) and stay within the margin.
+    E inside = both(le(iint(lo), start), le(add(start, iint(width)), iint(hi)));
+    top.push_back(mk_if(inside, path(false), path(true)));
+    f.body = top;
+    p.kernels.push_back(f);
+
+    // ---- the host side
+    Stmts tiled;
+    std::map<Name, Name> tmp;
+    for (auto& a : arrays)
+      if (a.written) {
+        auto al = std::make_shared<Stmt>();
+        al->k = Stmt::Alloc;
+        al->id = tmp[a.host] = gen.fresh(a.host.s + "_next");
+        al->ty = Type::scalar(a.sz);
+        al->iv = a.n;
+        tiled.push_back(al);
+      }
+    Name pair = gen.fresh("pair");
+    auto launch = [&](int64_t which) {
+      auto l = std::make_shared<Stmt>();
+      l->k = Stmt::Launch;
+      l->fname = f.name;
+      l->grid = f.grid;
+      l->block = f.block;
+      l->i = loop->i;
+      for (auto& a : arrays) l->args.push_back(mk_var(which == 1 && a.written ? tmp[a.host] : a.host, Type::pointer(a.sz)));
+      for (auto& a : arrays) if (a.written) l->args.push_back(mk_var(which == 1 ? a.host : tmp[a.host], Type::pointer(a.sz)));
+      E number = add(mk_binop(BinOp::Mul, mk_var(pair, ity), iint(2), ity), iint(which));
+      l->args.push_back(extra == 0 ? iint(base_steps) : add(iint(base_steps), mk_binop(BinOp::Lt, number, iint(extra), bty)));
+      return S(l);
+    };
+    tiled.push_back(mk_for(pair, iint(0), iint(pairs), 1, {launch(0), launch(1)}, LoopPar(), loop->i));
+    for (auto& kv : tmp) {
+      auto fr = std::make_shared<Stmt>();
+      fr->k = Stmt::Free;
+      fr->id = kv.second;
+      tiled.push_back(fr);
+    }
+    // A run that may allocate nothing has a fixed amount of scratch memory for all temporaries of the plan: when the
+    // second set of arrays may not fit, the loop of launches stays beside the tiled one and the runtime picks.
+    int64_t others = 0;
+    visit_stmts(p.host, [&](const S& s) { if (s->k == Stmt::Alloc) others += s->iv * elem_bytes(s->ty.sz) + 256; });
+    if (others + second_set > SCRATCH_BYTES) {
+      auto fits = std::make_shared<Expr>(*mk_raw("parpy_temporaries_fit(" + std::to_string(second_set) + ")", bty));
+      fits->iv = second_set;
+      return mk_scope({mk_if(fits, tiled, {loop})});
+    }
+    return mk_scope(tiled);
+  }
+
+  Stmts walk(const Stmts& ss) {
+    Stmts out;
+    for (auto& s : ss) {
+      if (S t = tile(s)) { for (auto& q : t->body) out.push_back(q); continue; }
+      auto r = clone(s);
+      if (s->k == Stmt::For || s->k == Stmt::While || s->k == Stmt::If) {
+        r->body = walk(s->body);
+        r->els = walk(s->els);
+      }
+      out.push_back(r);
+    }
+    return out;
+  }
+
+  void run() {
+    p.host = walk(p.host);
+    // kernels that nothing launches any more
+    std::set<std::string> used;
+    visit_stmts(p.host, [&](const S& s) { if (s->k == Stmt::Launch) used.insert(s->fname); });
+    std::vector<Kernel> keep;
+    for (auto& k : p.kernels) if (used.count(k.name)) keep.push_back(k);
+    p.kernels = keep;
+  }
+};
+
+}  // namespace
+
+void time_tile(Program& p, const Options& opts, NameGen& gen) { TimeTile(p, opts, gen).run(); }
+
+}  // namespace hipopt
+}  // namespace parpy

@@ -133,6 +133,21 @@ __device__ __forceinline__ float parpy_fmax3(float a, float b, float c) { float 
 __device__ __forceinline__ float parpy_fmin3(float a, float b, float c) { float r; asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c)); return r; }
 __device__ __forceinline__ float parpy_fmax3c(float a, float b, float c) { float r; asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c)); return r; }
 __device__ __forceinline__ float parpy_fmin3c(float a, float b, float c) { float r; asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c)); return r; }
+// x / c for an integral constant c: the product with the reciprocal r = 1 / c (rounded), corrected by the remainder
+// x - c * q, which is exact (Markstein's division: a quotient within one unit of the last place and a correctly rounded
+// reciprocal give the correctly rounded quotient after one correction; FIX is two where the reciprocal's own error can
+// put the product further off).  div_fixup settles zeros, infinities and NaN.  Results are those of the division bit for
+// bit, except that a quotient below the normal range which lies exactly between two numbers may round to the other one.
+template <int FIX> __device__ __forceinline__ float parpy_div_const(float x, float c, float r) {
+  float q = x * r;
+  for (int k = 0; k < FIX; ++k) q = __builtin_fmaf(__builtin_fmaf(-c, q, x), r, q);
+  return __builtin_amdgcn_div_fixupf(q, c, x);
+}
+template <int FIX> __device__ __forceinline__ double parpy_div_const(double x, double c, double r) {
+  double q = x * r;
+  for (int k = 0; k < FIX; ++k) q = __builtin_fma(__builtin_fma(-c, q, x), r, q);
+  return __builtin_amdgcn_div_fixup(q, c, x);
+}
 // reduce over each row of 16 lanes; afterwards every lane of a row holds the row's result
 template <class Op, class T> __device__ __forceinline__ T parpy_row_reduce(T v) {
   Op op;
@@ -526,7 +541,17 @@ struct DevicePrinter {
         }
       }
       case Expr::IfExpr: return "(" + pexpr(e->args[0]) + " ? " + pexpr(e->args[1]) + " : " + pexpr(e->args[2]) + ")";
-      case Expr::Convert: return "((" + std::string(elem_ctype(e->ty.sz)) + ")" + paren(pexpr(e->args[0])) + ")";
+      case Expr::Convert: {
+        // float32(float64(x) / c) with a single-precision x and c: the quotient of 24-bit numbers rounded to 53 bits and
+        // then to 24 is the one rounded to 24 at once, so the division is done in single precision (as the device
+        // compiler does with a division that it can see)
+        const E& d = e->args[0];
+        if (e->ty.is_scalar() && e->ty.sz == ElemSize::F32 && d->k == Expr::BinOpE && d->bop == BinOp::Div && d->ty.is_scalar() && d->ty.sz == ElemSize::F64 &&
+            d->args[0]->k == Expr::Convert && d->args[0]->args[0]->ty.is_scalar() && d->args[0]->args[0]->ty.sz == ElemSize::F32 &&
+            d->args[1]->k == Expr::Float && (double)(float)d->args[1]->fv == d->args[1]->fv)
+          return pexpr(mk_binop(BinOp::Div, d->args[0]->args[0], mk_float(d->args[1]->fv, ElemSize::F32), e->ty, d->i));
+        return "((" + std::string(elem_ctype(e->ty.sz)) + ")" + paren(pexpr(e->args[0])) + ")";
+      }
       case Expr::Index: {
         if (!as_lvalue) {
           if (cur_pack_loads) {
@@ -1202,6 +1227,8 @@ struct DevicePrinter {
       r.lo = 0;
       r.hi = k.block.x - 1;
       ranges[Name{"threadIdx.x", -1}] = r;
+      r.hi = k.grid.x - 1;
+      ranges[Name{"blockIdx.x", -1}] = r;
     }
     stream_out.clear();
     if (opts.opt_nontemporal && !k.cached_stores) {
@@ -1286,6 +1313,7 @@ struct PlanPrinter {
       }
       case Expr::IfExpr: return "(ite " + hexpr(e->args[0]) + " " + hexpr(e->args[1]) + " " + hexpr(e->args[2]) + ")";
       case Expr::Convert: return std::string("(cvt ") + elem_tag(e->ty.sz) + " " + hexpr(e->args[0]) + ")";
+      case Expr::Raw: return "(fits " + std::to_string(e->iv) + ")";   // whether temporaries of that many bytes can be had
       case Expr::AddrOf: return "(addr " + hexpr(e->args[0]) + " " + hexpr(e->args[1]) + " " + std::to_string(elem_bytes(e->ty.sz)) + ")";
       default: fail_rt(e->i, "Expression " + print_expr(e) + " is not supported in host code");
     }

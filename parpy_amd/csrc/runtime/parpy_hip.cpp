@@ -67,7 +67,7 @@ struct Val {
 };
 
 struct HExpr {
-  enum Op : uint8_t { Var, Lit, Neg, Not, BitNeg, Bin, Ite, Cvt, Addr } op = Lit;
+  enum Op : uint8_t { Var, Lit, Neg, Not, BitNeg, Bin, Ite, Cvt, Addr, Fits } op = Lit;
   int slot = -1;
   Val lit;
   std::string bin;
@@ -243,6 +243,9 @@ struct PlanBuilder {
       e.args.push_back(expr(x->at(1)));
       e.args.push_back(expr(x->at(2)));
       e.elem_bytes = x->at(3)->as_int();
+    } else if (h == "fits") {
+      e.op = HExpr::Fits;
+      e.lit.i = x->at(1)->as_int();
     } else {
       throw std::runtime_error("unknown host expression '" + h + "' in launch plan");
     }
@@ -375,6 +378,11 @@ Val eval(const Plan& p, const HExpr& e) {
         default: break;
       }
       r.i = v;
+      return r;
+    }
+    case HExpr::Fits: {   // temporaries of so many bytes can be had: always, unless this run may only carve scratch memory
+      Val r;
+      r.i = !p.scratch_base || ((p.scratch_top + 255) & ~int64_t(255)) + e.lit.i <= (int64_t)PARPY_HIP_SCRATCH_BYTES;
       return r;
     }
     case HExpr::Addr: {

@@ -1,0 +1,84 @@
+"""Time loops over element-wise updates from shifted elements: several steps per launch against one launch per update
+(`opt_tile_steps` off), at array lengths around the stretches of a wavefront."""
+import numpy as np
+import pytest
+
+import parpy_amd as parpy
+from parpy_amd.compile import hiprtc_compile
+from parpy_amd.operators import float32, max
+
+HIP = parpy.CompileBackend.Hip
+
+
+def jacobi(A, B, C, n, steps):
+    for t in range(1, steps):
+        parpy.label('N')
+        B[1:-1] = (A[:-2] + A[1:-1] + A[2:]) / 3.0
+        parpy.label('N')
+        A[1:-1] = (B[:-2] + B[1:-1] + B[2:]) / 3.0
+
+
+def wave_equation(A, B, C, n, steps):
+    """One update per step, reach two, a coefficient array, the own element of the array it writes."""
+    for t in range(steps):
+        parpy.label('N')
+        for i in range(2, n - 3):
+            s = A[i - 2] + A[i + 2] - A[i] * 2.0
+            B[i] = A[i] * 1.5 - B[i] * 0.5 + C[i] * s / 7.0
+        parpy.label('N')
+        for i in range(1, n):
+            A[i] = max(B[i - 1], A[i] * 0.25) + 0.001 * B[i]
+
+
+def lopsided(A, B, C, n, steps):
+    """Two arrays written by one launch, one-sided reach, the iteration number as a value."""
+    for t in range(steps):
+        parpy.label('N')
+        for i in range(n - 1):
+            A[i] = C[i + 1] * 0.5 + A[i] * 0.5
+            B[i] = A[i] + float32(i % 5)
+        parpy.label('N')
+        for i in range(3, n):
+            C[i] = B[i - 3] * 0.125 + C[i] * 0.875
+
+
+PROGRAMS = [jacobi, wave_equation, lopsided]
+
+
+def run(f, arrays, n, steps, **kw):
+    o = parpy.par({'N': parpy.threads(n)})
+    o.backend = HIP
+    for k, v in kw.items():
+        setattr(o, k, v)
+    got = [a.copy() for a in arrays]
+    parpy.jit(f)(*got, n, steps, opts=o)
+    return got
+
+
+@pytest.mark.parametrize("f", PROGRAMS, ids=lambda f: f.__name__)
+def test_steps_of_a_stencil_share_a_launch(f):
+    o = parpy.par({'N': parpy.threads(5000)})
+    o.backend = HIP
+    args = [np.zeros(5000), np.zeros(5000), np.zeros(5000), 5000, 20]
+    s = parpy.print_compiled(f, args, o)
+    hiprtc_compile(s[:s.index("// host side")], o)
+    assert "parpy_lane_before" in s and s[s.index("// host side"):].count("<<<") == 2
+    o.opt_tile_steps = False
+    s = parpy.print_compiled(f, args, o)
+    assert "parpy_lane_before(" not in s[s.index('extern "C"'):]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f", PROGRAMS, ids=lambda f: f.__name__)
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=lambda d: np.dtype(d).name)
+def test_tiled_steps_match_one_launch_per_update(f, dtype):
+    rng = np.random.default_rng(7)
+    for n, steps in [(512, 3), (513, 50), (1000, 2), (1024, 17), (4093, 64), (20000, 7), (65537, 33), (800001, 12)]:
+        arrays = [rng.standard_normal(n).astype(dtype) for _ in range(3)]
+        arrays[0][n // 2] = 0.0
+        arrays[0][n // 3] = 1e-42 if dtype == np.float32 else 5e-324
+        want, got = run(f, arrays, n, steps, opt_tile_steps=False), run(f, arrays, n, steps)
+        for w, g in zip(want, got):
+            # (products and sums may be contracted to fused multiply-adds differently)
+            same = np.array_equal(w, g) if f is jacobi else np.allclose(w, g, rtol=1e-12 if dtype == np.float64 else 1e-4, atol=1e-13 if dtype == np.float64 else 1e-5)
+            assert same, (f.__name__, n, steps, np.abs(w - g).max())
