@@ -119,6 +119,12 @@ def _expand_arg(arg):
     return [arg]
 
 
+def raise_runtime_error():
+    """Raise what the runtime library reported for the last call of this thread."""
+    from .runtime import load_hip_runtime_lib
+    raise RuntimeError(f"{load_hip_runtime_lib().parpy_get_error_message().decode('ascii', 'replace')}")
+
+
 def get_wrapper(name, key, plan_text, opts):
     """Callable that runs the launch plan of a compiled function on its (validated) arguments."""
     from .buffer import Buffer
@@ -172,6 +178,7 @@ def get_wrapper(name, key, plan_text, opts):
     wrapper.run_noalloc = run_noalloc
     wrapper.timed = timed
     wrapper.plan = plan
+    wrapper.lib = lib
     wrapper.launch_count = lambda: lib.parpy_hip_plan_launch_count(plan)
     wrapper.graph_replays = lambda: lib.parpy_hip_plan_graph_replays(plan)
     wrapper.persistent_launches = lambda: lib.parpy_hip_plan_persistent_launches(plan)

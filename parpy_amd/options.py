@@ -168,6 +168,8 @@ class LoopPar:
     a multiple of the 64-lane wavefront instead of the 32-lane warp.
     """
 
+    __slots__ = ("nthreads", "reduction", "_tpb")
+
     def __init__(self, nthreads=0, reduction=False, tpb=DEFAULT_TPB):
         self.nthreads = nthreads
         self.reduction = reduction
@@ -200,31 +202,33 @@ class LoopPar:
     __str__ = __repr__
 
 
-_options_clock = [0]
+_LISTS = ("includes", "libs", "extra_flags")
 
 
 class CompileOptions:
-    """src/option.rs:14-108; __str__ feeds the in-memory cache key (python/parpy/key.py:29-30)."""
+    """src/option.rs:14-108; __str__ feeds the in-memory cache key (python/parpy/key.py:29-30).
 
-    def __setattr__(self, name, value):
-        # every assignment to any options object gets a stamp that no other assignment has;
-        # the stamp tells when the cached part of the fast key is stale
-        _options_clock[0] += 1
-        object.__setattr__(self, "_stamp", _options_clock[0])
-        object.__setattr__(self, name, value)
+    An object holds only what was set on it: defaults are attributes of the class, the containers are made when they
+    are first asked for.  Building one is part of many calls (`opts=parpy.par(...)`), filling in thirty-five fields
+    would be most of its cost."""
+
+    def __getattr__(self, name):   # (only for what neither the object nor the class has)
+        if name in _LISTS:
+            value = self.__dict__[name] = []
+        elif name == "parallelize":
+            value = self.__dict__[name] = {}
+        else:
+            raise AttributeError(f"'CompileOptions' object has no attribute '{name}'")
+        return value
 
     def _fast_key(self):
         """Hashable value of the whole options state: equal for two objects that hold equal settings,
-        so that a call with a freshly built options object finds the code compiled for an earlier one.
-        The fields assigned through attributes are cached per stamp; the containers, which can be
-        changed in place, are read every time."""
+        so that a call with a freshly built options object finds the code compiled for an earlier one."""
         d = self.__dict__
-        if d.get("_key_stamp") != d["_stamp"]:
-            d["_key_fields"] = tuple(v for k, v in d.items()
-                                     if (k[0] != "_" or k in CompileOptions._DEFAULTS) and not isinstance(v, (dict, list)))
-            d["_key_stamp"] = d["_stamp"]
-        return (d["_key_fields"], tuple(d["includes"]), tuple(d["libs"]), tuple(d["extra_flags"]),
-                tuple((k, p.nthreads, p.reduction, p._tpb) for k, p in d["parallelize"].items()))
+        fields = [(k, v) for k, v in d.items() if k in CompileOptions._DEFAULTS and v is not CompileOptions._DEFAULTS[k]]
+        fields.sort(key=lambda kv: kv[0])
+        return (tuple(fields), tuple(tuple(d.get(k, ())) for k in _LISTS),
+                tuple((k, p.nthreads, p.reduction, p._tpb) for k, p in self.parallelize.items()))
 
     # opt_*: HIP memory-codegen switches; None keeps the compiler's default.  They exist so that
     # tests and benchmarks can measure what each buys.
@@ -272,19 +276,6 @@ class CompileOptions:
         'assume_aligned': None,   # set by the driver: False when an array argument is not 16-byte aligned
     }
 
-    def __init__(self):
-        # written into the instance dictionary directly: building an options object is part of
-        # many calls (`opts=parpy.par(...)`) and thirty stamped assignments would dominate them
-        d = self.__dict__
-        d.update(CompileOptions._DEFAULTS)
-        d["parallelize"] = {}
-        d["includes"] = []
-        d["libs"] = []
-        d["extra_flags"] = []
-        _options_clock[0] += 1
-        d["_stamp"] = d["_key_stamp"] = _options_clock[0]
-        d["_key_fields"] = CompileOptions._DEFAULT_KEY
-
     @property
     def max_thread_blocks_per_cluster(self):
         return self._max_thread_blocks_per_cluster
@@ -329,7 +320,8 @@ class CompileOptions:
                 f"includes: {self.includes}, libs: {self.libs}, extra_flags: {self.extra_flags} }}")
 
 
-CompileOptions._DEFAULT_KEY = tuple(CompileOptions._DEFAULTS.values())
+for _name, _value in CompileOptions._DEFAULTS.items():
+    setattr(CompileOptions, _name, _value)
 
 
 class ScalarSizes:
@@ -342,9 +334,9 @@ class ScalarSizes:
 
 def par(p):
     """Default options carrying the parallelisation mapping `p` (src/option.rs:157-162)."""
-    opts = CompileOptions()
     for k, v in p.items():
-        if not isinstance(k, str) or not isinstance(v, LoopPar):
+        if type(v) is not LoopPar and not isinstance(v, LoopPar) or not isinstance(k, str):
             raise TypeError("parallelization specification must map label strings to LoopPar values")
-    opts.__dict__["parallelize"] = dict(p)   # (no stamp needed: the fast key reads the mapping itself)
+    opts = CompileOptions()
+    opts.__dict__["parallelize"] = dict(p)
     return opts

@@ -1,0 +1,78 @@
+"""The call extension: which calls it takes for the same, and that what it runs is what the Python path would run."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import parpy_amd as parpy
+from parpy_amd.options import CompileOptions, LoopPar
+
+torch = pytest.importorskip("torch")
+HIP = parpy.CompileBackend.Hip
+
+
+def opts(n=64, **kw):
+    o = parpy.par({'N': parpy.threads(n)})
+    for k, v in kw.items():
+        setattr(o, k, v)
+    return o
+
+
+def test_calls_that_differ_in_anything_are_different_calls():
+    from parpy_amd import fastcall
+    ran = []
+    run = ctypes.CFUNCTYPE(ctypes.c_int32, ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p), ctypes.c_int32)(lambda plan, p, n: ran.append(plan) or 0)
+    table = fastcall._load().CallTable(CompileOptions, LoopPar, ctypes.cast(run, ctypes.c_void_p).value)
+    f32 = lambda v: torch.tensor(v, dtype=torch.float32)
+    calls = [((1,), opts()), ((1.0,), opts()), ((True,), opts()), ((2,), opts()), ((1, 1), opts()), (({"a": 1},), opts()), (({"b": 1},), opts()),
+             (({"a": 1, "b": 2},), opts()), (({"a": 12},), opts()), ((f32(1.0),), opts()), ((f32(2.0),), opts()), ((torch.tensor(1.0, dtype=torch.float64),), opts()),
+             ((1,), opts(128)), ((1,), opts(backend=HIP)), ((1,), opts(opt_vectorize=False)), ((1,), opts(opt_vectorize=True)), ((1,), opts(reg_budget=40)),
+             ((1,), parpy.par({'M': parpy.threads(64)})), ((1,), parpy.par({'N': parpy.threads(64).reduce()})), ((1,), parpy.par({'N': parpy.threads(64).tpb(64)}))]
+    for q, (args, o) in enumerate(calls):
+        assert table.run(args, {"opts": o}) is None, q
+        assert table.add(args, o, 1000 + q, ())
+    for q, (args, o) in enumerate(calls):
+        assert table.run(args, {"opts": o}) == 0 and ran[-1] == 1000 + q
+    assert table.run((1,), {"opts": parpy.par({'N': parpy.threads(64)})}) == 0 and ran[-1] == 1000     # a fresh object with equal settings
+    # what it leaves to the Python path
+    for args, kw in [((1,), {}), ((1,), {"opts": opts(), "extra": 1}), ((1,), {"opts": None}), ((np.zeros(3),), {"opts": opts()}), ((torch.zeros(3),), {"opts": opts()}),
+                     (({"a": {"b": 1}},), {"opts": opts()}), (({1: 1},), {"opts": opts()}), ((1 << 70,), {"opts": opts()}), ((1,), {"opts": opts(includes=["x"])})]:
+        assert table.run(args, kw) is None
+    table.clear()
+    assert table.run((1,), {"opts": opts()}) is None
+
+
+def test_plan_pointers_follow_the_sorted_fields():
+    from parpy_amd import fastcall
+    a, b, c, s = (torch.zeros(k) for k in (1, 2, 3, 4))
+    assert fastcall.pointer_order((a, {"z": b, "n": 3, "c": c, "d": torch.tensor(1.0)}, 5, s)) == (0, 2, 1, 3)
+
+
+def scale(d, out, n):
+    parpy.label('N')
+    for i in range(n):
+        out[i] = d["x"][i] * d["w"] + d["b"][i]
+
+
+@pytest.mark.gpu
+def test_warm_calls_run_on_the_arguments_of_the_call():
+    f = parpy.jit(scale)
+    for rep in range(3):
+        for n in (64, 65, 1000):
+            for w in (2.0, 4.0):   # (exact products: a fused multiply-add rounds like the two operations)
+                x, b = (torch.randn(n + 1, device="cuda") for _ in range(2))
+                out = torch.full((n + 1,), -1.0, device="cuda")
+                for off in (0, 1):                      # whole allocations and views that are only 4-byte aligned
+                    xv, bv, ov = x[off:off + n], b[off:off + n], out[off:off + n]
+                    fields = {"x": xv, "w": w, "b": bv} if rep % 2 else {"b": bv, "x": xv, "w": w}
+                    f(fields, ov, n, opts=opts(256))
+                    assert torch.equal(ov, xv * w + bv), (rep, n, w, off)
+    z = torch.randn(64, device="cuda", requires_grad=True)
+    with pytest.raises(Exception):
+        f({"x": z, "w": 2.0, "b": z}, z, 64, opts=opts(256))
+    parpy.clear_cache()
+    out = torch.zeros(64, device="cuda")
+    x = torch.randn(64, device="cuda")
+    f({"x": x, "w": 2.0, "b": x}, out, 64, opts=opts(256))
+    f({"x": x, "w": 2.0, "b": x}, out, 64, opts=opts(256))
+    assert torch.equal(out, x * 2.0 + x)
