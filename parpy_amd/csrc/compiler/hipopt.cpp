@@ -63,6 +63,7 @@ void hip_optimize(Program& p, const Options& opts, NameGen& gen) {
     if (opts.opt_unswitch_uniform) k.body = pass.hoist_uniform_conditions(k.body);
     if (opts.opt_if_convert) k.body = pass.if_convert(k.body);
     if (opts.opt_lds_rows) pass.lds_rows();
+    k.body = pass.widen_half_sums(k.body);
     if (opts.opt_vectorize) k.body = pass.vectorize(k.body);
     int64_t budget = pass.reg_budget();
     if (opts.opt_hoist_invariant) k.body = pass.hoist_invariant(k.body, &budget, false);

@@ -104,6 +104,7 @@ struct Pass {
   int vector_width(const S& loop);
   static int64_t strided_run(const E& idx, const Name& d);
   Stmts vectorize(const Stmts& ss);
+  Stmts widen_half_sums(const Stmts& ss);
   Stmts mfma_dot(const Stmts& ss);
 
   // hipopt_regs.cpp: values kept in registers: the register budget, loads hoisted out of sequential loops, sections cached between loops

@@ -147,6 +147,15 @@ template <int FIX> __device__ __forceinline__ double parpy_div_const(double x, d
   for (int k = 0; k < FIX; ++k) q = __builtin_fma(__builtin_fma(-c, q, x), r, q);
   return __builtin_amdgcn_div_fixup(q, c, x);
 }
+// Quotient of halves, correctly rounded: a quotient in single precision after one correction by the remainder is off by
+// 2^-24 of its value at most, two 11-bit numbers' quotient keeps 2^-23 away from every tie that it does not hit exactly,
+// so rounding it to a half is rounding the quotient (half the instructions of the general sequence).
+__device__ __forceinline__ _Float16 parpy_div_half(_Float16 a, _Float16 b) {
+  const float x = (float)a, y = (float)b, r = __builtin_amdgcn_rcpf(y);
+  float q = x * r;
+  q = __builtin_fmaf(__builtin_fmaf(-y, q, x), r, q);
+  return __builtin_amdgcn_div_fixuph((_Float16)q, b, a);
+}
 // reduce over each row of 16 lanes; afterwards every lane of a row holds the row's result
 template <class Op, class T> __device__ __forceinline__ T parpy_row_reduce(T v) {
   Op op;
@@ -164,6 +173,10 @@ template <class Op, class T> __device__ __forceinline__ T parpy_wave_reduce(T v)
   v = op(v, parpy_dpp<0x143>(v));  // row_bcast:31 (lane 31 into rows 2 and 3)
   return parpy_readlane(v, 63);
 }
+// halves are combined in single precision (the partial results of the lanes rounded once instead of in every step, and
+// one instruction per step instead of four)
+template <class Op> __device__ __forceinline__ _Float16 parpy_wave_reduce(_Float16 v) { return (_Float16)parpy_wave_reduce<Op>((float)v); }
+template <class Op> __device__ __forceinline__ _Float16 parpy_row_reduce(_Float16 v) { return (_Float16)parpy_row_reduce<Op>((float)v); }
 // block reduction: one LDS slot per wavefront, then every wavefront reduces the partials
 template <class Op, int NWAVES, class T>
 __device__ __forceinline__ T parpy_block_reduce(T v, T neutral, T* slots, bool sync_after) {
@@ -505,6 +518,8 @@ struct DevicePrinter {
             return std::string("parpy_") + base + "<" + elem_ctype(sz) + ">(" + a + ", " + b + ")";
           }
           case BinOp::FloorDiv: case BinOp::Div: case BinOp::Rem: {
+            if (e->bop == BinOp::Div && e->ty.is_scalar() && e->ty.sz == ElemSize::F16 && e->args[1]->ty.is_scalar() && e->args[1]->ty.sz == ElemSize::F16)
+              return "parpy_div_half(" + a + ", " + b + ")";
             // Division by an integral constant: 4 to 6 instructions instead of the 11 of the general division (a
             // three-point average in float64 held in registers: 93 -> 62 us for 98 updates of 10^6 elements).  Powers of
             // two are exact products, which the device compiler makes of them; constants with a fraction keep the
@@ -587,7 +602,8 @@ struct DevicePrinter {
           ranges[x->name] = r;
         }
         std::string out = pexpr(e->args[0]) + "[" + pexpr(e->args[1]) + "]";
-        if (opts.opt_offset32 && e->args[0]->ty.mem != Mem::LDS && read_only_param(e->args[0]) && !walks_sequentially(e->args[1])) {
+        if (opts.opt_offset32 && e->args[0]->ty.mem != Mem::LDS && read_only_param(e->args[0]) && !walks_sequentially(e->args[1]) &&
+            !(in_unrolled > 0 && elem_bytes(e->ty.sz) < 4)) {
           // An element whose byte offset provably fits 32 bits is addressed as base + 32-bit offset, the
           // form the global memory instructions take (64-bit scalar base, 32-bit per-lane offset): no
           // sign extension and no 64-bit add per access.  Matters where address arithmetic competes with
@@ -597,7 +613,8 @@ struct DevicePrinter {
           // were serialised (softmax over rows of 10^6 floats on 64 threads: 2.8 -> 3.6 ms).  For the same
           // reason an index that advances with a sequential loop keeps its plain form: there the device
           // compiler's own strength reduction and wide loads are worth more (one thread summing a row of
-          // 10^5 floats: 0.7 ms against 1.1 ms).
+          // 10^5 floats: 0.7 ms against 1.1 ms).  And neighbouring elements of one or two bytes keep it: with offsets that
+          // wrap they are only joined to one access when the vector is known to be aligned.
           Interval r = expr_range(e->args[1], ranges);
           int64_t eb = elem_bytes(e->ty.sz);
           if (r.known && r.lo >= 0 && r.hi * eb + eb <= (int64_t)UINT32_MAX) {
@@ -640,6 +657,8 @@ struct DevicePrinter {
     }
   }
 
+  std::vector<S> kept_alive;
+  int in_unrolled = 0;            // unrolled loops over the elements of a vector around the statement being printed
   std::set<Name> seq_loop_vars;   // variables of the enclosing sequential loops that are kept as loops
 
   bool walks_sequentially(const E& idx) const {
@@ -713,11 +732,29 @@ struct DevicePrinter {
     const char* cmp = s->step > 0 ? " < " : " > ";
     std::string los = pexpr(s->lo), his = pexpr(s->hi);
 
+    if (s->map.k == GpuMap::None && s->unroll && s->args.size() == 2) {
+      // the elements of one vector, some of which may lie past the end: all of them without a test where the vector is
+      // whole, one test each where it is not
+      os << ind(n) << "if (" << pexpr(s->args[0]) << ") {\n";
+      auto plain = std::make_shared<Stmt>(*s);
+      plain->args.clear();
+      kept_alive.push_back(plain);
+      pfor(plain, n + 2);
+      os << ind(n) << "} else {\n";
+      auto tested = std::make_shared<Stmt>(*plain);
+      tested->body = {s->body[0], mk_if(s->args[1], Stmts(s->body.begin() + 1, s->body.end()), {})};
+      kept_alive.push_back(tested);   // (places in its statement lists are keys of the packing plan)
+      pfor(tested, n + 2);
+      os << ind(n) << "}\n";
+      return;
+    }
     if (s->map.k == GpuMap::None) {
       if (s->unroll) os << ind(n) << "#pragma unroll\n";
       os << ind(n) << "for (" << vty << " " << v << " = " << los << "; " << v << cmp << his << "; " << v << " += " << s->step << ") {\n";
       bool fresh = !s->unroll && seq_loop_vars.insert(s->id).second;
+      in_unrolled += s->unroll;
       pstmts(s->body, n + 2);
+      in_unrolled -= s->unroll;
       if (fresh) seq_loop_vars.erase(s->id);
       os << ind(n) << "}\n";
       return;
