@@ -238,6 +238,7 @@ struct GpuMap {
   int64_t n = 0;          // Thread: #threads; Block: #blocks; ThreadBlock: #threads total
   int64_t tpb = 0;        // ThreadBlock: threads per block
   int64_t mult = 1;       // Block: divisor when several loops share one grid dimension
+  int64_t per = 1;        // Block: iterations of a workgroup, one wavefront (threadIdx.y) each
 };
 
 struct Stmt {
@@ -432,6 +433,7 @@ struct Kernel {
   bool cached_stores = false;   // what this kernel writes is read by the next one: no non-temporal stores
   bool opaque_body = false;     // the body is a call of a device helper: parameters are described by the creator
   bool no_restrict = false;     // workgroups exchange data through the parameters during the kernel: no no-alias promise
+  bool wave_rows = false;       // every wavefront of a workgroup has an iteration of its own: barriers only order its own accesses
   bool fence_lds_iterations = false;  // keep a thread's LDS load / compute / store groups apart when the code is scheduled
   std::vector<std::vector<Name>> distinct_pointers;  // local pointer variables that never name the same array while both are in scope
 };

@@ -21,7 +21,7 @@
 //                   `if (c) for x: A else for x: B`;
 //   drop_barriers   barriers between regions that share no written array go.
 //
-// Five rewrites work on the whole program because they change a launch:
+// Six rewrites work on the whole program because they change a launch:
 //   TimeTile        several steps of a host loop of element-wise launches over
 //                   shifted elements run in one launch;
 //   GatherTranspose column gathers X[d, c] over an innermost sequential d read a
@@ -30,6 +30,8 @@
 //                   the rows, whole workgroups the very long ones;
 //   LaneSplit       eight adjacent lanes share one iteration's sequential sum
 //                   over constant bounds, 16-byte pieces of each line each;
+//   RowThreads      short rows that are reduced get fewer threads than asked for,
+//                   down to a wavefront per row and several rows per workgroup;
 //   Coarsen         a large element-wise launch with one element per thread is
 //                   cut to a quarter so that vectorize gives each thread four.
 //
@@ -51,6 +53,7 @@ void hip_optimize(Program& p, const Options& opts, NameGen& gen) {
   if (opts.opt_lane_split) hipopt::ragged_sum(p, opts, gen);
   if (opts.opt_lane_split && !opts.opt_mfma_sddmm) hipopt::lane_split(p, opts, gen);
   if (opts.opt_vectorize) hipopt::coarsen(p, opts, gen);
+  if (opts.opt_vectorize && !opts.persistent_loops) hipopt::row_threads(p, opts, gen);
   for (auto& k : p.kernels) {
     if (k.opaque_body) { k.aligned_params = opts.assume_aligned; continue; }
     hipopt::Pass pass(k, opts, gen);

@@ -493,8 +493,112 @@ struct Coarsen {
   }
 };
 
+// ================================================================ threads for short rows
+// `{'N': threads(n), 'M': threads(512)}` on rows of 300 elements starts eight wavefronts per row, most of them for one
+// element per lane or none, and each takes part in every reduction: cross-lane steps, a round trip through LDS and a
+// barrier, around a hundred instructions per wavefront and reduction.  A row that is reduced and then needs no more than
+// a vector per thread gets fewer threads; a row that fits one wavefront reduces without LDS or barriers, and several
+// such rows share a workgroup.
+struct RowThreads {
+  Program& p;
+  const Options& opts;
+  NameGen& gen;
+  RowThreads(Program& prog, const Options& o, NameGen& g) : p(prog), opts(o), gen(g) {}
+
+  bool apply(Kernel& k, const StmtP& launch) {
+    if (k.body.size() != 1 || k.block.y != 1 || k.block.z != 1 || k.opaque_body) return false;
+    const S& root = k.body[0];
+    if (!(root->k == Stmt::For && root->map.k == GpuMap::Block && root->map.mult == 1 && root->step == 1 && root->lo->k == Expr::Int &&
+          root->lo->iv == 0 && root->hi->k == Expr::Int && root->els.empty()))
+      return false;
+    const int64_t rows = root->hi->iv, threads = k.block.x;
+    if (root->map.n != rows || k.grid.x * k.grid.y * k.grid.z != rows) return false;
+    // straight through the row: element loops and reductions over the whole workgroup, no loop around them
+    bool ok = true, reduces = false;
+    int64_t longest = 0, bytes = 0;
+    Pass probe(k, opts, gen);
+    std::function<void(const Stmts&)> walk = [&](const Stmts& ss) {
+      for (auto& s : ss) {
+        switch (s->k) {
+          case Stmt::Def: case Stmt::Assign: case Stmt::Sync: break;
+          case Stmt::WaveReduce:
+            reduces = true;
+            if (s->iv != threads) ok = false;
+            break;
+          case Stmt::If: walk(s->body); walk(s->els); break;
+          case Stmt::For: {
+            if (!thread_mapped(s) || s->map.dim != 0 || s->map.n != threads || !s->els.empty()) { ok = false; break; }
+            const int64_t extent = const_extent(s);
+            if (extent <= 0) { ok = false; break; }
+            visit_stmts(s->body, [&](const S& c) { if (c->k == Stmt::For || c->k == Stmt::While || c->k == Stmt::Sync || c->k == Stmt::RawStmt || c->k == Stmt::WaveReduce) ok = false; });
+            longest = std::max(longest, extent);
+            if (const int v = probe.vector_width(s)) bytes = std::max<int64_t>(bytes, 16 / v);
+            break;
+          }
+          default: ok = false;
+        }
+      }
+    };
+    walk(root->body);
+    if (!ok || !reduces || longest == 0 || bytes == 0) return false;
+    // (a launch of four wavefronts per SIMD or less starts all of them at once: nothing to gain)
+    if (rows * (threads / WAVE_SIZE) <= 4096) return false;
+    // At least 24 bytes of the row per thread: 16384 rows of 1000 floats 27.6 us on 512 threads, 20.0 / 20.8 / 21.5 on
+    // 256 / 128 / 64 (softmax); 1000 halves 20.2 us on 256 threads, 15.0 on 64; 300 doubles 23.6 and 14.7; sums of 20000
+    // rows of 300 floats 31.4 us on 1024 threads, 14.4 on 64.
+    int64_t want = WAVE_SIZE;
+    while (want * 2 * 24 <= longest * bytes) want *= 2;
+    want = std::min(want, threads);
+    // Workgroups start at about two per nanosecond, which is what small ones wait for: four rows each where a row is a
+    // wavefront's (the sums above 7.1 us, 6.7 with eight; softmax over 30000 rows of 200 floats 16.0 -> 8.7 us).
+    const int64_t group = want == WAVE_SIZE ? 4 : 1;
+    if (want == threads && group == 1) return false;
+    std::function<Stmts(const Stmts&)> cut = [&](const Stmts& ss) {
+      Stmts out;
+      for (auto& s : ss) {
+        auto r = clone(s);
+        if (s->k == Stmt::WaveReduce) r->iv = want;
+        if (s->k == Stmt::For) r->map.n = want;
+        r->body = cut(s->body);
+        r->els = cut(s->els);
+        out.push_back(r);
+      }
+      return out;
+    };
+    auto nr = clone(root);
+    nr->body = cut(root->body);
+    k.block = Dim3{want, group, 1};
+    if (group > 1) {
+      const int64_t blocks = (rows + group - 1) / group;
+      nr->map.per = group;
+      nr->map.n = blocks * group;
+      (root->map.dim == 0 ? k.grid.x : root->map.dim == 1 ? k.grid.y : k.grid.z) = blocks;
+      k.wave_rows = true;
+    }
+    k.body = {S(nr)};
+    launch->grid = k.grid;
+    launch->block = k.block;
+    return true;
+  }
+
+  void run() {
+    Stmts host;
+    for (auto& s : p.host) {
+      if (s->k != Stmt::Launch) { host.push_back(s); continue; }
+      Kernel* k = nullptr;
+      for (auto& kk : p.kernels)
+        if (kk.name == s->fname) k = &kk;
+      auto ns = std::make_shared<Stmt>(*s);
+      if (k) apply(*k, ns);
+      host.push_back(ns);
+    }
+    p.host = host;
+  }
+};
+
 }  // namespace
 
+void row_threads(Program& p, const Options& opts, NameGen& gen) { RowThreads(p, opts, gen).run(); }
 void gather_transpose(Program& p, const Options& opts, NameGen& gen) { GatherTranspose(p, opts, gen).run(); }
 void lane_split(Program& p, const Options& opts, NameGen& gen) { LaneSplit(p, opts, gen).run(); }
 void coarsen(Program& p, const Options& opts, NameGen& gen) { Coarsen(p, opts, gen).run(); }

@@ -141,6 +141,7 @@ struct Pass {
 void gather_transpose(Program& p, const Options& opts, NameGen& gen);   // hipopt_launch.cpp
 void time_tile(Program& p, const Options& opts, NameGen& gen);          // hipopt_timetile.cpp
 void ragged_sum(Program& p, const Options& opts, NameGen& gen);         // hipopt_ragged.cpp
+void row_threads(Program& p, const Options& opts, NameGen& gen);        // hipopt_launch.cpp
 void lane_split(Program& p, const Options& opts, NameGen& gen);         // hipopt_launch.cpp
 void coarsen(Program& p, const Options& opts, NameGen& gen);            // hipopt_launch.cpp
 void persistent_loops(Program& p, const Options& opts, NameGen& gen);   // hipopt_persist.cpp

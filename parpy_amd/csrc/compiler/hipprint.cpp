@@ -680,6 +680,7 @@ struct DevicePrinter {
       case GpuMap::Block: {
         int64_t tot = m.dim == 0 ? kernel->grid.x : m.dim == 1 ? kernel->grid.y : kernel->grid.z;
         std::string b = "(int)blockIdx." + std::string(1, "xyz"[m.dim]);
+        if (m.per > 1) return "(" + b + " * " + std::to_string(m.per) + " + (int)threadIdx.y)";
         if (tot > m.n) return "((" + b + " / " + std::to_string(m.mult) + ") % " + std::to_string(m.n) + ")";
         return b;
       }
@@ -956,7 +957,10 @@ struct DevicePrinter {
         }
         os << ind(n) << "}\n";
         break;
-      case Stmt::Sync: os << ind(n) << "__syncthreads();\n"; break;
+      case Stmt::Sync:
+        if (kernel->wave_rows) os << ind(n) << "__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, \"workgroup\");\n";
+        else os << ind(n) << "__syncthreads();\n";
+        break;
       case Stmt::Return: os << ind(n) << "return " << pexpr(s->expr) << ";\n"; break;   // (device functions only)
       case Stmt::Scope:
         if (!s->args.empty()) {
