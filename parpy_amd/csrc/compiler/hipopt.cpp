@@ -21,7 +21,7 @@
 //                   `if (c) for x: A else for x: B`;
 //   drop_barriers   barriers between regions that share no written array go.
 //
-// Six rewrites work on the whole program because they change a launch:
+// Seven rewrites work on the whole program because they change a launch:
 //   TimeTile        several steps of a host loop of element-wise launches over
 //                   shifted elements run in one launch;
 //   GatherTranspose column gathers X[d, c] over an innermost sequential d read a
@@ -30,6 +30,8 @@
 //                   the rows, whole workgroups the very long ones;
 //   LaneSplit       eight adjacent lanes share one iteration's sequential sum
 //                   over constant bounds, 16-byte pieces of each line each;
+//   Stages          reductions over several workgroups take vectors and finish in
+//                   one launch;
 //   RowThreads      short rows that are reduced get fewer threads than asked for,
 //                   down to a wavefront per row and several rows per workgroup;
 //   Coarsen         a large element-wise launch with one element per thread is
@@ -42,7 +44,7 @@
 // branches, aliases), hipopt_prefetch.cpp, hipopt_lds.cpp, hipopt_vector.cpp,
 // hipopt_regs.cpp (budget, hoisting, register caching), hipopt_keep.cpp and
 // hipopt_alias.cpp; the whole-program rewrites are in hipopt_launch.cpp,
-// hipopt_ragged.cpp, hipopt_timetile.cpp and hipopt_persist.cpp.
+// hipopt_ragged.cpp, hipopt_timetile.cpp, hipopt_stages.cpp and hipopt_persist.cpp.
 #include "hipopt_pass.hpp"
 
 namespace parpy {
@@ -50,6 +52,7 @@ namespace parpy {
 void hip_optimize(Program& p, const Options& opts, NameGen& gen) {
   if (opts.opt_gather_transpose) hipopt::gather_transpose(p, opts, gen);
   if (opts.opt_tile_steps && !opts.persistent_loops) hipopt::time_tile(p, opts, gen);
+  if (opts.opt_vectorize) hipopt::reduction_stages(p, opts, gen);
   if (opts.opt_lane_split) hipopt::ragged_sum(p, opts, gen);
   if (opts.opt_lane_split && !opts.opt_mfma_sddmm) hipopt::lane_split(p, opts, gen);
   if (opts.opt_vectorize) hipopt::coarsen(p, opts, gen);

@@ -147,10 +147,10 @@ void Pass::mark_read_only() {
       if (s->k == Stmt::Assign && s->dst->k == Expr::Var && (s->dst->ty.is_array() || s->dst->ty.is_pointer()))
         bases(s->expr, alias_of[s->dst->name]);
       if (s->k == Stmt::Assign && s->dst->k == Expr::Index) bases(s->dst->args[0], written);
-      // an array handed to an external device function may be written by it
+      // an array handed to an external device function may be written by it, one handed to the device-scope store is
       auto calls = [&](const E& root) {
         visit_exprs(root, [&](const E& x) {
-          if (x->k != Expr::Call || !x->ext) return;
+          if (x->k != Expr::Call || !(x->ext || x->sval == "parpy_device_store")) return;
           for (auto& a : x->args)
             if (a->k == Expr::AddrOf || (a->k == Expr::Var && !a->ty.is_scalar())) bases(a, written);
         });

@@ -181,7 +181,9 @@ Stmts Pass::expand_short_loops(const Stmts& ss0, bool in_par) {
   Stmts out;
   for (auto& s : ss) {
     int64_t n = s->k == Stmt::For && s->map.k == GpuMap::None ? const_extent(s) : -1;
-    if (in_par && n >= 1 && n <= 8 && straight_line(s->body) && count_stmts(s->body) * (size_t)n <= 256) {
+    // (a vector that may start anywhere stays a loop: its elements are addressed so that they join to one access)
+    const bool vector = s->unroll && s->iv != 0;
+    if (in_par && !vector && n >= 1 && n <= 8 && straight_line(s->body) && count_stmts(s->body) * (size_t)n <= 256) {
       std::vector<Name> locals;
       visit_stmts(s->body, [&](const S& c) { if (c->k == Stmt::Def) locals.push_back(c->id); });
       for (int64_t it = 0; it < n; ++it) {

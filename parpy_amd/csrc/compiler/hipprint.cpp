@@ -254,6 +254,26 @@ __device__ __forceinline__ bool parpy_grid_barrier(unsigned* counter, unsigned* 
   __syncthreads();
   return parpy_bar_ok != 0;
 }
+// What workgroups of one launch hand to each other: stored and loaded at device scope, past the caches of the dies.
+template <class T> __device__ __forceinline__ bool parpy_device_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); return true; }
+template <class T> __device__ __forceinline__ T parpy_device_load(const T* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// Whether this workgroup is the last of `n` to get here, for the counter `which`: its first thread waits until what it
+// stored has been performed and counts the workgroup in.  The last one finds n - 1 and puts the counter back to zero for
+// the next launch (launches of a program follow each other on one stream).  What is handed over goes through the two
+// functions above, so neither side writes its caches back or drops them.
+__device__ __forceinline__ bool parpy_last_workgroup(unsigned* counters, int which, unsigned n) {
+  __shared__ bool parpy_last;
+  if (threadIdx.x == 0) {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const unsigned before = __hip_atomic_fetch_add(counters + which, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    parpy_last = before == n - 1u;
+    if (before == n - 1u) __hip_atomic_store(counters + which, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return parpy_last;
+}
 typedef float parpy_f32x4 __attribute__((ext_vector_type(4)));
 template <class T> using parpy_vec4 = T __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ int parpy_lane_id() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
@@ -603,7 +623,7 @@ struct DevicePrinter {
         }
         std::string out = pexpr(e->args[0]) + "[" + pexpr(e->args[1]) + "]";
         if (opts.opt_offset32 && e->args[0]->ty.mem != Mem::LDS && read_only_param(e->args[0]) && !walks_sequentially(e->args[1]) &&
-            !(in_unrolled > 0 && elem_bytes(e->ty.sz) < 4)) {
+            !(in_unrolled > 0 && (elem_bytes(e->ty.sz) < 4 || in_unaligned > 0))) {
           // An element whose byte offset provably fits 32 bits is addressed as base + 32-bit offset, the
           // form the global memory instructions take (64-bit scalar base, 32-bit per-lane offset): no
           // sign extension and no 64-bit add per access.  Matters where address arithmetic competes with
@@ -613,8 +633,9 @@ struct DevicePrinter {
           // were serialised (softmax over rows of 10^6 floats on 64 threads: 2.8 -> 3.6 ms).  For the same
           // reason an index that advances with a sequential loop keeps its plain form: there the device
           // compiler's own strength reduction and wide loads are worth more (one thread summing a row of
-          // 10^5 floats: 0.7 ms against 1.1 ms).  And neighbouring elements of one or two bytes keep it: with offsets that
-          // wrap they are only joined to one access when the vector is known to be aligned.
+          // 10^5 floats: 0.7 ms against 1.1 ms).  And the elements of a vector keep it when they are one or two
+          // bytes wide or the vector may start anywhere: with offsets that wrap they are only joined to one access
+          // when the vector is known to be aligned.
           Interval r = expr_range(e->args[1], ranges);
           int64_t eb = elem_bytes(e->ty.sz);
           if (r.known && r.lo >= 0 && r.hi * eb + eb <= (int64_t)UINT32_MAX) {
@@ -659,6 +680,7 @@ struct DevicePrinter {
 
   std::vector<S> kept_alive;
   int in_unrolled = 0;            // unrolled loops over the elements of a vector around the statement being printed
+  int in_unaligned = 0;           // those whose vectors start at any element
   std::set<Name> seq_loop_vars;   // variables of the enclosing sequential loops that are kept as loops
 
   bool walks_sequentially(const E& idx) const {
@@ -754,8 +776,10 @@ struct DevicePrinter {
       os << ind(n) << "for (" << vty << " " << v << " = " << los << "; " << v << cmp << his << "; " << v << " += " << s->step << ") {\n";
       bool fresh = !s->unroll && seq_loop_vars.insert(s->id).second;
       in_unrolled += s->unroll;
+      in_unaligned += s->unroll && s->iv != 0;
       pstmts(s->body, n + 2);
       in_unrolled -= s->unroll;
+      in_unaligned -= s->unroll && s->iv != 0;
       if (fresh) seq_loop_vars.erase(s->id);
       os << ind(n) << "}\n";
       return;
