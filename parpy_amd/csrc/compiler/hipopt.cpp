@@ -33,7 +33,8 @@
 //   Stages          reductions over several workgroups take vectors and finish in
 //                   one launch;
 //   RowThreads      short rows that are reduced get fewer threads than asked for,
-//                   down to a wavefront per row and several rows per workgroup;
+//                   down to a wavefront per row and several rows per workgroup,
+//                   a few long ones more;
 //   Coarsen         a large element-wise launch with one element per thread is
 //                   cut to a quarter so that vectorize gives each thread four.
 //

@@ -514,7 +514,7 @@ struct RowThreads {
     const int64_t rows = root->hi->iv, threads = k.block.x;
     if (root->map.n != rows || k.grid.x * k.grid.y * k.grid.z != rows) return false;
     // straight through the row: element loops and reductions over the whole workgroup, no loop around them
-    bool ok = true, reduces = false;
+    bool ok = true, reduces = false, strided = false;
     int64_t longest = 0, bytes = 0;
     Pass probe(k, opts, gen);
     std::function<void(const Stmts&)> walk = [&](const Stmts& ss) {
@@ -532,6 +532,7 @@ struct RowThreads {
             if (extent <= 0) { ok = false; break; }
             visit_stmts(s->body, [&](const S& c) { if (c->k == Stmt::For || c->k == Stmt::While || c->k == Stmt::Sync || c->k == Stmt::RawStmt || c->k == Stmt::WaveReduce) ok = false; });
             longest = std::max(longest, extent);
+            strided = strided || s->step != 1;
             if (const int v = probe.vector_width(s)) bytes = std::max<int64_t>(bytes, 16 / v);
             break;
           }
@@ -541,17 +542,25 @@ struct RowThreads {
     };
     walk(root->body);
     if (!ok || !reduces || longest == 0 || bytes == 0) return false;
-    // (a launch of four wavefronts per SIMD or less starts all of them at once: nothing to gain)
-    if (rows * (threads / WAVE_SIZE) <= 4096) return false;
-    // At least 24 bytes of the row per thread: 16384 rows of 1000 floats 27.6 us on 512 threads, 20.0 / 20.8 / 21.5 on
-    // 256 / 128 / 64 (softmax); 1000 halves 20.2 us on 256 threads, 15.0 on 64; 300 doubles 23.6 and 14.7; sums of 20000
-    // rows of 300 floats 31.4 us on 1024 threads, 14.4 on 64.
-    int64_t want = WAVE_SIZE;
-    while (want * 2 * 24 <= longest * bytes) want *= 2;
-    want = std::min(want, threads);
+    int64_t want = threads;
+    if (rows * (threads / WAVE_SIZE) > 4096) {
+      // At least 24 bytes of the row per thread: 16384 rows of 1000 floats 27.6 us on 512 threads, 20.0 / 20.8 / 21.5 on
+      // 256 / 128 / 64 (softmax); 1000 halves 20.2 us on 256 threads, 15.0 on 64; 300 doubles 23.6 and 14.7; sums of 20000
+      // rows of 300 floats 31.4 us on 1024 threads, 14.4 on 64.
+      want = WAVE_SIZE;
+      while (want * 2 * 24 <= longest * bytes) want *= 2;
+      want = std::min(want, threads);
+    } else {
+      // A launch of less than two wavefronts per SIMD, and rows of four 16-byte vectors per thread and more: twice the
+      // threads, and again.  Sums of one row of 100000 floats 15.8 us on 64 threads, 5.0 on 1024; of 30 such rows 19.1 and 5.9; of 100
+      // rows of 150000 29.5 us on 128, 13.7 on 1024; softmax over 300 rows of 30000 doubles 75 us on 256, 39 on 512.
+      // (With a limit of four per SIMD 300 rows of 100000 took 23.9 us instead of 22.2.)
+      while (!strided && want < 1024 && rows * (want / WAVE_SIZE) < 2048 && longest * bytes >= 64 * want) want *= 2;
+    }
     // Workgroups start at about two per nanosecond, which is what small ones wait for: four rows each where a row is a
     // wavefront's (the sums above 7.1 us, 6.7 with eight; softmax over 30000 rows of 200 floats 16.0 -> 8.7 us).
-    const int64_t group = want == WAVE_SIZE ? 4 : 1;
+    // (a launch of four wavefronts per SIMD or less starts all of them at once)
+    const int64_t group = want == WAVE_SIZE && rows > 4096 ? 4 : 1;
     if (want == threads && group == 1) return false;
     std::function<Stmts(const Stmts&)> cut = [&](const Stmts& ss) {
       Stmts out;

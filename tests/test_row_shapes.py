@@ -60,6 +60,21 @@ def test_rows_of_all_lengths(n, threads, dtype, tol):
 parpy_centred = parpy.jit(centred)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 4e-3), (torch.float32, 1e-5), (torch.float64, 1e-12)], ids=["f16", "f32", "f64"])
+def test_few_long_rows_get_more_threads(dtype, tol):
+    for n, m, threads in ((1, 8191, 64), (3, 20003, 64), (7, 4100, 128), (500, 33000, 128)):
+        x = torch.rand((n, m), device="cuda", dtype=torch.float32).to(dtype)
+        y = torch.empty_like(x)
+        sums = torch.zeros(n, device="cuda", dtype=dtype)
+        W.sum_rows(x, sums, n, opts=opts(n, threads))
+        assert torch.allclose(sums.double(), x.double().sum(1), rtol=tol), (n, m)
+        W.softmax(x, n, m, y, opts=opts(n, threads))
+        e = torch.exp(x.double() - x.double().max(1, keepdim=True).values)
+        want = e / e.sum(1, keepdim=True)
+        assert ((y.double() - want).norm() / want.norm()) < tol, (n, m)
+
+
 @parpy.jit
 def quotient(a, b, out):
     parpy.label('N')
