@@ -399,7 +399,7 @@ struct Options {  // src/option.rs:14-108
   bool opt_if_convert = true;       // branches that only assign cheap scalar values become selects
   bool opt_drop_barriers = true;   // barriers between regions that share no written array are removed
   bool opt_lane_split = true;      // eight lanes share each long per-thread dot product
-  bool opt_nontemporal = true;   // non-temporal stores to arrays a kernel only writes
+  bool opt_nontemporal = true;   // non-temporal stores to arrays a kernel only writes, loads of large arrays it reads once
   bool opt_guard_bounds = true;       // `for t: if t < X: work` with X fixed and uniform runs to min(hi, X) without the test
   bool opt_prefetch_steps = true;     // loads indexed by the counter of a barrier-stepped loop are issued one step ahead
   bool opt_pack_accesses = true;      // four adjacent 4-byte accesses of one iteration become one 16-byte access
@@ -430,6 +430,7 @@ struct Kernel {
   Dim3 grid, block;
   int64_t lds_bytes = 0;
   bool aligned_params = false;  // every pointer argument is 16-byte aligned (checked by the caller)
+  std::set<Name> read_once;     // large inputs of which the launch reads every element once: non-temporal loads
   bool cached_stores = false;   // what this kernel writes is read by the next one: no non-temporal stores
   bool opaque_body = false;     // the body is a call of a device helper: parameters are described by the creator
   bool no_restrict = false;     // workgroups exchange data through the parameters during the kernel: no no-alias promise

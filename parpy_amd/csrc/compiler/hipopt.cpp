@@ -52,6 +52,9 @@ namespace parpy {
 
 void hip_optimize(Program& p, const Options& opts, NameGen& gen) {
   if (opts.opt_gather_transpose) hipopt::gather_transpose(p, opts, gen);
+  if (opts.opt_nontemporal)
+    for (auto& k : p.kernels)
+      if (!k.opaque_body) hipopt::Pass(k, opts, gen).mark_read_once();
   if (opts.opt_tile_steps && !opts.persistent_loops) hipopt::time_tile(p, opts, gen);
   if (opts.opt_vectorize) hipopt::reduction_stages(p, opts, gen);
   if (opts.opt_lane_split) hipopt::ragged_sum(p, opts, gen);

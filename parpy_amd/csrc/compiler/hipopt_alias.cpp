@@ -161,5 +161,79 @@ void Pass::mark_read_only() {
   for (auto& p : k.params) p.read_only = p.ty.is_pointer() && !written.count(p.id);
 }
 
+// Large inputs whose elements a launch reads once each.  One access in the kernel, each of its dimensions indexed by a
+// loop of its own, every loop around it one of these or a division of one of these into shares: nothing is read again
+// that a cache could keep, and reads from HBM are faster with non-temporal loads (10 rows of 10^7 floats 69.9 -> 64.8 us,
+// 1024 of 65536 45.2 -> 42.2; a plain reading kernel reaches 6.0 and 6.75 TB/s).  Only from the 256 MB on that the
+// memory-side cache holds: a smaller array that has just been written or read is found there or in L2, and non-temporal
+// loads are the slower ones then (1000 rows of 20000 floats, 80 MB: 14.8 and 17.2 us, read again and again 12.2 and 15.0;
+// 2000 of 10000 doubles, 160 MB: 27.4 and 26.1, 22.9 and 23.7; at 256 MB read again and again 39.3 and 40.2).  And only in
+// kernels that write little: a copy of 200 MB takes 76 and 71 us from HBM, but 50 and 69 between the same two arrays.
+void Pass::mark_read_once() {
+  struct Site { int count = 0; bool ok = false; int64_t bytes = 0; };
+  std::map<Name, Site> reads;
+  int64_t stored = 0;
+  std::set<Name> barred;   // written, aliased or handed to a call
+  auto size = [](const E& x) {
+    int64_t n = elem_bytes(x->ty.sz);
+    for (int64_t d : x->dim_shape) n *= d;
+    return n;
+  };
+  std::vector<S> loops;
+  bool seen_while = false;
+  auto once = [&](const E& x) {
+    if (seen_while || x->dim_idx.empty() || x->dim_idx.size() != x->dim_shape.size() || x->ty.sz == ElemSize::Bool) return false;
+    std::set<Name> used;
+    for (E d : x->dim_idx) {
+      while (d->k == Expr::Convert) d = d->args[0];
+      if (d->k != Expr::Var || !used.insert(d->name).second) return false;
+    }
+    // innermost first: a loop counts when its variable indexes a dimension or bounds a loop that counts
+    for (size_t q = loops.size(); q-- > 0;) {
+      if (!used.count(loops[q]->id)) return false;
+      for (const E& b : {loops[q]->lo, loops[q]->hi})
+        visit_exprs(b, [&](const E& y) { if (y->k == Expr::Var) used.insert(y->name); });
+    }
+    return true;
+  };
+  auto scan = [&](const E& root, bool is_dst) {
+    if (!root) return;
+    visit_exprs(root, [&](const E& x) {
+      if (x->k == Expr::Index && x->args[0]->k == Expr::Var) {
+        if (is_dst && x == root) { barred.insert(x->args[0]->name); stored = std::max(stored, size(x)); return; }
+        Site& s = reads[x->args[0]->name];
+        s.ok = ++s.count == 1 && once(x);
+        s.bytes = size(x);
+      }
+      if (x->k == Expr::AddrOf || x->k == Expr::Call || x->k == Expr::Raw)
+        for (auto& a : x->args) visit_exprs(a, [&](const E& y) { if (y->k == Expr::Var && !y->ty.is_scalar()) barred.insert(y->name); });
+    });
+  };
+  std::function<void(const Stmts&)> walk = [&](const Stmts& ss) {
+    for (auto& s : ss) {
+      scan(s->dst, s->k == Stmt::Assign);
+      scan(s->expr, false);
+      scan(s->lo, false);
+      scan(s->hi, false);
+      if ((s->k == Stmt::Def && !s->ty.is_scalar()) || (s->k == Stmt::Assign && s->dst->k == Expr::Var && !s->dst->ty.is_scalar()))
+        visit_exprs(s->expr, [&](const E& y) { if (y->k == Expr::Var) barred.insert(y->name); });
+      const bool outer = seen_while;
+      seen_while = seen_while || s->k == Stmt::While;
+      if (s->k == Stmt::For) loops.push_back(s);
+      walk(s->body);
+      walk(s->els);
+      if (s->k == Stmt::For) loops.pop_back();
+      seen_while = outer;
+    }
+  };
+  walk(k.body);
+  k.read_once.clear();
+  for (auto& p : k.params) {
+    auto r = reads.find(p.id);
+    if (!p.ty.is_pointer() || r == reads.end() || !r->second.ok || barred.count(p.id)) continue;
+    if (r->second.bytes >= (int64_t(256) << 20) && stored <= r->second.bytes / 8) k.read_once.insert(p.id);
+  }
+}
+
 }  // namespace hipopt
 }  // namespace parpy

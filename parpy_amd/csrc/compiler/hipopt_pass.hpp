@@ -129,12 +129,13 @@ struct Pass {
   std::set<Name> lds_array_names() const;
   Stmts keep_in_iteration(const Stmts& B, int64_t* budget, const S& seq_loop, Stmts* pre);
 
-  // hipopt_alias.cpp: what the target compiler may assume about pointers: distinct arrays, read-only parameters
+  // hipopt_alias.cpp: what the target compiler may assume about pointers: distinct arrays, read-only parameters, inputs that stream through
   static bool is_alias_type(const Type& t);
   static bool alias_target(const E& e, const AliasCfg& cfg, Name* out);
   static bool apply_alias_stmt(const S& st, std::vector<AliasCfg>& cfgs, std::vector<Name>& order);
   Stmts noalias_scopes(const Stmts& ss, bool wrap);
   void mark_read_only();
+  void mark_read_once();
 };
 
 // ---- rewrites of the whole program (they change a launch)

@@ -438,6 +438,10 @@ struct DevicePrinter {
     if (base->ty.mem == Mem::LDS || elem_bytes(e->ty.sz) < 4) return false;
     return !read_only_param(base);
   }
+  // an element of an input that the launch reads once
+  bool streams_in(const E& e) const {
+    return kernel && e->args[0]->k == Expr::Var && kernel->read_once.count(e->args[0]->name) && read_only_param(e->args[0]);
+  }
 
   // fp32 values that come straight from memory (a load, or a variable that only names one): what the compiler
   // would have to quiet before a max / min; maxima and minima of such values count as well, since they are
@@ -653,6 +657,7 @@ struct DevicePrinter {
         // unit or a die), so the barrier itself needs no cache write-back or invalidation.
         if (exchanged(e) && !as_lvalue)
           return "__hip_atomic_load(&" + out + ", __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)";
+        if (!as_lvalue && streams_in(e)) return "__builtin_nontemporal_load(&" + out + ")";
         return out;
       }
       case Expr::AddrOf: return "(&" + pexpr(e->args[0]) + "[" + pexpr(e->args[1]) + "])";
@@ -1202,7 +1207,7 @@ struct DevicePrinter {
       pk.first = acc[first].pos;
       pk.last = acc[last].pos;
       pk.owner = &ss;
-      pk.streamed = a0.store && stream_out.count(a0.base) > 0;   // write-once data keeps bypassing the caches
+      pk.streamed = a0.store ? stream_out.count(a0.base) > 0 : streams_in(e0);   // write-once data keeps bypassing the caches
       pk.decl_ty = std::string("parpy_vec4<") + elem_ctype(e0->ty.sz) + ">";
       as_lvalue = true;
       std::string elem = pexpr(e0);
@@ -1236,6 +1241,7 @@ struct DevicePrinter {
       for (size_t p = first_pack; p < packs.size(); ++p)
         if (packs[p].owner == &ss && packs[p].first == i) {
           if (packs[p].is_store) os << ind(n) << packs[p].decl_ty << " " << packs[p].var << ";\n";
+          else if (packs[p].streamed) os << ind(n) << "const " << packs[p].decl_ty << " " << packs[p].var << " = __builtin_nontemporal_load(" << packs[p].addr << ");\n";
           else os << ind(n) << "const " << packs[p].decl_ty << " " << packs[p].var << " = *" << packs[p].addr << ";\n";
         }
       {
