@@ -285,11 +285,17 @@ template <class T, int ROWS, int COLS> __device__ __forceinline__ void parpy_tra
   __shared__ T tile[64][65];
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   const int c0 = (int)blockIdx.x * 64, r0 = (int)blockIdx.y * 64;
+  // (past the edges the last row and column are read again: tests around the loads would let one go at a time)
+  T v[16];
   #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    const int r = r0 + j * 4 + ty, c = c0 + tx;
-    if ((ROWS % 64 == 0 || r < ROWS) && (COLS % 64 == 0 || c < COLS)) tile[j * 4 + ty][tx] = src[(long long)r * COLS + c];
+    int r = r0 + j * 4 + ty, c = c0 + tx;
+    if (ROWS % 64 != 0 && r >= ROWS) r = ROWS - 1;
+    if (COLS % 64 != 0 && c >= COLS) c = COLS - 1;
+    v[j] = src[(long long)r * COLS + c];
   }
+  #pragma unroll
+  for (int j = 0; j < 16; ++j) tile[j * 4 + ty][tx] = v[j];
   __syncthreads();
   #pragma unroll
   for (int j = 0; j < 16; ++j) {
