@@ -139,6 +139,65 @@ struct Restructure {
     return out;
   }
 
+  // ---- 0. a few long rows: several workgroups each
+  // Rows that are reduced by a workgroup each leave compute units idle when there are fewer rows than those, and one
+  // workgroup reads 50 to 80 GB/s at best.  Such a reduction, alone under its loops, is asked for on as many workgroups of
+  // 256 threads as make four for every compute unit, up to 128 per row, with eight 16-byte vectors per thread and more.
+  // Handing over the partial results costs 1 to 3 us, so only for rows of 320 KB, and of 8 KB for each row there is: one
+  // row of 190000 doubles 15.8 -> 3.8 us, 30 of 150001 doubles 19.3 -> 14.0, 30 of 100000 floats 7.9 -> 6.8, 100 of 1000001
+  // floats 143 -> 69 (on 256 threads asked for; the whole workgroup of 1024 that a program asks for by that number it
+  // gets, one workgroup and no more: the shape that the row-sum example compares with several); but 30 of 40000 floats 4.6 -> 5.5, 100 of 150000 13.3 -> 16.3, 255 of 390000 65.4 -> 67.9.
+  static int64_t literal_extent(const S& s) {
+    return s->step == 1 && s->lo->k == Expr::Int && s->lo->iv == 0 && s->hi->k == Expr::Int ? s->hi->iv : 0;
+  }
+  S spread_row(const S& s, int64_t rows) {
+    const int64_t n = literal_extent(s);
+    if (!is_par_for(s) || s->par.reduction || n <= 0 || s->par.nthreads != n || s->par.tpb != DEFAULT_TPB) return s;
+    rows *= n;
+    if (rows >= 256) return s;
+    size_t at = s->body.size();
+    for (size_t q = 0; q < s->body.size(); ++q) {
+      const S& b = s->body[q];
+      if (b->k == Stmt::For) {
+        if (at < s->body.size()) return s;
+        at = q;
+      } else if (!((b->k == Stmt::Def && b->ty.is_scalar()) || b->k == Stmt::Assign)) {
+        return s;
+      }
+    }
+    if (at == s->body.size()) return s;
+    const S& b = s->body[at];
+    S inner = b;
+    if (!b->par.reduction) {
+      if (s->body.size() != 1) return s;
+      inner = spread_row(b, rows);
+    } else if (b->par.is_parallel() && b->par.tpb == DEFAULT_TPB && b->par.nthreads < DEFAULT_TPB && literal_extent(b) > 0) {
+      E lhs, rhs;
+      BinOp op;
+      ElemSize sz;
+      extract_reduction(b, &lhs, &op, &rhs, &sz);
+      if (elem_bytes(sz) < 4) return s;   // (partial results of halves would be rounded)
+      const int64_t bytes = literal_extent(b) * elem_bytes(sz), vectors = bytes / 16;
+      if (bytes < std::max<int64_t>(320000, rows * 8192)) return s;
+      int64_t blocks = 1;
+      while (blocks < 128 && rows * blocks < 1024 && vectors / (2 * blocks * 256) >= 8) blocks *= 2;
+      if (blocks < 2) return s;
+      auto r = clone(b);
+      r->par.tpb = 256;
+      r->par.nthreads = 256 * blocks;
+      inner = r;
+    }
+    if (inner == b) return s;
+    auto r = clone(s);
+    r->body[at] = inner;
+    return r;
+  }
+  Stmts spread_rows(const Stmts& ss) {
+    Stmts out;
+    for (auto& s : ss) out.push_back(spread_row(s, 1));
+    return out;
+  }
+
   // ---- 3. multi-block reductions (inter_block.rs:150-433)
   static BinOp non_short_circuit(BinOp op) { return op == BinOp::And ? BinOp::BitAnd : op == BinOp::Or ? BinOp::BitOr : op; }
 
@@ -659,7 +718,7 @@ struct Restructure {
 
  public:
   Stmts run(const Stmts& body0, const std::vector<Param>& params) {
-    Stmts body = insert_sync(body0);
+    Stmts body = insert_sync(opts.opt_vectorize && !opts.persistent_loops ? spread_rows(body0) : body0);
     body = classify(body);
     body = split_reductions(body);
     body = hoist(body);

@@ -50,3 +50,27 @@ def test_planes_and_neighbouring_loops(k):
     parpy.jit(scaled_row_sums)(x, y, out, 5, k, opts=opts(5, 4096))
     want = x.double() * 2.0 + 1.0
     assert torch.allclose(out.double(), want.sum(1), rtol=1e-5) and torch.allclose(y.double(), want / want.sum(1, keepdim=True), rtol=2e-5)
+
+
+def test_a_few_long_rows_take_several_workgroups():
+    # (rows, row length, element type) and whether one workgroup per row is enough
+    for n, m, dtype, spread in ((1, 100000, np.float32, True), (1, 79999, np.float32, False), (30, 100001, np.float32, True), (3, 40000, np.float64, True),
+                                (64, 100000, np.float32, False), (64, 131072, np.float32, True), (3, 200000, np.float16, False)):
+        x, out = np.zeros((n, m), dtype=dtype), np.zeros(n, dtype=dtype)
+        s = parpy.print_compiled(sum_rows, [x, out, n], opts(n, 256))
+        assert s.count("<<<") == 1 and ("parpy_last_workgroup(" in s.split("extern", 1)[1]) == spread, (n, m, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tol", [(torch.int32, 0.0), (torch.float32, 1e-5), (torch.float64, 1e-12)], ids=["i32", "f32", "f64"])
+@pytest.mark.parametrize("n,m", [(1, 80000), (1, 100001), (2, 1000003), (31, 163841), (64, 262147), (127, 300002)])
+def test_a_few_long_rows(n, m, dtype, tol):
+    x = torch.randint(1, 100, (n, m), device="cuda").to(dtype)
+    for call in range(2):
+        for threads in (64, 512):
+            out = torch.full((3, n), -1, device="cuda", dtype=dtype)
+            for f, o in ((sum_rows, out[0]), (max_rows, out[1]), (min_rows, out[2])):
+                parpy.jit(f)(x, o, n, opts=opts(n, threads))
+            assert torch.allclose(out[0].double(), x.double().sum(1), rtol=tol, atol=0.0), (threads, call)
+            assert torch.equal(out[1], x.max(1).values) and torch.equal(out[2], x.min(1).values), (threads, call)
+        x[:, -1] += 150
