@@ -168,7 +168,8 @@ void Pass::mark_read_only() {
 // memory-side cache holds: a smaller array that has just been written or read is found there or in L2, and non-temporal
 // loads are the slower ones then (1000 rows of 20000 floats, 80 MB: 14.8 and 17.2 us, read again and again 12.2 and 15.0;
 // 2000 of 10000 doubles, 160 MB: 27.4 and 26.1, 22.9 and 23.7; at 256 MB read again and again 39.3 and 40.2).  And only in
-// kernels that write little: a copy of 200 MB takes 76 and 71 us from HBM, but 50 and 69 between the same two arrays.
+// kernels that write little and gather nothing: five million indices and values of a sparse product 38.9 us with plain
+// loads, 49.0 with these (rows share lines), 671744 sampled products 33.6 and 37.5; a copy of 200 MB takes 76 and 71 us from HBM, but 50 and 69 between the same two arrays.
 void Pass::mark_read_once() {
   struct Site { int count = 0; bool ok = false; int64_t bytes = 0; };
   std::map<Name, Site> reads;
@@ -180,7 +181,9 @@ void Pass::mark_read_once() {
     return n;
   };
   std::vector<S> loops;
-  bool seen_while = false;
+  bool seen_while = false, gathers = false;
+  std::set<Name> loop_vars;
+  visit_stmts(k.body, [&](const S& s) { if (s->k == Stmt::For) loop_vars.insert(s->id); });
   auto once = [&](const E& x) {
     if (seen_while || x->dim_idx.empty() || x->dim_idx.size() != x->dim_shape.size() || x->ty.sz == ElemSize::Bool) return false;
     std::set<Name> used;
@@ -191,6 +194,7 @@ void Pass::mark_read_once() {
     // innermost first: a loop counts when its variable indexes a dimension or bounds a loop that counts
     for (size_t q = loops.size(); q-- > 0;) {
       if (!used.count(loops[q]->id)) return false;
+      if (has_load(loops[q]->lo) || has_load(loops[q]->hi)) return false;
       for (const E& b : {loops[q]->lo, loops[q]->hi})
         visit_exprs(b, [&](const E& y) { if (y->k == Expr::Var) used.insert(y->name); });
     }
@@ -199,6 +203,7 @@ void Pass::mark_read_once() {
   auto scan = [&](const E& root, bool is_dst) {
     if (!root) return;
     visit_exprs(root, [&](const E& x) {
+      if (x->k == Expr::Index) visit_exprs(x->args[1], [&](const E& y) { if (y->k == Expr::Index || (y->k == Expr::Var && !loop_vars.count(y->name))) gathers = true; });
       if (x->k == Expr::Index && x->args[0]->k == Expr::Var) {
         if (is_dst && x == root) { barred.insert(x->args[0]->name); stored = std::max(stored, size(x)); return; }
         Site& s = reads[x->args[0]->name];
@@ -228,6 +233,7 @@ void Pass::mark_read_once() {
   };
   walk(k.body);
   k.read_once.clear();
+  if (gathers) return;
   for (auto& p : k.params) {
     auto r = reads.find(p.id);
     if (!p.ty.is_pointer() || r == reads.end() || !r->second.ok || barred.count(p.id)) continue;

@@ -32,6 +32,19 @@ def scaled(x, out, N):
         out[i] = 1.0
 
 
+def between(x, out, first, N):
+    parpy.label('outer')
+    for i in range(N):
+        for j in range(first[i], first[i + 1]):
+            out[i] += x[j]
+
+
+def picked(x, out, first, N):
+    parpy.label('outer')
+    for i in range(N):
+        out[first[i]] = x[i]
+
+
 def opts(n, m):
     return parpy.par({'outer': parpy.threads(n), 'inner': parpy.threads(m)})
 
@@ -50,6 +63,12 @@ def test_which_inputs_stream(f, n, m, threads, streams):
     plain = opts(n, threads)
     plain.opt_nontemporal = False
     assert "__builtin_nontemporal_load(" not in parpy.print_compiled(f, args, plain)
+
+
+@pytest.mark.parametrize("f", [between, picked])
+def test_sums_over_data_do_not_stream(f):
+    args = [np.zeros(1 << 26, dtype=np.float32), np.zeros(1 << 10, dtype=np.float32), np.zeros((1 << 10) + 1, dtype=np.int64), 1 << 10]
+    assert "__builtin_nontemporal_load(" not in parpy.print_compiled(parpy.jit(f), args, opts(1 << 10, 64))
 
 
 @pytest.mark.gpu
