@@ -27,7 +27,7 @@ namespace {
 // flight 547 us, in teams 39 us.  Five million 8-byte gathers out of L2 are then what bounds it: 128 lines per
 // nanosecond, the rate at which random lines come out of L2 on this part.  20 000 rows of 24 on average (longest 3400)
 // times a 128-column matrix: one workgroup per row with the sum read and written back in LDS per element 840 us, in
-// teams 42 us: the workgroups that share the longest rows pull 1.7 MB each through one compute unit.
+// teams 42 us, with the longest rows first (below) 33: they pull 1.7 MB each through one compute unit.
 struct RaggedSum {
   Program& p;
   const Options& opts;
@@ -250,6 +250,15 @@ struct RaggedSum {
     // and the waves that have no such row wait for it: 256 elements for single sums (128 costs 5 to 20 %), fewer when
     // every element moves a row of columns (64 against 256 elements: 17.4 and 20.1 us for the 32-column product above).
     const int64_t longest = r.has_col ? std::max<int64_t>(64, 2 * avg) : std::max<int64_t>(256, 4 * avg);
+    // A launch of more wavefronts than run at once starts its rows one after the other, and the longest may start last.
+    // Where rows of columns are moved, 256 workgroups in front of the others look for rows that stand out by another factor
+    // of four and share each of them as above; the teams pass those by.  20 000 rows of 24 on average times 128 columns:
+    // 41.5 -> 33.3 us (rows of equal length 24.6 and 24.8), 20 000 of 20 times 99: 43.0 -> 32.1, 100 000 of 15 times 64:
+    // 73 -> 61; 2 and 8 instead of 4 measure 33.6 and 37.7 on the first, 1024 workgroups 34.5.  Without columns the
+    // longest row is over before the last rows have started (38.9 and 38.5 us; 10^6 rows of 10 124.7 and 127.1).
+    const int64_t huge = 4 * longest;
+    const int64_t scouts = r.has_col && r.n * T > 256 * 2048 ? std::max<int64_t>(256, (r.n + 1023) / 1024) : 0;
+    const int64_t looked = scouts ? (r.n + scouts - 1) / scouts : 0;   // rows for each of them
     // element numbers in 32 bits when the array they walk is known to be small enough
     const bool small = r.elements > 0 && r.elements < (int64_t(1) << 29);
     const ElemSize esz = small && isz == ElemSize::I64 ? ElemSize::I32 : isz;
@@ -382,7 +391,7 @@ struct RaggedSum {
       d->k = Stmt::LdsDecl;
       d->id = queue;
       d->ty = Type::scalar(ElemSize::I32);
-      d->iv = teams;
+      d->iv = std::max(teams, looked);
       top.push_back(d);
       auto e = std::make_shared<Stmt>(*d);
       e->id = count;
@@ -397,7 +406,9 @@ struct RaggedSum {
     E lv = mk_var(lane, ity), qv = mk_var(q, ity);
     {
       Stmts body;
-      body.push_back(mk_def(r.row, ity, mk_binop(BinOp::FloorDiv, lv, iint(T), ity), r.loop->i));
+      E team = mk_binop(BinOp::FloorDiv, lv, iint(T), ity);
+      if (scouts) team = mk_binop(BinOp::Max, mk_binop(BinOp::Sub, team, iint(scouts * teams), ity), iint(0), ity);   // (known not to be negative)
+      body.push_back(mk_def(r.row, ity, team, r.loop->i));
       body.push_back(mk_def(q, ity, mk_binop(BinOp::Rem, lv, iint(T), ity), r.loop->i));
       E lo, hi;
       bounds(body, &lo, &hi);
@@ -413,18 +424,31 @@ struct RaggedSum {
       Stmts f = finish_slots(l);
       if (P > 1) own.push_back(mk_if(mk_binop(BinOp::Lt, qv, iint(L), bty), f, {}));
       else own.insert(own.end(), f.begin(), f.end());
-      Stmts defer{mk_if(mk_binop(BinOp::Eq, qv, iint(0), bty),
-                        {mk_rawstmt(queue.str() + "[atomicAdd(&" + count.str() + "[0], 1)] = (int)" + r.row.str() + ";")}, {})};
+      const S enqueue = mk_rawstmt(queue.str() + "[atomicAdd(&" + count.str() + "[0], 1)] = (int)" + r.row.str() + ";");
+      auto longer = [&](const E& a, const E& b) { return mk_binop(BinOp::Gt, mk_binop(BinOp::Sub, b, a, ety), eint(huge), bty); };
+      Stmts defer{mk_if(mk_binop(BinOp::Eq, qv, iint(0), bty), {scouts ? mk_if(longer(lo, hi), {}, {enqueue}) : enqueue}, {})};
       body.push_back(mk_if(mk_binop(BinOp::Leq, mk_binop(BinOp::Sub, hi, lo, ety), eint(longest), bty), own, defer));
       auto nr = clone(k.body[0]);
       nr->id = lane;
-      nr->hi = iint(r.n * T);
+      nr->hi = iint(r.n * T + scouts * tpb);
       nr->body = body;
+      if (scouts) {
+        Name at = gen.fresh(r.row.s + "_at"), slice = gen.fresh("slice");
+        const E first = mk_binop(BinOp::Mul, mk_var(slice, ity), iint(looked), ity);
+        Stmts look{mk_def(r.row, ity, mk_var(at, ity), r.loop->i)};
+        E a, b;
+        bounds(look, &a, &b);
+        look.push_back(mk_if(longer(a, b), {enqueue}, {}));
+        nr->body = {mk_if(mk_binop(BinOp::Lt, lv, iint(scouts * tpb), bty),
+                          {mk_def(slice, ity, mk_binop(BinOp::FloorDiv, lv, iint(tpb), ity)),
+                           mk_for(at, add(first, mk_binop(BinOp::Rem, lv, iint(tpb), ity)), mk_binop(BinOp::Min, add(first, iint(looked)), iint(r.n), ity), tpb, look, LoopPar(), r.loop->i)},
+                          body)};
+      }
       nr->els.clear();
       nr->map = GpuMap();
       nr->map.k = GpuMap::ThreadBlock;
       nr->map.tpb = tpb;
-      nr->map.n = (r.n * T + WAVE_SIZE - 1) / WAVE_SIZE * WAVE_SIZE;
+      nr->map.n = (r.n * T + scouts * tpb + WAVE_SIZE - 1) / WAVE_SIZE * WAVE_SIZE;
       top.push_back(nr);
     }
     top.push_back(mk_sync());
@@ -490,10 +514,10 @@ struct RaggedSum {
       }
       top.push_back(mk_for(h, iint(0), mk_raw("((int64_t)" + count.str() + "[0])", ity), 1, body, LoopPar()));
     }
-    k.lds_bytes += (teams + 1) * 4;
+    k.lds_bytes += (std::max(teams, looked) + 1) * 4;
     k.body = top;
     k.block = Dim3{tpb, 1, 1};
-    k.grid = Dim3{(r.n + teams - 1) / teams, 1, 1};
+    k.grid = Dim3{(r.n + teams - 1) / teams + scouts, 1, 1};
     launch->grid = k.grid;
     launch->block = k.block;
     return true;

@@ -108,3 +108,38 @@ def test_start_value_of_a_shared_sum_counts_once():
     out = np.zeros(300, dtype=np.float32)
     parpy.jit(fixed_length)(x, out, 300, 132, opts=opts_for({'i': parpy.threads(300)}))
     assert np.allclose(out, 3.0 + x.astype(np.float64).sum(1), atol=1e-4)
+
+
+def outliers(n, dtype, long, seed):
+    """Short rows and, at the places given, rows around and beyond the length that workgroups of their own look for."""
+    rng = np.random.default_rng(seed)
+    lens = rng.integers(0, 8, size=n)
+    for row, length in long.items():
+        lens[row] = length
+    rows = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    return {"values": rng.standard_normal(rows[-1]).astype(dtype), "rows": rows, "cols": rng.integers(0, 300, rows[-1]).astype(np.int64), "nrows": n}
+
+
+LONG = {0: 20000, 1: 1024, 2: 1025, 3: 1026, 77: 256, 78: 257, 79: 64, 80: 65, 81: 258, 5000: 4097, 5001: 4096, 5002: 4095, 60001: 12345, -2: 3000, -1: 9999}
+
+
+def test_outliers_are_looked_for_where_not_all_rows_run_at_once():
+    for n, found in ((8192, False), (8193, True)):   # (a wavefront per row)
+        A, z = outliers(n, np.float32, {}, 1), np.zeros(n, dtype=np.float32)
+        B = {"values": np.zeros((300, 33), dtype=np.float32), "ncols": 33}
+        s = parpy.print_compiled(columns, [A, B, np.zeros((n, 33), dtype=np.float32), z], opts_for({"i": parpy.threads(n), "j": parpy.threads(33)}))
+        assert ("slice_" in s) == found
+        hiprtc_compile(s[:s.index("// host side")], opts_for({}))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,cols", [(70000, 33), (8193, 33), (9001, 256), (17000, 128)])
+def test_outliers_with_columns(n, cols):
+    for long in ({k if k < n else n - 5: min(v, 5000) for k, v in LONG.items()}, {}, {n // 2: 20000}, {r: 300 for r in range(1000, 1200)}):
+        A = outliers(n, np.float32, long, n)
+        rng = np.random.default_rng(cols)
+        B, z, C = rng.standard_normal((300, cols)).astype(np.float32), rng.standard_normal(n).astype(np.float32), np.full((n, cols), np.nan, dtype=np.float32)
+        parpy.jit(columns)(A, {"values": B, "ncols": cols}, C, z, opts=opts_for({"i": parpy.threads(n), "j": parpy.threads(cols)}))
+        want = (0.5 * z[:, None] + row_sums(A, A["values"].astype(np.float64)[:, None] * B[A["cols"]])) * z[:, None] + 1.0
+        # (a sum of 20000 products of order one is off by 20000 * 2^-24 * 100 at the very most: 0.1; 5e-3 is what their random signs leave)
+        assert np.allclose(C, want, atol=5e-3)
