@@ -219,7 +219,10 @@ struct Stages {
     // threads: 29.5 us on 32 workgroups, 11.0 on 128, 13.7 on 256, 18.6 on 512 -- all of them count in one word).
     int64_t results = 1;
     for (auto& o : f.outer) results *= o->hi->iv;
-    while (nb < 128 && results * nb * threads < 2048 * WAVE_SIZE && vectors / (nb * threads) >= 16) { split *= 2; nb *= 2; }
+    // Workgroups of fewer than 256 threads are there only because the program names that size: the split it names with it,
+    // two launches and the temporary between them (which callers of the entry without allocations make room for) stay.
+    const bool named = threads < 256;
+    while (!named && nb < 128 && results * nb * threads < 2048 * WAVE_SIZE && vectors / (nb * threads) >= 16) { split *= 2; nb *= 2; }
     const int64_t share = (vectors + nb - 1) / nb;
     const E bv = mk_var(f.blocks->id, ity);
     auto mapped = [&](const Name& id, E lo, E hi, const Stmts& body) {
@@ -270,7 +273,7 @@ struct Stages {
     // workgroup takes the value itself, the initialising stores disappear.  (Workgroups on different dies must not store
     // to one element.)  From five elements per thread on; with fewer, a share is little more than one access, the time
     // is that of the launches themselves and both forms stay as they are.
-    bool fuse = f.elements >= 5 * nb * threads && elem_bytes(f.reduce->ty.sz) >= 4 && !opts.persistent_loops;
+    bool fuse = !named && f.elements >= 5 * nb * threads && elem_bytes(f.reduce->ty.sz) >= 4 && !opts.persistent_loops;
     std::vector<std::pair<E, E>> known;   // element -> value
     std::map<Name, E> defs;
     for (auto& b : f.prefix) {

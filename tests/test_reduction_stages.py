@@ -52,6 +52,12 @@ def test_planes_and_neighbouring_loops(k):
     assert torch.allclose(out.double(), want.sum(1), rtol=1e-5) and torch.allclose(y.double(), want / want.sum(1, keepdim=True), rtol=2e-5)
 
 
+def test_a_split_with_small_workgroups_stays_as_it_is_named():
+    x, out = np.zeros((100, 65536), dtype=np.float32), np.zeros(100, dtype=np.float32)
+    s = parpy.print_compiled(sum_rows, [x, out, 100], parpy.par({'outer': parpy.threads(100), 'inner': parpy.threads(1024).tpb(128)}))
+    assert s.count("<<<") == 2 and "parpy_alloc_buffer(3200)" in s
+
+
 def test_a_few_long_rows_take_several_workgroups():
     # (rows, row length, element type) and whether one workgroup per row is enough
     for n, m, dtype, spread in ((1, 100000, np.float32, True), (1, 79999, np.float32, False), (30, 100001, np.float32, True), (3, 40000, np.float64, True),
