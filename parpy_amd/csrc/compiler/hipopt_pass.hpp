@@ -29,6 +29,12 @@ int64_t per_thread_trips(const S& loop);                  // iterations every th
 E counter_var(const S& loop, ElemSize isz);               // the per-thread iteration counter of a mapped loop as the printer names it
 E subst_vars(const E& e, const std::map<Name, E>& m);
 
+// operand q of e may be left unevaluated (the branches of a selection, the right side of `and` / `or`): an index in it
+// need only be in bounds where it is evaluated, so nothing may be loaded from there ahead of the test
+inline bool may_skip(const E& e, size_t q) {
+  return q > 0 && (e->k == Expr::IfExpr || (e->k == Expr::BinOpE && (e->bop == BinOp::And || e->bop == BinOp::Or)));
+}
+
 template <class F> E rewrite_expr(const E& e, F f) {  // bottom-up rewrite
   if (!e) return e;
   E r = map_children(e, [&](const E& c) { return rewrite_expr(c, f); });

@@ -51,6 +51,7 @@ struct RaggedSum {
     E acc, term, start;       // accumulator, summand, value the sum starts from
     Stmts post;               // statements after the sum
     int64_t elements = 0;     // length of the array that the loop variable walks, 0 when there is none
+    bool bounded = false;     // the loop variable stays below it (not when all its accesses are under tests)
     int64_t tpb = 0;          // threads per workgroup
     bool one_group = false;   // the launch was a single workgroup
   };
@@ -83,19 +84,22 @@ struct RaggedSum {
     const Name& acc_name = scalar_acc ? acc->name : acc->args[0]->name;
     bool ok = !mentions(term, acc_name) && !mentions(s->lo, acc_name) && !mentions(s->hi, acc_name);
     int loads = 0;
-    auto scan = [&](const E& e) {
-      visit_exprs(e, [&](const E& x) {
-        if (x->k == Expr::Call || x->k == Expr::AddrOf || x->k == Expr::Raw || x->k == Expr::RegElem) ok = false;
-        if (x->k != Expr::Index) return;
+    std::function<void(const E&, bool)> scan = [&](const E& x, bool always) {
+      if (x->k == Expr::Call || x->k == Expr::AddrOf || x->k == Expr::Raw || x->k == Expr::RegElem) ok = false;
+      E rest;
+      if (x->k == Expr::Index) {
         ++loads;
-        E rest;
-        if (x->dim_shape.size() == 1 && affine_unit(x->args[1], s->id, &rest) && rest->k == Expr::Int)
+        if (x->dim_shape.size() == 1 && affine_unit(x->args[1], s->id, &rest) && rest->k == Expr::Int) {
           r.elements = std::max(r.elements, x->dim_shape[0]);
-      });
+          r.bounded = r.bounded || always;
+        }
+      }
+      for (size_t q = 0; q < x->args.size(); ++q)
+        if (x->args[q]) scan(x->args[q], always && !may_skip(x, q));
     };
-    scan(term);
+    scan(term, true);
     for (size_t q = 0; q + 1 < s->body.size(); ++q) {
-      scan(s->body[q]->expr);
+      scan(s->body[q]->expr, true);
       if (mentions(s->body[q]->expr, acc_name)) ok = false;
     }
     if (!ok || loads < 1) return false;
@@ -260,7 +264,7 @@ struct RaggedSum {
     const int64_t scouts = r.has_col && r.n * T > 256 * 2048 ? std::max<int64_t>(256, (r.n + 1023) / 1024) : 0;
     const int64_t looked = scouts ? (r.n + scouts - 1) / scouts : 0;   // rows for each of them
     // element numbers in 32 bits when the array they walk is known to be small enough
-    const bool small = r.elements > 0 && r.elements < (int64_t(1) << 29);
+    const bool small = r.bounded && r.elements < (int64_t(1) << 29);
     const ElemSize esz = small && isz == ElemSize::I64 ? ElemSize::I32 : isz;
     const Type ety = Type::scalar(esz);
     auto eint = [&](int64_t v) { return mk_int(v, esz); };
@@ -309,22 +313,25 @@ struct RaggedSum {
       Stmts batch;
       batch.push_back(mk_def(at, ety, mk_binop(BinOp::Min, iv, mk_binop(BinOp::Sub, hi, eint(1), ety), ety), r.loop->i));
       std::map<Name, E> to_clamped{{r.loop->id, widen(atv)}};
-      // loaded values that select other elements get a name: an index is in bounds by contract, and a named one takes
-      // part in 32-bit address arithmetic
+      // Loaded values that select other elements get a name, which lets them take part in 32-bit address arithmetic.  A
+      // name is evaluated in front of the term whatever the term's tests say, so operands that a selection or a
+      // short-circuit operator may skip make none (`x[perm[c]] if c >= 0 else 0`: c may be anything where it is not used).
       std::vector<std::pair<E, Name>> named;
       auto bind = [&](const E& e0, Stmts& to) {
         E e = subst_vars(e0, to_clamped);
-        std::function<E(const E&, bool)> go = [&](const E& x, bool inside) -> E {
+        std::function<E(const E&, bool, bool)> go = [&](const E& x, bool inside, bool always) -> E {
           if (!x) return x;
-          E y = map_children(x, [&](const E& ch) { return go(ch, inside || x->k == Expr::Index); });
+          size_t q = 0;
+          E y = map_children(x, [&](const E& ch) { return go(ch, inside || x->k == Expr::Index, always && !may_skip(x, q++)); });
           if (!(inside && y->k == Expr::Index && is_int(y->ty.sz))) return y;
           for (auto& nv : named) if (expr_eq(nv.first, y)) return mk_var(nv.second, y->ty);
+          if (!always) return y;
           Name nm = gen.fresh("sel");
           named.push_back({y, nm});
           to.push_back(mk_def(nm, y->ty, y, r.loop->i));
           return mk_var(nm, y->ty);
         };
-        return go(e, false);
+        return go(e, false, true);
       };
       auto summand = [&](const E& c) {
         Stmts ss;

@@ -500,7 +500,7 @@ struct Pass::OwnIterations {
       return mk_var(n, e->ty, e->i);
     }
     // what a selection or a short-circuit operator may skip stays where it is (a test can guard an index)
-    if (e->k == Expr::IfExpr || (e->k == Expr::BinOpE && (e->bop == BinOp::And || e->bop == BinOp::Or))) {
+    if (may_skip(e, 1)) {
       auto n = std::make_shared<Expr>(*e);
       n->args[0] = lift(e->args[0]);
       return n;

@@ -42,6 +42,43 @@ def fixed_length(x, out, N, M):
         out[i] = t
 
 
+def padded(A, x, perm, y):
+    """Padding marked by -1, an index array that is shorter than the sums, and a test that is a load itself."""
+    parpy.label('row')
+    for row in range(A["nrows"]):
+        y[row] = 0.0
+        parpy.label('i')
+        for i in range(A["rows"][row], A["rows"][row + 1]):
+            y[row] += x[perm[A["cols"][i]]] if A["cols"][i] >= 0 else 0.0
+
+
+def summed(A, x, y):
+    parpy.label('row')
+    for row in range(A["nrows"]):
+        y[row] = 0.0
+        parpy.label('i')
+        for i in range(A["rows"][row], A["rows"][row + 1]):
+            y[row] += A["values"][i] * (x[i] if i < 100 else 0.0)
+
+
+def guarded(A, x, y):
+    parpy.label('row')
+    for row in range(A["nrows"]):
+        y[row] = 0.0
+        parpy.label('i')
+        for i in range(A["rows"][row], A["rows"][row + 1]):
+            y[row] += x[i] if i < 100 else 0.0
+
+
+def bounded(A, x, perm, y):
+    parpy.label('row')
+    for row in range(A["nrows"]):
+        y[row] = 0.0
+        parpy.label('i')
+        for i in range(A["rows"][row], A["rows"][row + 1]):
+            y[row] += x[A["cols"][perm[i]]] if i < 100 and perm[i] >= 0 and A["cols"][perm[i]] > 3 else 0.5
+
+
 def matrix(n, m, dtype, seed):
     """Row lengths: empty, one, around a team, around the longest row a team keeps, and one that dwarfs the rest."""
     rng = np.random.default_rng(seed)
@@ -76,6 +113,46 @@ def test_long_rows_are_queued_for_the_workgroup():
     s = parpy.print_compiled(columns, [A, B, np.zeros((5000, 64), dtype=np.float32), v], opts_for({"i": parpy.threads(5000), "j": parpy.threads(64)}))
     hiprtc_compile(s[:s.index("// host side")], opts_for({}))
     assert "parpy_team_sum<16, 64>" in s and "long_sums" in s
+
+
+def test_loads_under_a_test_stay_under_it():
+    """What a selection or a short-circuit operator may skip is not evaluated in front of the term: its index need not be one."""
+    import re
+    A, x, perm, y = matrix(5000, 300, np.float64, 1), np.zeros(300), np.zeros(300, dtype=np.int64), np.zeros(5000)
+    for f, skipped in ((padded, ("perm",)), (bounded, ("perm", "cols"))):
+        s = parpy.print_compiled(f, [A, x, perm, y], opts_for({"row": parpy.threads(5000)}))
+        s = s[:s.index("// host side")]
+        hiprtc_compile(s, opts_for({}))
+        kernel = s[s.rindex('extern "C"'):]
+        assert "parpy_block_reduce" in kernel    # (the form with teams of lanes)
+        for line in kernel.splitlines():
+            for name in skipped:
+                at, test = re.search(rf"parpy_at\(\w*{name}_\d+,|\w*{name}_\d+\[", line), re.search(r"\?|&&", line)
+                assert at is None or (test is not None and test.start() < at.start()), line
+
+
+def test_loop_variables_are_narrowed_by_arrays_that_every_element_reads():
+    """An array that is read under a test only says nothing about how far the rows go."""
+    A, x, y = matrix(5000, 300, np.float64, 1), np.zeros(100), np.zeros(5000)
+
+    def kernel(f):
+        s = parpy.print_compiled(f, [A, x, y], opts_for({"row": parpy.threads(5000)}))
+        return s[:s.index("// host side")]
+
+    assert "int32_t end_" in kernel(summed) and "int64_t end_" in kernel(guarded)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [65, 1025, 20001])
+def test_sums_of_padded_rows(n):
+    A = matrix(n, 300, np.float64, n)
+    rng = np.random.default_rng(n + 2)
+    A["cols"][rng.random(len(A["cols"])) < 0.3] = -1
+    x, perm, y = rng.standard_normal(300), rng.permutation(300).astype(np.int64), np.full(n, np.nan)
+    parpy.jit(padded)(A, x, perm, y, opts=opts_for({"row": parpy.threads(n)}))
+    want = row_sums(A, np.where(A["cols"] >= 0, x[perm[A["cols"]]], 0.0))
+    # (partial sums of the whole vector, at most 400000 terms of order one: 400000 * 2^-53 * 600 at the very most)
+    assert np.allclose(y, want, atol=1e-7)
 
 
 @pytest.mark.gpu
