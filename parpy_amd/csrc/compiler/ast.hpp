@@ -247,7 +247,7 @@ struct Stmt {
     Assign,     // dst = expr
     For,        // for id in lo..hi step: body  (labels / par)
     While,      // while expr: body
-    If,         // if expr: body else els
+    If,         // if expr: body else els (host: fname, when given, says what els stands for)
     WithGpu,    // with gpu: body
     CallStmt,   // fname(args)
     Label,      // fname = label text

@@ -1413,6 +1413,12 @@ struct PlanPrinter {
       case Expr::IfExpr: return "(ite " + hexpr(e->args[0]) + " " + hexpr(e->args[1]) + " " + hexpr(e->args[2]) + ")";
       case Expr::Convert: return std::string("(cvt ") + elem_tag(e->ty.sz) + " " + hexpr(e->args[0]) + ")";
       case Expr::Raw: return "(fits " + std::to_string(e->iv) + ")";   // whether temporaries of that many bytes can be had
+      case Expr::Call: {   // whether two stretches of memory, given by start and bytes, have nothing in common
+        if (e->sval != "parpy_disjoint") fail_rt(e->i, "Expression " + print_expr(e) + " is not supported in host code");
+        std::string r = "(disjoint";
+        for (auto& a : e->args) r += " " + hexpr(a);
+        return r + ")";
+      }
       case Expr::AddrOf: return "(addr " + hexpr(e->args[0]) + " " + hexpr(e->args[1]) + " " + std::to_string(elem_bytes(e->ty.sz)) + ")";
       default: fail_rt(e->i, "Expression " + print_expr(e) + " is not supported in host code");
     }
@@ -1527,7 +1533,11 @@ void list_host(std::ostringstream& os, const Stmts& ss, int n) {
       case Stmt::If:
         os << pad << "if (" << print_expr(s->expr) << ") {\n";
         list_host(os, s->body, n + 2);
-        if (!s->els.empty()) {
+        if (!s->fname.empty()) {   // the launches that the other branch stands for, named only
+          os << pad << "} else {   // " << s->fname << ":";
+          visit_stmts(s->els, [&](const S& l) { if (l->k == Stmt::Launch) os << " " << l->fname; });
+          os << "\n";
+        } else if (!s->els.empty()) {
           os << pad << "} else {\n";
           list_host(os, s->els, n + 2);
         }

@@ -67,7 +67,7 @@ struct Val {
 };
 
 struct HExpr {
-  enum Op : uint8_t { Var, Lit, Neg, Not, BitNeg, Bin, Ite, Cvt, Addr, Fits } op = Lit;
+  enum Op : uint8_t { Var, Lit, Neg, Not, BitNeg, Bin, Ite, Cvt, Addr, Fits, Disjoint } op = Lit;
   int slot = -1;
   Val lit;
   std::string bin;
@@ -246,6 +246,9 @@ struct PlanBuilder {
     } else if (h == "fits") {
       e.op = HExpr::Fits;
       e.lit.i = x->at(1)->as_int();
+    } else if (h == "disjoint") {
+      e.op = HExpr::Disjoint;
+      for (int k = 1; k <= 4; ++k) e.args.push_back(expr(x->at(k)));
     } else {
       throw std::runtime_error("unknown host expression '" + h + "' in launch plan");
     }
@@ -383,6 +386,12 @@ Val eval(const Plan& p, const HExpr& e) {
     case HExpr::Fits: {   // temporaries of so many bytes can be had: always, unless this run may only carve scratch memory
       Val r;
       r.i = !p.scratch_base || ((p.scratch_top + 255) & ~int64_t(255)) + e.lit.i <= (int64_t)PARPY_HIP_SCRATCH_BYTES;
+      return r;
+    }
+    case HExpr::Disjoint: {   // (start, bytes) twice
+      const uintptr_t a = (uintptr_t)eval(p, e.args[0]).p, b = (uintptr_t)eval(p, e.args[2]).p;
+      Val r;
+      r.i = a < b ? b - a >= (uint64_t)eval(p, e.args[1]).as_i() : a - b >= (uint64_t)eval(p, e.args[3]).as_i();
       return r;
     }
     case HExpr::Addr: {

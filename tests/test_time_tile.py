@@ -42,6 +42,15 @@ def lopsided(A, B, C, n, steps):
             C[i] = B[i - 3] * 0.125 + C[i] * 0.875
 
 
+def driven(A, B, C, n, steps):
+    """An array that the loop only reads, which a caller may pass a second time under the name of one it writes."""
+    for t in range(steps):
+        parpy.label('N')
+        B[1:-1] = (A[:-2] + A[2:]) * 0.5
+        parpy.label('N')
+        A[1:-1] = B[1:-1] * 0.25 + C[2:]
+
+
 PROGRAMS = [jacobi, wave_equation, lopsided]
 
 
@@ -82,3 +91,51 @@ def test_tiled_steps_match_one_launch_per_update(f, dtype):
             # (products and sums may be contracted to fused multiply-adds differently)
             same = np.array_equal(w, g) if f is jacobi else np.allclose(w, g, rtol=1e-12 if dtype == np.float64 else 1e-4, atol=1e-13 if dtype == np.float64 else 1e-5)
             assert same, (f.__name__, n, steps, np.abs(w - g).max())
+
+
+def plan_of(f, args, o):
+    o = parpy.backend._resolve_backend(o, False)
+    return parpy.compiler.compile_ir(parpy._ir_asts[parpy.jit(f)], parpy.validate.check_arguments(args, o, False), o, {}).plan
+
+
+def test_a_written_array_must_not_be_reachable_under_another_name():
+    """The plan tests every pair of arrays of which one is written, over their whole length, and keeps the loop of launches."""
+    import re
+    o = parpy.par({'N': parpy.threads(5000)})
+    o.backend = HIP
+    plan = plan_of(driven, [np.zeros(5000, dtype=np.float32) for _ in range(3)] + [5000, 20], o)
+    pairs = re.findall(r'\(disjoint \(v "?(\w)_\d+"?\) \(i 20000\) \(v "?(\w)_\d+"?\) \(i 20000\)\)', plan)
+    assert sorted("".join(sorted(p)) for p in pairs) == ["AB", "AC", "BC"]
+    tiled, updates = re.search(r"\(then (.*)\) \(else (.*)\)\)", plan).groups()
+    assert tiled.count("(launch") == 2 and updates.count("(launch") == 2 and "(i 20)" in updates
+
+
+@pytest.mark.gpu
+def test_arrays_passed_under_two_names():
+    torch = pytest.importorskip("torch")
+    n, steps = 4000, 12
+    f = parpy.jit(driven)
+
+    def call(arrays, **kw):
+        o = parpy.par({'N': parpy.threads(n)})
+        for k, v in kw.items():
+            setattr(o, k, v)
+        f(*arrays, n, steps, opts=o)
+        parpy.sync(HIP)
+        o = parpy.backend._resolve_backend(o, True)
+        return parpy._compile_function(parpy._ir_asts[f], parpy.validate.check_arguments([*arrays, n, steps], o, True), o).launch_count()
+
+    def arrays(overlap, seed):
+        """A and B apart; C is B (None) or starts `overlap` elements before B ends."""
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        buf = torch.randn(3 * n, generator=g, device="cuda")
+        A, B = buf[:n], buf[n:2 * n]
+        return buf, [A, B, B if overlap is None else buf[2 * n - overlap:3 * n - overlap]]
+
+    for q, (overlap, tiled) in enumerate([(None, False), (0, True), (4, False), (n, False)]):
+        whole, a = arrays(overlap, q)
+        want, b = arrays(overlap, q)
+        assert call(a) == (2 if tiled else 2 * steps), overlap
+        call(b, opt_tile_steps=False)
+        # (products and sums may be contracted to fused multiply-adds differently)
+        assert torch.allclose(whole, want, rtol=1e-4, atol=1e-5), overlap
