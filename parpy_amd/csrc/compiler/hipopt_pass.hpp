@@ -35,6 +35,11 @@ inline bool may_skip(const E& e, size_t q) {
   return q > 0 && (e->k == Expr::IfExpr || (e->k == Expr::BinOpE && (e->bop == BinOp::And || e->bop == BinOp::Or)));
 }
 
+// Launches that are merged into one keep the order that launches have among accesses of one name only.  The host test that
+// no array which is written can be reached under another name: address ranges of every such pair; null when there is none.
+struct HostArray { Name name; int64_t bytes = 0; bool written = false; };
+E arrays_disjoint(const Program& p, const std::vector<HostArray>& arrays);
+
 template <class F> E rewrite_expr(const E& e, F f) {  // bottom-up rewrite
   if (!e) return e;
   E r = map_children(e, [&](const E& c) { return rewrite_expr(c, f); });

@@ -163,11 +163,23 @@ struct PersistentLoops {
     l->iv = groups;   // counters the barrier needs
     for (auto& q : f.params) l->args.push_back(mk_var(q.id, q.ty));
     l->body = {loop};
+    // (only what is written by name is loaded at device scope)
+    std::vector<HostArray> ranges;
+    for (auto& q : f.params) {
+      if (q.ty.k != Type::Pointer && !q.ty.is_array()) continue;
+      HostArray a{q.id, INT64_MAX, !q.read_only};   // (of unknown length unless it is an argument)
+      for (auto& e : p.entry_params) if (e.id == q.id) a.bytes = e.ty.numel() * elem_bytes(e.ty.sz);
+      ranges.push_back(a);
+    }
+    const E usable = arrays_disjoint(p, ranges);
     f.params.push_back(counter);
     f.params.push_back(status);
     f.params.push_back(limit);
     p.kernels.push_back(f);
-    return l;
+    if (!usable) return l;
+    auto either = clone(mk_if(usable, {S(l)}, {loop}));
+    either->fname = "one launch per step";
+    return either;
   }
 
   Stmts walk(const Stmts& ss) {

@@ -360,32 +360,17 @@ struct TimeTile {
     // reachable under two names when one of them is written: `C is B`, or views that overlap, is legal in a loop of
     // launches none of which writes an array that it reads under another name.  Names say nothing about that and a plan
     // serves any pointers, so it tests the address ranges and holds the loop of launches for those that meet.
-    std::set<Name> made_here;
-    int64_t others = 0;
-    visit_stmts(p.host, [&](const S& s) {
-      if (s->k != Stmt::Alloc) return;
-      made_here.insert(s->id);
-      others += s->iv * elem_bytes(s->ty.sz) + 256;
-    });
-    E usable;
-    auto also = [&](const E& c) { usable = usable ? both(usable, c) : c; };
-    for (size_t x = 0; x < arrays.size(); ++x)
-      for (size_t y = x + 1; y < arrays.size(); ++y) {
-        const Arr &a = arrays[x], &b = arrays[y];
-        if (!(a.written || b.written) || made_here.count(a.host) || made_here.count(b.host)) continue;
-        auto c = std::make_shared<Expr>();
-        c->k = Expr::Call;
-        c->ty = bty;
-        c->sval = "parpy_disjoint";
-        c->args = {mk_var(a.host, Type::pointer(a.sz)), iint(a.n * elem_bytes(a.sz)), mk_var(b.host, Type::pointer(b.sz)), iint(b.n * elem_bytes(b.sz))};
-        also(E(c));
-      }
+    std::vector<HostArray> ranges;
+    for (auto& a : arrays) ranges.push_back({a.host, a.n * elem_bytes(a.sz), a.written});
+    E usable = arrays_disjoint(p, ranges);
     // A run that may allocate nothing has a fixed amount of scratch memory for all temporaries of the plan, which the
     // second set of arrays may not fit.
+    int64_t others = 0;
+    visit_stmts(p.host, [&](const S& s) { if (s->k == Stmt::Alloc) others += s->iv * elem_bytes(s->ty.sz) + 256; });
     if (others + second_set > SCRATCH_BYTES) {
       auto fits = std::make_shared<Expr>(*mk_raw("parpy_temporaries_fit(" + std::to_string(second_set) + ")", bty));
       fits->iv = second_set;
-      also(E(fits));
+      usable = usable ? both(usable, E(fits)) : E(fits);
     }
     if (!usable) return mk_scope(tiled);
     auto either = clone(mk_if(usable, tiled, {loop}));

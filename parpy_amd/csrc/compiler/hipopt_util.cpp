@@ -58,5 +58,24 @@ E subst_vars(const E& e, const std::map<Name, E>& m) {
   return map_children(e, [&](const E& c) { return subst_vars(c, m); });
 }
 
+E arrays_disjoint(const Program& p, const std::vector<HostArray>& arrays) {
+  std::set<Name> made_here;   // temporaries of the plan meet nothing
+  visit_stmts(p.host, [&](const S& s) { if (s->k == Stmt::Alloc) made_here.insert(s->id); });
+  const Type bty = Type::scalar(ElemSize::Bool);
+  E all;
+  for (size_t x = 0; x < arrays.size(); ++x)
+    for (size_t y = x + 1; y < arrays.size(); ++y) {
+      const HostArray &a = arrays[x], &b = arrays[y];
+      if (!(a.written || b.written) || made_here.count(a.name) || made_here.count(b.name)) continue;
+      auto c = std::make_shared<Expr>();
+      c->k = Expr::Call;
+      c->ty = bty;
+      c->sval = "parpy_disjoint";
+      c->args = {mk_var(a.name, Type::pointer(ElemSize::I8)), mk_int(a.bytes), mk_var(b.name, Type::pointer(ElemSize::I8)), mk_int(b.bytes)};
+      all = all ? mk_binop(BinOp::And, all, E(c), bty) : E(c);
+    }
+  return all;
+}
+
 }  // namespace hipopt
 }  // namespace parpy

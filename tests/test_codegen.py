@@ -607,6 +607,31 @@ def test_persistent_loops_let_the_workgroups_of_one_read_meet_among_themselves()
     assert re.search(r"parpy_grid_barrier\(parpy_bar_counter_\d+ \+ 32u \* blockIdx\.y, parpy_bar_status_\d+, 16u,", s)
 
 
+def test_persistent_loops_keep_the_loop_of_launches_for_arrays_that_overlap():
+    """Workgroups load what the steps write at device scope, by name: the same array under the name of one that is only
+    read would be read out of a cache.  The plan tests every pair of arrays of which one is written."""
+    a, c = np.zeros((2, 4096), dtype=np.float32), np.zeros(4096, dtype=np.float32)
+
+    @parpy.jit
+    def pingpong(a, b, c, N, M, T):
+        parpy.label('i')
+        for i in range(N):
+            for t in range(T):
+                src = a
+                dst = b
+                if t & 1:
+                    src = b
+                    dst = a
+                parpy.label('j')
+                for j in range(M):
+                    dst[i, j] = src[i, (j + 1) % M] + c[j]
+    o = opts_for({'i': parpy.threads(2), 'j': parpy.threads(4096).tpb(256)}, persistent_loops=True, backend=parpy.CompileBackend.Hip)
+    plan = _plan_of(pingpong, [a, a.copy(), c, 2, 4096, 10], o)
+    pairs = re.findall(r'\(disjoint \(v "?(\w)_\d+"?\) \(i (\d+)\) \(v "?(\w)_\d+"?\) \(i (\d+)\)\)', plan)
+    assert sorted(tuple(sorted([p[:2], p[2:]])) for p in pairs) == [(("a", "32768"), ("b", "32768")), (("a", "32768"), ("c", "16384")), (("b", "32768"), ("c", "16384"))]
+    assert re.search(r"\(then \(persist .*\) 2\) \) \(else \(for ", plan)
+
+
 def test_persistent_loops_keep_the_loop_of_launches_for_arrays_of_narrow_elements():
     """Workgroups exchange data through device-scope loads and stores, which exist for elements of four bytes and
     more: a ping-pong step over float16 or int8 vectors stays a loop of launches, the float32 one becomes one kernel."""
