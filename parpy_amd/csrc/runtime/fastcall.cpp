@@ -4,13 +4,14 @@
 // settings of the options object -- is written into a byte string, looked up, and the plan runs on the tensors' device
 // pointers.  The Python statement of the same key (a tuple per argument, hashed) took 4.5 of the 7.2 us that a call
 // with two tensors costs, the launch itself the rest; this file takes 0.4 us.  What it does not recognise (host arrays,
-// sliced or gradient-tracking tensors, unusual option values) it leaves to the Python path, which decides everything
+// sliced or gradient-tracking tensors, tensors without memory of their own, unusual option values) it leaves to the Python path, which decides everything
 // and adds what it compiled.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
+#include <new>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -77,7 +78,7 @@ bool put_value(std::string& k, PyObject* v, Pointers& ps) {
     }
     if (!t.is_cuda() || t.layout() != c10::kStrided || !t.is_contiguous() || t.requires_grad()) return false;
     if (ps.n == MAX_POINTERS) return false;
-    void* p = const_cast<void*>(t.const_data_ptr());
+    void* p = t.mutable_data_ptr();   // (a tensor that shares its memory until it is written gets its own, as `data_ptr()` does)
     ps.p[ps.n++] = p;
     ps.aligned = ps.aligned && (uintptr_t)p % 16 == 0;
     put_tag(k, 't');
@@ -169,12 +170,20 @@ bool put_options(std::string& k, PyObject* opts, PyObject* loop_par_type) {
   return ok;
 }
 
-bool make_key(Table* self, PyObject* args, PyObject* opts, Pointers& ps) {
-  std::string& k = *self->key;
-  k.clear();
-  if (!put_args(k, args, ps)) return false;
-  put_tag(k, ps.aligned ? '|' : '!');
-  return put_options(k, opts, self->loop_par_type);
+// What is asked of a tensor throws where it has no memory to point at (inside torch.vmap and the like the type is
+// torch.Tensor all the same), and nothing may be thrown through the interpreter's frames: such a call is not for this
+// path, the Python path asks again and reports it.
+bool make_key(Table* self, PyObject* args, PyObject* opts, Pointers& ps) noexcept {
+  try {
+    std::string& k = *self->key;
+    k.clear();
+    if (!put_args(k, args, ps)) return false;
+    put_tag(k, ps.aligned ? '|' : '!');
+    return put_options(k, opts, self->loop_par_type);
+  } catch (...) {
+    PyErr_Clear();   // (an exception that Python code under the tensor raised)
+    return false;
+  }
 }
 
 // run(args, kwargs) -> None: a call this table does not know; else the status of the run
@@ -208,17 +217,25 @@ PyObject* table_add(PyObject* o, PyObject* const* a, Py_ssize_t na) {
   if ((PyObject*)Py_TYPE(a[1]) != self->opts_type) Py_RETURN_FALSE;
   Pointers ps;
   if (!make_key(self, a[0], a[1], ps)) Py_RETURN_FALSE;
-  Entry e;
-  e.plan = PyLong_AsVoidPtr(a[2]);
+  void* plan = PyLong_AsVoidPtr(a[2]);
   if (PyErr_Occurred()) return nullptr;
   if ((size_t)PyTuple_GET_SIZE(a[3]) != ps.n) Py_RETURN_FALSE;
+  int32_t order[MAX_POINTERS];
   for (size_t q = 0; q < ps.n; ++q) {
     long v = PyLong_AsLong(PyTuple_GET_ITEM(a[3], q));
-    if (v < 0 || (size_t)v >= ps.n) { PyErr_SetString(PyExc_ValueError, "order out of range"); return nullptr; }
-    e.order.push_back((int32_t)v);
+    if (v < 0 || (size_t)v >= ps.n) {
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "order out of range");
+      return nullptr;
+    }
+    order[q] = (int32_t)v;
   }
-  if (self->entries->size() >= MAX_ENTRIES) self->entries->clear();
-  (*self->entries)[*self->key] = std::move(e);
+  try {
+    if (self->entries->size() >= MAX_ENTRIES) self->entries->clear();
+    Entry e{plan, {order, order + ps.n}};
+    (*self->entries)[*self->key] = std::move(e);
+  } catch (...) {
+    return PyErr_NoMemory();
+  }
   Py_RETURN_TRUE;
 }
 
@@ -234,8 +251,9 @@ PyObject* table_new(PyTypeObject* type, PyObject* args, PyObject*) {
   if (PyErr_Occurred()) return nullptr;
   Table* self = (Table*)type->tp_alloc(type, 0);
   if (!self) return nullptr;
-  self->entries = new std::unordered_map<std::string, Entry>();
-  self->key = new std::string();
+  self->entries = new (std::nothrow) std::unordered_map<std::string, Entry>();
+  self->key = new (std::nothrow) std::string();
+  if (!self->entries || !self->key) { Py_DECREF(self); return PyErr_NoMemory(); }
   Py_INCREF(opts_type);
   Py_INCREF(loop_par_type);
   self->opts_type = opts_type;

@@ -42,6 +42,24 @@ def test_calls_that_differ_in_anything_are_different_calls():
     assert table.run((1,), {"opts": opts()}) is None
 
 
+def test_tensors_without_memory_of_their_own_are_left_to_the_python_path():
+    """Inside torch.vmap an argument is of type torch.Tensor and has no address; asking for it throws a C++ exception."""
+    from parpy_amd import fastcall
+    run = ctypes.CFUNCTYPE(ctypes.c_int32, ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p), ctypes.c_int32)(lambda plan, p, n: 0)
+    table = fastcall._load().CallTable(CompileOptions, LoopPar, ctypes.cast(run, ctypes.c_void_p).value)
+    answers = []
+
+    def inside(v):
+        for args in ((v,), ({"a": v, "b": 1},)):
+            answers.append((type(v) is torch.Tensor, table.add(args, opts(), 1000, ()), table.run(args, {"opts": opts()})))
+        return v
+    torch.vmap(inside)(torch.zeros(3))                # 0-d
+    torch.vmap(inside)(torch.zeros(3, 4))
+    torch.func.grad(lambda v: inside(v) * 1.0)(torch.tensor(2.0))
+    assert answers == [(True, False, None)] * 6
+    assert table.add((torch.tensor(2.0),), opts(), 1000, ()) and table.run((torch.tensor(2.0),), {"opts": opts()}) == 0
+
+
 def test_plan_pointers_follow_the_sorted_fields():
     from parpy_amd import fastcall
     a, b, c, s = (torch.zeros(k) for k in (1, 2, 3, 4))
@@ -76,3 +94,20 @@ def test_warm_calls_run_on_the_arguments_of_the_call():
     f({"x": x, "w": 2.0, "b": x}, out, 64, opts=opts(256))
     f({"x": x, "w": 2.0, "b": x}, out, 64, opts=opts(256))
     assert torch.equal(out, x * 2.0 + x)
+
+
+@pytest.mark.gpu
+def test_warm_calls_on_tensors_that_share_or_lack_memory():
+    f = parpy.jit(scale)
+    x, b = (torch.randn(64, device="cuda") for _ in range(2))
+    out = torch.full((64,), -1.0, device="cuda")
+    call = lambda o: f({"x": x, "w": 2.0, "b": b}, o, 64, opts=opts(64))
+    call(out.clone())
+    shared = torch._lazy_clone(out)                   # shares the memory of `out` until one of them is written
+    call(shared)                                      # (a warm call)
+    parpy.sync(HIP)
+    assert torch.equal(shared, x * 2.0 + b) and bool((out == -1.0).all())
+    with pytest.raises(RuntimeError):
+        torch.vmap(lambda o: (call(o), o)[1])(torch.zeros(3, 64, device="cuda"))
+    call(out)
+    assert torch.equal(out, x * 2.0 + b)
