@@ -79,7 +79,8 @@ int32_t parpy_hip_plan_create(void* module, const char* plan_text, void** plan);
  * the error message is per thread.  Temporaries stay allocated between runs up
  * to 1 GiB per plan and 8 GiB over all plans of the process (beyond that they
  * are allocated and freed per run); a run that fails half way frees what it
- * had allocated for itself. */
+ * had allocated for itself.  Where a plan can do without some of them (a branch
+ * under `fits`), a run that cannot have them takes the other branch. */
 int32_t parpy_hip_plan_run(void* plan, void* const* args, int32_t nargs);
 
 /* Same as parpy_hip_plan_run, bracketed by HIP events recorded on the null

@@ -47,8 +47,6 @@ struct TimeTile {
     int64_t radius = 0;
   };
 
-  static constexpr int64_t SCRATCH_BYTES = int64_t(16) << 20;   // PARPY_HIP_SCRATCH_BYTES of the runtime
-
   E iint(int64_t v) { return mk_int(v, isz); }
   E add(E a, E b) { return mk_binop(BinOp::Add, a, b, ity); }
   static int64_t pow2_at_least(int64_t n) { int64_t q = 1; while (q < n) q *= 2; return q; }
@@ -146,6 +144,11 @@ struct TimeTile {
       for (auto& u : ups) if (u.hi > a.n) { bool w = false; for (auto& st : u.body) if (st->dst && st->dst->k == Expr::Index && u.host[st->dst->args[0]->name] == a.host) w = true; if (w) return S(); }
     }
     if (n < 512 || n > (int64_t(1) << 30) || steps * (int64_t)ups.size() < 4 || steps < 2) return S();
+    // The second set is kept between runs up to 1 GiB per plan; a larger one is obtained and given back by every call, out of
+    // the device's pool, which costs a tenth of a millisecond up to some size and then hundreds (ten Jacobi steps, float64,
+    // tiled and as launches: 1.6 GB 1.6 and 6.6 ms, 4.3 GB 5.2 and 17.9, 6.4 GB 6.7 and 26.3, 9.6 GB 10 and 39 with single
+    // calls of 149, 14.4 GB 390 and 58.6).
+    if (second_set > (int64_t(6) << 30)) return S();
     // Elements per lane: eight where that leaves every SIMD a wavefront or two, four for smaller arrays, where the
     // latency of a step is what counts (98 updates of a three-point average, float64: 10^6 elements 153 / 73 / 56 / 51 /
     // 68 us for 1 / 2 / 4 / 8 / 16 elements per lane, 6 * 10^5: 35 on four, 38 on eight, 10^5: 15 and 24).
@@ -362,18 +365,12 @@ struct TimeTile {
     // serves any pointers, so it tests the address ranges and holds the loop of launches for those that meet.
     std::vector<HostArray> ranges;
     for (auto& a : arrays) ranges.push_back({a.host, a.n * elem_bytes(a.sz), a.written});
-    E usable = arrays_disjoint(p, ranges);
-    // A run that may allocate nothing has a fixed amount of scratch memory for all temporaries of the plan, which the
-    // second set of arrays may not fit.
-    int64_t others = 0;
-    visit_stmts(p.host, [&](const S& s) { if (s->k == Stmt::Alloc) others += s->iv * elem_bytes(s->ty.sz) + 256; });
-    if (others + second_set > SCRATCH_BYTES) {
-      auto fits = std::make_shared<Expr>(*mk_raw("parpy_temporaries_fit(" + std::to_string(second_set) + ")", bty));
-      fits->iv = second_set;
-      usable = usable ? both(usable, E(fits)) : E(fits);
-    }
-    if (!usable) return mk_scope(tiled);
-    auto either = clone(mk_if(usable, tiled, {loop}));
+    const E apart = arrays_disjoint(p, ranges);
+    // Nor must the call fail for the second set: what the device has left, or the fixed amount of scratch memory of a run
+    // that may allocate nothing, may not hold it.
+    auto fits = std::make_shared<Expr>(*mk_raw("parpy_temporaries_fit(" + std::to_string(second_set) + ")", bty));
+    fits->iv = second_set;
+    auto either = clone(mk_if(apart ? both(apart, E(fits)) : E(fits), tiled, {loop}));
     either->fname = "one launch per update";
     return mk_scope({S(either)});
   }

@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdlib>
@@ -90,7 +91,8 @@ struct HStmt {
   int64_t step = 1;
   int64_t nbytes = 0;
   std::vector<HStmt> body, els;   // Persist: body = the loop of launches that the kernel stands for
-  bool fits = false;              // Persist: every workgroup of the launch can be resident at once (checked at creation)
+  bool fits = false;              // Persist: every workgroup of the launch can be resident at once (checked at creation).
+                                  // If: the temporaries that `body` begins with may be refused, `els` does without them
   int64_t groups = 1;            // Persist: groups of workgroups that meet among themselves at the barrier (one counter each)
 };
 
@@ -255,6 +257,12 @@ struct PlanBuilder {
     return e;
   }
 
+  static bool asks_for_temporaries(const HExpr& e) {
+    if (e.op == HExpr::Fits) return true;
+    for (auto& a : e.args) if (asks_for_temporaries(a)) return true;
+    return false;
+  }
+
   std::vector<HStmt> stmts(const SXP& lst, size_t from) {
     std::vector<HStmt> out;
     for (size_t k = from; k < lst->size(); ++k) out.push_back(stmt(lst->at(k)));
@@ -328,6 +336,7 @@ struct PlanBuilder {
     } else if (h == "if") {
       s.op = HStmt::If;
       s.a = expr(x->at(1));
+      s.fits = asks_for_temporaries(s.a);
       s.body = stmts(x->at(2), 1);
       s.els = stmts(x->at(3), 1);
     } else if (h == "def") {
@@ -383,7 +392,7 @@ Val eval(const Plan& p, const HExpr& e) {
       r.i = v;
       return r;
     }
-    case HExpr::Fits: {   // temporaries of so many bytes can be had: always, unless this run may only carve scratch memory
+    case HExpr::Fits: {   // temporaries of so many bytes can be had: what a run that allocates finds out when it does
       Val r;
       r.i = !p.scratch_base || ((p.scratch_top + 255) & ~int64_t(255)) + e.lit.i <= (int64_t)PARPY_HIP_SCRATCH_BYTES;
       return r;
@@ -468,7 +477,41 @@ union Packed {
   bool b;
 };
 
-int32_t run_stmts(Plan& p, const std::vector<HStmt>& ss);
+int32_t run_stmts(Plan& p, const std::vector<HStmt>& ss, size_t from = 0);
+int32_t run_stmt(Plan& p, const HStmt& s);
+
+// A branch that begins with temporaries and can be done without: whether it has them now.  Those obtained before one is
+// refused go back to the device, also where they would be kept between runs.
+bool obtain_temporaries(Plan& p, const std::vector<HStmt>& ss, size_t* count) {
+  const int64_t top = p.scratch_top;
+  const size_t carved = p.carved.size();
+  for (*count = 0; *count < ss.size() && ss[*count].op == HStmt::Alloc; ++*count) {
+    if (run_stmt(p, ss[*count]) == 0) continue;
+    p.scratch_top = top;
+    p.carved.resize(carved);
+    for (size_t k = 0; k < *count && !p.scratch_base; ++k) {
+      void* ptr = p.env[ss[k].slot].p;
+      Plan::Kept& kp = p.kept[ss[k].slot];
+      if (p.capturing) {   // (an earlier run's: nothing is allocated or released inside a capture)
+        kp.in_use = false;
+        continue;
+      }
+      if (kp.ptr == ptr) {
+        p.kept_bytes -= kp.nbytes;
+        g_kept_all -= kp.nbytes;
+        kp = Plan::Kept();
+      } else {
+        p.unkept.erase(std::remove(p.unkept.begin(), p.unkept.end(), ptr), p.unkept.end());
+      }
+      if (hipFreeAsync(ptr, nullptr) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(ptr);
+      }
+    }
+    return false;
+  }
+  return true;
+}
 
 int32_t run_stmt(Plan& p, const HStmt& s) {
   switch (s.op) {
@@ -534,8 +577,11 @@ int32_t run_stmt(Plan& p, const HStmt& s) {
       while (eval(p, s.a).as_i() != 0)
         if (int32_t rc = run_stmts(p, s.body)) return rc;
       return 0;
-    case HStmt::If:
-      return run_stmts(p, eval(p, s.a).as_i() != 0 ? s.body : s.els);
+    case HStmt::If: {
+      size_t done = 0;
+      const bool then = eval(p, s.a).as_i() != 0 && (!s.fits || obtain_temporaries(p, s.body, &done));
+      return then ? run_stmts(p, s.body, done) : run_stmts(p, s.els);
+    }
     case HStmt::Def: case HStmt::Set:
       p.env[s.slot] = eval(p, s.a);
       return 0;
@@ -610,9 +656,9 @@ int32_t run_stmt(Plan& p, const HStmt& s) {
   return 0;
 }
 
-int32_t run_stmts(Plan& p, const std::vector<HStmt>& ss) {
-  for (auto& s : ss) {
-    if (int32_t rc = run_stmt(p, s)) return rc;
+int32_t run_stmts(Plan& p, const std::vector<HStmt>& ss, size_t from) {
+  for (size_t k = from; k < ss.size(); ++k) {
+    if (int32_t rc = run_stmt(p, ss[k])) return rc;
     if (g_div_by_zero) return fail("division by zero in the host part of the launch plan");
   }
   return 0;

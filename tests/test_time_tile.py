@@ -110,6 +110,70 @@ def test_a_written_array_must_not_be_reachable_under_another_name():
     assert tiled.count("(launch") == 2 and updates.count("(launch") == 2 and "(i 20)" in updates
 
 
+def decay(A, n, steps):
+    for t in range(steps):
+        parpy.label('N')
+        for i in range(n):
+            A[i] = A[i] * 0.5 + 1.0
+        parpy.label('N')
+        A[1:] = A[1:] - 0.25
+
+
+def test_a_call_does_not_need_memory_for_the_second_set_of_arrays():
+    """Whatever its size, the plan holds the loop of launches for a run that cannot have it."""
+    import re
+    o = parpy.par({'N': parpy.threads(5000)})
+    o.backend = HIP
+    for f, args in ((decay, [np.zeros(5000)]), (driven, [np.zeros(5000) for _ in range(3)]), (jacobi, [np.zeros(3000000) for _ in range(3)])):
+        plan = plan_of(f, args + [len(args[0]), 20], o)
+        assert re.search(r"\(if .*\(fits \d+\)\)? \(then \(alloc .*\(launch .*\) \(else \(for .*\(launch ", plan)
+
+
+def test_second_sets_that_no_pool_hands_out_quickly_are_not_asked_for():
+    o = parpy.par({'N': parpy.threads(5000)})
+    o.backend = HIP
+    for n, tiled in ((400_000_000, True), (600_000_000, False)):   # two float64 arrays: 6.4 and 9.6 GB
+        a = np.empty(n)   # (never touched)
+        assert ("parpy_lane_before(" in parpy.print_compiled(jacobi, [a, a, a, n, 10], o).split('extern "C"', 1)[1]) == tiled
+
+
+@pytest.mark.gpu
+def test_a_branch_whose_temporaries_are_refused_is_not_taken():
+    """Through the runtime's own entry points: the first temporary can be had, the second (4 TiB) cannot."""
+    import ctypes
+    torch = pytest.importorskip("torch")
+    from parpy_amd import runtime
+    o = parpy.par({})
+    o.backend = HIP
+    lib = runtime._compile_runtime_lib(HIP)
+    code = hiprtc_compile('extern "C" __global__ void add(float* x, float v) { if (threadIdx.x == 0) x[0] += v; }', o)
+    buf, module = ctypes.create_string_buffer(code, len(code)), ctypes.c_void_p()
+    assert lib.parpy_hip_module_load(buf, len(code), ctypes.byref(module)) == 0
+    x = torch.zeros(1, device="cuda")
+    arr = (ctypes.c_void_p * 1)(x.data_ptr())
+
+    def plan(second):
+        text = ('(plan "f" (params ("x" ptr)) (kernels ("add" (params ptr f32))) (body (if (bin and i (i 1) (fits 1)) (then (alloc "t" 1024) '
+                f'(alloc "u" {second}) (launch 0 1 1 1 64 1 1 (args (v "t") (f 1))) (launch 0 1 1 1 64 1 1 (args (v "x") (f 1))) (free "t") (free "u") ) '
+                '(else (launch 0 1 1 1 64 1 1 (args (v "x") (f 100))) )) (launch 0 1 1 1 64 1 1 (args (v "x") (f 1000))) ))')
+        h = ctypes.c_void_p()
+        assert lib.parpy_hip_plan_create(module, text.encode(), ctypes.byref(h)) == 0, lib.parpy_get_error_message()
+        return h
+
+    total = 0.0
+    for second, run, adds in ((4096, lib.parpy_hip_plan_run, 1001.0), (1 << 42, lib.parpy_hip_plan_run, 1100.0),
+                              (4096, lib.parpy_hip_plan_run_noalloc, 1001.0), (1 << 24, lib.parpy_hip_plan_run_noalloc, 1100.0)):
+        h = plan(second)
+        for graph in (0, 1) if run is lib.parpy_hip_plan_run else (0,):
+            lib.parpy_hip_plan_set_graph(h, graph)
+            for _ in range(4):
+                assert run(h, arr, 1) == 0, lib.parpy_get_error_message()
+                total += adds
+                assert lib.parpy_sync() == 0 and x.item() == total, (second, graph)
+            assert lib.parpy_hip_plan_launch_count(h) == (3 if adds == 1001.0 else 2)
+        assert lib.parpy_hip_plan_destroy(h) == 0
+
+
 @pytest.mark.gpu
 def test_arrays_passed_under_two_names():
     torch = pytest.importorskip("torch")
