@@ -143,7 +143,14 @@ struct TimeTile {
       if (a.written) second_set += (a.n * elem_bytes(a.sz) + 255) / 256 * 256;
       for (auto& u : ups) if (u.hi > a.n) { bool w = false; for (auto& st : u.body) if (st->dst && st->dst->k == Expr::Index && u.host[st->dst->args[0]->name] == a.host) w = true; if (w) return S(); }
     }
-    if (n < 512 || n > (int64_t(1) << 30) || steps * (int64_t)ups.size() < 4 || steps < 2) return S();
+    // Four updates cost what two launches save, except for long arrays of float64, where the launches move as much as the
+    // updates did and the division's arithmetic comes on top (Jacobi, tiled and as launches: 1000 6.8 and 12.0 us, 300 000
+    // 8.6 and 11.6, 10^6 21.3 and 17.9, 2 * 10^6 34.8 and 26.6, 4 * 10^6 59 and 62, 3 * 10^7 470 and 417; six updates of
+    // 10^6 21.0 and 26.2; float32 12.7 and 13.6 for 10^6, 205 and 285 for 3 * 10^7).
+    bool wide = false;
+    for (auto& a : arrays) wide = wide || elem_bytes(a.sz) == 8;
+    const int64_t updates = steps * (int64_t)ups.size();
+    if (n < 512 || n > (int64_t(1) << 30) || steps < 2 || updates < (wide && n >= 800000 ? 6 : 4)) return S();
     // The second set is kept between runs up to 1 GiB per plan; a larger one is obtained and given back by every call, out of
     // the device's pool, which costs a tenth of a millisecond up to some size and then hundreds (ten Jacobi steps, float64,
     // tiled and as launches: 1.6 GB 1.6 and 6.6 ms, 4.3 GB 5.2 and 17.9, 6.4 GB 6.7 and 26.3, 9.6 GB 10 and 39 with single

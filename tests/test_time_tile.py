@@ -129,6 +129,15 @@ def test_a_call_does_not_need_memory_for_the_second_set_of_arrays():
         assert re.search(r"\(if .*\(fits \d+\)\)? \(then \(alloc .*\(launch .*\) \(else \(for .*\(launch ", plan)
 
 
+def test_few_updates_of_long_arrays_stay_launches():
+    o = parpy.par({'N': parpy.threads(5000)})
+    o.backend = HIP
+    for n, dtype, steps, tiled in ((5000, np.float64, 3, True), (799999, np.float64, 3, True), (800000, np.float64, 3, False),
+                                   (800000, np.float64, 4, True), (800000, np.float32, 3, True), (5000, np.float64, 2, False)):
+        a = np.empty(n, dtype=dtype)
+        assert ("parpy_lane_before(" in parpy.print_compiled(jacobi, [a, a, a, n, steps], o).split('extern "C"', 1)[1]) == tiled, (n, dtype, steps)
+
+
 def test_second_sets_that_no_pool_hands_out_quickly_are_not_asked_for():
     o = parpy.par({'N': parpy.threads(5000)})
     o.backend = HIP
