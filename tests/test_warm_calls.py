@@ -60,6 +60,57 @@ def test_tensors_without_memory_of_their_own_are_left_to_the_python_path():
     assert table.add((torch.tensor(2.0),), opts(), 1000, ()) and table.run((torch.tensor(2.0),), {"opts": opts()}) == 0
 
 
+def plain_calls(monkeypatch, f):
+    """`f` as a jitted function of scalars whose calls reach the warm path without a device; returns it and the list of its runs."""
+    from parpy_amd import runtime
+    ran = []
+
+    def wrapper(*args):
+        ran.append("checked")
+    wrapper.run_pointers = lambda ptrs: ran.append("pointers")
+    wrapper.lib, wrapper.plan = ctypes.CDLL(str(runtime.PARPY_HIP_BASE_LIB_PATH)), ctypes.c_void_p(1)
+    monkeypatch.setattr(parpy, "_compile_function", lambda ir, args, opts: wrapper)
+    monkeypatch.setattr(parpy.backend, "_resolve_backend", lambda opts, execute: opts)
+    return parpy.jit(f), ran
+
+
+def nothing(n):
+    parpy.label('N')
+    for i in range(n):
+        t = i
+
+
+def test_calls_run_without_the_extension(monkeypatch):
+    """No compiler, no headers, a folder that cannot be written: said once, and not by a call that fails after its work is done."""
+    import warnings
+    from parpy_amd import fastcall
+    tried = []
+
+    def no_compiler(*a, **k):
+        tried.append(1)
+        raise RuntimeError("no compiler")
+    monkeypatch.setattr(fastcall, "_module", None)
+    monkeypatch.setattr(fastcall, "_unavailable", False, raising=False)
+    monkeypatch.setattr(fastcall, "_command", no_compiler)
+    f, ran = plain_calls(monkeypatch, nothing)
+    with pytest.warns(RuntimeWarning, match="no compiler"):
+        f(3, opts=opts())
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        f(3, opts=opts())
+        f(4, opts=opts())
+    assert ran == ["checked", "pointers", "checked"] and len(tried) == 1
+
+
+def test_looking_for_the_extension_does_not_import_the_build_tools():
+    import os
+    import subprocess
+    import sys
+    code = "import sys, torch; from parpy_amd import fastcall; fastcall._load(); assert 'torch.utils.cpp_extension' not in sys.modules"
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    assert subprocess.run([sys.executable, "-W", "error::RuntimeWarning", "-c", code], cwd=root, timeout=300).returncode == 0
+
+
 def test_plan_pointers_follow_the_sorted_fields():
     from parpy_amd import fastcall
     a, b, c, s = (torch.zeros(k) for k in (1, 2, 3, 4))
