@@ -102,6 +102,21 @@ def test_calls_run_without_the_extension(monkeypatch):
     assert ran == ["checked", "pointers", "checked"] and len(tried) == 1
 
 
+def test_calls_that_the_extension_declines_are_offered_once(monkeypatch):
+    from parpy_amd import fastcall
+    offered = []
+    order = fastcall.pointer_order
+    monkeypatch.setattr(fastcall, "pointer_order", lambda args: offered.append(args) or order(args))
+    f, ran = plain_calls(monkeypatch, nothing)
+    for k in range(5):
+        f(3, opts=opts(includes=["/usr/include"]))
+    assert ran == ["checked"] + 4 * ["pointers"]
+    assert len(offered) == 2      # under the state that was passed and the one after the backend was chosen
+    for k in range(3):
+        f(5, opts=opts(includes=["/usr/include"]))
+    assert len(offered) == 4
+
+
 def test_looking_for_the_extension_does_not_import_the_build_tools():
     import os
     import subprocess
