@@ -29,12 +29,6 @@ int64_t per_thread_trips(const S& loop);                  // iterations every th
 E counter_var(const S& loop, ElemSize isz);               // the per-thread iteration counter of a mapped loop as the printer names it
 E subst_vars(const E& e, const std::map<Name, E>& m);
 
-// operand q of e may be left unevaluated (the branches of a selection, the right side of `and` / `or`): an index in it
-// need only be in bounds where it is evaluated, so nothing may be loaded from there ahead of the test
-inline bool may_skip(const E& e, size_t q) {
-  return q > 0 && (e->k == Expr::IfExpr || (e->k == Expr::BinOpE && (e->bop == BinOp::And || e->bop == BinOp::Or)));
-}
-
 // Launches that are merged into one keep the order that launches have among accesses of one name only.  The host test that
 // no array which is written can be reached under another name: address ranges of every such pair; null when there is none.
 struct HostArray { Name name; int64_t bytes = 0; bool written = false; };

@@ -1122,25 +1122,27 @@ struct DevicePrinter {
     return false;
   }
 
-  struct Access { size_t pos; const Expr* e; const Stmt* st; bool store; Name base; Mem mem; E f; int64_t c; bool tracked; };
+  struct Access { size_t pos; const Expr* e; const Stmt* st; bool store; Name base; Mem mem; E f; int64_t c; bool tracked; bool always; };
 
   void plan_packs(const Stmts& ss, size_t lo, size_t hi) {
     // every element access of the run in program order (an assignment evaluates its right-hand side first)
     std::vector<Access> acc;
     for (size_t i = lo; i < hi; ++i) {
       const S& st = ss[i];
-      auto scan = [&](const E& root) {
-        visit_exprs(root, [&](const E& x) {
-          if (x->k != Expr::Index) return;
-          Access a{i, x.get(), st.get(), false, x->args[0]->k == Expr::Var ? x->args[0]->name : Name(), x->args[0]->ty.mem, E(), 0, false};
+      std::function<void(const E&, bool)> visit = [&](const E& x, bool always) {
+        if (!x) return;
+        if (x->k == Expr::Index) {
+          Access a{i, x.get(), st.get(), false, x->args[0]->k == Expr::Var ? x->args[0]->name : Name(), x->args[0]->ty.mem, E(), 0, false, always};
           a.tracked = x->args[0]->k == Expr::Var && split_offset(x->args[1], &a.f, &a.c);
           acc.push_back(a);
-        });
+        }
+        for (size_t q = 0; q < x->args.size(); ++q) visit(x->args[q], always && !may_skip(x, q));
       };
+      auto scan = [&](const E& root) { visit(root, true); };
       if (st->expr) scan(st->expr);
       if (st->k == Stmt::Assign && st->dst->k == Expr::Index) {
         scan(st->dst->args[1]);
-        Access a{i, st->dst.get(), st.get(), true, st->dst->args[0]->k == Expr::Var ? st->dst->args[0]->name : Name(), st->dst->args[0]->ty.mem, E(), 0, false};
+        Access a{i, st->dst.get(), st.get(), true, st->dst->args[0]->k == Expr::Var ? st->dst->args[0]->name : Name(), st->dst->args[0]->ty.mem, E(), 0, false, true};
         a.tracked = st->dst->args[0]->k == Expr::Var && split_offset(st->dst->args[1], &a.f, &a.c);
         acc.push_back(a);
       } else if (st->dst) {
@@ -1183,6 +1185,11 @@ struct DevicePrinter {
         ok = found;
       }
       if (!ok) continue;
+      // Four loads under tests are not one load in front of them: their index need only be one where a test holds.  (Next to
+      // one element that is read anyhow the other three of its 16 bytes may be read as well.)
+      bool safe = a0.store;
+      for (int c = 0; c < 4; ++c) safe = safe || acc[member[c]].always;
+      if (!safe) continue;
       // each element of the array may appear once in the group's direction (a second load of a[4q] keeps its place)
       size_t first = i, last = i;
       for (int c = 0; c < 4; ++c) { first = std::min(first, member[c]); last = std::max(last, member[c]); }

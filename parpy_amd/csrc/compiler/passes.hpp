@@ -67,4 +67,10 @@ std::string hip_print_listing(const Program& p, const Options& opts);
 
 using DebugHook = std::function<void(const std::string& stage, const std::string& text)>;
 
+// operand q of e may be left unevaluated (the branches of a selection, the right side of `and` / `or`): an index in it
+// need only be in bounds where it is evaluated, so nothing may be loaded from there ahead of the test
+inline bool may_skip(const E& e, size_t q) {
+  return q > 0 && (e->k == Expr::IfExpr || (e->k == Expr::BinOpE && (e->bop == BinOp::And || e->bop == BinOp::Or)));
+}
+
 }  // namespace parpy
