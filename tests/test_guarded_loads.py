@@ -38,7 +38,7 @@ def ragged_groups(idx, x, y, N):
         k = idx[i]
         s = x[4 * k]
         for c in range(1, 4):
-            s = s + (x[4 * k + c] if y[i] > float(c) else float32(0.0))
+            s = s + (x[4 * k + c] if y[i] > float32(0.5) else float32(0.0))
         y[i] = s
 
 
