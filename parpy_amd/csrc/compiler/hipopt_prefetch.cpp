@@ -154,6 +154,20 @@ Stmts Pass::prefetch_selected_rows(const Stmts& ss, int64_t* budget) {
         }
       };
       collect_defs(*is.body);
+      // elements that every iteration reads: a row of which tests let some be read only may not be there to fetch
+      std::vector<std::pair<Name, E>> read_anyhow;
+      std::function<void(const E&)> note_loads = [&](const E& x) {
+        if (!x) return;
+        if (x->k == Expr::Index && x->args[0]->k == Expr::Var) read_anyhow.push_back({x->args[0]->name, fold_expr(subst_vars(x->args[1], defs))});
+        for (size_t q = 0; q < x->args.size(); ++q) if (!may_skip(x, q)) note_loads(x->args[q]);
+      };
+      std::function<void(const Stmts&)> note = [&](const Stmts& b) {
+        for (auto& d : b) {
+          for (const E& e : {d->expr, d->dst, d->lo, d->hi}) note_loads(e);
+          if (d->k == Stmt::For && const_extent(d) > 0) note(d->body);
+        }
+      };
+      note(*is.body);
       struct Row { E load; Name reg; ElemSize sz; };
       std::vector<Row> rows;
       auto take = [&](const E& e) -> E {
@@ -168,6 +182,9 @@ Stmts Pass::prefetch_selected_rows(const Stmts& ss, int64_t* budget) {
           if (x->k == Expr::Index || x->k == Expr::RegElem || x->k == Expr::ThreadIdx || x->k == Expr::Call || x->k == Expr::Raw) ok = false;
         });
         if (!selected || !ok) return e;
+        bool anyhow = false;
+        for (auto& l : read_anyhow) anyhow = anyhow || (l.first == base && expr_eq(l.second, idx));
+        if (!anyhow) return e;
         auto elem = [&](const Name& reg) {
           auto re = std::make_shared<Expr>();
           re->k = Expr::RegElem;

@@ -47,3 +47,49 @@ def test_four_loads_under_tests_are_not_packed():
     assert "parpy_vec4<float> pk_" not in kernel(padded_groups, args, {'i': parpy.threads(1000)})
     # one of them is read anyhow: the others lie in the same 16 bytes
     assert "parpy_vec4<float> pk_" in kernel(ragged_groups, args, {'i': parpy.threads(1000)})
+
+
+def padded_steps(data, lens, tab, a, b, N, S, T):
+    parpy.label('i')
+    for i in range(N):
+        parpy.label('s')
+        for s in range(S):
+            a[i, s] = 0.0
+        for t in range(1, T):
+            src = a
+            dst = b
+            if t & 1:
+                src = b
+                dst = a
+            o = data[i, t]
+            parpy.label('s')
+            for s in range(S):
+                dst[i, s] = src[i, (s + 1) % S] + (tab[o, s] if o >= 0 else float32(0.0))
+
+
+def steps(data, lens, tab, a, b, N, S, T):
+    parpy.label('i')
+    for i in range(N):
+        parpy.label('s')
+        for s in range(S):
+            a[i, s] = 0.0
+        for t in range(1, T):
+            src = a
+            dst = b
+            if t & 1:
+                src = b
+                dst = a
+            o = data[i, t]
+            parpy.label('s')
+            for s in range(S):
+                dst[i, s] = src[i, (s + 1) % S] + tab[o, s]
+
+
+STEP_ARGS = [np.zeros((8, 50), np.int8), np.zeros(8, np.int64), np.zeros((101, 256), np.float32), np.zeros((8, 256), np.float32), np.zeros((8, 256), np.float32), 8, 256, 50]
+
+
+def test_rows_read_under_a_test_are_not_fetched_a_step_ahead():
+    par = {'i': parpy.threads(8), 's': parpy.threads(256)}
+    k = kernel(padded_steps, STEP_ARGS, par)
+    assert "row_tab" not in k and re.search(r"o_\d+\) >= 0\) \? (tab_\d+\[|parpy_at\(tab_)", k)
+    assert "row_tab" in kernel(steps, STEP_ARGS, par)
