@@ -13,7 +13,9 @@ namespace hipopt {
 // emission row).  The array is never written and the address is a function of t and of values that
 // do not change in the loop, so the load for step t + 1 is issued at the start of step t into a second
 // variable: its latency passes behind a whole step of work.  The index must be provably in bounds
-// over the static range of the loop (the last iteration re-reads its own element instead of t + 1).
+// over the static range of the loop.  The last iteration re-reads its own element instead of t + 1: where
+// the loop ends at run time (a read's length), what stands behind its end may be padding that nothing
+// else may be selected with.
 Stmts Pass::prefetch_counter_loads(const Stmts& ss, RangeEnv env) {
   std::set<Name> params = param_names();
   std::set<Name> written = written_arrays();
@@ -47,6 +49,8 @@ Stmts Pass::prefetch_counter_loads(const Stmts& ss, RangeEnv env) {
       tr.hi = HI - 1;
       le[s->id] = tr;
       Stmts pre, body;
+      E last = mk_int(HI - 1, s->lo->ty.sz);
+      if (s->hi->k != Expr::Int) last = mk_var(gen.fresh(s->id.s + "_last"), s->lo->ty);
       for (auto& c : s->body) {
         E ld = c->k == Stmt::Def && c->expr ? strip_converts(c->expr) : E();
         bool ok = ld && ld->k == Expr::Index && c->ty.is_scalar() && !reassigned.count(c->id) && ld->args[0]->k == Expr::Var &&
@@ -72,10 +76,15 @@ Stmts Pass::prefetch_counter_loads(const Stmts& ss, RangeEnv env) {
         Name nxt = gen.fresh(c->id.s + "_next");
         pre.push_back(mk_def(nxt, c->ty, at(s->lo), c->i));
         body.push_back(mk_def(c->id, c->ty, mk_var(nxt, c->ty), c->i));
-        E t1 = mk_binop(BinOp::Min, mk_binop(BinOp::Add, mk_var(s->id, ity), mk_int(1, ity.sz), ity), mk_int(HI - 1, ity.sz), ity);
+        E t1 = mk_binop(BinOp::Min, mk_binop(BinOp::Add, mk_var(s->id, ity), mk_int(1, ity.sz), ity), last, ity);
         body.push_back(mk_assign(mk_var(nxt, c->ty), at(t1), c->i));
       }
       if (!pre.empty()) {
+        if (last->k == Expr::Var) {   // (within the static range also where there is no iteration: the address stays in 32 bits)
+          E end = mk_binop(BinOp::Min, mk_binop(BinOp::Sub, s->hi, mk_int(1, s->hi->ty.sz), s->hi->ty), mk_int(HI - 1, s->hi->ty.sz), s->hi->ty);
+          if (end->ty.sz != last->ty.sz) end = mk_convert(end, last->ty.sz);
+          out.push_back(mk_def(last->name, last->ty, mk_binop(BinOp::Max, end, s->lo, last->ty), s->i));
+        }
         for (auto& d : pre) out.push_back(d);
         auto r = clone(s);
         r->body = body;
@@ -249,7 +258,9 @@ Stmts Pass::prefetch_selected_rows(const Stmts& ss, int64_t* budget) {
         d->iv = is.slots;
         pre.push_back(d);
       }
-      pre.push_back(fill_nest());
+      // (a loop that ends at run time may have no first step, whose row might then be any)
+      if (s->lo->k == Expr::Int && s->hi->k == Expr::Int && s->lo->iv < s->hi->iv) pre.push_back(fill_nest());
+      else pre.push_back(mk_if(mk_binop(BinOp::Lt, s->lo, s->hi, Type::scalar(ElemSize::Bool)), {fill_nest()}, {}));
       auto nc = clone(c);
       nc->unroll = true;
       if (is.inner) {
