@@ -106,6 +106,26 @@ def ended_steps(data, lens, tab, a, b, N, S, T):
                     dst[i, s] = src[i, (s + 1) % S] + tab[o, s]
 
 
+def offset_steps(data, lens, tab, a, b, N, S, T):
+    parpy.label('i')
+    for i in range(N):
+        parpy.label('s')
+        for s in range(S):
+            a[i, s] = 0.0
+            b[i, s] = 0.0
+        for t in range(1, T):
+            src = a
+            dst = b
+            if t & 1:
+                src = b
+                dst = a
+            o = data[i, t]
+            parpy.label('s')
+            for s in range(S):
+                if t < lens[i]:
+                    dst[i, s] = src[i, (s + 1) % S] + tab[o - 1, s]
+
+
 STEP_ARGS = [np.zeros((8, 50), np.int8), np.zeros(8, np.int64), np.zeros((101, 256), np.float32), np.zeros((8, 256), np.float32), np.zeros((8, 256), np.float32), 8, 256, 50]
 
 
@@ -123,6 +143,11 @@ def test_the_step_past_the_end_selects_nothing():
     assert re.search(r"int t_last_\d+ = parpy_max<int64_t>\(parpy_min<int64_t>\(\(t_end_\d+ - \(int64_t\)\(1\)\), ", k)
     assert re.search(r"o_next_\d+ = .*parpy_min<int>\(\(t_\d+ \+ 1\), t_last_\d+\)", k)
     first = k[:k.index("for (int t_")]
+    assert re.search(r"o_first_\d+ = \(\(1 < t_end_\d+\) \? o_next_\d+ : \(\(int8_t\)0\)\);", first)
+    assert re.search(r"row_tab_\d+\[0\] = tab_\d+\[\(\(\(int\)\(o_first_\d+\) \* 256\)", first) and first.count("row_tab") == 2
+    # an index that is more than the observation itself: no number stands for a row that is there
+    first = kernel(offset_steps, STEP_ARGS, {'i': parpy.threads(8), 's': parpy.threads(256)})
+    first = first[:first.index("for (int t_")]
     assert re.search(r"if \(1 < t_end_\d+\) \{\s*\{[^}]*row_tab_\d+\[0\] = ", first) and first.count("row_tab") == 2
 
 
