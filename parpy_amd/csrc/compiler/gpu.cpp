@@ -145,8 +145,13 @@ struct Restructure {
   // 256 threads as make four for every compute unit, up to 128 per row, with eight 16-byte vectors per thread and more.
   // Handing over the partial results costs 1 to 3 us, so only for rows of 320 KB, and of 8 KB for each row there is: one
   // row of 190000 doubles 15.8 -> 3.8 us, 30 of 150001 doubles 19.3 -> 14.0, 30 of 100000 floats 7.9 -> 6.8, 100 of 1000001
-  // floats 143 -> 69 (on 256 threads asked for; the whole workgroup of 1024 that a program asks for by that number it
-  // gets, one workgroup and no more: the shape that the row-sum example compares with several); but 30 of 40000 floats 4.6 -> 5.5, 100 of 150000 13.3 -> 16.3, 255 of 390000 65.4 -> 67.9.
+  // floats 143 -> 69 (on 256 threads asked for); but 30 of 40000 floats 4.6 -> 5.5, 100 of 150000 13.3 -> 16.3, 255 of 390000
+  // 65.4 -> 67.9.
+  // The whole workgroup of 1024 threads, asked for by that number, stays one workgroup.  It is the shape that programs compare
+  // with a split of their own, and the line would lie elsewhere, because it reads faster than a smaller one: spread by this
+  // rule, 100 rows of 1000001 floats 141 -> 67, 2 of 10^6 29.5 -> 5.0, one of 190000 doubles 11.8 -> 4.0, but 200 of 500000
+  // floats 59 -> 68, 64 of 65536 doubles 7.1 -> 9.5, 30 of 100000 floats 5.6 -> 6.1.  (So more threads asked for can be the
+  // slower request: the 100 rows take 67 us on 512.)
   static int64_t literal_extent(const S& s) {
     return s->step == 1 && s->lo->k == Expr::Int && s->lo->iv == 0 && s->hi->k == Expr::Int ? s->hi->iv : 0;
   }

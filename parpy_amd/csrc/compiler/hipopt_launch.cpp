@@ -263,14 +263,16 @@ struct LaneSplit {
   // memory.  Neighbours mostly have one row in common (non-zeros sorted by rows or columns): the group loads it once and
   // tests whether the second iteration's is another one; a quarter of the 16-byte pieces that pass through L1 go away.
   // 655360 products over 128 floats out of a 4 MiB table: 27.9 -> 21.6 us (four iterations 22.4), over 64 floats 19.4 ->
-  // 15.1, 262144 over 128 out of 1 MiB 10.7 -> 8.8.  Not for rows of more than 512 bytes (256 floats: 37.4 -> 43.1, the
-  // registers of three rows), nor for tables that one die's L2 does not hold (8 MiB: 43.9 -> 45.7), nor for launches that run
-  // at once as they are.
+  // 15.1, 262144 over 128 out of 1 MiB 10.7 -> 8.8.  Three rows are in registers at a time, 16 bytes of each per lane and
+  // round, and 48 registers of them leave a SIMD its wavefronts: not for rows of more than 512 bytes (256 floats: 37.4 ->
+  // 43.1).  Nor for tables that the 4 MiB L2 of a die does not hold, where the pieces come from farther than L1 anyway (8 MiB:
+  // 43.9 -> 45.7), nor for launches that run at once as they are.
+  static constexpr int64_t ROW_REGISTERS = 48, L2_OF_A_DIE = int64_t(4) << 20;
   bool pair(Kernel& k, const StmtP& launch, const S& root, size_t pos, int vec, const E& term) {
     const S& loop = root->body[pos];
     const E& acc = loop->body[0]->dst;
     const int64_t N = root->hi->iv, K = loop->hi->iv, rounds = K / (vec * G);
-    if (acc->k != Expr::Var || K % (vec * G) != 0 || rounds > 4 || N * G <= 2 * 256 * 2048) return false;
+    if (acc->k != Expr::Var || K % (vec * G) != 0 || 3 * rounds * 4 > ROW_REGISTERS || N * G <= 2 * 256 * 2048) return false;
     if (!(term->k == Expr::BinOpE && term->bop == BinOp::Mul)) return false;
     E x = term->args[0], y = term->args[1];
     for (const E& e : {x, y})
@@ -284,7 +286,7 @@ struct LaneSplit {
     if (swapped) std::swap(x, y);
     int64_t table = elem_bytes(y->ty.sz);
     for (int64_t d : y->dim_shape) table *= d;
-    if (y->dim_shape.empty() || table > (int64_t(4) << 20)) return false;
+    if (y->dim_shape.empty() || table > L2_OF_A_DIE) return false;
     std::set<Name> from_memory;
     bool zero = false;
     for (size_t q = 0; q < pos; ++q) {

@@ -220,7 +220,10 @@ struct Stages {
     int64_t results = 1;
     for (auto& o : f.outer) results *= o->hi->iv;
     // Workgroups of fewer than 256 threads are there only because the program names that size: the split it names with it,
-    // two launches and the temporary between them (which callers of the entry without allocations make room for) stay.
+    // two launches and the temporary between them, stay.  Split further and in one launch they are no faster on the whole:
+    // 100 rows of 65536 floats on 1024 threads in workgroups of 128 6.8 us as named, 11.2 so; 10 of 10^6 on 8192 in 128 12.6
+    // and 16.3; 1000 of 65536 on 512 in 128 40.3 and 40.9; 37 of 3000 on 256 in 128 6.3 and 5.2; 10 of 10^6 on 2048 in 64
+    // 17.9 and 16.5; one of 10^7 on 8192 in 64 28.5 and 26.2.
     const bool named = threads < 256;
     while (!named && nb < 128 && results * nb * threads < 2048 * WAVE_SIZE && vectors / (nb * threads) >= 16) { split *= 2; nb *= 2; }
     const int64_t share = (vectors + nb - 1) / nb;
