@@ -25,8 +25,9 @@ namespace {
 //   * The arithmetic of an element is that of the statement as written: same operations, same order.
 //
 // A three-point average back and forth over 10^6 float64 elements, 98 updates: 447 us as launches of 4.5 us each, 51 us
-// in two launches of 25 steps; the vector ALU is then what bounds it (two additions and a division in four
-// instructions per element and update, a quarter of them in the margins).
+// in two launches of 25 steps.  Two additions and a division in four instructions per element and update, a quarter of them
+// in the margins: counted, a SIMD issues vector instructions 52 % of the time, 63 % where three of the 2504 wavefronts share
+// it; the rest is the latency of dependent steps.
 struct TimeTile {
   Program& p;
   const Options& opts;
