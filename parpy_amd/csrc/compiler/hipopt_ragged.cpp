@@ -228,6 +228,15 @@ struct RaggedSum {
 
   static int64_t pow2_at_least(int64_t n) { int64_t q = 1; while (q < n) q *= 2; return q; }
 
+  // a[v + c] and a[v + c + 1]
+  static bool adjacent(E a, E b, const Name& v) {
+    while (a->k == Expr::Convert) a = a->args[0];
+    while (b->k == Expr::Convert) b = b->args[0];
+    if (a->k != Expr::Index || b->k != Expr::Index || !expr_eq(a->args[0], b->args[0])) return false;
+    E ra, rb;
+    return affine_unit(a->args[1], v, &ra) && affine_unit(b->args[1], v, &rb) && ra->k == Expr::Int && rb->k == Expr::Int && rb->iv == ra->iv + 1;
+  }
+
   bool apply(Kernel& k, const StmtP& launch) {
     Rows r;
     if (!match(k, r)) return false;
@@ -385,9 +394,19 @@ struct RaggedSum {
     };
     auto bounds = [&](Stmts& ss, E* lo, E* hi) {
       for (auto& st : r.pre) ss.push_back(st);
-      Name ln = gen.fresh("first"), hn = gen.fresh("end");
-      ss.push_back(mk_def(ln, ety, narrow(r.loop->lo), r.loop->i));
-      ss.push_back(mk_def(hn, ety, narrow(r.loop->hi), r.loop->i));
+      // (the bounds of a row without elements may be anything, a marker like 2^63 - 1 and 0: what is cut to 32 bits of them, or
+      // passes the largest integer when a lane's place is added, must not become a row)
+      Name lw = gen.fresh("lo"), hw = gen.fresh("hi"), any = gen.fresh("any"), ln = gen.fresh("first"), hn = gen.fresh("end");
+      E l = mk_var(lw, ity), h = mk_var(hw, ity), some = mk_var(any, bty);
+      // (`rows[row] .. rows[row + 1]` in the plain form of an index, whose neighbours the device compiler joins to one load: with
+      // 32-bit offsets two loads of eight bytes, 52.0 us for SpMV with 100 000 rows of 50, 50.4 so, 50.0 unchecked)
+      std::map<Name, E> plain;
+      if (adjacent(r.loop->lo, r.loop->hi, r.row)) plain[r.row] = mk_raw(r.row.str(), ity);
+      ss.push_back(mk_def(lw, ity, subst_vars(r.loop->lo, plain), r.loop->i));
+      ss.push_back(mk_def(hw, ity, subst_vars(r.loop->hi, plain), r.loop->i));
+      ss.push_back(mk_def(any, bty, mk_binop(BinOp::Lt, l, h, bty), r.loop->i));
+      ss.push_back(mk_def(ln, ety, narrow(mk_ifexpr(some, l, iint(0), ity)), r.loop->i));
+      ss.push_back(mk_def(hn, ety, narrow(mk_ifexpr(some, h, iint(0), ity)), r.loop->i));
       *lo = mk_var(ln, ety);
       *hi = mk_var(hn, ety);
     };

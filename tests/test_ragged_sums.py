@@ -1,6 +1,8 @@
 """Sums over rows of uneven length (bounds that are data): teams of lanes per row, very long rows shared by a workgroup,
 with and without columns; row counts, row lengths and column counts at the edges of what a team, a batch, a wavefront
 and the queue of long rows hold.  The expectation is NumPy in float64."""
+import re
+
 import numpy as np
 import pytest
 
@@ -70,6 +72,16 @@ def guarded(A, x, y):
             y[row] += x[i] if i < 100 else 0.0
 
 
+def ranges(first, end, x, y, n):
+    """Every row with a first and a last element of its own."""
+    parpy.label('row')
+    for row in range(n):
+        y[row] = 0.0
+        parpy.label('i')
+        for i in range(first[row], end[row]):
+            y[row] += x[i]
+
+
 def bounded(A, x, perm, y):
     parpy.label('row')
     for row in range(A["nrows"]):
@@ -117,7 +129,6 @@ def test_long_rows_are_queued_for_the_workgroup():
 
 def test_loads_under_a_test_stay_under_it():
     """What a selection or a short-circuit operator may skip is not evaluated in front of the term: its index need not be one."""
-    import re
     A, x, perm, y = matrix(5000, 300, np.float64, 1), np.zeros(300), np.zeros(300, dtype=np.int64), np.zeros(5000)
     for f, skipped in ((padded, ("perm",)), (bounded, ("perm", "cols"))):
         s = parpy.print_compiled(f, [A, x, perm, y], opts_for({"row": parpy.threads(5000)}))
@@ -140,6 +151,32 @@ def test_loop_variables_are_narrowed_by_arrays_that_every_element_reads():
         return s[:s.index("// host side")]
 
     assert "int32_t end_" in kernel(summed) and "int64_t end_" in kernel(guarded)
+
+
+def test_rows_without_elements_have_bounds_of_zero():
+    v = np.zeros(5000, dtype=np.int64)
+    for f, args in ((ranges, [v, v.copy(), np.zeros(100000), np.zeros(5000), 5000]), (guarded, [matrix(5000, 300, np.float64, 1), np.zeros(100), np.zeros(5000)])):
+        s = parpy.print_compiled(f, args, opts_for({"row": parpy.threads(5000)}))
+        s = s[:s.index("// host side")]
+        hiprtc_compile(s, opts_for({}))
+        bounds = re.findall(r"int\d+_t (?:first|end)_\d+ = (.*);", s[s.rindex('extern "C"'):])
+        assert len(bounds) == 4 and all(re.search(r"any_\d+ \? (lo|hi)_\d+ : 0", b) for b in bounds), bounds
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [64, 1000, 20001])
+def test_rows_whose_bounds_mark_that_they_are_empty(n):
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(5000)
+    first = rng.integers(0, 4900, n)
+    end = first + rng.integers(1, 100, n)
+    end[:3], first[:3] = 5000, 0
+    for q, (a, b) in enumerate([(2**63 - 1, 0), (2**63 - 1, -2**63), (2**32, 3), (7, 7), (2**31 + 5, 4), (100, 50), (-1, -1)]):
+        first[q + 5::11], end[q + 5::11] = a, b
+    y = np.full(n, np.nan)
+    parpy.jit(ranges)(first, end, x, y, n, opts=opts_for({"row": parpy.threads(n)}))
+    want = np.array([x[a:b].sum() if a < b else 0.0 for a, b in zip(first.tolist(), end.tolist())])
+    assert np.allclose(y, want, atol=1e-10)   # (5000 terms of order one: 5000 * 5000 * 2^-53)
 
 
 @pytest.mark.gpu
