@@ -69,6 +69,7 @@ struct Pointers {
 bool put_value(std::string& k, PyObject* v, Pointers& ps) {
   if (Py_TYPE(v) == (PyTypeObject*)THPVariableClass) {
     const at::Tensor& t = THPVariable_Unpack(v);
+    if (t.is_neg() || t.is_conj()) return false;   // (what stands in memory is not the value)
     if (t.dim() == 0) {
       if (t.is_cuda() || t.layout() != c10::kStrided || !t.device().is_cpu()) return false;
       put_tag(k, 's');

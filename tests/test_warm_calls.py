@@ -60,6 +60,16 @@ def test_tensors_without_memory_of_their_own_are_left_to_the_python_path():
     assert table.add((torch.tensor(2.0),), opts(), 1000, ()) and table.run((torch.tensor(2.0),), {"opts": opts()}) == 0
 
 
+def test_a_scalar_whose_memory_holds_its_negative_is_left_to_the_python_path():
+    from parpy_amd import fastcall
+    run = ctypes.CFUNCTYPE(ctypes.c_int32, ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p), ctypes.c_int32)(lambda plan, p, n: 0)
+    table = fastcall._load().CallTable(CompileOptions, LoopPar, ctypes.cast(run, ctypes.c_void_p).value)
+    v = torch.tensor(1 + 2j).conj().imag
+    assert v.is_neg() and v.item() == -2.0
+    assert not table.add((v,), opts(), 1000, ()) and table.run((torch.tensor(2.0),), {"opts": opts()}) is None
+    assert table.run((v,), {"opts": opts()}) is None
+
+
 def plain_calls(monkeypatch, f):
     """`f` as a jitted function of scalars whose calls reach the warm path without a device; returns it and the list of its runs."""
     from parpy_amd import runtime
