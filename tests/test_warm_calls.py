@@ -70,6 +70,14 @@ def test_a_scalar_whose_memory_holds_its_negative_is_left_to_the_python_path():
     assert table.run((v,), {"opts": opts()}) is None
 
 
+def test_the_two_zeros_are_different_values():
+    from parpy_amd.key import _describe_argument
+    from parpy_amd.validate import check_arguments
+    values = (0.0, -0.0, torch.tensor(0.0), torch.tensor(-0.0), 0, False, 1.5, 1, True)
+    assert len({parpy._call_signature((x,))[0] for x in values}) == len(values)
+    assert len({_describe_argument(check_arguments((x,), opts(backend=HIP), False)[0]) for x in values}) == len(values)
+
+
 def plain_calls(monkeypatch, f):
     """`f` as a jitted function of scalars whose calls reach the warm path without a device; returns it and the list of its runs."""
     from parpy_amd import runtime
