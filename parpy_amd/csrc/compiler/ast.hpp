@@ -281,6 +281,7 @@ struct Stmt {
   std::vector<E> args;
   Dim3 grid, block;
   bool unroll = false;    // For: emit an unroll pragma
+  bool in_pairs = false;  // For: a time loop whose iterations are compiled once for odd and once for even values of its variable
 };
 
 S mk_def(const Name& id, const Type& ty, E expr, const Info& i = Info());
@@ -406,6 +407,7 @@ struct Options {  // src/option.rs:14-108
   bool opt_share_iterations = true;   // what all iterations of one thread have in common is evaluated once per thread
   bool opt_keep_own = false;     // ... and across steps when source and destination swap every step (own elements never re-read from LDS)
   bool opt_keep_stored = true;   // values a thread stores and reads back itself later in the same step stay in registers
+  bool opt_pair_steps = true;         // a time loop whose steps swap two arrays in LDS is written out for two steps
   bool opt_fence_iterations = true;   // the unrolled iterations of a thread that read and write LDS are scheduled one after the other
   bool opt_tile_steps = true;         // several steps of a host loop of element-wise launches run in one launch
   bool opt_expand_short_loops = true; // counted loops of <= 8 iterations inside a parallel iteration are expanded in place

@@ -88,6 +88,9 @@ void hip_optimize(Program& p, const Options& opts, NameGen& gen) {
     if (opts.opt_drop_barriers) pass.drop_barriers();
     k.distinct_pointers.clear();
     k.body = pass.noalias_scopes(k.body, opts.opt_noalias_scopes);
+    // (where the passes above have taken the registers, what two steps share and load early does not fit beside it: the
+    // headline kernel would spill six, the reference form of 7-mers runs 11.4 -> 12.3 ms, 16 layers of 5-mers 11.9 -> 12.5)
+    if (opts.opt_pair_steps && budget >= 16) k.body = pass.pair_steps(k.body);
     k.fence_lds_iterations = opts.opt_fence_iterations && !pass.step_has_transcendentals();
     pass.mark_read_only();
     k.aligned_params = opts.assume_aligned;

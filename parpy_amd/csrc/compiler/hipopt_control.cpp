@@ -225,6 +225,51 @@ Stmts Pass::expand_short_loops(const Stmts& ss0, bool in_par) {
   return out;
 }
 
+// ================================================================ steps that swap two arrays, two at a time
+// `for t: src = a; dst = b; if (t & 1) { src = b; dst = a; } <step>`: the step is written out twice, once for each parity,
+// and the arrays of each are known (the base of an LDS access becomes part of the instruction, and a load and a store are
+// seen not to coincide).  100 reads of 1000 to 3000 samples, scaled form: 16-layer models of 3- / 4- / 5-mers 1733 -> 1069 us,
+// 2335 -> 1547, 3487 -> 2955; single layer, 4- / 5- / 6-mers 587 -> 503, 810 -> 725, 1256 -> 1090; reference form, 3- / 4- /
+// 5-mers 531 -> 398, 655 -> 530, 1034 -> 926.  One of 21 got slower: 16 layers of 3-mers, reference form, 1169 -> 1219.
+Stmts Pass::pair_steps(const Stmts& ss) {
+  static const char* const PARITY = "parpy_odd.value";
+  Stmts out;
+  for (auto& s : ss) {
+    auto r = clone(s);
+    r->body = pair_steps(s->body);
+    if (s->k != Stmt::For || s->map.k == GpuMap::None) r->els = pair_steps(s->els);
+    bool swaps = false, barrier = false, plain = true;
+    if (s->k == Stmt::For && s->map.k == GpuMap::None && !s->unroll && s->step == 1 && s->lo->k == Expr::Int && s->els.empty()) {
+      for (auto& c : s->body) {
+        if (c->k == Stmt::Sync) barrier = true;
+        if (c->k == Stmt::If && alternates(c->expr, s))
+          for (auto& d : c->body)
+            if (d->k == Stmt::Assign && d->dst->k == Expr::Var && d->dst->ty.is_pointer() && d->dst->ty.mem == Mem::LDS) swaps = true;
+      }
+      visit_stmts(s->body, [&](const S& c) { if ((c->k == Stmt::RawStmt && c->fname.rfind("__builtin_amdgcn_wave_barrier", 0) != 0) || c->k == Stmt::Return || (c->k == Stmt::Assign && c->dst->k == Expr::Var && c->dst->name == s->id)) plain = false; });
+    }
+    if (!(swaps && barrier && plain)) { out.push_back(r); continue; }
+    // the tests of the parity become constants of the copy
+    const Type bty = Type::scalar(ElemSize::Bool);
+    const E is_odd = mk_raw(PARITY, bty);
+    auto counter = [&](const E& e) { const E v = strip_converts(e); return v->k == Expr::Var && v->name == s->id; };
+    r->body = rewrite_stmts(r->body, [&](const E& e) -> E {
+      if (e->k != Expr::BinOpE || e->args[1]->k != Expr::Int) return e;
+      const int64_t c = e->args[1]->iv;
+      if (e->bop == BinOp::BitAnd && c == 1 && counter(e->args[0])) return is_odd;
+      if (e->bop == BinOp::Eq && c % 2 == 0) {   // `t % 8 == 0`
+        const E rem = strip_converts(e->args[0]);
+        if (rem->k == Expr::BinOpE && rem->bop == BinOp::Rem && counter(rem->args[0]) && rem->args[1]->k == Expr::Int && rem->args[1]->iv > 0 && rem->args[1]->iv % 2 == 0)
+          return mk_binop(BinOp::And, mk_unop(UnOp::Not, is_odd, bty), e, bty, e->i);
+      }
+      return e;
+    });
+    r->in_pairs = true;
+    out.push_back(r);
+  }
+  return out;
+}
+
 // ================================================================ guards that only ever switch off
 // `for t in range(lo, hi): ... if t < X: <work>` where X does not change while the loop runs, every
 // effect of the body sits under that test and X is the same for all threads of the workgroup: once

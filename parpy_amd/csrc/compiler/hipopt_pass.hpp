@@ -90,6 +90,7 @@ struct Pass {
   Stmts expand_short_loops(const Stmts& ss0, bool in_par);
   static E strip_converts(const E& e);
   Stmts guards_to_bounds(const Stmts& ss);
+  Stmts pair_steps(const Stmts& ss);
   Stmts hoist_uniform_conditions(const Stmts& ss);
   Stmts if_convert(const Stmts& ss);
   Stmts if_convert(const Stmts& ss, const std::set<Name>& nonzero_const);

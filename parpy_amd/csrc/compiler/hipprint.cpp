@@ -102,6 +102,7 @@ template <class T> __device__ __forceinline__ T parpy_readlane(T v, int lane) {
     return __builtin_bit_cast(T, (unsigned char)__builtin_amdgcn_readlane((int)__builtin_bit_cast(unsigned char, v), lane));
   }
 }
+template <bool B> struct parpy_flag { static constexpr bool value = B; };   // a constant that a function object is called with
 struct parpy_op_add { template <class T> __device__ __forceinline__ T operator()(T a, T b) const { return a + b; } };
 struct parpy_op_mul { template <class T> __device__ __forceinline__ T operator()(T a, T b) const { return a * b; } };
 struct parpy_op_and { template <class T> __device__ __forceinline__ T operator()(T a, T b) const { return a & b; } };
@@ -788,7 +789,23 @@ struct DevicePrinter {
       bool fresh = !s->unroll && seq_loop_vars.insert(s->id).second;
       in_unrolled += s->unroll;
       in_unaligned += s->unroll && s->iv != 0;
-      pstmts(s->body, n + 2);
+      if (s->in_pairs) {
+        // the step as a function of the parity and of the counter; the inner loop runs pairs, the odd one out stands behind
+        // it (behind a test between the two steps of a pair, the loads that the first one issues for the second would be
+        // moved to where they are used)
+        const bool odd = s->lo->iv & 1;
+        const std::string end = v + "_stop";
+        auto call = [&](bool o, const std::string& t) { return "parpy_step(parpy_flag<" + std::string(o ? "true" : "false") + ">(), " + t + ");\n"; };
+        os << ind(n + 2) << "const auto parpy_step = [&](auto parpy_odd, const " << vty << " " << v << ") __attribute__((always_inline)) {\n";
+        pstmts(s->body, n + 4);
+        os << ind(n + 2) << "};\n";
+        os << ind(n + 2) << "const " << vty << " " << end << " = " << his << ";\n";
+        os << ind(n + 2) << "for (; " << v << " + 1 < " << end << "; " << v << " += 2) {\n";
+        os << ind(n + 4) << call(odd, v) << ind(n + 4) << call(!odd, v + " + 1") << ind(n + 2) << "}\n";
+        os << ind(n + 2) << "if (" << v << " < " << end << ") " << call(odd, v);
+      } else {
+        pstmts(s->body, n + 2);
+      }
       in_unrolled -= s->unroll;
       in_unaligned -= s->unroll && s->iv != 0;
       if (fresh) seq_loop_vars.erase(s->id);

@@ -96,6 +96,7 @@ Options parse_options(const std::string& sexpr) {
     else if (h == "opt_guard_bounds") o.opt_guard_bounds = flag();
     else if (h == "opt_pack_accesses") o.opt_pack_accesses = flag();
     else if (h == "opt_share_iterations") o.opt_share_iterations = flag();
+    else if (h == "opt_pair_steps") o.opt_pair_steps = flag();
     else if (h == "opt_fence_iterations") o.opt_fence_iterations = flag();
     else if (h == "opt_tile_steps") o.opt_tile_steps = flag();
     else if (h == "opt_keep_stored") o.opt_keep_stored = flag();

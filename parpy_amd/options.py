@@ -264,6 +264,7 @@ class CompileOptions:
         'opt_guard_bounds': None,
         'opt_pack_accesses': None,
         'opt_share_iterations': None,
+        'opt_pair_steps': None,
         'opt_fence_iterations': None,
         'opt_keep_stored': None,
         'opt_keep_own': None,

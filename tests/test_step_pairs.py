@@ -1,0 +1,57 @@
+"""Time loops whose steps swap two arrays in LDS, compiled once for odd and once for even steps: reads that end in the first,
+the second and the odd step out, against the float64 oracle and the loop that is not taken apart."""
+import numpy as np
+import pytest
+
+import oracle
+import parpy_amd as parpy
+from parpy_amd import workloads as W
+
+torch = pytest.importorskip("torch")
+
+
+def opts(n, threads, **kw):
+    o = parpy.par({'inst': parpy.threads(n), 'state': parpy.threads(threads)})
+    for name, value in kw.items():
+        setattr(o, name, value)
+    return o
+
+
+def text(k, threads, **kw):
+    hmm, seqs = W.synthetic_hmm(k, n_inst=4, min_len=10, max_len=30)
+    a = np.zeros((4, hmm["num_states"]), dtype=np.float32)
+    o = opts(4, threads, **kw)
+    return parpy.print_compiled(W.forward_syn, [hmm, seqs, np.zeros(4, dtype=np.float32), a, a.copy()], o)
+
+
+def test_one_text_for_both_parities():
+    s = text(5, 1024)
+    assert s.count("const auto parpy_step = [&](auto parpy_odd, const int t_") == 1 and s.count("if (parpy_odd.value) {") == 1
+    assert "parpy_step(parpy_flag<true>()" in s and "parpy_step(parpy_flag<false>()" in s
+    assert "parpy_step" not in text(5, 1024, opt_pair_steps=False)
+    assert "parpy_step" not in text(7, 1024)      # the registers of a thread are taken by its tables
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["reference", "grouped", "scaled"])
+@pytest.mark.parametrize("k,threads", [(3, 64), (4, 64), (5, 256)])
+def test_reads_of_odd_and_even_length(k, threads, form):
+    n = 12
+    hmm, seqs = W.synthetic_hmm(k, n_inst=n, min_len=20, max_len=41)
+    seqs["lens"][:6] = [1, 2, 3, 4, 5, 6]
+    got = {}
+    for pairs in (True, False):
+        hd, sd = W.to_device(hmm), W.to_device(seqs)
+        if form != "reference":
+            hd = W.scaled_tables_on_device(hd)
+        a1 = torch.zeros((n, hmm["num_states"]), dtype=torch.float32, device="cuda")
+        a2 = torch.zeros_like(a1)
+        res = torch.zeros(n, dtype=torch.float64 if form == "scaled" else torch.float32, device="cuda")
+        f = {"reference": W.forward_syn, "grouped": W.forward_syn4, "scaled": W.forward_scaled}[form]
+        f(hd, sd, res, a1, a2, opts=opts(n, threads, opt_pair_steps=pairs))
+        got[pairs] = [x.double().cpu().numpy() for x in (res, a1, a2)]
+    want = oracle.hmm_syn_forward(hmm, seqs, np.float64)
+    # 41 steps of half a unit in the last place of scores up to 256 (single precision); the scaled form keeps 1e-4
+    assert np.abs(got[True][0] - want).max() < (1e-4 if form == "scaled" else 41 * 2.0 ** -16)
+    for with_pairs, without in zip(got[True], got[False]):
+        np.testing.assert_allclose(with_pairs, without, rtol=1e-5, atol=1e-5 if form != "scaled" else 1e-30)
