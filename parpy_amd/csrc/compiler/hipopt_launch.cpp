@@ -686,7 +686,7 @@ struct RowThreads {
     if (root->map.n != rows || k.grid.x * k.grid.y * k.grid.z != rows) return false;
     // straight through the row: element loops and reductions over the whole workgroup, no loop around them
     bool ok = true, reduces = false, strided = false;
-    int64_t longest = 0, bytes = 0;
+    int64_t longest = 0, bytes = 0, loops = 0;
     Pass probe(k, opts, gen);
     std::function<void(const Stmts&)> walk = [&](const Stmts& ss) {
       for (auto& s : ss) {
@@ -703,6 +703,7 @@ struct RowThreads {
             if (extent <= 0) { ok = false; break; }
             visit_stmts(s->body, [&](const S& c) { if (c->k == Stmt::For || c->k == Stmt::While || c->k == Stmt::Sync || c->k == Stmt::RawStmt || c->k == Stmt::WaveReduce) ok = false; });
             longest = std::max(longest, extent);
+            ++loops;
             strided = strided || s->step != 1;
             if (const int v = probe.vector_width(s)) bytes = std::max<int64_t>(bytes, 16 / v);
             break;
@@ -728,6 +729,9 @@ struct RowThreads {
       // (With a limit of four per SIMD 300 rows of 100000 took 23.9 us instead of 22.2.)
       while (!strided && want < 1024 && rows * (want / WAVE_SIZE) < 2048 && longest * bytes >= 64 * want) want *= 2;
     }
+    // Rows that several loops walk stay in registers where a thread runs 32 vectors of them at most (softmax, doubles, 256
+    // threads asked for: 644 rows of 29553 165 -> 78 us, 2000 of 20001 349 -> 138, 1000 of 17001 147 -> 57).
+    while (loops > 1 && !strided && want < 1024 && longest * bytes > 32 * 16 * want) want *= 2;
     // Workgroups start at about two per nanosecond, which is what small ones wait for: four rows each where a row is a
     // wavefront's (the sums above 7.1 us, 6.7 with eight; softmax over 30000 rows of 200 floats 16.0 -> 8.7 us).
     // (a launch of four wavefronts per SIMD or less starts all of them at once)

@@ -109,6 +109,7 @@ struct Pass {
   // hipopt_vector.cpp: several consecutive elements per thread; MFMA dot products
   int vector_width(const S& loop);
   static int64_t strided_run(const E& idx, const Name& d);
+  Stmts whole_lines(const S& loop, int V);
   Stmts vectorize(const Stmts& ss);
   Stmts widen_half_sums(const Stmts& ss);
   Stmts mfma_dot(const Stmts& ss);

@@ -57,7 +57,70 @@ int64_t Pass::strided_run(const E& idx, const Name& d) {
   return 0;
 }
 
+// A long loop over a row that is no whole number of vectors: rows start anywhere.  The vectors begin where a line of the
+// memory does, so that no two accesses share a line, and what stands in front of them and behind them (less than a line and
+// a vector) is a loop of its own, one element to a thread.  Sums of 542 rows of 115 669 floats on 128 threads 70.5 -> 49.9 us,
+// 300 of 100 001 on 512 34.8 -> 26.9, 16 of 1 000 001 on 1024 79.7 -> 44.4; with vectors that start where the row does 27.8 on
+// the second, and 55.0 instead of 51.7 for 2000 of 40 001 on 256.  Doubles stay as they are: vectors of two were slower by the
+// clock (200 rows of 200 001: 53.8 -> 63.1 us, 1500 of 33 001: 64.9 -> 66.9).
+Stmts Pass::whole_lines(const S& s, int V) {
+  const int64_t extent = const_extent(s), N = s->map.n;
+  if (!s->els.empty() || s->lo->iv != 0 || extent % V == 0 || counted_trips(extent, N) > 0 || extent < 2 * V * N) return {};
+  // the first element of the row, by the first array that is walked
+  E row;
+  int64_t line = 0;
+  bool ok = true;
+  for (auto& c : s->body)
+    if (c->k != Stmt::Def && c->k != Stmt::Assign) ok = false;
+  visit_stmts(s->body, [&](const S& c) {
+    for (const E& e : {c->expr, c->dst})
+      visit_exprs(e, [&](const E& x) {
+        E rest;
+        if (row || x->k != Expr::Index || x->args[0]->ty.mem == Mem::LDS || !affine_unit(x->args[1], s->id, &rest)) return;
+        row = rest;
+        line = 128 / elem_bytes(x->ty.sz);
+      });
+  });
+  if (!ok || !row || has_load(row) || N < line + V) return {};
+  visit_exprs(row, [&](const E& x) { if (x->k != Expr::Var && x->k != Expr::Int && x->k != Expr::BinOpE && x->k != Expr::Convert) ok = false; });
+  if (!ok) return {};
+  Type ity = Type::scalar(isz), bty = Type::scalar(ElemSize::Bool);
+  auto num = [&](int64_t v) { return mk_int(v, isz); };
+  auto bin = [&](BinOp op, E a, E b) { return mk_binop(op, a, b, ity); };
+  const Name front = gen.fresh(s->id.s + "_front"), vectors = gen.fresh(s->id.s + "_vectors"), q = gen.fresh(s->id.s + "_q"), u = gen.fresh(s->id.s + "_u"), o = gen.fresh(s->id.s + "_o");
+  const E fv = mk_var(front, ity), nv = mk_var(vectors, ity), qv = mk_var(q, ity), ov = mk_var(o, ity);
+  Stmts out;
+  out.push_back(mk_def(front, ity, bin(BinOp::Min, bin(BinOp::Max, bin(BinOp::Rem, bin(BinOp::Sub, num(line), bin(BinOp::Rem, row, num(line))), num(line)), num(0)), num(line - 1)), s->i));
+  out.push_back(mk_def(vectors, ity, bin(BinOp::FloorDiv, bin(BinOp::Sub, num(extent), fv), num(V)), s->i));
+  Stmts ib{mk_def(s->id, ity, bin(BinOp::Add, fv, bin(BinOp::Add, bin(BinOp::Mul, qv, num(V)), mk_var(u, ity))), s->i)};
+  ib.insert(ib.end(), s->body.begin(), s->body.end());
+  auto inner = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(mk_for(u, num(0), num(V), 1, ib, LoopPar(), s->i)));
+  inner->unroll = true;
+  inner->iv = 1;   // (the vectors are not known to be aligned)
+  auto main = clone(s);
+  main->id = q;
+  main->hi = nv;
+  main->body = {S(inner)};
+  out.push_back(main);
+  // the other elements, numbered: those in front, then those behind the vectors
+  auto rest = clone(s);
+  rest->id = o;
+  rest->hi = num(line + V - 2);
+  const E at = mk_ifexpr(mk_binop(BinOp::Lt, ov, fv, bty), ov, bin(BinOp::Add, ov, bin(BinOp::Mul, nv, num(V))), ity);
+  rest->body = {mk_def(s->id, ity, at, s->i), mk_if(mk_binop(BinOp::Lt, mk_var(s->id, ity), num(extent), bty), s->body, {})};
+  out.push_back(rest);
+  return out;
+}
+
 Stmts Pass::vectorize(const Stmts& ss) {
+  bool stores_rows = false;   // a loop of the kernel writes element after element of an array
+  visit_stmts(k.body, [&](const S& s) {
+    if (thread_mapped(s))
+      visit_stmts(s->body, [&](const S& c) {
+        E rest;
+        if (c->k == Stmt::Assign && c->dst->k == Expr::Index && c->dst->args[0]->ty.mem != Mem::LDS && affine_unit(c->dst->args[1], s->id, &rest)) stores_rows = true;
+      });
+  });
   Stmts out;
   for (auto& s : ss) {
     bool done = false;
@@ -72,20 +135,29 @@ Stmts Pass::vectorize(const Stmts& ss) {
       // fill its launch exactly, since it has no bounds guard.  Where 16-byte vectors would leave more than a quarter of
       // the threads without one, narrower vectors are taken.  Elements of four bytes and more move 256 bytes per
       // wavefront and access as they are, so only narrower ones take vectors that do not divide the loop: the last one
-      // is then tested element by element.  (Rows need not start on 16 bytes: the memory instructions take any
+      // is then tested element by element.  So do wider ones where rows are written and threads take two vectors and more
+      // (softmax, floats on 256 threads: 30000 rows of 501 / 999 / 1001 21.3 / 57.9 / 58.1 -> 19.2 / 40.3 / 40.0 us, 2000 of 20001
+      // 182 -> 61; 63305 rows of 202 on one vector a thread 20.7 -> 25.7; sums of 20000 rows of 999 13.9 -> 15.6).  (Rows need not start on 16 bytes: the memory instructions take any
       // element-aligned address.  Softmax over 1000 rows of 20001 halves on 512 threads per row: 40.2 -> 21.6 us, over
       // 3000 rows of 999 on 256: 10.3 -> 6.7.)
       int V = 0;
       for (int v = widest; v >= 2 && V == 0 && !nested; v /= 2) {
         const int64_t vectors = (extent + v - 1) / v;
         const bool whole = extent % v == 0;
-        if (grid_wide ? whole && extent % (s->map.n * v) == 0 : (extent % widest == 0 || widest > 4) && 4 * vectors >= 3 * s->map.n) V = v;
+        if (grid_wide ? whole && extent % (s->map.n * v) == 0 : (extent % widest == 0 || widest > 4 || (stores_rows && v == widest && vectors > s->map.n)) && 4 * vectors >= 3 * s->map.n) V = v;
         if (grid_wide) break;
       }
       // (a long loop whose trip count is not the same for all threads is not counted: its last vector would put a test
       // into every iteration)
       const bool partial = V > 0 && extent % V != 0;
       if (partial && counted_trips((extent + V - 1) / V, s->map.n) < 0) V = 0;
+      if (V == 0 && !grid_wide && !nested && widest >= 4) {
+        Stmts lines = whole_lines(s, widest);
+        if (!lines.empty()) {
+          out.insert(out.end(), lines.begin(), lines.end());
+          continue;
+        }
+      }
       if (V > 0) {
         Type ity = Type::scalar(isz), bty = Type::scalar(ElemSize::Bool);
         Name q = gen.fresh(s->id.s + "_q"), u = gen.fresh(s->id.s + "_u");
@@ -97,8 +169,9 @@ Stmts Pass::vectorize(const Stmts& ss) {
         auto inner = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(
             mk_for(u, mk_int(0, isz), mk_int(V, isz), 1, ib, LoopPar(), s->i)));
         inner->unroll = true;
-        if (partial)   // (whole vector, element in range): printed as two loops
-          inner->args = {mk_binop(BinOp::Leq, first, mk_int(extent - V, isz), bty), mk_binop(BinOp::Lt, mk_var(s->id, ity), s->hi, bty)};
+        if (partial) inner->iv = 1;   // (rows that are no whole vectors start anywhere)
+        if (partial)   // (whole vector, element in range, end): printed as two loops
+          inner->args = {mk_binop(BinOp::Leq, first, mk_int(extent - V, isz), bty), mk_binop(BinOp::Lt, mk_var(s->id, ity), s->hi, bty), s->hi};
         auto outer = clone(s);
         outer->id = q;
         outer->lo = mk_int(0, isz);

@@ -9,7 +9,7 @@
 #include <cinttypes>
 #include <sstream>
 
-#include "passes.hpp"
+#include "hipopt_pass.hpp"
 
 namespace parpy {
 
@@ -276,6 +276,25 @@ __device__ __forceinline__ bool parpy_last_workgroup(unsigned* counters, int whi
   return parpy_last;
 }
 typedef float parpy_f32x4 __attribute__((ext_vector_type(4)));
+template <class T, int V> using parpy_vec = T __attribute__((ext_vector_type(V)));
+// Elements first, first + 1, ... of p for a thread whose vector may reach past `end` (V elements at least stand in front of
+// it).  All threads issue the same access: where the vector is not whole, the one that ends at `end`, and its elements are
+// moved down (those past the end then hold what the others hold).
+// The elements are loaded one by one, for the device compiler to join: a vector that starts at any element has no alignment
+// that a pointer to it could promise (a scalar load drops the low bits of an address that it takes for a multiple of four).
+template <class T, int V> __device__ __forceinline__ const T* parpy_vector_within(const T* p, int first, int end, bool whole) {
+  return p + (whole || first <= end - V ? first : end - V);
+}
+template <class T, int V> __device__ __forceinline__ parpy_vec<T, V> parpy_moved_down(parpy_vec<T, V> v, int first, int end, bool whole) {
+  if (whole) return v;
+  const int past = first <= end - V ? 0 : first - (end - V);
+  #pragma unroll
+  for (int s = 1; s < V; s *= 2) {
+    #pragma unroll
+    for (int e = 0; e + s < V; ++e) v[e] = past & s ? v[e + s] : v[e];
+  }
+  return v;
+}
 template <class T> using parpy_vec4 = T __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ int parpy_lane_id() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 // dst[c][r] = src[r][c] for a ROWS x COLS matrix in 64 x 64 tiles: a 256-thread workgroup reads
@@ -599,6 +618,8 @@ struct DevicePrinter {
       }
       case Expr::Index: {
         if (!as_lvalue) {
+          auto joined = tail_loads.find(e.get());
+          if (joined != tail_loads.end()) return joined->second;
           if (cur_pack_loads) {
             auto pk = cur_pack_loads->find(e.get());
             if (pk != cur_pack_loads->end()) return pk->second;
@@ -692,6 +713,9 @@ struct DevicePrinter {
 
   std::vector<S> kept_alive;
   int in_unrolled = 0;            // unrolled loops over the elements of a vector around the statement being printed
+  std::map<const Expr*, std::string> tail_loads;   // elements of vectors loaded in front of the loop over them
+  int next_tail = 0;
+  std::string not_last_trip;      // holds in all trips of the counted loop being printed but the last
   int in_unaligned = 0;           // those whose vectors start at any element
   std::set<Name> seq_loop_vars;   // variables of the enclosing sequential loops that are kept as loops
 
@@ -767,10 +791,52 @@ struct DevicePrinter {
     const char* cmp = s->step > 0 ? " < " : " > ";
     std::string los = pexpr(s->lo), his = pexpr(s->hi);
 
-    if (s->map.k == GpuMap::None && s->unroll && s->args.size() == 2) {
+    if (s->map.k == GpuMap::None && s->unroll && s->args.size() == 3) {
       // the elements of one vector, some of which may lie past the end: all of them without a test where the vector is
       // whole, one test each where it is not
-      os << ind(n) << "if (" << pexpr(s->args[0]) << ") {\n";
+      // What the vector is made of is loaded in front of the test, by one access that ends with the loop where the vector
+      // would reach past it: in the two branches, one would wait for its loads before the other issues its own.
+      std::vector<const Expr*> joined;
+      const S head = s->body.empty() ? S() : s->body[0];
+      if (head && head->k == Stmt::Def) {
+        const Name elem = head->id;
+        std::set<Name> inside{s->id};   // what is known inside the loop only
+        visit_stmts(s->body, [&](const S& c) { if (c->k == Stmt::Def || c->k == Stmt::For) inside.insert(c->id); });
+        auto known = [&](const E& x) {
+          bool ok = !hipopt::has_load(x);
+          visit_exprs(x, [&](const E& y) { if (y->k == Expr::Var && inside.count(y->name)) ok = false; });
+          return ok;
+        };
+        std::vector<std::pair<E, std::string>> loaded;
+        std::function<void(const E&)> find = [&](const E& e) {
+          if (!e) return;
+          E rest;
+          if (e->k == Expr::Index && e->args[0]->k == Expr::Var && e->args[0]->ty.mem != Mem::LDS && read_only_param(e->args[0]) &&
+              hipopt::affine_unit(e->args[1], elem, &rest) && known(rest)) {
+            std::string var;
+            for (auto& l : loaded) if (expr_eq(l.first, e)) var = l.second;
+            if (var.empty()) {
+              var = "tail_" + std::to_string(next_tail++);
+              loaded.push_back({e, var});
+              const std::string T = elem_ctype(e->ty.sz), V = std::to_string(hipopt::const_extent(s)), TV = "<" + T + ", " + V + ">";
+              std::map<Name, E> zero{{s->id, mk_int(0, s->lo->ty.sz)}};
+              const std::string where = pexpr(fold_expr(hipopt::subst_vars(head->expr, zero))) + ", " + pexpr(s->args[2]) + ", " + (not_last_trip.empty() ? "false" : not_last_trip);
+              os << ind(n) << "const " << T << "* " << var << "_at = parpy_vector_within" << TV << "(" << pexpr(e->args[0]) << " + " << paren(pexpr(rest)) << ", " << where << ");\n";
+              os << ind(n) << "const parpy_vec" << TV << " " << var << " = parpy_moved_down" << TV << "(parpy_vec" << TV << "{";
+              for (int64_t q = 0; q < hipopt::const_extent(s); ++q)
+                os << (q ? ", " : "") << (streams_in(e) ? "__builtin_nontemporal_load(&" : "") << var << "_at[" << q << "]" << (streams_in(e) ? ")" : "");
+              os << "}, " << where << ");\n";
+            }
+            tail_loads[e.get()] = var + "[" + s->id.str() + "]";
+            joined.push_back(e.get());
+            return;
+          }
+          for (size_t q = 0; q < e->args.size(); ++q) if (!may_skip(e, q)) find(e->args[q]);
+        };
+        for (size_t q = 1; q < s->body.size(); ++q)
+          if (s->body[q]->k == Stmt::Def || s->body[q]->k == Stmt::Assign) find(s->body[q]->expr);
+      }
+      os << ind(n) << "if (" << (not_last_trip.empty() ? "" : not_last_trip + " || ") << pexpr(s->args[0]) << ") {\n";
       auto plain = std::make_shared<Stmt>(*s);
       plain->args.clear();
       kept_alive.push_back(plain);
@@ -781,6 +847,7 @@ struct DevicePrinter {
       kept_alive.push_back(tested);   // (places in its statement lists are keys of the packing plan)
       pfor(tested, n + 2);
       os << ind(n) << "}\n";
+      for (auto e : joined) tail_loads.erase(e);
       return;
     }
     if (s->map.k == GpuMap::None) {
@@ -900,9 +967,13 @@ struct DevicePrinter {
         }
         os << ind(n) << "#pragma unroll " << factor << "\n";
       }
+      // (the device compiler does not see by itself that all other trips are in range)
+      const std::string outer_not_last = not_last_trip;
+      not_last_trip = peeled ? "true" : per > 1 ? k + " < " + std::to_string(per - 1) : "";
       os << ind(n) << "for (int " << k << " = 0; " << k << " < " << (peeled ? per - 1 : per) << "; ++" << k << ") {\n";
       os << ind(n + 2) << vty << " " << v << " = " << init("(" + (shared_first ? v + "_g" : idx) + " + " + k + " * " + std::to_string(N) + ")") << ";\n";
       if (ragged && !peeled) {
+        if (per > 1) os << ind(n + 2) << "__builtin_assume(" << k << " == " << per - 1 << " || " << v << cmp << his << ");\n";
         os << ind(n + 2) << "if (" << v << cmp << his << ") {\n";
         pstmts(s->body, n + 4);
         os << ind(n + 2) << "}\n";
@@ -919,6 +990,7 @@ struct DevicePrinter {
         os << ind(n + 2) << "__builtin_amdgcn_sched_barrier(0);\n";
       }
       os << ind(n) << "}\n";
+      not_last_trip = outer_not_last;
       if (peeled) {
         os << ind(n) << "{\n";
         os << ind(n + 2) << "const int " << k << " = " << per - 1 << ";\n";

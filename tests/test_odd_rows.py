@@ -1,0 +1,61 @@
+"""Rows that are no whole number of vectors: the last vector of a counted loop ends with the row, a long loop's vectors begin
+where a line of memory does, and neither sees the elements of the next row."""
+import numpy as np
+import pytest
+
+import parpy_amd as parpy
+from parpy_amd import workloads as W
+from parpy_amd.compile import hiprtc_compile
+
+torch = pytest.importorskip("torch")
+
+
+def opts(n, threads):
+    return parpy.par({'N': parpy.threads(n), 'M': parpy.threads(threads), 'outer': parpy.threads(n), 'inner': parpy.threads(threads)})
+
+
+def softmax_text(n, m, threads, dtype=np.float32):
+    x = np.zeros((n, m), dtype)
+    s = parpy.print_compiled(W.softmax, [x, n, m, x.copy()], opts(n, threads))
+    hiprtc_compile(s[:s.index("// host side")], opts(n, threads))
+    return s[s.index('extern "C" __global__'):]
+
+
+def sums_text(n, m, threads, dtype=np.float32):
+    s = parpy.print_compiled(W.sum_rows, [np.zeros((n, m), dtype), np.zeros(n, dtype), n], opts(n, threads))
+    hiprtc_compile(s[:s.index("// host side")], opts(n, threads))
+    return s[s.index('extern "C" __global__'):]
+
+
+def test_which_rows_take_vectors():
+    for m, dtype, taken in ((1001, np.float32, True), (1000, np.float32, False), (777, np.float64, True), (1777, np.float16, True),
+                            (202, np.float32, False)):   # (whole vectors; a vector a thread)
+        assert ("parpy_vector_within<" in softmax_text(5000, m, 256, dtype)) == taken, (m, dtype)
+    assert "_front_" in sums_text(3, 40001, 1024) and "_front_" not in sums_text(3, 40000, 1024)
+    assert "_front_" not in sums_text(3, 10001, 1024) and "_front_" not in sums_text(3, 40001, 1024, np.float64)
+
+
+def test_long_rows_of_several_loops_fit_the_registers():
+    assert "dim3(512, 1, 1)" in softmax_text(700, 29553, 256, np.float64) and "dim3(256, 1, 1)" in sums_text(700, 29553, 256, np.float64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 4e-3), (torch.float32, 1e-5), (torch.float64, 1e-12)], ids=["f16", "f32", "f64"])
+@pytest.mark.parametrize("n,threads", [(4200, 256), (6, 1024)])
+def test_rows_do_not_see_their_neighbours(n, threads, dtype, tol):
+    """Every other row holds infinities; the ones between are compared with float64."""
+    lengths = (257, 258, 259, 515, 1025, 1026, 1027, 2051, 4097, 4099) + ((40001, 40002, 40003, 40031, 33333) if n < 100 else ())
+    for m in lengths:
+        g = torch.Generator(device="cuda").manual_seed(m)
+        x = torch.randn((n, m), generator=g, device="cuda", dtype=torch.float32).to(dtype)
+        x[1::2] = float("inf")
+        out = torch.full_like(x, -1.0)
+        W.softmax(x, n, m, out, opts=opts(n, threads))
+        mine = x[::2].double()
+        e = torch.exp(mine - mine.max(1, keepdim=True).values)
+        want = e / e.sum(1, keepdim=True)
+        assert ((out[::2].double() - want).norm() / want.norm()) < tol, m
+        sums = torch.full((n,), -1.0, device="cuda", dtype=dtype)
+        W.sum_rows(x, sums, n, opts=opts(n, threads))
+        assert torch.allclose(sums[::2].double(), mine.sum(1), rtol=tol, atol=tol * 30), m
+        assert torch.isinf(sums[1::2]).all(), m
