@@ -24,10 +24,15 @@ namespace {
 //     most one.
 //   * The arithmetic of an element is that of the statement as written: same operations, same order.
 //
-// A three-point average back and forth over 10^6 float64 elements, 98 updates: 447 us as launches of 4.5 us each, 51 us
-// in two launches of 25 steps.  Two additions and a division in four instructions per element and update, a quarter of them
-// in the margins: counted, a SIMD issues vector instructions 52 % of the time, 63 % where three of the 2504 wavefronts share
-// it; the rest is the latency of dependent steps.
+//   * A lane's neighbouring elements come and go through LDS where they are more than 16 bytes, so that memory is read and
+//     written in whole lines; a wavefront's part of LDS is its own, without barriers.
+//   * At the ends of the arrays an update covers a part of a stretch: there the new value is blended with the old one under
+//     a mask kept in a register.
+//
+// A three-point average back and forth over 10^6 float64 elements, 98 updates, two launches of 25 steps: 447 us as launches
+// of 4.5 us each, 45.6 on eight elements per lane with their own accesses and a division of four instructions one of which
+// takes as long as four, 39.1 as it is (33 on arrays in the memory-side cache): 1852 wavefronts, two to a SIMD.  The vector ALU bounds it: 7.2 instructions per
+// element and update, an eighth of them in the margins.
 struct TimeTile {
   Program& p;
   const Options& opts;
@@ -157,21 +162,30 @@ struct TimeTile {
     // tiled and as launches: 1.6 GB 1.6 and 6.6 ms, 4.3 GB 5.2 and 17.9, 6.4 GB 6.7 and 26.3, 9.6 GB 10 and 39 with single
     // calls of 149, 14.4 GB 390 and 58.6).
     if (second_set > (int64_t(6) << 30)) return S();
-    // Elements per lane: eight where that leaves every SIMD a wavefront or two, four for smaller arrays, where the
-    // latency of a step is what counts (98 updates of a three-point average, float64: 10^6 elements 153 / 73 / 56 / 51 /
-    // 68 us for 1 / 2 / 4 / 8 / 16 elements per lane, 6 * 10^5: 35 on four, 38 on eight, 10^5: 15 and 24).
-    int64_t Es = n >= 800000 ? 8 : 4;
-    while (Es * words > 64 && Es > 1) Es /= 2;
-    Es = std::max(Es, pow2_at_least(std::max<int64_t>(1, reach)));
-    if (Es * words > 64 || per_step > 8 * Es) return S();
-    // Steps per launch: a margin of up to a quarter of the stretch on either side.  Launches cost more than the margins
-    // (10^5 elements: margins of 1/16, 1/8 and 1/4 of the stretch 32, 22 and 15 us; 10^6 elements: 60, 52, 51).
+    // Elements per lane, and with them steps per launch (a margin of up to a quarter of the stretch on either side) and
+    // wavefronts: what is expected to be over first.  A wavefront takes an element through an update in 12.2 ns, a SIMD in
+    // 10 ns (6.5 ns for words of four bytes); its share is a whole number of wavefronts; a launch
+    // costs 2.7 us and its bytes at 7 TB/s.  98 updates of a three-point average, two launches, doubles: 10^6 elements
+    // 48.7 / 38.6 / 37.6 / 33.3 / 37.2 / 46.4 us on 4 / 6 / 8 / 10 / 12 / 16 elements per lane (7, 4, 3, 2, 2, 2 wavefronts to a
+    // SIMD), 4 * 10^6 148 / 114 / 103 / 102 / 105 / 103, 10^5 11.5 / 14.3 / 16.3 / 18.8.
+    int64_t Es = 0;
+    double best = 0;
+    for (int64_t e : {1, 2, 3, 4, 6, 8, 10, 12}) {
+      if (e * words > 64 || e < reach || per_step > 8 * e) continue;
+      const int64_t most = per_step > 0 ? 16 * e / per_step : steps, pairs = (steps + 2 * most - 1) / (2 * most);
+      const int64_t margin = ((steps + 2 * pairs - 1) / (2 * pairs) * per_step + e - 1) / e * e, useful = WAVE_SIZE * e - 2 * margin;
+      if (useful < WAVE_SIZE * e / 4) continue;
+      const int64_t waves = (n + useful - 1) / useful, share = (waves + 1023) / 1024;
+      const double time = std::max(12.2, (wide ? 10.0 : 6.5) * (double)share) * (double)(updates * e) +
+                          (double)(2 * pairs) * (2700.0 + (double)(n * words * 4 * 2) / 7000.0);
+      if (Es == 0 || time < best) Es = e, best = time;
+    }
+    if (Es == 0) return S();
     const int64_t most = per_step > 0 ? 16 * Es / per_step : steps;
     const int64_t pairs = (steps + 2 * most - 1) / (2 * most), launches = 2 * pairs;
     const int64_t base_steps = steps / launches, extra = steps % launches;
     const int64_t margin = ((base_steps + (extra > 0)) * per_step + Es - 1) / Es * Es;
     const int64_t width = WAVE_SIZE * Es, useful = width - 2 * margin;
-    if (useful < width / 4) return S();
     const int64_t tpb = 256;
 
     // ---- the kernel
@@ -225,7 +239,20 @@ struct TimeTile {
     top.push_back(mk_def(lane, ity, mk_binop(BinOp::Rem, index_reg(Expr::ThreadIdx), iint(WAVE_SIZE), ity)));
     top.push_back(mk_def(wave, ity, add(mk_binop(BinOp::Mul, index_reg(Expr::BlockIdx), iint(tpb / WAVE_SIZE), ity),
                                         mk_binop(BinOp::FloorDiv, index_reg(Expr::ThreadIdx), iint(WAVE_SIZE), ity))));
-    E start = mk_binop(BinOp::Sub, mk_binop(BinOp::Mul, wv, iint(useful), ity), iint(margin), ity);
+    const Name first = gen.fresh("start"), meeting = gen.fresh("stretch");
+    top.push_back(mk_def(first, ity, mk_binop(BinOp::Sub, mk_binop(BinOp::Mul, wv, iint(useful), ity), iint(margin), ity)));
+    E start = mk_var(first, ity);
+    int64_t widest = 4;
+    for (auto& a : arrays) widest = std::max<int64_t>(widest, elem_bytes(a.sz));
+    const int64_t part = WAVE_SIZE * (Es * widest + 16);   // bytes of LDS for a wavefront
+    top.push_back(mk_rawstmt("__shared__ __attribute__((aligned(16))) unsigned char " + meeting.str() + "[" + std::to_string(part * (tpb / WAVE_SIZE)) + "];"));
+    f.lds_bytes = part * (tpb / WAVE_SIZE);
+    auto through_lds = [&](const Arr& a) {
+      return std::string("parpy_stretch<") + elem_ctype(a.sz) + ", " + std::to_string(Es) + ">::";
+    };
+    auto lds_of_wave = [&](const Arr& a) {
+      return std::string("(") + elem_ctype(a.sz) + "*)(" + meeting.str() + " + threadIdx.x / 64 * " + std::to_string(part) + "), " + lane.str();
+    };
     top.push_back(mk_def(at, ity, add(start, mk_binop(BinOp::Mul, lv, iint(Es), ity))));
     for (auto& a : arrays) {
       auto d = std::make_shared<Stmt>();
@@ -250,12 +277,30 @@ struct TimeTile {
     // the path of a stretch: `edge` tests every element against the bounds of the arrays and of the updates
     auto path = [&](bool edge) {
       Stmts ss;
-      for (auto& a : arrays)
+      for (auto& a : arrays) {
+        if (!edge && Es * elem_bytes(a.sz) > 16) {
+          ss.push_back(mk_rawstmt(through_lds(a) + "in(" + reg[a.host].str() + ", " + a.host.str() + " + " + first.str() + ", " + lds_of_wave(a) + ");"));
+          continue;
+        }
         for (int64_t e = 0; e < Es; ++e) {
           S ld = mk_assign(slot(a, e), elem(a.host, a, e));
-          ss.push_back(edge ? mk_if(within(e, 0, a.n), {ld}, {mk_assign(slot(a, e), is_float(a.sz) ? mk_float(0.0, a.sz) : mk_int(0, a.sz))}) : ld);
+          ss.push_back(!edge ? ld : mk_if(within(e, 0, a.n), {ld}, {mk_assign(slot(a, e), is_float(a.sz) ? mk_float(0.0, a.sz) : mk_int(0, a.sz))}));
         }
-      Stmts step;
+      }
+      Stmts step, masks;
+      std::vector<std::pair<std::vector<int64_t>, E>> known;
+      auto covered = [&](int64_t e, int64_t from, int64_t to) {
+        for (auto& kn : known) if (kn.first == std::vector<int64_t>{e, from, to}) return kn.second;
+        auto call = std::make_shared<Expr>();
+        call->k = Expr::Call;
+        call->ty = Type::scalar(ElemSize::I32);
+        call->sval = "parpy_mask";
+        call->args = {within(e, from, to)};
+        Name m = gen.fresh("covered");
+        masks.push_back(mk_def(m, call->ty, E(call)));
+        known.push_back({{e, from, to}, mk_var(m, call->ty)});
+        return known.back().second;
+      };
       for (auto& u : ups) {
         // what the neighbouring lanes hold
         std::map<std::pair<Name, int64_t>, E> from;
@@ -307,24 +352,39 @@ struct TimeTile {
               names[st->id] = mk_var(nm, st->ty);
             } else {
               E to = slot(arr_of(u.host[st->dst->args[0]->name]), e);
-              // (computed for every element and kept where the update covers it: no branches between the elements)
-              one.push_back(mk_assign(to, edge ? mk_ifexpr(within(e, u.lo, u.hi), v, to, to->ty) : v, st->i));
+              // computed for every element and kept where the update covers it, bit by bit: of a selection the device compiler
+              // makes a branch around the element, and the stretches at the ends took twice as long as the others
+              if (edge) {
+                auto blend = std::make_shared<Expr>();
+                blend->k = Expr::Call;
+                blend->ty = to->ty;
+                blend->sval = "parpy_blend";
+                blend->args = {covered(e, u.lo, u.hi), v, to};
+                v = E(blend);
+              }
+              one.push_back(mk_assign(to, v, st->i));
             }
           }
           step.insert(step.end(), one.begin(), one.end());
         }
       }
+      ss.insert(ss.end(), masks.begin(), masks.end());
       Name s = gen.fresh("s");
       ss.push_back(mk_for(s, mk_int(0, ElemSize::I32), mk_var(count.id, Type::scalar(ElemSize::I32)), 1, step, LoopPar()));
       Stmts put;
-      for (auto& a : arrays)
-        if (a.written)
-          for (int64_t e = 0; e < Es; ++e) {
-            S stt = mk_assign(elem(dst[a.host], a, e), slot(a, e));
-            put.push_back(edge ? mk_if(within(e, 0, a.n), {stt}, {}) : stt);
-          }
+      for (auto& a : arrays) {
+        if (!a.written) continue;
+        if (!edge && Es * elem_bytes(a.sz) > 16) {
+          ss.push_back(mk_rawstmt(through_lds(a) + "out(" + reg[a.host].str() + ", " + dst[a.host].str() + " + " + first.str() + ", " + lds_of_wave(a) + ", " + std::to_string(margin) + ");"));
+          continue;
+        }
+        for (int64_t e = 0; e < Es; ++e) {
+          S stt = mk_assign(elem(dst[a.host], a, e), slot(a, e));
+          put.push_back(edge ? mk_if(within(e, 0, a.n), {stt}, {}) : stt);
+        }
+      }
       const int64_t outer = margin / Es;
-      ss.push_back(mk_if(both(le(iint(outer), lv), lt(lv, iint(WAVE_SIZE - outer))), put, {}));
+      if (!put.empty()) ss.push_back(mk_if(both(le(iint(outer), lv), lt(lv, iint(WAVE_SIZE - outer))), put, {}));
       return ss;
     };
     // A stretch that lies inside all bounds takes the plain path.  Values next to the bounds of a stretch are wrong (its
