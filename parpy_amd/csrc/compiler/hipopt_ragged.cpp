@@ -24,7 +24,7 @@ namespace {
 //     barrier all waves share each of them.
 //
 // Measured (100 000 rows of 50 non-zeros on average, the longest 15 800, float64): eight lanes per row, one element in
-// flight 547 us, in teams 39 us.  The gathers out of L2 are then what bounds it: 5.5 million lines requested (counted, 87 %
+// flight 547 us, in teams 34 us.  The gathers out of L2 are then what bounds it: 5.5 million lines requested (counted, 87 %
 // of them hits), 141 per nanosecond.  20 000 rows of 24 on average (longest 3400)
 // times a 128-column matrix: one workgroup per row with the sum read and written back in LDS per element 840 us, in
 // teams 42 us, with the longest rows first (below) 33: they pull 1.7 MB each through one compute unit, and 165 of the 261 MB
@@ -256,7 +256,12 @@ struct RaggedSum {
     // columns: 22.4 / 17.7 / 17.4 / 20.9 us for 1 / 2 / 4 / 8 subteams.)  Rows that were the threads of one workgroup
     // are too few to fill the chip in any case: 10.3 us on 16 lanes, 11.0 on eight.
     const int64_t P = r.one_group ? 8 : std::min<int64_t>(WAVE_SIZE / L, std::max<int64_t>(pow2_at_least((avg + 1) / 2), r.has_col ? 1 : 4));
-    const int64_t T = L * P, tpb = r.tpb;
+    const int64_t T = L * P;
+    // more wavefronts than run at once
+    const bool queues = r.n * T > 256 * 2048;
+    // (single sums: a workgroup is over with its slowest wavefront; 1024 / 512 / 256 threads 36.6 / 34.2 / 34.2 us for the 50
+    // non-zeros above, 29.9 / 28.2 / 30.2 in floats, 99.8 / 91.2 / 91.9 for 10^6 rows of 10 floats)
+    const int64_t tpb = !r.has_col && queues ? std::min<int64_t>(r.tpb, 512) : r.tpb;
     if (tpb % WAVE_SIZE != 0 || tpb < L * V || r.n * T > (int64_t(1) << 30)) return false;
     const int64_t teams = tpb / T, waves = tpb / WAVE_SIZE;
     if (r.has_col && (tpb < r.cols || waves * L * K * elem_bytes(r.acc->ty.sz) > 64 * 1024)) return false;
@@ -269,9 +274,12 @@ struct RaggedSum {
     // of four and share each of them as above; the teams pass those by.  20 000 rows of 24 on average times 128 columns:
     // 41.5 -> 33.3 us (rows of equal length 24.6 and 24.8), 20 000 of 20 times 99: 43.0 -> 32.1, 100 000 of 15 times 64:
     // 73 -> 61; 2 and 8 instead of 4 measure 33.6 and 37.7 on the first, 1024 workgroups 34.5.  Without columns the
-    // longest row is over before the last rows have started (38.9 and 38.5 us; 10^6 rows of 10 124.7 and 127.1).
-    const int64_t huge = 4 * longest;
-    const int64_t scouts = r.has_col && r.n * T > 256 * 2048 ? std::max<int64_t>(256, (r.n + 1023) / 1024) : 0;
+    // workgroups in front take every row that is not a team's, 512 of them, and the teams' workgroups have no queue to wait
+    // for: a row shared there holds sixteen wavefronts for three microseconds, and half of the workgroups have one (100 000
+    // rows of 50 on average, doubles: 39.5 us with the queues, 36.3 without, 37.5 with 1024 workgroups in front, 39.1 with only
+    // the rows in front that stand out by four; floats 32.6 and 29.8; 10 000 of 100, floats, 12.5 and 10.6).
+    const int64_t huge = r.has_col ? 4 * longest : longest;
+    const int64_t scouts = queues ? std::max<int64_t>(r.has_col ? 256 : 512, (r.n + 1023) / 1024) : 0;
     const int64_t looked = scouts ? (r.n + scouts - 1) / scouts : 0;   // rows for each of them
     // element numbers in 32 bits when the array they walk is known to be small enough
     const bool small = r.bounded && r.elements < (int64_t(1) << 29);
@@ -425,6 +433,7 @@ struct RaggedSum {
       e->iv = 1;
       top.push_back(e);
     }
+    const bool all_in_front = scouts > 0 && huge == longest;
     top.push_back(mk_rawstmt("if (threadIdx.x == 0) " + count.str() + "[0] = 0;"));
     top.push_back(mk_sync());
 
@@ -453,7 +462,8 @@ struct RaggedSum {
       else own.insert(own.end(), f.begin(), f.end());
       const S enqueue = mk_rawstmt(queue.str() + "[atomicAdd(&" + count.str() + "[0], 1)] = (int)" + r.row.str() + ";");
       auto longer = [&](const E& a, const E& b) { return mk_binop(BinOp::Gt, mk_binop(BinOp::Sub, b, a, ety), eint(huge), bty); };
-      Stmts defer{mk_if(mk_binop(BinOp::Eq, qv, iint(0), bty), {scouts ? mk_if(longer(lo, hi), {}, {enqueue}) : enqueue}, {})};
+      Stmts defer;
+      if (!all_in_front) defer = {mk_if(mk_binop(BinOp::Eq, qv, iint(0), bty), {scouts ? mk_if(longer(lo, hi), {}, {enqueue}) : enqueue}, {})};
       body.push_back(mk_if(mk_binop(BinOp::Leq, mk_binop(BinOp::Sub, hi, lo, ety), eint(longest), bty), own, defer));
       auto nr = clone(k.body[0]);
       nr->id = lane;
@@ -478,6 +488,7 @@ struct RaggedSum {
       nr->map.n = (r.n * T + scouts * tpb + WAVE_SIZE - 1) / WAVE_SIZE * WAVE_SIZE;
       top.push_back(nr);
     }
+    if (all_in_front) top.push_back(mk_rawstmt("if (blockIdx.x >= " + std::to_string(scouts) + ") return;"));
     top.push_back(mk_sync());
 
     // long rows, one after the other, by all threads of the workgroup
