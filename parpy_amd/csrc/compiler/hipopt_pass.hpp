@@ -123,6 +123,7 @@ struct Pass {
   Stmts hoist_invariant(const Stmts& ss, int64_t* budget, bool in_seq);
   struct OwnIterations;
   bool distinct_names(const Name& a, const Name& b) const;
+  Stmts issue_ahead(const OwnIterations& oi, const S& loop, Stmts* pre, bool* any);
   Stmts share_own_iterations(const Stmts& ss);
   void reg_cache(int64_t* budget);
 
