@@ -8,8 +8,10 @@
 // and adds what it compiled.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <structmember.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cstring>
 #include <new>
 #include <string>
@@ -31,6 +33,7 @@ struct Table {
   std::string* key;             // built per call; calls hold the interpreter lock while they use it
   PyObject* opts_type;
   PyObject* loop_par_type;
+  Py_ssize_t par_fields[3];     // where a LoopPar keeps nthreads, reduction and _tpb: slots, read without a look-up by name
   RunFn run;
 };
 
@@ -125,7 +128,7 @@ bool put_args(std::string& k, PyObject* args, Pointers& ps) {
 }
 
 // settings of an options object: the fields that its own dictionary holds (a field that is not there has its default)
-bool put_options(std::string& k, PyObject* opts, PyObject* loop_par_type) {
+bool put_options(std::string& k, PyObject* opts, PyObject* loop_par_type, const Py_ssize_t* par_fields) {
   PyObject* d = PyObject_GenericGetDict(opts, nullptr);   // new reference
   if (!d) { PyErr_Clear(); return false; }
   bool ok = PyDict_CheckExact(d);
@@ -146,12 +149,9 @@ bool put_options(std::string& k, PyObject* opts, PyObject* loop_par_type) {
       Py_ssize_t q = 0;
       while (ok && PyDict_Next(v, &q, &label, &par)) {
         ok = (PyObject*)Py_TYPE(par) == loop_par_type && put_str(k, label);
-        PyObject* const names[3] = {s_nthreads, s_reduction, s_tpb};
         for (int f = 0; ok && f < 3; ++f) {
-          PyObject* x = PyObject_GetAttr(par, names[f]);
-          if (!x) { PyErr_Clear(); ok = false; break; }
-          ok = PyLong_Check(x) && put_long(k, x);
-          Py_DECREF(x);
+          PyObject* x = *(PyObject**)((char*)par + par_fields[f]);   // (null: deleted)
+          ok = x && PyLong_Check(x) && put_long(k, x);
         }
       }
     } else if (v == Py_None || PyBool_Check(v)) {
@@ -180,7 +180,7 @@ bool make_key(Table* self, PyObject* args, PyObject* opts, Pointers& ps) noexcep
     k.clear();
     if (!put_args(k, args, ps)) return false;
     put_tag(k, ps.aligned ? '|' : '!');
-    return put_options(k, opts, self->loop_par_type);
+    return put_options(k, opts, self->loop_par_type, self->par_fields);
   } catch (...) {
     PyErr_Clear();   // (an exception that Python code under the tensor raised)
     return false;
@@ -250,8 +250,19 @@ PyObject* table_new(PyTypeObject* type, PyObject* args, PyObject*) {
   if (!PyArg_ParseTuple(args, "OOO", &opts_type, &loop_par_type, &run)) return nullptr;
   void* fn = PyLong_AsVoidPtr(run);
   if (PyErr_Occurred()) return nullptr;
+  Py_ssize_t fields[3];
+  PyObject* const names[3] = {s_nthreads, s_reduction, s_tpb};
+  for (int f = 0; f < 3; ++f) {
+    PyObject* slot = PyObject_GetAttr(loop_par_type, names[f]);
+    if (!slot) return nullptr;
+    const bool object = Py_TYPE(slot) == &PyMemberDescr_Type && ((PyMemberDescrObject*)slot)->d_member->type == T_OBJECT_EX;
+    fields[f] = object ? ((PyMemberDescrObject*)slot)->d_member->offset : 0;
+    Py_DECREF(slot);
+    if (!object) { PyErr_SetString(PyExc_TypeError, "CallTable: the fields of the second type are not slots"); return nullptr; }
+  }
   Table* self = (Table*)type->tp_alloc(type, 0);
   if (!self) return nullptr;
+  std::copy(fields, fields + 3, self->par_fields);
   self->entries = new (std::nothrow) std::unordered_map<std::string, Entry>();
   self->key = new (std::nothrow) std::string();
   if (!self->entries || !self->key) { Py_DECREF(self); return PyErr_NoMemory(); }
