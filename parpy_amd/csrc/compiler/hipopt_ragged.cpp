@@ -27,7 +27,7 @@ namespace {
 // flight 547 us, in teams 34 us.  The gathers out of L2 are then what bounds it: 5.5 million lines requested (counted, 87 %
 // of them hits), 141 per nanosecond.  20 000 rows of 24 on average (longest 3400)
 // times a 128-column matrix: one workgroup per row with the sum read and written back in LDS per element 840 us, in
-// teams 42 us, with the longest rows first (below) 33: they pull 1.7 MB each through one compute unit, and 165 of the 261 MB
+// teams 42 us, with the long rows in front (below) 34: the longest pulls 1.7 MB through one compute unit, and 165 of the 261 MB
 // that the L2s deliver come from behind them, since the 10 MB matrix does not fit a die's 4 MB.
 struct RaggedSum {
   Program& p;
@@ -237,6 +237,33 @@ struct RaggedSum {
     return affine_unit(a->args[1], v, &ra) && affine_unit(b->args[1], v, &rb) && ra->k == Expr::Int && rb->k == Expr::Int && rb->iv == ra->iv + 1;
   }
 
+  // Loads of every element that depend on its number alone (`cols[i]`, `values[i]`): each is executed for all elements of
+  // a row, and nothing in the kernel writes there.
+  std::vector<E> element_loads(const Kernel& k, const Rows& r) {
+    std::set<Name> params, written;
+    for (auto& q : k.params) if (q.ty.is_pointer()) params.insert(q.id);
+    visit_stmts(k.body, [&](const S& c) {
+      if (c->k == Stmt::Assign && c->dst->k == Expr::Index && c->dst->args[0]->k == Expr::Var) written.insert(c->dst->args[0]->name);
+    });
+    std::vector<E> out;
+    std::function<void(const E&, bool)> scan = [&](const E& x, bool always) {
+      if (!x) return;
+      E rest;
+      if (always && x->k == Expr::Index && x->args[0]->k == Expr::Var && params.count(x->args[0]->name) && !written.count(x->args[0]->name) &&
+          !k.no_restrict && x->ty.is_scalar() && x->ty.sz != ElemSize::Bool && affine_unit(x->args[1], r.loop->id, &rest) &&
+          rest->k == Expr::Int) {
+        bool known = false;
+        for (auto& e : out) known = known || expr_eq(e, x);
+        if (!known) out.push_back(x);
+        return;
+      }
+      for (size_t q = 0; q < x->args.size(); ++q) scan(x->args[q], always && !may_skip(x, q));
+    };
+    for (auto& d : r.defs) scan(d->expr, true);
+    scan(r.term, true);
+    return out;
+  }
+
   bool apply(Kernel& k, const StmtP& launch) {
     Rows r;
     if (!match(k, r)) return false;
@@ -258,7 +285,8 @@ struct RaggedSum {
     const int64_t P = r.one_group ? 8 : std::min<int64_t>(WAVE_SIZE / L, std::max<int64_t>(pow2_at_least((avg + 1) / 2), r.has_col ? 1 : 4));
     const int64_t T = L * P;
     // more wavefronts than run at once
-    const bool queues = r.n * T > 256 * 2048;
+    constexpr int64_t RESIDENT = 256 * 2048;
+    const bool queues = r.n * T > RESIDENT;
     // (single sums: a workgroup is over with its slowest wavefront; 1024 / 512 / 256 threads 36.6 / 34.2 / 34.2 us for the 50
     // non-zeros above, 29.9 / 28.2 / 30.2 in floats, 99.8 / 91.2 / 91.9 for 10^6 rows of 10 floats)
     const int64_t tpb = !r.has_col && queues ? std::min<int64_t>(r.tpb, 512) : r.tpb;
@@ -269,17 +297,25 @@ struct RaggedSum {
     // and the waves that have no such row wait for it: 256 elements for single sums (128 costs 5 to 20 %), fewer when
     // every element moves a row of columns (64 against 256 elements: 17.4 and 20.1 us for the 32-column product above).
     const int64_t longest = r.has_col ? std::max<int64_t>(64, 2 * avg) : std::max<int64_t>(256, 4 * avg);
-    // A launch of more wavefronts than run at once starts its rows one after the other, and the longest may start last.
-    // Where rows of columns are moved, 256 workgroups in front of the others look for rows that stand out by another factor
-    // of four and share each of them as above; the teams pass those by.  20 000 rows of 24 on average times 128 columns:
-    // 41.5 -> 33.3 us (rows of equal length 24.6 and 24.8), 20 000 of 20 times 99: 43.0 -> 32.1, 100 000 of 15 times 64:
-    // 73 -> 61; 2 and 8 instead of 4 measure 33.6 and 37.7 on the first, 1024 workgroups 34.5.  Without columns the
-    // workgroups in front take every row that is not a team's, 512 of them, and the teams' workgroups have no queue to wait
-    // for: a row shared there holds sixteen wavefronts for three microseconds, and half of the workgroups have one (100 000
-    // rows of 50 on average, doubles: 39.5 us with the queues, 36.3 without, 37.5 with 1024 workgroups in front, 39.1 with only
-    // the rows in front that stand out by four; floats 32.6 and 29.8; 10 000 of 100, floats, 12.5 and 10.6).
-    const int64_t huge = r.has_col ? 4 * longest : longest;
-    const int64_t scouts = queues ? std::max<int64_t>(r.has_col ? 256 : 512, (r.n + 1023) / 1024) : 0;
+    // The rows longer than that go to workgroups in front of the others, which look for them and share each as above: started
+    // in order, the longest may start last, and in the others' workgroups sixteen wavefronts would wait for them.  Where more
+    // wavefronts are launched than run at once, 1024 such workgroups for rows of columns (20 000 rows of 24 on average times
+    // 128 columns: 34.1 us, 35.1 with 512, 33.8 with 2048, 37.9 with 256; 20 000 of 24 times 64: 20.7, 20.9, 21.0, 23.3) and
+    // 512 for single sums (100 000 rows of 50, doubles: 36.3, 37.5 with 1024; 39.5 us with every long row shared where it is).
+    // Before, rows of columns had 256, for the rows that stand out by another factor of four: 34.7 us for the first and 21.3
+    // for the second, 100 000 of 4 times 256: 85.4 -> 79.5, 50 000 of 20 times 37: 50.4 -> 45.6; 9529 of 41 times 101 loses
+    // by it, 31.0 -> 33.6 (40.8 before the elements of a shared row stood in LDS, below).  Otherwise there is room beside the teams' workgroups: one for eight rows as long as they run at once
+    // (1021 rows of 35 times 256 columns 20.3 -> 13.0 us, 1000 of 64 times 64: 12.9 -> 8.6, 5000 of 64 times 256: 70.4 -> 59.2;
+    // one for 4 / 16 / 32 rows: 13.1 / 13.6 / 15.0, 7.6 / 8.5 / 10.5, 59.4 / 59.2 / 65.5, but 2000 of 64 times 256: 34.8 / 26.2 /
+    // 27.3 and 26.2 with eight), one for sixteen rows for single sums (3000 rows of 60, doubles 6.3 -> 4.9 us, 5.5 with one for
+    // four; 20 000 of 30: 9.8 -> 9.0).  Where the teams leave no room, single sums keep the queues (8000 rows of 150: 18.0 us,
+    // 20.0 with 64 in front) and rows of columns have 512 in front (7500 of 30 times 200: 43.5 -> 32.4, 8000 of 10 times 64:
+    // 8.1 -> 7.3; 256 of them 35.4 and 7.3, 1024 31.5 and 8.1), but for a launch that fills the device exactly.
+    const int64_t groups = (r.n + teams - 1) / teams, room = RESIDENT / tpb - groups;
+    const int64_t scouts = queues ? std::max<int64_t>(r.has_col ? 1024 : 512, (r.n + 1023) / 1024)
+                           : r.one_group ? 0
+                           : room >= 64 ? std::max<int64_t>(1, std::min<int64_t>(room, r.n / (r.has_col ? 8 : 16)))
+                                        : r.has_col && room > 0 ? 512 : 0;
     const int64_t looked = scouts ? (r.n + scouts - 1) / scouts : 0;   // rows for each of them
     // element numbers in 32 bits when the array they walk is known to be small enough
     const bool small = r.bounded && r.elements < (int64_t(1) << 29);
@@ -316,7 +352,9 @@ struct RaggedSum {
     };
     const bool partial = L * K != r.cols;   // lanes or slots past the last column exist
     // statements that add the elements first, first + stride, ... of the row to the lane's sums
-    auto walk = [&](Stmts& out, const E& lo, const E& hi, const E& first, int64_t stride, const E& l) {
+    // (staged: loads of the elements that stand in LDS, from element `lo` on)
+    struct Staged { E load; Name lds; };
+    auto sums_from_zero = [&](Stmts& out) {
       out.push_back([&] {
         auto d = std::make_shared<Stmt>();
         d->k = Stmt::RegDecl;
@@ -326,6 +364,8 @@ struct RaggedSum {
         return S(d);
       }());
       out.push_back(per_slot([&](const E& c) { return Stmts{mk_assign(part(c), mk_float(0.0, sty.sz))}; }));
+    };
+    auto walk = [&](Stmts& out, const E& lo, const E& hi, const E& first, int64_t stride, const E& l, const std::vector<Staged>& staged = {}) {
       Name b = gen.fresh(r.loop->id.s + "_b"), at = gen.fresh(r.loop->id.s + "_at");
       E bv = mk_var(b, ety), iv = mk_var(r.loop->id, ety), atv = mk_var(at, ety);
       Stmts batch;
@@ -336,7 +376,12 @@ struct RaggedSum {
       // short-circuit operator may skip make none (`x[perm[c]] if c >= 0 else 0`: c may be anything where it is not used).
       std::vector<std::pair<E, Name>> named;
       auto bind = [&](const E& e0, Stmts& to) {
-        E e = subst_vars(e0, to_clamped);
+        E e = rewrite_expr(e0, [&](const E& x) -> E {
+          for (auto& st : staged)
+            if (expr_eq(st.load, x)) return mk_index(mk_var(st.lds, Type::pointer(x->ty.sz, Mem::LDS)), widen(mk_binop(BinOp::Sub, atv, lo, ety)), x->ty);
+          return x;
+        });
+        e = subst_vars(e, to_clamped);
         std::function<E(const E&, bool, bool)> go = [&](const E& x, bool inside, bool always) -> E {
           if (!x) return x;
           size_t q = 0;
@@ -400,18 +445,24 @@ struct RaggedSum {
         return ss;
       })};
     };
-    auto bounds = [&](Stmts& ss, E* lo, E* hi) {
-      for (auto& st : r.pre) ss.push_back(st);
-      // (the bounds of a row without elements may be anything, a marker like 2^63 - 1 and 0: what is cut to 32 bits of them, or
-      // passes the largest integer when a lane's place is added, must not become a row)
-      Name lw = gen.fresh("lo"), hw = gen.fresh("hi"), any = gen.fresh("any"), ln = gen.fresh("first"), hn = gen.fresh("end");
-      E l = mk_var(lw, ity), h = mk_var(hw, ity), some = mk_var(any, bty);
+    auto limits = [&](Stmts& ss, E* lo, E* hi) {
+      Name lw = gen.fresh("lo"), hw = gen.fresh("hi");
       // (`rows[row] .. rows[row + 1]` in the plain form of an index, whose neighbours the device compiler joins to one load: with
       // 32-bit offsets two loads of eight bytes, 52.0 us for SpMV with 100 000 rows of 50, 50.4 so, 50.0 unchecked)
       std::map<Name, E> plain;
       if (adjacent(r.loop->lo, r.loop->hi, r.row)) plain[r.row] = mk_raw(r.row.str(), ity);
       ss.push_back(mk_def(lw, ity, subst_vars(r.loop->lo, plain), r.loop->i));
       ss.push_back(mk_def(hw, ity, subst_vars(r.loop->hi, plain), r.loop->i));
+      *lo = mk_var(lw, ity);
+      *hi = mk_var(hw, ity);
+    };
+    auto bounds = [&](Stmts& ss, E* lo, E* hi) {
+      for (auto& st : r.pre) ss.push_back(st);
+      // (the bounds of a row without elements may be anything, a marker like 2^63 - 1 and 0: what is cut to 32 bits of them, or
+      // passes the largest integer when a lane's place is added, must not become a row)
+      Name any = gen.fresh("any"), ln = gen.fresh("first"), hn = gen.fresh("end");
+      E l, h, some = mk_var(any, bty);
+      limits(ss, &l, &h);
       ss.push_back(mk_def(any, bty, mk_binop(BinOp::Lt, l, h, bty), r.loop->i));
       ss.push_back(mk_def(ln, ety, narrow(mk_ifexpr(some, l, iint(0), ity)), r.loop->i));
       ss.push_back(mk_def(hn, ety, narrow(mk_ifexpr(some, h, iint(0), ity)), r.loop->i));
@@ -433,7 +484,6 @@ struct RaggedSum {
       e->iv = 1;
       top.push_back(e);
     }
-    const bool all_in_front = scouts > 0 && huge == longest;
     top.push_back(mk_rawstmt("if (threadIdx.x == 0) " + count.str() + "[0] = 0;"));
     top.push_back(mk_sync());
 
@@ -455,15 +505,15 @@ struct RaggedSum {
         own.push_back(mk_def(ln, ity, l));
         l = mk_var(ln, ity);
       }
+      sums_from_zero(own);
       walk(own, lo, hi, narrow(sub), P, l);
       if (P > 1) own.push_back(team_sum(L == 1 && P == 8 ? "parpy_sum8" : "parpy_team_sum<" + std::to_string(L) + ", " + std::to_string(T) + ">"));
       Stmts f = finish_slots(l);
       if (P > 1) own.push_back(mk_if(mk_binop(BinOp::Lt, qv, iint(L), bty), f, {}));
       else own.insert(own.end(), f.begin(), f.end());
       const S enqueue = mk_rawstmt(queue.str() + "[atomicAdd(&" + count.str() + "[0], 1)] = (int)" + r.row.str() + ";");
-      auto longer = [&](const E& a, const E& b) { return mk_binop(BinOp::Gt, mk_binop(BinOp::Sub, b, a, ety), eint(huge), bty); };
       Stmts defer;
-      if (!all_in_front) defer = {mk_if(mk_binop(BinOp::Eq, qv, iint(0), bty), {scouts ? mk_if(longer(lo, hi), {}, {enqueue}) : enqueue}, {})};
+      if (!scouts) defer = {mk_if(mk_binop(BinOp::Eq, qv, iint(0), bty), {enqueue}, {})};
       body.push_back(mk_if(mk_binop(BinOp::Leq, mk_binop(BinOp::Sub, hi, lo, ety), eint(longest), bty), own, defer));
       auto nr = clone(k.body[0]);
       nr->id = lane;
@@ -473,9 +523,11 @@ struct RaggedSum {
         Name at = gen.fresh(r.row.s + "_at"), slice = gen.fresh("slice");
         const E first = mk_binop(BinOp::Mul, mk_var(slice, ity), iint(looked), ity);
         Stmts look{mk_def(r.row, ity, mk_var(at, ity), r.loop->i)};
+        for (auto& st : r.pre) look.push_back(st);
         E a, b;
-        bounds(look, &a, &b);
-        look.push_back(mk_if(longer(a, b), {enqueue}, {}));
+        limits(look, &a, &b);
+        const E more = mk_binop(BinOp::Gt, mk_binop(BinOp::Sub, b, a, ity), iint(longest), bty);
+        look.push_back(mk_if(mk_binop(BinOp::And, mk_binop(BinOp::Lt, a, b, bty), more, bty), {enqueue}, {}));
         nr->body = {mk_if(mk_binop(BinOp::Lt, lv, iint(scouts * tpb), bty),
                           {mk_def(slice, ity, mk_binop(BinOp::FloorDiv, lv, iint(tpb), ity)),
                            mk_for(at, add(first, mk_binop(BinOp::Rem, lv, iint(tpb), ity)), mk_binop(BinOp::Min, add(first, iint(looked)), iint(r.n), ity), tpb, look, LoopPar(), r.loop->i)},
@@ -488,7 +540,7 @@ struct RaggedSum {
       nr->map.n = (r.n * T + scouts * tpb + WAVE_SIZE - 1) / WAVE_SIZE * WAVE_SIZE;
       top.push_back(nr);
     }
-    if (all_in_front) top.push_back(mk_rawstmt("if (blockIdx.x >= " + std::to_string(scouts) + ") return;"));
+    if (scouts) top.push_back(mk_rawstmt("if (blockIdx.x >= " + std::to_string(scouts) + ") return;"));
     top.push_back(mk_sync());
 
     // long rows, one after the other, by all threads of the workgroup
@@ -505,7 +557,53 @@ struct RaggedSum {
       E lo, hi;
       bounds(body, &lo, &hi);
       E l = L == 1 ? iint(0) : mk_binop(BinOp::Rem, tv, iint(L), ity), sub = L == 1 ? tv : mk_binop(BinOp::FloorDiv, tv, iint(L), ity);
-      walk(body, lo, hi, narrow(sub), tpb / L, l);
+      sums_from_zero(body);
+      // An element costs two dependent round trips, its column and what the column selects, and the longest row makes them one
+      // batch after the other.  Where lanes along the columns leave few elements to a batch, the workgroup loads the columns
+      // and values of as many elements as it has threads at once, those of the next piece while this one is summed, and the
+      // batches wait for the selected rows alone.  The order of the sum stays.  9529 rows of 41 on average times 101 columns
+      // 40.7 -> 31.8 us, 1021 of 35 times 256 23.2 -> 20.3, 20 000 of 24 times 128 35.4 -> 34.5; twice the elements in a batch
+      // instead of that or beside it are registers: 75 and 46 us for the first and the last.
+      std::vector<Staged> staged;
+      int64_t bytes = 0;
+      if (r.has_col && U <= L)
+        for (auto& e : element_loads(k, r)) {
+          staged.push_back({e, gen.fresh("staged")});
+          bytes += elem_bytes(e->ty.sz);
+        }
+      if (staged.empty() || bytes > 16) {
+        walk(body, lo, hi, narrow(sub), tpb / L, l);
+      } else {
+        Name from = gen.fresh("from"), upto = gen.fresh("upto");
+        E fv = mk_var(from, ety), uv = mk_var(upto, ety);
+        Stmts put;
+        Stmts fetch_next;
+        for (auto& st : staged) {
+          auto d = std::make_shared<Stmt>();
+          d->k = Stmt::LdsDecl;
+          d->id = st.lds;
+          d->ty = st.load->ty;
+          d->iv = tpb;
+          top.push_back(d);
+          k.lds_bytes += tpb * elem_bytes(st.load->ty.sz);
+          Name next = gen.fresh(st.lds.s + "_next");
+          auto load_at = [&](const E& start, int64_t ahead) {
+            // (the last element where the thread has none: loads without a test, which the walk does not wait for)
+            E i = mk_binop(BinOp::Min, mk_binop(BinOp::Add, narrow(tv), eint(ahead), ety), mk_binop(BinOp::Sub, mk_binop(BinOp::Sub, hi, eint(1), ety), start, ety), ety);
+            std::map<Name, E> at{{r.loop->id, widen(mk_binop(BinOp::Add, start, i, ety))}};
+            return subst_vars(st.load, at);
+          };
+          body.push_back(mk_def(next, st.load->ty, load_at(lo, 0)));
+          fetch_next.push_back(mk_assign(mk_var(next, st.load->ty), load_at(fv, tpb)));
+          put.push_back(mk_assign(mk_index(mk_var(st.lds, Type::pointer(st.load->ty.sz, Mem::LDS)), tv, st.load->ty), mk_var(next, st.load->ty)));
+        }
+        Stmts piece{mk_def(upto, ety, mk_binop(BinOp::Min, mk_binop(BinOp::Add, fv, eint(tpb), ety), hi, ety)), mk_sync()};
+        piece.insert(piece.end(), put.begin(), put.end());
+        piece.push_back(mk_sync());
+        piece.insert(piece.end(), fetch_next.begin(), fetch_next.end());
+        walk(piece, fv, uv, narrow(sub), tpb / L, l, staged);
+        body.push_back(mk_for(from, lo, hi, tpb, piece, LoopPar(), r.loop->i));
+      }
       if (!r.has_col) {
         Name w = gen.fresh("whole");
         body.push_back(mk_def(w, sty, part(iint(0))));
@@ -555,7 +653,7 @@ struct RaggedSum {
     k.lds_bytes += (std::max(teams, looked) + 1) * 4;
     k.body = top;
     k.block = Dim3{tpb, 1, 1};
-    k.grid = Dim3{(r.n + teams - 1) / teams + scouts, 1, 1};
+    k.grid = Dim3{groups + scouts, 1, 1};
     launch->grid = k.grid;
     launch->block = k.block;
     return true;

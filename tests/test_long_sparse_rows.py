@@ -51,9 +51,11 @@ def test_long_rows_stand_in_front():
     s = parpy.print_compiled(spmv, [A, np.zeros(n, np.float32), np.zeros(n, np.float32)], opts(n))
     hiprtc_compile(s[:s.index("// host side")], opts(n))
     assert "if (blockIdx.x >= 512) return;" in s and "dim3(512, 1, 1)" in s
-    n = 20000     # all at once: shared where they are
-    A = matrix(n, lengths_of("ends", n), np.float32)
-    assert ") return;" not in parpy.print_compiled(spmv, [A, np.zeros(n, np.float32), np.zeros(n, np.float32)], opts(n))
+    # all at once: as many in front as have room beside the others, none where there is none
+    for n, each, in_front in ((20000, 7, 433), (4000, 7, 250), (8000, 150, 0), (65536, 16, 0)):
+        A = matrix(n, np.full(n, each), np.float32)
+        s = parpy.print_compiled(spmv, [A, np.zeros(n, np.float32), np.zeros(n, np.float32)], opts(n))
+        assert (f"if (blockIdx.x >= {in_front}) return;" in s) if in_front else ") return;" not in s, n
 
 
 @pytest.mark.gpu
@@ -70,3 +72,48 @@ def test_sums(kind, dtype, tol):
         want[A["rows"][1:] == A["rows"][:-1]] = 0.0
         # rounding of sums of up to 5000 products of size one
         assert np.abs(y - want).max() < tol * np.sqrt(5000) * 4, (n, tpb)
+
+
+@parpy.jit
+def spmm(A, B, C):
+    parpy.label('i')
+    for i in range(A["nrows"]):
+        parpy.label('j')
+        for j in range(B["ncols"]):
+            C[i, j] = 0.0
+            parpy.label('k')
+            for k in range(A["rows"][i], A["rows"][i + 1]):
+                C[i, j] += A["values"][k] * B["values"][A["cols"][k], j]
+
+
+def column_opts(n, cols):
+    o = parpy.par({'i': parpy.threads(n), 'j': parpy.threads(cols)})
+    o.backend = HIP
+    return o
+
+
+def test_elements_of_long_rows_stand_in_lds():
+    for n, cols, staged, in_front in ((1000, 256, 2, 125), (1000, 37, 2, 125), (8192, 128, 2, 0), (8100, 128, 2, 512), (20000, 64, 2, 1024), (1000, 4, 0, 125)):
+        A = matrix(n, np.full(n, 20), np.float32)
+        args = [A, {"values": np.zeros((n, cols), np.float32), "ncols": cols}, np.zeros((n, cols), np.float32)]
+        s = parpy.print_compiled(spmm, args, column_opts(n, cols))
+        hiprtc_compile(s[:s.index("// host side")], column_opts(n, cols))
+        assert s.count(" staged_") - s.count(" staged_next") >= staged and ("staged_" in s) == (staged > 0), (n, cols)
+        assert (f"if (blockIdx.x >= {in_front}) return;" in s) if in_front else ") return;" not in s, (n, cols)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["ends", "bound", "slice", "even"])
+@pytest.mark.parametrize("n,cols", [(4000, 256), (4000, 37), (8100, 100), (8192, 128), (20000, 64), (4000, 4)])
+def test_sums_of_columns(kind, n, cols):
+    lengths = lengths_of(kind, n)
+    lengths[50:53] = [1023, 1024, 1025]          # whole pieces of a row and one more
+    A = matrix(n, lengths, np.float32)
+    B = np.random.default_rng(2).standard_normal((n, cols)).astype(np.float32)
+    C = np.full((n, cols), -1.0, np.float32)
+    spmm(A, {"values": B, "ncols": cols}, C, opts=column_opts(n, cols))
+    terms = A["values"].astype(np.float64)[:, None] * B[A["cols"]]
+    want = np.add.reduceat(np.vstack([terms, np.zeros((1, cols))]), A["rows"][:-1])
+    want[A["rows"][1:] == A["rows"][:-1]] = 0.0
+    # rounding of sums of up to 5000 products of size one
+    assert np.abs(C - want).max() < 2e-5 * np.sqrt(5000) * 4
