@@ -686,17 +686,20 @@ struct RowThreads {
     if (root->map.n != rows || k.grid.x * k.grid.y * k.grid.z != rows) return false;
     // straight through the row: element loops and reductions over the whole workgroup, no loop around them
     bool ok = true, reduces = false, strided = false;
+    bool meets_in_test = false;   // a barrier under a test that not all rows of a workgroup need pass
     int64_t longest = 0, bytes = 0, loops = 0;
     Pass probe(k, opts, gen);
-    std::function<void(const Stmts&)> walk = [&](const Stmts& ss) {
+    std::function<void(const Stmts&, bool)> walk = [&](const Stmts& ss, bool tested) {
       for (auto& s : ss) {
         switch (s->k) {
-          case Stmt::Def: case Stmt::Assign: case Stmt::Sync: break;
+          case Stmt::Def: case Stmt::Assign: break;
+          case Stmt::Sync: meets_in_test = meets_in_test || tested; break;
           case Stmt::WaveReduce:
             reduces = true;
+            meets_in_test = meets_in_test || tested;
             if (s->iv != threads) ok = false;
             break;
-          case Stmt::If: walk(s->body); walk(s->els); break;
+          case Stmt::If: walk(s->body, true); walk(s->els, true); break;
           case Stmt::For: {
             if (!thread_mapped(s) || s->map.dim != 0 || s->map.n != threads || !s->els.empty()) { ok = false; break; }
             const int64_t extent = const_extent(s);
@@ -712,7 +715,7 @@ struct RowThreads {
         }
       }
     };
-    walk(root->body);
+    walk(root->body, false);
     if (!ok || !reduces || longest == 0 || bytes == 0) return false;
     int64_t want = threads;
     if (rows * (threads / WAVE_SIZE) > 4096) {
@@ -735,7 +738,18 @@ struct RowThreads {
     // Workgroups start at about two per nanosecond, which is what small ones wait for: four rows each where a row is a
     // wavefront's (the sums above 7.1 us, 6.7 with eight; softmax over 30000 rows of 200 floats 16.0 -> 8.7 us).
     // (a launch of four wavefronts per SIMD or less starts all of them at once)
-    const int64_t group = want == WAVE_SIZE && rows > 4096 ? 4 : 1;
+    int64_t group = want == WAVE_SIZE && rows > 4096 ? 4 : 1;
+    // Rows of one loop, four vectors per thread at most: what such a workgroup moves is over before the next has started, and
+    // what they wait for is the start.  Up to eight rows and 1024 threads each, the rows still on threads of their own: the
+    // order of a row's sum stays.  Floats, rows x length, one row against this: 400 x 4000 5.0 -> 3.5 us, 1000 x 1708 4.8 -> 3.4,
+    // 5000 x 1000 7.9 -> 5.0, 5000 x 1001 7.5 -> 5.4, 9001 x 1777 14.0 -> 12.1, 12000 x 1500 15.0 -> 11.8, 16384 x 3000
+    // 35.0 -> 33.2; doubles 4001 x 333 5.3 -> 3.5, 16384 x 500 12.3 -> 11.2 (11.0 with four wavefronts' rows, but 5000 x 1000
+    // floats 5.3).  At most 256 rows start at once.  Where memory is the bound it is no gain: 7602 x 2236 doubles 23.9 and 23.9
+    // us, 512 threads and 134 MB 24.2 and 24.6.  Rows that several loops walk lose by waiting for each other at the barriers:
+    // softmax over 8000 x 1024 floats 11.6 us alone, 12.9 in eights; over 16384 x 1500 32.3 and 34.4.
+    const int64_t total = rows * longest * bytes;
+    if (loops == 1 && rows > 256 && !meets_in_test && longest * bytes <= 64 * want && total < (int64_t(1) << (want > 256 ? 27 : 28)))
+      group = std::max<int64_t>(group, std::min<int64_t>(8, 1024 / want));
     if (want == threads && group == 1) return false;
     std::function<Stmts(const Stmts&)> cut = [&](const Stmts& ss) {
       Stmts out;
@@ -757,7 +771,7 @@ struct RowThreads {
       nr->map.per = group;
       nr->map.n = blocks * group;
       (root->map.dim == 0 ? k.grid.x : root->map.dim == 1 ? k.grid.y : k.grid.z) = blocks;
-      k.wave_rows = true;
+      k.wave_rows = want == WAVE_SIZE;
     }
     k.body = {S(nr)};
     launch->grid = k.grid;

@@ -980,7 +980,13 @@ struct DevicePrinter {
       os << ind(n) << "{\n";
       os << ind(n + 2) << vty << " " << v << " = " << init(idx) << ";\n";
       std::string cond;
-      if (extent < launched) cond = v + cmp + his;
+      if (extent < launched && m.per > 1 && !kernel->wave_rows) {
+        // a workgroup with several rows that meets at barriers: the wavefronts without a row end here, a barrier waits for
+        // those that are left
+        os << ind(n + 2) << "if (__builtin_amdgcn_readfirstlane(" << v << ") >= " << his << ") return;\n";
+      } else if (extent < launched) {
+        cond = v + cmp + his;
+      }
       if (!guard.empty() && cond.empty()) cond = guard;  // v < hi already implies the launch guard (extent <= N)
       if (!cond.empty()) {
         os << ind(n + 2) << "if (" << cond << ") {\n";
@@ -1196,10 +1202,12 @@ struct DevicePrinter {
           os << ind(n) << v << " = parpy_wave_reduce<" << op << ">(" << v << ");\n";
         } else {
           std::string slots = "parpy_red_" + std::to_string(red_sites++);
-          lds_decls.push_back("__shared__ " + ty + " " + slots + "[" + std::to_string(nwaves) + "];");
+          // (a workgroup with several rows has slots for each)
+          const int64_t rows = s->iv == kernel->block.x ? kernel->block.y : 1;
+          lds_decls.push_back("__shared__ " + ty + " " + slots + "[" + std::to_string(nwaves * rows) + "];");
           E ne = neutral_element(s->bop == BinOp::And ? BinOp::BitAnd : s->bop == BinOp::Or ? BinOp::BitOr : s->bop, s->ty.sz, s->i);
           os << ind(n) << v << " = parpy_block_reduce<" << op << ", " << nwaves << ">(" << v << ", (" << ty << ")" << pexpr(ne)
-             << ", " << slots << ", " << (s->unroll ? "true" : "false") << ");\n";
+             << ", " << slots << (rows > 1 ? " + " + std::to_string(nwaves) + " * (int)threadIdx.y" : "") << ", " << (s->unroll ? "true" : "false") << ");\n";
         }
         break;
       }
