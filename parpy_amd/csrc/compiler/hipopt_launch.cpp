@@ -737,8 +737,9 @@ struct RowThreads {
     while (loops > 1 && !strided && want < 1024 && longest * bytes > 32 * 16 * want) want *= 2;
     // Workgroups start at about two per nanosecond, which is what small ones wait for: four rows each where a row is a
     // wavefront's (the sums above 7.1 us, 6.7 with eight; softmax over 30000 rows of 200 floats 16.0 -> 8.7 us).
-    // (a launch of four wavefronts per SIMD or less starts all of them at once)
-    int64_t group = want == WAVE_SIZE && rows > 4096 ? 4 : 1;
+    // Fewer of them start at once in time where a wavefront has more than four vectors per lane to move; below that they
+    // share workgroups too (softmax over 4000 rows of 700 floats 5.4 -> 5.0 us, over 3000 of 300 3.85 -> 3.57).
+    int64_t group = want == WAVE_SIZE && (rows > 4096 || (rows > 256 && longest * bytes <= 64 * want)) ? 4 : 1;
     // Rows of one loop, four vectors per thread at most: what such a workgroup moves is over before the next has started, and
     // what they wait for is the start.  Up to eight rows and 1024 threads each, the rows still on threads of their own: the
     // order of a row's sum stays.  Floats, rows x length, one row against this: 400 x 4000 5.0 -> 3.5 us, 1000 x 1708 4.8 -> 3.4,

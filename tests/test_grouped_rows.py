@@ -71,6 +71,9 @@ def test_rows_of_a_workgroup(n, m, threads, want):
 
 
 def test_rows_that_stay_alone():
+    for n, m, rows in ((257, 500, 4), (256, 500, 1), (4096, 2000, 1), (4097, 700, 4)):      # a wavefront each, no barriers
+        x = np.zeros((n, m), np.float32)
+        assert block(two_loops, [x, x.copy(), n], n, 64)[0] == (64, rows), (n, m)
     x, out = np.zeros((5000, 1500), np.float32), np.zeros(5000, np.float32)
     assert block(two_loops, [x, x.copy(), 5000], 5000, 256)[0][1] == 1
     assert block(chosen, [x, np.ones(5000, np.int32), out, 5000], 5000, 256)[0][1] == 1     # a barrier that not every row meets
