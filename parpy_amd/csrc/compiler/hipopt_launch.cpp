@@ -684,6 +684,7 @@ struct RowThreads {
       return false;
     const int64_t rows = root->hi->iv, threads = k.block.x;
     if (root->map.n != rows || k.grid.x * k.grid.y * k.grid.z != rows) return false;
+    if (share_starts(k, root, launch, rows, threads)) return true;
     // straight through the row: element loops and reductions over the whole workgroup, no loop around them
     bool ok = true, reduces = false, strided = false;
     bool meets_in_test = false;   // a barrier under a test that not all rows of a workgroup need pass
@@ -767,16 +768,38 @@ struct RowThreads {
     auto nr = clone(root);
     nr->body = cut(root->body);
     k.block = Dim3{want, group, 1};
+    if (group > 1) k.wave_rows = want == WAVE_SIZE;
+    several(k, nr, launch, rows, group);
+    return true;
+  }
+
+  static void several(Kernel& k, const StmtP& root, const StmtP& launch, int64_t rows, int64_t group) {
     if (group > 1) {
       const int64_t blocks = (rows + group - 1) / group;
-      nr->map.per = group;
-      nr->map.n = blocks * group;
+      root->map.per = group;
+      root->map.n = blocks * group;
       (root->map.dim == 0 ? k.grid.x : root->map.dim == 1 ? k.grid.y : k.grid.z) = blocks;
-      k.wave_rows = want == WAVE_SIZE;
     }
-    k.body = {S(nr)};
+    k.body = {S(root)};
     launch->grid = k.grid;
     launch->block = k.block;
+  }
+
+  // Rows on a wavefront or two whose threads never meet (the row numbers of a compressed matrix, written to its elements): how
+  // long they are may stand in memory, so they share workgroups where those are still as many as the device has compute
+  // units.  SDDMM with a compressed mask, whose row numbers are filled in first: 8192 rows of 82, 128 deep, 34.8 -> 32.1 us;
+  // 2491 rows of 5, 174 deep, doubles 13.8 -> 13.0.
+  bool share_starts(Kernel& k, const S& root, const StmtP& launch, int64_t rows, int64_t threads) {
+    bool apart = threads <= 128 && rows >= 2048;
+    visit_stmts(root->body, [&](const S& s) {
+      const bool plain = s->k == Stmt::Def || s->k == Stmt::Assign || s->k == Stmt::If ||
+                         (s->k == Stmt::For && (s->map.k == GpuMap::None || (s->map.k == GpuMap::Thread && s->map.dim == 0 && s->map.n == threads && !s->par.reduction)));
+      apart = apart && plain;
+    });
+    if (!apart) return false;
+    const int64_t group = 512 / threads;
+    k.block = Dim3{threads, group, 1};
+    several(k, clone(root), launch, rows, group);
     return true;
   }
 

@@ -49,6 +49,15 @@ def two_loops(x, out, N):
         out[i, :] = exp(x[i, :] - m)
 
 
+@parpy.jit
+def numbers(first, rows, N):
+    parpy.label('i')
+    for i in range(N):
+        parpy.label('j')
+        for q in range(first[i], first[i + 1]):
+            rows[q] = rows[q] + i
+
+
 def opts(n, threads):
     o = parpy.par({'i': parpy.threads(n), 'j': parpy.threads(threads)})
     o.backend = parpy.CompileBackend.Hip
@@ -77,6 +86,22 @@ def test_rows_that_stay_alone():
     x, out = np.zeros((5000, 1500), np.float32), np.zeros(5000, np.float32)
     assert block(two_loops, [x, x.copy(), 5000], 5000, 256)[0][1] == 1
     assert block(chosen, [x, np.ones(5000, np.int32), out, 5000], 5000, 256)[0][1] == 1     # a barrier that not every row meets
+
+
+def test_rows_that_never_meet():
+    for n, threads, rows in ((2047, 64, 1), (2048, 64, 8), (5001, 128, 4), (5001, 256, 1)):
+        (width, group), s = block(numbers, [np.zeros(n + 1, np.int64), np.zeros(9, np.int64), n], n, threads)
+        assert (width, group) == (threads, rows) and ("readfirstlane(i_" in s) == (rows > 1 and n % rows != 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [2047, 2048, 5001])
+def test_row_numbers(n):
+    for threads in (64, 128):
+        first = np.concatenate([[0], np.cumsum(np.random.default_rng(n).integers(0, 200, n))]).astype(np.int64)
+        rows = np.arange(first[-1], dtype=np.int64)
+        numbers(first, rows, n, opts=opts(n, threads))
+        assert np.array_equal(rows - np.arange(first[-1]), np.repeat(np.arange(n), np.diff(first)))
 
 
 @pytest.mark.gpu
