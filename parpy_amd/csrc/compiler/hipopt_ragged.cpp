@@ -20,12 +20,12 @@ namespace {
 //     each where the columns allow it), P subteams take every P-th element of the row.
 //   * A subteam issues U elements at a time: index loads first, then what they select.  The last batch is clamped to
 //     the row's last element instead of branching, so that its loads are issued together as well.
-//   * A row longer than `longest` elements is left to the workgroup: its teams queue such rows in LDS, and after a
-//     barrier all waves share each of them.
+//   * A row longer than `longest` elements is shared by all waves of a workgroup: by one of those in front of the others,
+//     which look for such rows and queue them in LDS, or, where there are none, by that of its own team.
 //
 // Measured (100 000 rows of 50 non-zeros on average, the longest 15 800, float64): eight lanes per row, one element in
 // flight 547 us, in teams 34 us.  The gathers out of L2 are then what bounds it: 5.5 million lines requested (counted, 87 %
-// of them hits), 141 per nanosecond.  20 000 rows of 24 on average (longest 3400)
+// of them hits), 158 per nanosecond.  20 000 rows of 24 on average (longest 3400)
 // times a 128-column matrix: one workgroup per row with the sum read and written back in LDS per element 840 us, in
 // teams 42 us, with the long rows in front (below) 34: the longest pulls 1.7 MB through one compute unit, and 165 of the 261 MB
 // that the L2s deliver come from behind them, since the 10 MB matrix does not fit a die's 4 MB.
