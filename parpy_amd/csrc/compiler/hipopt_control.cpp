@@ -230,7 +230,9 @@ Stmts Pass::expand_short_loops(const Stmts& ss0, bool in_par) {
 // and the arrays of each are known (the base of an LDS access becomes part of the instruction, and a load and a store are
 // seen not to coincide).  100 reads of 1000 to 3000 samples, scaled form: 16-layer models of 3- / 4- / 5-mers 1733 -> 1069 us,
 // 2335 -> 1547, 3487 -> 2955; single layer, 4- / 5- / 6-mers 587 -> 503, 810 -> 725, 1256 -> 1090; reference form, 3- / 4- /
-// 5-mers 531 -> 398, 655 -> 530, 1034 -> 926.  One of 21 got slower: 16 layers of 3-mers, reference form, 1169 -> 1219.
+// 5-mers 531 -> 398, 655 -> 530, 1034 -> 926.  A step under a test (`if t < len: <step> elif t == len: <copy>`) gains with several
+// elements per thread (16 layers of 4-mers, reference form, 3274 -> 3031) and loses with one, where the test is most of
+// what a second copy adds (of 3-mers 1170 -> 1224): that one stays as it is.
 Stmts Pass::pair_steps(const Stmts& ss) {
   static const char* const PARITY = "parpy_odd.value";
   Stmts out;
@@ -242,6 +244,12 @@ Stmts Pass::pair_steps(const Stmts& ss) {
     if (s->k == Stmt::For && s->map.k == GpuMap::None && !s->unroll && s->step == 1 && s->lo->k == Expr::Int && s->els.empty()) {
       for (auto& c : s->body) {
         if (c->k == Stmt::Sync) barrier = true;
+        if (c->k == Stmt::If && !c->els.empty())
+          for (auto& d : c->body) {
+            bool one = thread_mapped(d) && per_thread_trips(d) == 1;
+            if (one) visit_stmts(d->body, [&](const S& e) { one = one && e->k != Stmt::For; });
+            if (one) plain = false;
+          }
         if (c->k == Stmt::If && alternates(c->expr, s))
           for (auto& d : c->body)
             if (d->k == Stmt::Assign && d->dst->k == Expr::Var && d->dst->ty.is_pointer() && d->dst->ty.mem == Mem::LDS) swaps = true;

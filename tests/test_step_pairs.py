@@ -32,6 +32,14 @@ def test_one_text_for_both_parities():
     assert "parpy_step" not in text(7, 1024)      # the registers of a thread are taken by its tables
 
 
+@pytest.mark.parametrize("k,taken", [(3, False), (4, True)])
+def test_a_step_under_a_test_needs_several_elements_per_thread(k, taken):
+    hmm, seqs = W.random_reference_model(k, n_reads=2, min_len=3, max_len=6)
+    a = np.zeros((2, hmm["num_states"]), np.float32)
+    s = parpy.print_compiled(W.forward_kernel, [hmm, seqs, a, a.copy(), np.zeros(2, np.float32)], opts(2, 1024))
+    assert ("parpy_step" in s) == taken
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", ["reference", "grouped", "scaled"])
 @pytest.mark.parametrize("k,threads", [(3, 64), (4, 64), (5, 256)])
