@@ -790,7 +790,7 @@ struct RowThreads {
   // units.  SDDMM with a compressed mask, whose row numbers are filled in first: 8192 rows of 82, 128 deep, 34.8 -> 32.1 us;
   // 2491 rows of 5, 174 deep, doubles 13.8 -> 13.0.
   bool share_starts(Kernel& k, const S& root, const StmtP& launch, int64_t rows, int64_t threads) {
-    bool apart = threads <= 128 && rows >= 2048;
+    bool apart = threads <= 128 && rows >= 2048 && rows < (int64_t(1) << 30);
     visit_stmts(root->body, [&](const S& s) {
       const bool plain = s->k == Stmt::Def || s->k == Stmt::Assign || s->k == Stmt::If ||
                          (s->k == Stmt::For && (s->map.k == GpuMap::None || (s->map.k == GpuMap::Thread && s->map.dim == 0 && s->map.n == threads && !s->par.reduction)));
