@@ -232,7 +232,8 @@ Stmts Pass::expand_short_loops(const Stmts& ss0, bool in_par) {
 // 2335 -> 1547, 3487 -> 2955; single layer, 4- / 5- / 6-mers 587 -> 503, 810 -> 725, 1256 -> 1090; reference form, 3- / 4- /
 // 5-mers 531 -> 398, 655 -> 530, 1034 -> 926.  A step under a test (`if t < len: <step> elif t == len: <copy>`) gains with several
 // elements per thread (16 layers of 4-mers, reference form, 3274 -> 3031) and loses with one, where the test is most of
-// what a second copy adds (of 3-mers 1170 -> 1224): that one stays as it is.
+// what a second copy adds (of 3-mers 1170 -> 1224): that one stays as it is.  Of loops inside each other the inner one: the
+// outer one's parity has no name there, and every level would double the text.
 Stmts Pass::pair_steps(const Stmts& ss) {
   static const char* const PARITY = "parpy_odd.value";
   Stmts out;
@@ -241,7 +242,8 @@ Stmts Pass::pair_steps(const Stmts& ss) {
     r->body = pair_steps(s->body);
     if (s->k != Stmt::For || s->map.k == GpuMap::None) r->els = pair_steps(s->els);
     bool swaps = false, barrier = false, plain = true;
-    if (s->k == Stmt::For && s->map.k == GpuMap::None && !s->unroll && s->step == 1 && s->lo->k == Expr::Int && s->els.empty()) {
+    visit_stmts(r->body, [&](const S& c) { if (c->in_pairs) plain = false; });
+    if (plain && s->k == Stmt::For && s->map.k == GpuMap::None && !s->unroll && s->step == 1 && s->lo->k == Expr::Int && s->els.empty()) {
       for (auto& c : s->body) {
         if (c->k == Stmt::Sync) barrier = true;
         if (c->k == Stmt::If && !c->els.empty())

@@ -1,11 +1,14 @@
 """Time loops whose steps swap two arrays in LDS, compiled once for odd and once for even steps: reads that end in the first,
-the second and the odd step out, against the float64 oracle and the loop that is not taken apart."""
+the second and the odd step out, against the float64 oracle and the loop that is not taken apart; loops inside each other."""
+import re
+
 import numpy as np
 import pytest
 
 import oracle
 import parpy_amd as parpy
 from parpy_amd import workloads as W
+from parpy_amd.compile import hiprtc_compile
 
 torch = pytest.importorskip("torch")
 
@@ -63,3 +66,70 @@ def test_reads_of_odd_and_even_length(k, threads, form):
     assert np.abs(got[True][0] - want).max() < (1e-4 if form == "scaled" else 41 * 2.0 ** -16)
     for with_pairs, without in zip(got[True], got[False]):
         np.testing.assert_allclose(with_pairs, without, rtol=1e-5, atol=1e-5 if form != "scaled" else 1e-30)
+
+
+@parpy.jit
+def loops_inside_each_other(a, b, out, N, M, U, T):
+    parpy.label('inst')
+    for i in range(N):
+        for u in range(1, U):
+            s = b
+            d = a
+            if u & 1:
+                s = a
+                d = b
+            parpy.label('state')
+            for j in range(M):
+                d[i, j] = s[i, (j + 1) % M] * 0.5
+            for t in range(u % 2, T):
+                s2 = b
+                d2 = a
+                if t & 1:
+                    s2 = a
+                    d2 = b
+                parpy.label('state')
+                for j in range(M):
+                    d2[i, j] = s2[i, (j + 1) % M] * (1.0 if u % 2 == 0 else 0.25) + s2[i, j] * (1.0 if u & 1 else 2.0)
+            for t in range(1, T):
+                s3 = b
+                d3 = a
+                if t & 1:
+                    s3 = a
+                    d3 = b
+                parpy.label('state')
+                for j in range(M):
+                    d3[i, j] = s3[i, (j + 2) % M] * (0.5 if u & 1 else 0.25)
+        parpy.label('state')
+        for j in range(M):
+            out[i, j] = a[i, j] - b[i, j]
+
+
+def test_of_loops_inside_each_other_the_inner_one():
+    a = np.zeros((4, 512), np.float32)
+    s = parpy.print_compiled(loops_inside_each_other, [a, a.copy(), a.copy(), 4, 512, 6, 7], opts(4, 256))
+    hiprtc_compile(s[:s.index("// host side")], opts(4, 256))
+    step = re.findall(r"const auto parpy_step = \[&\]\(auto parpy_odd, const \w+ (\w+)_\d+\)", s)
+    assert step and set(step) == {"t"}
+    assert len(re.findall(r"\(u_\d+ & 1\) \? ", s)) == 2 and not re.search(r"parpy_odd\.value\)* \?", s)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("U,T", [(2, 2), (5, 4), (6, 7)])
+def test_loops_inside_each_other(U, T):
+    n, m = 3, 512
+    rng = np.random.default_rng(U)
+    a, b = rng.random((n, m)).astype(np.float32), rng.random((n, m)).astype(np.float32)
+    out = np.zeros_like(a)
+    x, y = a.astype(np.float64), b.astype(np.float64)
+    loops_inside_each_other(a, b, out, n, m, U, T, opts=opts(n, 256))
+    for u in range(1, U):
+        (y if u & 1 else x)[:] = np.roll(x if u & 1 else y, -1, axis=1) * 0.5
+        for t in range(u % 2, T):
+            s = x if t & 1 else y
+            (y if t & 1 else x)[:] = np.roll(s, -1, axis=1) * (1.0 if u % 2 == 0 else 0.25) + s * (1.0 if u & 1 else 2.0)
+        for t in range(1, T):
+            (y if t & 1 else x)[:] = np.roll(x if t & 1 else y, -2, axis=1) * (0.5 if u & 1 else 0.25)
+    # every value is a sum of positive terms of at most 2 * U * T steps, each rounded once to 24 bits
+    for got, want in ((a, x), (b, y)):
+        np.testing.assert_allclose(got, want, rtol=2 * U * T * 2.0 ** -24)
+    assert np.array_equal(out, a - b)
