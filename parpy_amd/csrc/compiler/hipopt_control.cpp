@@ -259,14 +259,21 @@ Stmts Pass::pair_steps(const Stmts& ss) {
       visit_stmts(s->body, [&](const S& c) { if ((c->k == Stmt::RawStmt && c->fname.rfind("__builtin_amdgcn_wave_barrier", 0) != 0) || c->k == Stmt::Return || (c->k == Stmt::Assign && c->dst->k == Expr::Var && c->dst->name == s->id)) plain = false; });
     }
     if (!(swaps && barrier && plain)) { out.push_back(r); continue; }
-    // the tests of the parity become constants of the copy
+    // the tests of the parity become constants of the copy (where a number is made of it, its width counts: that stays)
     const Type bty = Type::scalar(ElemSize::Bool);
     const E is_odd = mk_raw(PARITY, bty);
     auto counter = [&](const E& e) { const E v = strip_converts(e); return v->k == Expr::Var && v->name == s->id; };
+    auto tested = [&](const E& e) { return alternates(e, s) ? is_odd : e; };
     r->body = rewrite_stmts(r->body, [&](const E& e) -> E {
-      if (e->k != Expr::BinOpE || e->args[1]->k != Expr::Int) return e;
+      if (e->k == Expr::IfExpr) {
+        auto n = std::make_shared<Expr>(*e);
+        n->args[0] = tested(e->args[0]);
+        return n;
+      }
+      if (e->k != Expr::BinOpE || e->args[1]->k != Expr::Int || !(e->bop == BinOp::Eq || e->bop == BinOp::Neq)) return e;
       const int64_t c = e->args[1]->iv;
-      if (e->bop == BinOp::BitAnd && c == 1 && counter(e->args[0])) return is_odd;
+      if ((c == 0 || c == 1) && alternates(e->args[0], s) && e->args[0]->ty.sz != ElemSize::Bool)
+        return (e->bop == BinOp::Eq) == (c == 1) ? is_odd : mk_unop(UnOp::Not, is_odd, bty);
       if (e->bop == BinOp::Eq && c % 2 == 0) {   // `t % 8 == 0`
         const E rem = strip_converts(e->args[0]);
         if (rem->k == Expr::BinOpE && rem->bop == BinOp::Rem && counter(rem->args[0]) && rem->args[1]->k == Expr::Int && rem->args[1]->iv > 0 && rem->args[1]->iv % 2 == 0)
@@ -274,6 +281,18 @@ Stmts Pass::pair_steps(const Stmts& ss) {
       }
       return e;
     });
+    std::function<Stmts(const Stmts&)> tests = [&](const Stmts& b) {
+      Stmts o;
+      for (auto& c : b) {
+        auto n = clone(c);
+        if (c->k == Stmt::If) n->expr = tested(c->expr);
+        n->body = tests(c->body);
+        n->els = tests(c->els);
+        o.push_back(n);
+      }
+      return o;
+    };
+    r->body = tests(r->body);
     r->in_pairs = true;
     out.push_back(r);
   }

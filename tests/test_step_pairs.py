@@ -133,3 +133,42 @@ def test_loops_inside_each_other(U, T):
     for got, want in ((a, x), (b, y)):
         np.testing.assert_allclose(got, want, rtol=2 * U * T * 2.0 ** -24)
     assert np.array_equal(out, a - b)
+
+
+@parpy.jit
+def parity_as_a_number(a, b, N, M, T):
+    parpy.label('inst')
+    for i in range(N):
+        for t in range(1, T):
+            s = b
+            d = a
+            if t & 1:
+                s = a
+                d = b
+            parpy.label('state')
+            for j in range(M):
+                d[i, j] = s[i, (j + 1) % M] + ((t & 1) << 40) - parpy.operators.max(t & 1, j) + (1 if (t & 1) == 0 else 3) + (5 if (t & 1) != 1 and j > 3 else 7) + (~(t & 1)) * (t & 1)
+
+
+def test_the_parity_as_a_number_keeps_its_width():
+    """A shift of a truth value is one of 32 bits."""
+    a = np.zeros((4, 512), np.int64)
+    s = parpy.print_compiled(parity_as_a_number, [a, a.copy(), 4, 512, 7], opts(4, 256))
+    hiprtc_compile(s[:s.index("// host side")], opts(4, 256))
+    assert "(int64_t)(t_" in s and "parpy_odd.value <<" not in s
+    assert s.count("if (parpy_odd.value) {") == 1 and "(!parpy_odd.value)" in s
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [2, 3, 8])
+def test_the_parity_as_a_number(T):
+    n, m = 3, 512
+    rng = np.random.default_rng(T)
+    a, b = rng.integers(-1000, 1000, (n, m)), rng.integers(-1000, 1000, (n, m))
+    x, y = a.copy(), b.copy()
+    parity_as_a_number(a, b, n, m, T, opts=opts(n, 256))
+    j = np.arange(m)
+    for t in range(1, T):
+        p = t & 1
+        (y if p else x)[:] = np.roll(x if p else y, -1, axis=1) + (p << 40) - np.maximum(p, j) + (1 if p == 0 else 3) + np.where((p != 1) & (j > 3), 5, 7) + ~p * p
+    assert np.array_equal(a, x) and np.array_equal(b, y)
