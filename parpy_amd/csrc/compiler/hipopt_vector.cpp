@@ -70,8 +70,15 @@ Stmts Pass::whole_lines(const S& s, int V) {
   E row;
   int64_t line = 0;
   bool ok = true;
-  for (auto& c : s->body)
+  // what the body names on the way (`base = i * M`) is written out: the names mean nothing in front of the loop
+  std::map<Name, E> named;
+  std::set<Name> assigned;
+  for (auto& c : s->body) {
     if (c->k != Stmt::Def && c->k != Stmt::Assign) ok = false;
+    if (c->k == Stmt::Def && c->expr) named[c->id] = subst_vars(c->expr, named);
+    if (c->k == Stmt::Assign && c->dst->k == Expr::Var) assigned.insert(c->dst->name);
+  }
+  for (auto& n : assigned) named.erase(n);
   visit_stmts(s->body, [&](const S& c) {
     for (const E& e : {c->expr, c->dst})
       visit_exprs(e, [&](const E& x) {
@@ -81,7 +88,11 @@ Stmts Pass::whole_lines(const S& s, int V) {
         line = 128 / elem_bytes(x->ty.sz);
       });
   });
-  if (!ok || !row || has_load(row) || N < line + V) return {};
+  if (!ok || !row || N < line + V) return {};
+  row = fold_expr(subst_vars(row, named));
+  if (has_load(row) || mentions(row, s->id)) return {};
+  for (auto& n : assigned)
+    if (mentions(row, n)) return {};
   visit_exprs(row, [&](const E& x) { if (x->k != Expr::Var && x->k != Expr::Int && x->k != Expr::BinOpE && x->k != Expr::Convert) ok = false; });
   if (!ok) return {};
   Type ity = Type::scalar(isz), bty = Type::scalar(ElemSize::Bool);

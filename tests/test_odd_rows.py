@@ -59,3 +59,93 @@ def test_rows_do_not_see_their_neighbours(n, threads, dtype, tol):
         W.sum_rows(x, sums, n, opts=opts(n, threads))
         assert torch.allclose(sums[::2].double(), mine.sum(1), rtol=tol, atol=tol * 30), m
         assert torch.isinf(sums[1::2]).all(), m
+
+
+@parpy.jit
+def flat(x, out, rows, N, M):
+    parpy.label('N')
+    for i in range(N):
+        parpy.label('M')
+        for j in range(M):
+            base = i * M
+            at = base + 1
+            out[at + j] = x[at + j] + 1.0
+
+
+@parpy.jit
+def every_other(x, out, rows, N, M):
+    parpy.label('N')
+    for i in range(N):
+        parpy.label('M')
+        for j in range(M):
+            r = i * 2
+            out[r, j] = x[r, j] + 1.0
+
+
+@parpy.jit
+def picked(x, out, rows, N, M):
+    parpy.label('N')
+    for i in range(N):
+        parpy.label('M')
+        for j in range(M):
+            r = rows[i]
+            out[i, j] = x[r, j] + 1.0
+
+
+@parpy.jit
+def zigzag(x, out, rows, N, M):
+    parpy.label('N')
+    for i in range(N):
+        parpy.label('M')
+        for j in range(M):
+            r = (i + j * 3) % N
+            out[i, j] = x[r, j] + 1.0
+
+
+def named_rows(name, x, rows, n, m):
+    """What the functions above write: the rows of the result, and which rows of it they are."""
+    i, j = np.arange(n)[:, None], np.arange(m)[None, :]
+    one = x.dtype.type(1.0)
+    if name == "flat":
+        return x.reshape(-1)[1:1 + n * m].reshape(n, m) + one
+    if name == "every_other":
+        return x[2 * np.arange(n)] + one
+    if name == "picked":
+        return x[rows] + one
+    return x[(i + j * 3) % n, j] + one
+
+
+NAMED = [flat, every_other, picked, zigzag]
+
+
+def named_arrays(fn, n, m, dtype):
+    rng = np.random.default_rng(m)
+    x = rng.random((2 * n, m)).astype(dtype)
+    return x.reshape(-1) if fn is flat else x, rng.permutation(2 * n)[:n].astype(np.int64)
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("threads", [128, 256, 512])
+def test_rows_named_inside_the_loop_compile(threads, dtype):
+    for fn in NAMED:
+        x, rows = named_arrays(fn, 20, 40001, dtype)
+        s = parpy.print_compiled(fn, [x, x.copy(), rows, 20, 40001], opts(20, threads))
+        hiprtc_compile(s[:s.index("// host side")], opts(20, threads))
+        if dtype == np.float32 and threads < 512:   # (the row of a pick is not known, nor is there one row in a zigzag)
+            assert ("_front_" in s[s.index('extern "C" __global__'):]) == (fn in (flat, every_other)), fn
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float16, np.float32], ids=["f16", "f32"])
+def test_rows_named_inside_the_loop(dtype):
+    for fn in NAMED:
+        for n, m, threads in ((7, 40001, 128), (20, 20003, 256), (300, 999, 64)):
+            x, rows = named_arrays(fn, n, m, dtype)
+            out = np.full_like(x, -1.0)
+            fn(x, out, rows, n, m, opts=opts(n, threads))
+            want = np.full_like(x, -1.0)
+            if fn is flat:
+                want[1:1 + n * m] = named_rows("flat", x, rows, n, m).reshape(-1)
+            else:
+                want[2 * np.arange(n) if fn is every_other else np.arange(n)] = named_rows(fn.__name__, x, rows, n, m)
+            assert np.array_equal(out, want), (fn.__name__, n, m)
