@@ -882,7 +882,10 @@ struct DevicePrinter {
       if (head && head->k == Stmt::Def) {
         const Name elem = head->id;
         std::set<Name> inside{s->id};   // what is known inside the loop only
-        visit_stmts(s->body, [&](const S& c) { if (c->k == Stmt::Def || c->k == Stmt::For) inside.insert(c->id); });
+        visit_stmts(s->body, [&](const S& c) {
+          if (c->k == Stmt::Def || c->k == Stmt::For) inside.insert(c->id);
+          if (c->k == Stmt::Assign && c->dst->k == Expr::Var) inside.insert(c->dst->name);
+        });
         auto known = [&](const E& x) {
           bool ok = !hipopt::has_load(x);
           visit_exprs(x, [&](const E& y) { if (y->k == Expr::Var && inside.count(y->name)) ok = false; });

@@ -102,6 +102,17 @@ def zigzag(x, out, rows, N, M):
             out[i, j] = x[r, j] + 1.0
 
 
+@parpy.jit
+def zigzag_assigned(x, out, rows, N, M):
+    parpy.label('N')
+    for i in range(N):
+        r = i
+        parpy.label('M')
+        for j in range(M):
+            r = (i + j * 3) % N
+            out[i, j] = x[r, j] + 1.0
+
+
 def named_rows(name, x, rows, n, m):
     """What the functions above write: the rows of the result, and which rows of it they are."""
     i, j = np.arange(n)[:, None], np.arange(m)[None, :]
@@ -115,7 +126,7 @@ def named_rows(name, x, rows, n, m):
     return x[(i + j * 3) % n, j] + one
 
 
-NAMED = [flat, every_other, picked, zigzag]
+NAMED = [flat, every_other, picked, zigzag, zigzag_assigned]
 
 
 def named_arrays(fn, n, m, dtype):
@@ -149,3 +160,11 @@ def test_rows_named_inside_the_loop(dtype):
             else:
                 want[2 * np.arange(n) if fn is every_other else np.arange(n)] = named_rows(fn.__name__, x, rows, n, m)
             assert np.array_equal(out, want), (fn.__name__, n, m)
+
+
+def test_rows_assigned_inside_the_loop_are_loaded_inside_it():
+    """A row that every iteration picks anew is not known in front of the vector's elements."""
+    x, rows = named_arrays(zigzag_assigned, 20, 1001, np.float32)
+    s = parpy.print_compiled(zigzag_assigned, [x, x.copy(), rows, 20, 1001], opts(20, 64))
+    hiprtc_compile(s[:s.index("// host side")], opts(20, 64))
+    assert "parpy_vector_within<" not in s[s.index('extern "C" __global__'):]
