@@ -358,7 +358,7 @@ struct TimeTile {
                 auto blend = std::make_shared<Expr>();
                 blend->k = Expr::Call;
                 blend->ty = to->ty;
-                blend->sval = "parpy_blend";
+                blend->sval = std::string("parpy_blend<") + elem_ctype(to->ty.sz) + ">";   // (integers may be computed in 32 bits)
                 blend->args = {covered(e, u.lo, u.hi), v, to};
                 v = E(blend);
               }

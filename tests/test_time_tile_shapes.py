@@ -54,3 +54,41 @@ def test_bit_for_bit(n, steps, dtype, per_lane):
             y[1:-1] = (x[:-2] + x[1:-1] + x[2:]) / dtype(3.0)
             x[2:-3] = (y[1:-4] + y[2:-3] + y[3:-2]) / dtype(-7.0)
     assert np.array_equal(A, x, equal_nan=True) and np.array_equal(B, y, equal_nan=True)
+
+
+@parpy.jit
+def counts(A, B, steps):
+    for t in range(steps):
+        parpy.label('N')
+        B[1:-1] = 1
+        parpy.label('N')
+        A[2:-2] = A[2:-2] * 3 + B[1:-3] - B[4:]
+        parpy.label('N')
+        B[3:-1] = A[4:]
+
+
+INTEGERS = [(np.int32, np.int32), (np.int64, np.int64), (np.int32, np.int64), (np.int64, np.int32)]
+
+
+@pytest.mark.parametrize("a,b", INTEGERS)
+def test_integers_compile(a, b):
+    for n, steps in ((600, 3), (9001, 20)):
+        s = parpy.print_compiled(counts, [np.zeros(n, a), np.zeros(n, b), steps], opts(n))
+        assert "parpy_blend<" in s[s.index('extern "C"'):]
+        hiprtc_compile(s[:s.index("// host side")], opts(n))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("a,b", INTEGERS)
+def test_integers(a, b):
+    for n, steps in ((600, 3), (9001, 20)):
+        rng = np.random.default_rng(n)
+        A, B = rng.integers(-9, 9, n).astype(a), rng.integers(-9, 9, n).astype(b)
+        x, y = A.copy(), B.copy()
+        counts(A, B, steps, opts=opts(n))
+        with np.errstate(all="ignore"):
+            for _ in range(steps):
+                y[1:-1] = 1
+                x[2:-2] = x[2:-2] * a(3) + y[1:-3].astype(a) - y[4:].astype(a)
+                y[3:-1] = x[4:]
+        assert np.array_equal(A, x) and np.array_equal(B, y), (n, steps)
