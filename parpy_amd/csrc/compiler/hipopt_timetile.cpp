@@ -55,7 +55,55 @@ struct TimeTile {
 
   E iint(int64_t v) { return mk_int(v, isz); }
   E add(E a, E b) { return mk_binop(BinOp::Add, a, b, ity); }
-  static int64_t pow2_at_least(int64_t n) { int64_t q = 1; while (q < n) q *= 2; return q; }
+
+  // Vector instructions for one element of an update: a product and the sum that it goes into are one, a division by a
+  // constant is five and a half (`DevicePrinter` has which constants), neighbours and own elements are registers.  `waits`
+  // counts what those that depend on each other wait where a SIMD has nothing else to issue.
+  static double instructions(const E& e, double* waits) {
+    if (!e->ty.is_scalar() || e->k == Expr::Index) return 0;
+    const bool f32 = e->ty.sz == ElemSize::F32, integer = is_int(e->ty.sz);
+    const double words = integer && elem_bytes(e->ty.sz) == 8 ? 2 : 1;
+    if (e->k == Expr::Convert) {
+      const E& d = e->args[0];
+      // float32(float64(x) / c) is a division in single precision
+      if (f32 && d->k == Expr::BinOpE && d->bop == BinOp::Div && d->args[1]->k == Expr::Float && d->args[0]->k == Expr::Convert && d->args[0]->args[0]->ty.sz == ElemSize::F32)
+        return instructions(mk_binop(BinOp::Div, d->args[0]->args[0], d->args[1], e->ty), waits);
+      if (d->k == Expr::Int || d->k == Expr::Float || d->k == Expr::Bool) return 0;
+      return instructions(d, waits) + (d->ty.sz == e->ty.sz ? 0 : words);
+    }
+    double n = 0;
+    for (auto& a : e->args) n += instructions(a, waits);
+    auto product = [](const E& x) { return x->k == Expr::BinOpE && x->bop == BinOp::Mul && x->ty.is_scalar() && is_float(x->ty.sz); };
+    if (e->k == Expr::IfExpr) return n + 1 + elem_bytes(e->ty.sz) / 4;
+    if (e->k == Expr::UnOpE) return n + (e->uop == UnOp::Sub || e->uop == UnOp::Abs || e->uop == UnOp::Not || e->uop == UnOp::BitNeg ? words : f32 ? 4 : 40);
+    if (e->k != Expr::BinOpE) return n;
+    switch (e->bop) {
+      case BinOp::Add: case BinOp::Sub: return n + (product(e->args[0]) || product(e->args[1]) ? 0 : words);
+      case BinOp::Mul: return n + (integer ? 4 * words : 1);
+      case BinOp::Div: case BinOp::FloorDiv: case BinOp::Rem:
+        if (integer) return n + 20 * words;
+        *waits += f32 ? 5 : 3;
+        return n + (e->args[1]->k != Expr::Float ? 12 : f32 ? 5 : 5.5);
+      case BinOp::Pow: case BinOp::Atan2: return n + 40;
+      default: return n + words;
+    }
+  }
+
+  // how far an update reads each array to the left and to the right
+  static std::map<Name, std::pair<int64_t, int64_t>> need_of(const Update& u) {
+    std::map<Name, std::pair<int64_t, int64_t>> need;
+    for (auto& st : u.body)
+      visit_exprs(st->expr, [&](const E& x) {
+        if (x->k != Expr::Index) return;
+        E rest;
+        affine_unit(x->args[1], u.id, &rest);
+        const int64_t d = rest->iv - u.c;
+        auto& nd = need[u.host.at(x->args[0]->name)];
+        nd.first = std::max(nd.first, -d);
+        nd.second = std::max(nd.second, d);
+      });
+    return need;
+  }
 
   bool update_of(const Kernel& k, const S& launch, Update& u, std::vector<Arr>& arrays) {
     if (k.opaque_body || k.body.size() != 1 || k.grid.y != 1 || k.grid.z != 1 || k.block.y != 1 || k.block.z != 1) return false;
@@ -163,11 +211,29 @@ struct TimeTile {
     // calls of 149, 14.4 GB 390 and 58.6).
     if (second_set > (int64_t(6) << 30)) return S();
     // Elements per lane, and with them steps per launch (a margin of up to a quarter of the stretch on either side) and
-    // wavefronts: what is expected to be over first.  A wavefront takes an element through an update in 12.2 ns, a SIMD in
-    // 10 ns (6.5 ns for words of four bytes); its share is a whole number of wavefronts; a launch
-    // costs 2.7 us and its bytes at 7 TB/s.  98 updates of a three-point average, two launches, doubles: 10^6 elements
-    // 48.7 / 38.6 / 37.6 / 33.3 / 37.2 / 46.4 us on 4 / 6 / 8 / 10 / 12 / 16 elements per lane (7, 4, 3, 2, 2, 2 wavefronts to a
-    // SIMD), 4 * 10^6 148 / 114 / 103 / 102 / 105 / 103, 10^5 11.5 / 14.3 / 16.3 / 18.8.
+    // wavefronts: what is expected to be over first.  A step is `work` instructions for every element, `taken` words from the
+    // neighbouring lanes and, next to the ends, a blend of `kept` words for every element.  A wavefront issues one in 1.0 ns,
+    // where a word from another lane counts as three and a blended one as four, and waits for the steps of a division; a SIMD
+    // takes 1.05 ns for each of its share, a whole number of wavefronts, and 1.5 for a lane's word.  A launch costs 2.4 us,
+    // 15 ns times the square of the elements (the ends of the arrays are loaded and stored one by one) and its bytes,
+    // margins included, at 8 TB/s.
+    // Fitted to 2040 times: two updates a step that copy, average three neighbours with and without a division, and add 2, 5,
+    // 10, 20 and 33 products and three far ones, floats and doubles, 2000 to 4 * 10^6 elements, 3 to 93 steps, each on 1 to 32
+    // elements per lane.  The choice then takes 1.2 % longer than the best of them on average and 16 % at most; a time
+    // per element that knows nothing of the update took 2.8 % and 39 % longer (98 updates, its choice and this one: copies of
+    // 403 337 doubles 14.0 and 10.1 us, ten products over 403 337 floats 66.8 and 52.2, over 10 007 doubles 42.5 and 35.5;
+    // 186 of 403 337 floats with a division 36.7 and 32.0; the one that loses most, five over 403 337 doubles, 25.8 and 29.9).
+    double work = 0, waits = 0;
+    int64_t taken = 0, kept = 0;
+    for (auto& u : ups) {
+      for (auto& st : u.body) {
+        const double v = instructions(st->expr, &waits);
+        work += st->k == Stmt::Assign ? std::max(1.0, v) : v;
+        if (st->k == Stmt::Assign) kept += elem_bytes(st->dst->ty.sz) / 4;
+      }
+      for (auto& kv : need_of(u))
+        for (auto& a : arrays) if (a.host == kv.first) taken += (kv.second.first + kv.second.second) * (elem_bytes(a.sz) / 4);
+    }
     int64_t Es = 0;
     double best = 0;
     for (int64_t e : {1, 2, 3, 4, 6, 8, 10, 12}) {
@@ -176,8 +242,10 @@ struct TimeTile {
       const int64_t margin = ((steps + 2 * pairs - 1) / (2 * pairs) * per_step + e - 1) / e * e, useful = WAVE_SIZE * e - 2 * margin;
       if (useful < WAVE_SIZE * e / 4) continue;
       const int64_t waves = (n + useful - 1) / useful, share = (waves + 1023) / 1024;
-      const double time = std::max(12.2, (wide ? 10.0 : 6.5) * (double)share) * (double)(updates * e) +
-                          (double)(2 * pairs) * (2700.0 + (double)(n * words * 4 * 2) / 7000.0);
+      const double lane = (work + waits + 4.0 * (double)kept) * (double)e + 3.0 * (double)taken;
+      const double simd = 1.05 * (double)share * (work * (double)e + 1.5 * (double)taken);
+      const double bytes = (double)(n * words * 4) * (1.0 + (double)(WAVE_SIZE * e) / (double)useful);
+      const double time = std::max(lane, simd) * (double)steps + (double)(2 * pairs) * (2400.0 + 15.0 * (double)(e * e) + bytes / 8000.0);
       if (Es == 0 || time < best) Es = e, best = time;
     }
     if (Es == 0) return S();
@@ -304,18 +372,7 @@ struct TimeTile {
       for (auto& u : ups) {
         // what the neighbouring lanes hold
         std::map<std::pair<Name, int64_t>, E> from;
-        std::map<Name, std::pair<int64_t, int64_t>> need;
-        for (auto& st : u.body)
-          visit_exprs(st->expr, [&](const E& x) {
-            if (x->k != Expr::Index) return;
-            E rest;
-            affine_unit(x->args[1], u.id, &rest);
-            int64_t d = rest->iv - u.c;
-            auto& nd = need[u.host[x->args[0]->name]];
-            nd.first = std::max(nd.first, -d);
-            nd.second = std::max(nd.second, d);
-          });
-        for (auto& kv : need) {
+        for (auto& kv : need_of(u)) {
           const Arr& a = arr_of(kv.first);
           auto fetch = [&](int64_t pos, int64_t own, const char* fn) {
             Name nm = gen.fresh(a.host.s + (pos < 0 ? "_left" : "_right"));

@@ -92,3 +92,53 @@ def test_integers(a, b):
                 x[2:-2] = x[2:-2] * a(3) + y[1:-3].astype(a) - y[4:].astype(a)
                 y[3:-1] = x[4:]
         assert np.array_equal(A, x) and np.array_equal(B, y), (n, steps)
+
+
+@parpy.jit
+def shifts(A, B, steps):
+    for t in range(steps):
+        parpy.label('N')
+        B[1:-1] = A[2:]
+        parpy.label('N')
+        A[1:-1] = B[:-2]
+
+
+@parpy.jit
+def ten_terms(A, B, steps):
+    for t in range(steps):
+        parpy.label('N')
+        B[5:-5] = (A[:-10] + A[1:-9] - A[2:-8] + A[3:-7] - A[4:-6] + A[6:-4] - A[7:-3] + A[8:-2] - A[9:-1] + A[10:]) * 0.25
+        parpy.label('N')
+        A[5:-5] = (B[:-10] - B[1:-9] + B[2:-8] - B[3:-7] + B[4:-6] - B[6:-4] + B[7:-3] - B[8:-2] + B[9:-1] - B[10:]) * 0.5
+
+
+# updates that cost less and more than an average of three: length, steps, element type -> elements per lane of each
+WORK = [(403337, 49, np.float64, 4, 6), (1000003, 49, np.float64, 4, 12), (10007, 49, np.float64, 4, 6), (3000001, 10, np.float32, 4, 10)]
+
+
+@pytest.mark.parametrize("n,steps,dtype,copies,terms", WORK)
+def test_elements_per_lane_by_the_work_of_an_update(n, steps, dtype, copies, terms):
+    got = {}
+    for fn in (shifts, ten_terms):
+        a = np.zeros(n, dtype)
+        s = parpy.print_compiled(fn, [a, a.copy(), steps], opts(n))
+        got[fn] = int(re.search(r"A_r_\d+\[(\d+)\];", s)[1])
+    assert got == {shifts: copies, ten_terms: terms}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,steps,dtype", [w[:3] for w in WORK])
+def test_copies_and_ten_terms(n, steps, dtype):
+    rng = np.random.default_rng(n)
+    for fn in (shifts, ten_terms):
+        A, B = rng.standard_normal(n).astype(dtype), rng.standard_normal(n).astype(dtype)
+        x, y = A.copy(), B.copy()
+        fn(A, B, steps, opts=opts(n))
+        for _ in range(steps):
+            if fn is shifts:
+                y[1:-1] = x[2:]
+                x[1:-1] = y[:-2]
+            else:   # sums in the type of the arrays, from the left
+                y[5:-5] = (((((((((x[:-10] + x[1:-9]) - x[2:-8]) + x[3:-7]) - x[4:-6]) + x[6:-4]) - x[7:-3]) + x[8:-2]) - x[9:-1]) + x[10:]) * dtype(0.25)
+                x[5:-5] = (((((((((y[:-10] - y[1:-9]) + y[2:-8]) - y[3:-7]) + y[4:-6]) - y[6:-4]) + y[7:-3]) - y[8:-2]) + y[9:-1]) - y[10:]) * dtype(0.5)
+        assert np.array_equal(A, x) and np.array_equal(B, y), fn
