@@ -236,17 +236,41 @@ struct TimeTile {
     }
     int64_t Es = 0;
     double best = 0;
-    for (int64_t e : {1, 2, 3, 4, 6, 8, 10, 12}) {
-      if (e * words > 64 || e < reach || per_step > 8 * e) continue;
+    auto consider = [&](int64_t e) {
+      if (e * words > 64 || e < reach || per_step > 8 * e) return;
       const int64_t most = per_step > 0 ? 16 * e / per_step : steps, pairs = (steps + 2 * most - 1) / (2 * most);
       const int64_t margin = ((steps + 2 * pairs - 1) / (2 * pairs) * per_step + e - 1) / e * e, useful = WAVE_SIZE * e - 2 * margin;
-      if (useful < WAVE_SIZE * e / 4) continue;
+      if (useful < WAVE_SIZE * e / 4) return;
       const int64_t waves = (n + useful - 1) / useful, share = (waves + 1023) / 1024;
       const double lane = (work + waits + 4.0 * (double)kept) * (double)e + 3.0 * (double)taken;
       const double simd = 1.05 * (double)share * (work * (double)e + 1.5 * (double)taken);
       const double bytes = (double)(n * words * 4) * (1.0 + (double)(WAVE_SIZE * e) / (double)useful);
       const double time = std::max(lane, simd) * (double)steps + (double)(2 * pairs) * (2400.0 + 15.0 * (double)(e * e) + bytes / 8000.0);
       if (Es == 0 || time < best) Es = e, best = time;
+    };
+    for (int64_t e : {1, 2, 3, 4, 6, 8, 10, 12}) consider(e);
+    // Updates that reach further than 12 elements take up to 32, where that beats a launch per update by a tenth: those take
+    // 3 us each behind the first, or their arrays at 3.6 TB/s or loads at 15.  Steps of two updates, tiled and as launches,
+    // three products 13 elements apart, doubles: three steps over 30 000 elements 13.5 and 15.3 us, over 4 * 10^6 52 and 94,
+    // ten over 30 000 16.6 and 57, fifty over 10^6 98 and 447; 32 apart, floats: three over 30 000 29.7 and 16.4 (stays
+    // launches), ten over 30 000 35 and 57, over 4 * 10^6 62 and 161; 33 neighbouring ones, ten over 10^6 doubles 61 and 349.
+    if (Es == 0) {
+      for (int64_t e : {14, 16, 20, 24, 28, 32}) consider(e);
+      double launches = -3000.0;
+      for (auto& u : ups) {
+        double loaded = 0, moved = 0;
+        std::set<Name> seen;
+        auto count = [&](const E& e) {
+          visit_exprs(e, [&](const E& x) {
+            if (x->k != Expr::Index) return;
+            loaded += elem_bytes(x->ty.sz);
+            if (seen.insert(x->args[0]->name).second) moved += elem_bytes(x->ty.sz);
+          });
+        };
+        for (auto& st : u.body) { count(st->expr); count(st->dst); }
+        launches += std::max({3000.0, (double)n * moved / 3600.0, (double)n * loaded / 15000.0}) * (double)steps;
+      }
+      if (1.1 * best > launches) return S();
     }
     if (Es == 0) return S();
     const int64_t most = per_step > 0 ? 16 * Es / per_step : steps;

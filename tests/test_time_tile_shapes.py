@@ -142,3 +142,43 @@ def test_copies_and_ten_terms(n, steps, dtype):
                 y[5:-5] = (((((((((x[:-10] + x[1:-9]) - x[2:-8]) + x[3:-7]) - x[4:-6]) + x[6:-4]) - x[7:-3]) + x[8:-2]) - x[9:-1]) + x[10:]) * dtype(0.25)
                 x[5:-5] = (((((((((y[:-10] - y[1:-9]) + y[2:-8]) - y[3:-7]) + y[4:-6]) - y[6:-4]) + y[7:-3]) - y[8:-2]) + y[9:-1]) - y[10:]) * dtype(0.5)
         assert np.array_equal(A, x) and np.array_equal(B, y), fn
+
+
+@parpy.jit
+def far(A, B, R, N, steps):
+    for t in range(steps):
+        parpy.label('N')
+        for i in range(R, N - R):
+            B[i] = (A[i - R] - A[i] + A[i + R]) * 0.5
+        parpy.label('N')
+        for i in range(R, N - R):
+            A[i] = (B[i - R] + B[i] - B[i + R]) * 0.5
+
+
+# reach, length, steps, element type -> elements per lane (None: a launch per update)
+FAR = [(13, 3001, 3, np.float64, 14), (16, 3001, 10, np.float64, 16), (13, 30001, 40, np.float32, 14), (16, 30001, 40, np.float32, 20),
+       (24, 30001, 40, np.float32, 24), (28, 3001, 10, np.float32, 28), (32, 30001, 40, np.float32, 32), (32, 1000003, 20, np.float32, 32),
+       (16, 3001, 3, np.float32, None), (32, 3001, 3, np.float32, None), (17, 3001, 10, np.float64, None), (33, 3001, 10, np.float32, None)]
+
+
+@pytest.mark.parametrize("reach,n,steps,dtype,per_lane", FAR)
+def test_updates_of_wide_reach(reach, n, steps, dtype, per_lane):
+    a = np.zeros(n, dtype)
+    s = parpy.print_compiled(far, [a, a.copy(), reach, n, steps], opts(n))
+    m = re.search(r"A_r_\d+\[(\d+)\];", s)
+    assert (int(m[1]) if m else None) == per_lane
+    hiprtc_compile(s[:s.index("// host side")], opts(n))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("reach,n,steps,dtype", [f[:4] for f in FAR if f[4]])
+def test_updates_of_wide_reach_bit_for_bit(reach, n, steps, dtype):
+    rng = np.random.default_rng(n + reach)
+    A, B = rng.standard_normal(n).astype(dtype), rng.standard_normal(n).astype(dtype)
+    x, y = A.copy(), B.copy()
+    far(A, B, reach, n, steps, opts=opts(n))
+    r = reach
+    for _ in range(steps):
+        y[r:-r] = (x[:-2 * r] - x[r:-r] + x[2 * r:]) * dtype(0.5)
+        x[r:-r] = (y[:-2 * r] + y[r:-r] - y[2 * r:]) * dtype(0.5)
+    assert np.array_equal(A, x) and np.array_equal(B, y)
