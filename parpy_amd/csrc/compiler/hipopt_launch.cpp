@@ -785,15 +785,23 @@ struct RowThreads {
     launch->block = k.block;
   }
 
-  // Rows on a wavefront or two whose threads never meet (the row numbers of a compressed matrix, written to its elements): how
-  // long they are may stand in memory, so they share workgroups where those are still as many as the device has compute
-  // units.  SDDMM with a compressed mask, whose row numbers are filled in first: 8192 rows of 82, 128 deep, 34.8 -> 32.1 us;
-  // 2491 rows of 5, 174 deep, doubles 13.8 -> 13.0.
+  // Rows on a wavefront or two whose threads never meet share workgroups where those are still as many as the device has
+  // compute units: short rows wait for the starts.  The row numbers of a compressed matrix, written to its elements (how long
+  // a row is stands in memory), 64 threads: 20 000 rows of 3 / 30 / 100 10.6 / 10.3 / 10.6 -> 3.5 / 3.8 / 5.0 us, 100 000 of 30
+  // 22.6 -> 11.8, 2048 the same; of 600 each up to 13 % slower, 600 on average 5 % faster.  Within SDDMM, 8192 rows of 82, 128
+  // deep, 34.8 -> 32.1 us; 2491 rows of 5, 174 deep, doubles 13.8 -> 13.0.  Element-wise rows of floats, halves and doubles,
+  // 20 000 of 20 / 64 / 100 10.2 / 9.8 / 10.5 -> 3.8 / 3.7 / 4.5; 8192 of 256 4.9 -> 3.4; 100 000 of 256 and 20 000 of 500 are
+  // bound by memory: 0.95 to 1.08 of the time.  Not with a loop inside the thread's element, where the row's own values
+  // are scalar loads as long as a workgroup has one row: products of half-precision sparse matrices 1.2 times as slow in the
+  // median (5000 rows of 60 times 128 columns 29.7 -> 54.2 us), dense products by rows 1.2 (5000 x 256 x 64 38.7 -> 56.7).
   bool share_starts(Kernel& k, const S& root, const StmtP& launch, int64_t rows, int64_t threads) {
     bool apart = threads <= 128 && rows >= 2048 && rows < (int64_t(1) << 30);
     visit_stmts(root->body, [&](const S& s) {
-      const bool plain = s->k == Stmt::Def || s->k == Stmt::Assign || s->k == Stmt::If ||
-                         (s->k == Stmt::For && (s->map.k == GpuMap::None || (s->map.k == GpuMap::Thread && s->map.dim == 0 && s->map.n == threads && !s->par.reduction)));
+      bool plain = s->k == Stmt::Def || s->k == Stmt::Assign || s->k == Stmt::If;
+      if (s->k == Stmt::For && s->map.k == GpuMap::Thread && s->map.dim == 0 && s->map.n == threads && !s->par.reduction) {
+        const int64_t extent = const_extent(s);
+        plain = extent <= 128 || rows * extent <= 6000000;   // (-1 where it is not constant)
+      }
       apart = apart && plain;
     });
     if (!apart) return false;

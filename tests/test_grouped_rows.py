@@ -122,3 +122,43 @@ def test_every_row_once(n, m, dtype):
     got = np.zeros(n, dtype)
     chosen(x, pick, got, n, opts=opts(n, 256))
     assert np.array_equal(got == -1.0, pick == 0) and np.allclose(got[pick > 0], x[pick > 0].astype(np.float64).sum(1), atol=0.25 * m * np.sqrt(m) * np.finfo(dtype).eps)
+
+
+@parpy.jit
+def scaled_rows(x, y, N, M):
+    parpy.label('i')
+    for i in range(N):
+        parpy.label('j')
+        for j in range(M):
+            y[i, j] = x[i, j] * 2.0
+
+
+@parpy.jit
+def row_products(x, w, y, N, M, K):
+    parpy.label('i')
+    for i in range(N):
+        parpy.label('j')
+        for j in range(M):
+            t = 0.0
+            for q in range(K):
+                t = t + x[i, q] * w[q, j]
+            y[i, j] = t
+
+
+def test_which_rows_that_never_meet_share():
+    for n, m, rows in ((20000, 100, 8), (20000, 128, 8), (8192, 500, 8), (100000, 256, 1), (20000, 500, 1), (2000, 100, 1)):
+        x = np.zeros((n, m), np.float32)
+        assert block(scaled_rows, [x, x.copy(), n, m], n, 64)[0] == (64, rows), (n, m)
+    x, w, y = np.zeros((5000, 256), np.float32), np.zeros((256, 64), np.float32), np.zeros((5000, 64), np.float32)
+    s = block(row_products, [x, w, y, 5000, 64, 256], 5000, 64)[1]
+    assert "<<<dim3(1, 5000, 1), dim3(64, 1, 1)" in s     # (the row's own values are scalar loads)
+
+
+@pytest.mark.gpu
+def test_element_wise_rows_once():
+    for n, m in ((20001, 100), (8193, 500), (2049, 65), (20001, 500)):
+        x = np.random.default_rng(m).random((n, m)).astype(np.float32)
+        for threads in (64, 128):
+            y = np.zeros_like(x)
+            scaled_rows(x, y, n, m, opts=opts(n, threads))
+            assert np.array_equal(y, x * np.float32(2.0)), (n, m, threads)
