@@ -796,7 +796,8 @@ struct DevicePrinter {
   int in_unrolled = 0;            // unrolled loops over the elements of a vector around the statement being printed
   std::map<const Expr*, std::string> tail_loads;   // elements of vectors loaded in front of the loop over them
   int next_tail = 0;
-  std::string not_last_trip;      // holds in all trips of the counted loop being printed but the last
+  std::string not_last_trip;      // holds in all trips but the last of the innermost counted loop around what is printed,
+  Name not_last_of;               // which has this variable
   int in_unaligned = 0;           // those whose vectors start at any element
   std::set<Name> seq_loop_vars;   // variables of the enclosing sequential loops that are kept as loops
 
@@ -878,6 +879,8 @@ struct DevicePrinter {
       // What the vector is made of is loaded in front of the test, by one access that ends with the loop where the vector
       // would reach past it: in the two branches, one would wait for its loads before the other issues its own.
       std::vector<const Expr*> joined;
+      // (of the loop over the row's vectors alone: a loop over several rows around it says nothing about them)
+      const std::string whole = hipopt::mentions(s->args[0], not_last_of) ? not_last_trip : "";
       const S head = s->body.empty() ? S() : s->body[0];
       if (head && head->k == Stmt::Def) {
         const Name elem = head->id;
@@ -904,7 +907,7 @@ struct DevicePrinter {
               loaded.push_back({e, var});
               const std::string T = elem_ctype(e->ty.sz), V = std::to_string(hipopt::const_extent(s)), TV = "<" + T + ", " + V + ">";
               std::map<Name, E> zero{{s->id, mk_int(0, s->lo->ty.sz)}};
-              const std::string where = pexpr(fold_expr(hipopt::subst_vars(head->expr, zero))) + ", " + pexpr(s->args[2]) + ", " + (not_last_trip.empty() ? "false" : not_last_trip);
+              const std::string where = pexpr(fold_expr(hipopt::subst_vars(head->expr, zero))) + ", " + pexpr(s->args[2]) + ", " + (whole.empty() ? "false" : whole);
               os << ind(n) << "const " << T << "* " << var << "_at = parpy_vector_within" << TV << "(" << pexpr(e->args[0]) << " + " << paren(pexpr(rest)) << ", " << where << ");\n";
               os << ind(n) << "const parpy_vec" << TV << " " << var << " = parpy_moved_down" << TV << "(parpy_vec" << TV << "{";
               for (int64_t q = 0; q < hipopt::const_extent(s); ++q)
@@ -920,7 +923,7 @@ struct DevicePrinter {
         for (size_t q = 1; q < s->body.size(); ++q)
           if (s->body[q]->k == Stmt::Def || s->body[q]->k == Stmt::Assign) find(s->body[q]->expr);
       }
-      os << ind(n) << "if (" << (not_last_trip.empty() ? "" : not_last_trip + " || ") << pexpr(s->args[0]) << ") {\n";
+      os << ind(n) << "if (" << (whole.empty() ? "" : whole + " || ") << pexpr(s->args[0]) << ") {\n";
       auto plain = std::make_shared<Stmt>(*s);
       plain->args.clear();
       kept_alive.push_back(plain);
@@ -1059,6 +1062,8 @@ struct DevicePrinter {
       }
       // (the device compiler does not see by itself that all other trips are in range)
       const std::string outer_not_last = not_last_trip;
+      const Name outer_not_last_of = not_last_of;
+      not_last_of = s->id;
       not_last_trip = peeled ? "true" : per > 1 ? k + " < " + std::to_string(per - 1) : "";
       os << ind(n) << "for (int " << k << " = 0; " << k << " < " << (peeled ? per - 1 : per) << "; ++" << k << ") {\n";
       os << ind(n + 2) << vty << " " << v << " = " << init("(" + (shared_first ? v + "_g" : idx) + " + " + k + " * " + std::to_string(N) + ")") << ";\n";
@@ -1081,6 +1086,7 @@ struct DevicePrinter {
       }
       os << ind(n) << "}\n";
       not_last_trip = outer_not_last;
+      not_last_of = outer_not_last_of;
       if (peeled) {
         os << ind(n) << "{\n";
         os << ind(n + 2) << "const int " << k << " = " << per - 1 << ";\n";

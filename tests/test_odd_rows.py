@@ -1,5 +1,7 @@
 """Rows that are no whole number of vectors: the last vector of a counted loop ends with the row, a long loop's vectors begin
 where a line of memory does, and neither sees the elements of the next row."""
+import re
+
 import numpy as np
 import pytest
 
@@ -168,3 +170,35 @@ def test_rows_assigned_inside_the_loop_are_loaded_inside_it():
     s = parpy.print_compiled(zigzag_assigned, [x, x.copy(), rows, 20, 1001], opts(20, 64))
     hiprtc_compile(s[:s.index("// host side")], opts(20, 64))
     assert "parpy_vector_within<" not in s[s.index('extern "C" __global__'):]
+
+
+# lengths and threads whose vectors are one to a thread, two, and many (the last trip apart), rows taken by fewer workgroups
+FEWER = [(777, 128, 10), (777, 64, 10), (2051, 128, 7), (8195, 128, 30)]
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32, np.float64])
+def test_a_loop_over_rows_says_nothing_about_their_vectors(dtype):
+    for m, threads, groups in FEWER:
+        x = np.zeros((100, m), dtype)
+        o = parpy.par({'N': parpy.threads(groups), 'M': parpy.threads(threads)})
+        s = parpy.print_compiled(W.softmax, [x, 100, m, x.copy()], o)
+        s = s[s.index('extern "C" __global__'):]
+        row = re.search(r"int (i_\d+) = \(\(int\)blockIdx", s)[1]
+        assert row + "_k" in s and not re.search(r"\(" + row + r"_k < \d+ \|\|", s) and not re.search(row + r"_k < \d+\)?;\n.*parpy_moved", s)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 4e-3), (torch.float32, 1e-5), (torch.float64, 1e-12)], ids=["f16", "f32", "f64"])
+def test_rows_taken_by_fewer_workgroups(dtype, tol):
+    """As above: every other row holds infinities, and a workgroup takes several rows."""
+    n = 100
+    for m, threads, groups in FEWER:
+        g = torch.Generator(device="cuda").manual_seed(m)
+        x = torch.randn((n, m), generator=g, device="cuda", dtype=torch.float32).to(dtype)
+        x[1::2] = float("inf")
+        out = torch.full_like(x, -1.0)
+        W.softmax(x, n, m, out, opts=parpy.par({'N': parpy.threads(groups), 'M': parpy.threads(threads)}))
+        mine = x[::2].double()
+        e = torch.exp(mine - mine.max(1, keepdim=True).values)
+        want = e / e.sum(1, keepdim=True)
+        assert ((out[::2].double() - want).norm() / want.norm()) < tol, (m, threads, groups)
