@@ -8,9 +8,11 @@ input that is already resident in HBM.  The default run (`all`) first measures
 the machine rates that the bound models use (LDS, vector ALU, the latency of a
 dependent step: hand-written microkernels, about two seconds), then times the
 headline workload -- the 7-mer HMM forward batch (4^7 = 16384 states, 100 reads
-of 5000..15000 samples) -- and then the other configurations, whose records go
-under `secondary` of the same JSON line and, as scalars, into `config`
-(`forms_ms`, `secondary_ms`, `secondary_frac`, `measured_rates`).  Every record
+of 5000..15000 samples) -- and then the other configurations, whose figures go
+as scalars into `config` of the one JSON line on stdout (`forms_ms`,
+`secondary_ms`, `secondary_frac`, `measured_rates`).  Their whole records and
+those of the headline's other forms are lines of stderr: with them in it, the
+line on stdout had 24 kB, more than a reader of a log's last few holds.  Every record
 carries the roofline of its dominant kernel (algorithmic bytes or flops /
 measured kernel time against the published peak) and a CPU baseline timed on
 the host cores (bounded sample).
@@ -887,6 +889,14 @@ def _apply_opt_flags(opts, args):
         opts.reg_budget = args.reg_budget
 
 
+def report(r):
+    """One line on stdout; the records of other forms and workloads go to stderr, a line each."""
+    for name in ("other_forms", "secondary"):
+        for record in r.get(name, []):
+            print(json.dumps({name: record}), file=sys.stderr)
+    print(json.dumps({k: v for k, v in r.items() if k not in ("other_forms", "secondary")}))
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -966,7 +976,7 @@ def main():
         r = runners[args.workload]()
         r.update(common)
         r.setdefault("data", "synthetic")
-    print(json.dumps(r))
+    report(r)
 
 
 if __name__ == "__main__":
