@@ -31,8 +31,9 @@ namespace {
 //
 // A three-point average back and forth over 10^6 float64 elements, 98 updates, two launches of 25 steps: 447 us as launches
 // of 4.5 us each, 45.6 on eight elements per lane with their own accesses and a division of four instructions one of which
-// takes as long as four, 39.1 as it is (33 on arrays in the memory-side cache): 1852 wavefronts, two to a SIMD.  The vector ALU bounds it: 7.2 instructions per
-// element and update, an eighth of them in the margins.
+// takes as long as four, 39.1 as it is (33 on arrays in the memory-side cache): 1852 wavefronts, 1.8 to a SIMD.  The vector
+// ALU and its latency bound it: 6.7 instructions per update and element of a stretch (counted), of whose 640 elements 100 are
+// margins.
 struct TimeTile {
   Program& p;
   const Options& opts;

@@ -321,7 +321,10 @@ template <class T> __device__ __forceinline__ T parpy_blend(int m, T a, T b) {
 // 25 steps each way and back: 41.8 -> 37.6 us).  Only lanes of one wavefront meet in its part of LDS: no barrier.
 template <class T, int E> struct parpy_stretch {
   static constexpr int V = sizeof(T) == 4 && E % 4 == 0 ? 4 : E % 2 == 0 ? 2 : 1;   // neighbours that a lane moves at once
-  static constexpr int W = E + 16 / (int)sizeof(T);                               // (a lane's place in LDS: the odd 16 bytes keep the banks apart)
+  // a lane's place in LDS: another 16 bytes, an odd number of 16 bytes in all where E is a multiple of 8 floats or 4 doubles, which
+  // keeps the banks apart; other lanes' places start in fewer of them (10 doubles in eight, which are half of the banks; 6 doubles
+  // and 12 floats in four)
+  static constexpr int W = E + 16 / (int)sizeof(T);
   static __device__ __forceinline__ void meet() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
