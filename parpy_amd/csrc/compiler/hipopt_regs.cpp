@@ -780,10 +780,18 @@ void Pass::reg_cache(int64_t* budget) {
     cands.push_back(c);
   }
   if (cands.size() < 2) return;
-  // loops must agree on extent, mapping and element width
+  // loops must agree on extent, mapping and element width, and those over vectors on the element that a slot is and on
+  // where the last vector ends (998 and 999 elements are 125 vectors of eight)
   auto same = [&](const Cand& a, const Cand& b) {
-    return const_extent(a.loop) == const_extent(b.loop) && a.loop->map.n == b.loop->map.n && a.is.slots == b.is.slots &&
-           a.loop->lo->iv == b.loop->lo->iv && (a.is.inner != nullptr) == (b.is.inner != nullptr);
+    if (const_extent(a.loop) != const_extent(b.loop) || a.loop->map.n != b.loop->map.n || a.is.slots != b.is.slots ||
+        a.loop->lo->iv != b.loop->lo->iv || (a.is.inner != nullptr) != (b.is.inner != nullptr))
+      return false;
+    if (!a.is.inner) return true;
+    const Type ity = Type::scalar(isz);
+    std::map<Name, E> names{{b.loop->id, mk_var(a.loop->id, ity)}, {b.is.inner->id, mk_var(a.is.inner->id, ity)}};
+    auto elem = [](const Cand& c) { return c.is.body->front()->expr; };
+    if (!elem(a) || !elem(b) || !expr_eq(elem(a), subst_vars(elem(b), names)) || a.is.inner->args.size() != b.is.inner->args.size()) return false;
+    return a.is.inner->args.size() < 3 || expr_eq(a.is.inner->args[2], b.is.inner->args[2]);
   };
   std::vector<Cand> group;
   for (auto& c : cands)
