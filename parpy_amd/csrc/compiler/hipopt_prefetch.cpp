@@ -258,6 +258,13 @@ Stmts Pass::prefetch_selected_rows(const Stmts& ss, int64_t* budget) {
           auto fi = clone(is.inner);
           fi->id = nu;
           fi->body = fills;
+          if (!fi->args.empty()) {   // the last vector is not whole: its tests, and the element that they name
+            const S& elem = is.body->front();
+            const Name ne = gen.fresh(elem->id.s);
+            fi->body.insert(fi->body.begin(), mk_def(ne, elem->ty, subst_vars(elem->expr, rv), elem->i));
+            rv[elem->id] = mk_var(ne, elem->ty);
+            for (auto& t : fi->args) t = subst_vars(t, rv);
+          }
           outer->body = {S(fi)};
         } else {
           outer->body = fills;

@@ -348,6 +348,7 @@ Stmts Pass::hoist_from_seq_loop(const S& seq, int64_t* budget) {
           auto fi = clone(is.inner);
           fi->id = nu;
           fi->body = fills;
+          fi->args.clear();   // (a last vector that is not whole: what is past the end is inside the array, as tested above)
           fill_outer->body = {S(fi)};
         } else {
           fill_outer->body = fills;

@@ -202,3 +202,51 @@ def test_rows_taken_by_fewer_workgroups(dtype, tol):
         e = torch.exp(mine - mine.max(1, keepdim=True).values)
         want = e / e.sum(1, keepdim=True)
         assert ((out[::2].double() - want).norm() / want.norm()) < tol, (m, threads, groups)
+
+
+@parpy.jit
+def steps_of_rows(table, obs, a, b, N, M, T):
+    parpy.label('N')
+    for i in range(N):
+        for t in range(T):
+            o = obs[i, t]
+            parpy.label('M')
+            for j in range(M):
+                a[i, j] = table[o, j] - a[i, j] + b[j]
+
+
+# lengths and threads: one vector to a thread, two, and the last trip apart
+STEPS = [(1001, 128), (999, 64), (4099, 256), (515, 64), (2050, 64)]
+
+
+def steps_arrays(m, dtype, n=6, steps=5):
+    rng = np.random.default_rng(m)
+    table, a, b = (rng.integers(-20, 20, shape).astype(dtype) for shape in ((7, m), (n, m), (m + 9,)))
+    obs = rng.integers(0, 7, (n, steps))
+    obs[:, -1] = 6   # (the last row: what is past its end is not the table's)
+    return table, obs, a, b
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32, np.int32])
+def test_rows_fetched_in_front_of_a_time_loop_compile(dtype):
+    for m, threads in STEPS:
+        table, obs, a, b = steps_arrays(m, dtype)
+        s = parpy.print_compiled(steps_of_rows, [table, obs, a, b, 6, m, 5], opts(6, threads))
+        hiprtc_compile(s[:s.index("// host side")], opts(6, threads))
+        s = s[s.index('extern "C" __global__'):]
+        assert "row_table_" in s and "inv_b_" in s
+        # every vector of the table that may not be whole is tested, in front of the loop and behind each step
+        assert len(re.findall(rf"if \(j_\d+ < {m}\) {{\n\s*row_table_", s)) == 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float16, np.float32, np.int32], ids=["f16", "f32", "i32"])
+def test_rows_fetched_in_front_of_a_time_loop(dtype):
+    """Small whole numbers: exact in every type."""
+    for m, threads in STEPS:
+        table, obs, a, b = steps_arrays(m, dtype)
+        want = a.copy()
+        for t in range(obs.shape[1]):
+            want = table[obs[:, t]] - want + b[:m]
+        steps_of_rows(table, obs, a, b, 6, m, 5, opts=opts(6, threads))
+        assert np.array_equal(a, want), (m, threads)
