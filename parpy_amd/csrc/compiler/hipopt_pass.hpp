@@ -109,6 +109,7 @@ struct Pass {
   // hipopt_vector.cpp: several consecutive elements per thread; MFMA dot products
   int vector_width(const S& loop);
   static int64_t strided_run(const E& idx, const Name& d);
+  bool part_of_a_vector_pays(const S& loop);
   Stmts whole_lines(const S& loop, int V);
   Stmts vectorize(const Stmts& ss);
   Stmts widen_half_sums(const Stmts& ss);

@@ -57,6 +57,61 @@ int64_t Pass::strided_run(const E& idx, const Name& d) {
   return 0;
 }
 
+// Whether a loop over elements of four bytes and more takes vectors that do not divide it.  In rows that stand in LDS it does
+// where neighbouring elements are read by neighbouring iterations: 300 rows of 1001 / 4099 floats, 128 / 256 threads, 100 steps
+// of `d[j] = f(s[j], s[(j + 1) % M])` 66 -> 36 / 102 -> 80 us, of `s[j / 2]` 54 -> 34 / 98 -> 64, and 300 steps with a row of a
+// table 151 -> 87 / 258 -> 140; of `s[4 j % M]` 76 -> 96 / 127 -> 371, whose lanes then meet in the banks (`s[M - 1 - j]` and
+// `s[p[j]]` gain on short rows and lose on long ones).  In rows that stand in memory it does where another loop walks the same
+// elements, which then stay in registers (20 000 000 floats: x / sum(x), rows of 1001 on 64 threads 36 -> 30, of 4099 on 256
+// 31 -> 28; two element-wise loops over two arrays 55 -> 46 and 46 -> 41); one loop alone is bound by memory and loses by
+// accesses that share lines (x + 1, rows of 4099 30 -> 38, a sum of three neighbours 30 -> 51, x[M - 1 - j] 30 -> 67).
+bool Pass::part_of_a_vector_pays(const S& loop) {
+  // neighbours of the loop's elements, wherever the row starts or wraps around
+  std::function<bool(const E&)> follows = [&](const E& x) {
+    if (x->k == Expr::Convert) return follows(x->args[0]);
+    if (x->k == Expr::Var) return x->name == loop->id;
+    if (x->k != Expr::BinOpE) return false;
+    const bool left = mentions(x->args[0], loop->id), right = mentions(x->args[1], loop->id);
+    if (left && right) return false;
+    if (x->bop == BinOp::Add) return follows(x->args[left ? 0 : 1]);
+    return left && (x->bop == BinOp::Sub || x->bop == BinOp::FloorDiv || x->bop == BinOp::Rem) && follows(x->args[0]);
+  };
+  std::map<Name, E> named;
+  std::vector<std::pair<Name, E>> rows;   // arrays in memory, and where the row starts
+  bool in_lds = false, ok = true;
+  visit_stmts(loop->body, [&](const S& c) {
+    for (const E& e : {c->expr, c->dst})
+      visit_exprs(e, [&](const E& x) {
+        if (x->k != Expr::Index) return;
+        const E at = subst_vars(x->args[1], named);
+        E rest;
+        if (x->args[0]->ty.mem == Mem::LDS) {
+          in_lds = true;
+          ok = ok && (!mentions(at, loop->id) || follows(at));
+        } else if (affine_unit(at, loop->id, &rest)) {
+          if (x->args[0]->k == Expr::Var) rows.push_back({x->args[0]->name, rest});
+        } else {
+          ok = ok && !mentions(at, loop->id);
+        }
+      });
+    if (c->k == Stmt::Def && c->expr) named[c->id] = subst_vars(c->expr, named);
+  });
+  if (!ok || in_lds) return ok;
+  bool shared = false;
+  visit_stmts(k.body, [&](const S& o) {
+    if (o == loop || !thread_mapped(o) || o->map.n != loop->map.n || !expr_eq(o->lo, loop->lo) || !expr_eq(o->hi, loop->hi)) return;
+    visit_stmts(o->body, [&](const S& c) {
+      for (const E& e : {c->expr, c->dst})
+        visit_exprs(e, [&](const E& x) {
+          E rest;
+          if (x->k != Expr::Index || x->args[0]->k != Expr::Var || !affine_unit(x->args[1], o->id, &rest)) return;
+          for (auto& r : rows) shared = shared || (r.first == x->args[0]->name && expr_eq(r.second, rest));
+        });
+    });
+  });
+  return shared;
+}
+
 // A long loop over a row that is no whole number of vectors: rows start anywhere.  The vectors begin where a line of the
 // memory does, so that no two accesses share a line, and what stands in front of them and behind them (less than a line and
 // a vector) is a loop of its own, one element to a thread.  Sums of 542 rows of 115 669 floats on 128 threads 70.5 -> 49.9 us,
@@ -146,8 +201,8 @@ Stmts Pass::vectorize(const Stmts& ss) {
       // fill its launch exactly, since it has no bounds guard.  Where 16-byte vectors would leave more than a quarter of
       // the threads without one, narrower vectors are taken.  Elements of four bytes and more move 256 bytes per
       // wavefront and access as they are, so only narrower ones take vectors that do not divide the loop: the last one
-      // is then tested element by element.  So do wider ones where rows are written and threads take two vectors and more
-      // (softmax, floats on 256 threads: 30000 rows of 501 / 999 / 1001 21.3 / 57.9 / 58.1 -> 19.2 / 40.3 / 40.0 us, 2000 of 20001
+      // is then tested element by element.  So do wider ones where rows are written, threads take two vectors and more and
+      // `part_of_a_vector_pays` (softmax, floats on 256 threads: 30000 rows of 501 / 999 / 1001 21.3 / 57.9 / 58.1 -> 19.2 / 40.3 / 40.0 us, 2000 of 20001
       // 182 -> 61; 63305 rows of 202 on one vector a thread 20.7 -> 25.7; sums of 20000 rows of 999 13.9 -> 15.6).  (Rows need not start on 16 bytes: the memory instructions take any
       // element-aligned address.  Softmax over 1000 rows of 20001 halves on 512 threads per row: 40.2 -> 21.6 us, over
       // 3000 rows of 999 on 256: 10.3 -> 6.7.)
@@ -155,7 +210,7 @@ Stmts Pass::vectorize(const Stmts& ss) {
       for (int v = widest; v >= 2 && V == 0 && !nested; v /= 2) {
         const int64_t vectors = (extent + v - 1) / v;
         const bool whole = extent % v == 0;
-        if (grid_wide ? whole && extent % (s->map.n * v) == 0 : (extent % widest == 0 || widest > 4 || (stores_rows && v == widest && vectors > s->map.n)) && 4 * vectors >= 3 * s->map.n) V = v;
+        if (grid_wide ? whole && extent % (s->map.n * v) == 0 : (extent % widest == 0 || widest > 4 || (stores_rows && v == widest && vectors > s->map.n && part_of_a_vector_pays(s))) && 4 * vectors >= 3 * s->map.n) V = v;
         if (grid_wide) break;
       }
       // (a long loop whose trip count is not the same for all threads is not counted: its last vector would put a test

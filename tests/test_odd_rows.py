@@ -250,3 +250,110 @@ def test_rows_fetched_in_front_of_a_time_loop(dtype):
             want = table[obs[:, t]] - want + b[:m]
         steps_of_rows(table, obs, a, b, 6, m, 5, opts=opts(6, threads))
         assert np.array_equal(a, want), (m, threads)
+
+
+@parpy.jit
+def one_loop(x, y, N, M):
+    parpy.label('N')
+    for i in range(N):
+        parpy.label('M')
+        for j in range(M):
+            y[i, j] = x[i, j] + 1.0
+
+
+@parpy.jit
+def two_loops(x, y, N, M):
+    parpy.label('N')
+    for i in range(N):
+        parpy.label('M')
+        for j in range(M):
+            y[i, j] = x[i, j] + 1.0
+        parpy.label('M')
+        for j in range(M):
+            x[i, j] = y[i, j] - x[i, j] * 2.0
+
+
+@parpy.jit
+def two_loops_apart(x, y, N, M):
+    parpy.label('N')
+    for i in range(N):
+        parpy.label('M')
+        for j in range(1, M - 1):
+            y[i, j] = x[i, j - 1] - x[i, j + 1]
+        parpy.label('M')
+        for j in range(2, M - 2):
+            x[i, j] = y[i, j - 1] + y[i, j + 1]
+
+
+@parpy.jit
+def ring(x, y, N, M):
+    parpy.label('N')
+    for i in range(N):
+        for t in range(5):
+            s = x
+            d = y
+            if t & 1:
+                s = y
+                d = x
+            parpy.label('M')
+            for j in range(M):
+                d[i, j] = s[i, (j + 1) % M] - s[i, j // 2]
+
+
+@parpy.jit
+def fourth(x, y, N, M):
+    parpy.label('N')
+    for i in range(N):
+        for t in range(5):
+            s = x
+            d = y
+            if t & 1:
+                s = y
+                d = x
+            parpy.label('M')
+            for j in range(M):
+                d[i, j] = s[i, (j * 4) % M] - s[i, j]
+
+
+def walked(fn, x, y, m):
+    j = np.arange(m)
+    if fn in (one_loop, two_loops):
+        y[:] = x + x.dtype.type(1)
+        if fn is two_loops:
+            x[:] = y - x * x.dtype.type(2)
+    elif fn is two_loops_apart:
+        y[:, 1:-1] = x[:, :-2] - x[:, 2:]
+        x[:, 2:-2] = y[:, 1:-3] + y[:, 3:-1]
+    else:
+        for t in range(5):
+            s, d = (y, x) if t & 1 else (x, y)
+            d[:] = s[:, (j + 1) % m] - s[:, j // 2] if fn is ring else s[:, (j * 4) % m] - s
+
+
+WALKS = [(one_loop, False), (two_loops, True), (two_loops_apart, False), (ring, True), (fourth, False)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_which_loops_take_a_part_of_a_vector(dtype):
+    """Rows of which a thread walks its elements twice, or which stand in LDS and are read in order."""
+    for m, threads in ((1001, 64), (4099, 256)):
+        for fn, taken in WALKS:
+            x = np.zeros((5, m), dtype)
+            s = parpy.print_compiled(fn, [x, x.copy(), 5, m], opts(5, threads))
+            hiprtc_compile(s[:s.index("// host side")], opts(5, threads))
+            loops = re.findall(r"\(int j_(q_)?\d+_k = 0", s)
+            assert loops and all((q == "q_") == taken for q in loops), (fn, m)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+def test_walks_of_odd_rows(dtype):
+    """Small whole numbers: exact in every type."""
+    for m, threads in ((129, 64), (257, 64), (1001, 64), (1003, 128), (4099, 256)):
+        for fn, _ in WALKS:
+            rng = np.random.default_rng(m)
+            x, y = (rng.integers(-9, 9, (21, m)).astype(dtype) for _ in range(2))
+            want_x, want_y = x.copy(), y.copy()
+            walked(fn, want_x, want_y, m)
+            fn(x, y, 21, m, opts=opts(21, threads))
+            assert np.array_equal(x, want_x) and np.array_equal(y, want_y), (fn, m, threads)
