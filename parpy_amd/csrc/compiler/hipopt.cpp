@@ -92,6 +92,7 @@ void hip_optimize(Program& p, const Options& opts, NameGen& gen) {
     // headline kernel would spill six, the reference form of 7-mers runs 11.4 -> 12.3 ms, 16 layers of 5-mers 11.9 -> 12.5)
     if (opts.opt_pair_steps && budget >= 16) k.body = pass.pair_steps(k.body);
     k.fence_lds_iterations = opts.opt_fence_iterations && !pass.step_has_transcendentals();
+    if (!k.no_restrict) k.body = pass.swapped_pointers(k.body);
     pass.mark_read_only();
     k.aligned_params = opts.assume_aligned;
   }

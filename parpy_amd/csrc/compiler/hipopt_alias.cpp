@@ -7,6 +7,43 @@
 namespace parpy {
 namespace hipopt {
 
+// ================================================================ pointers that change places while the kernel runs
+// `for t: src = a; dst = b; if (t & 1) { src = b; dst = a; } <step>` on arrays in memory: within a step nothing is stored to
+// what `src` names, and the device compiler takes that for all steps: it reads an element that all threads read, or a single
+// thread behind a test, by a scalar load.  The scalar cache does not see vector stores, and the element is that of an earlier
+// step.  (`s[i, 5]` in a step that also reduces the row, 2 rows of 2051 floats; `s[i, 4 j % 2051]` for j = 2049, which only
+// thread 0 of 512 has.)  The pointers get an offset of zero from a vector register, with which no address is the same for
+// all threads as far as the compiler knows.  Arrays in LDS and loops on the host are not concerned.
+Stmts Pass::swapped_pointers(const Stmts& ss0) {
+  auto in_memory = [](const Type& t) { return is_alias_type(t) && t.mem != Mem::LDS; };
+  std::function<Stmts(const Stmts&, bool, bool)> walk = [&](const Stmts& ss, bool in_loop, bool loop_body) {
+    std::set<Name> here, inside;       // pointers declared by these statements, and anywhere in them
+    std::map<Name, size_t> last;       // the last of these statements that sets a pointer
+    for (size_t i = 0; in_loop && i < ss.size(); ++i) {
+      if (ss[i]->k == Stmt::Def) here.insert(ss[i]->id);
+      visit_stmts({ss[i]}, [&](const S& c) { if (c->k == Stmt::Def) inside.insert(c->id); });
+      if (ss[i]->k == Stmt::For || ss[i]->k == Stmt::While) continue;
+      visit_stmts({ss[i]}, [&](const S& c) {
+        if (c->k == Stmt::Assign && c->dst->k == Expr::Var && in_memory(c->dst->ty)) last[c->dst->name] = i;
+        if (c->k == Stmt::Def && c->expr && c->expr->k == Expr::IfExpr && in_memory(c->ty)) last[c->id] = i;
+      });
+    }
+    Stmts out;
+    for (size_t i = 0; i < ss.size(); ++i) {
+      const S& s = ss[i];
+      const bool loop = s->k == Stmt::While || (s->k == Stmt::For && s->map.k == GpuMap::None && !s->unroll);
+      auto r = clone(s);
+      r->body = walk(s->body, in_loop || loop, loop);
+      r->els = walk(s->els, in_loop, false);
+      out.push_back(r);
+      for (auto& l : last)
+        if (l.second == i && (here.count(l.first) || (loop_body && !inside.count(l.first)))) out.push_back(mk_rawstmt(l.first.str() + " += parpy_vector_zero();"));
+    }
+    return out;
+  };
+  return walk(ss0, false, false);
+}
+
 // ================================================================ no-alias scopes for array aliases
 // `src = a; dst = b; if (c) { src = b; dst = a; } <rest>`: in <rest> the two aliases always name
 // different arrays, but the target compiler only sees two selected pointers that may be equal, so

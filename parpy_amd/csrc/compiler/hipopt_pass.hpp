@@ -143,6 +143,7 @@ struct Pass {
   static bool alias_target(const E& e, const AliasCfg& cfg, Name* out);
   static bool apply_alias_stmt(const S& st, std::vector<AliasCfg>& cfgs, std::vector<Name>& order);
   Stmts noalias_scopes(const Stmts& ss, bool wrap);
+  Stmts swapped_pointers(const Stmts& ss);
   void mark_read_only();
   void mark_read_once();
 };

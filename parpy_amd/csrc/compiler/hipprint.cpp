@@ -297,6 +297,8 @@ __device__ __forceinline__ bool parpy_last_workgroup(unsigned* counters, int whi
   __syncthreads();
   return parpy_last;
 }
+// zero, in a vector register (the device compiler does not know that it is the same for all lanes)
+__device__ __forceinline__ int parpy_vector_zero() { int z; asm("v_mov_b32 %0, 0" : "=v"(z)); return z; }
 // all bits or none, and the bits of a where they are set, of b elsewhere
 __device__ __forceinline__ int parpy_mask(bool c) {
   int m = c ? -1 : 0;
