@@ -22,13 +22,14 @@ namespace {
 //     the row's last element instead of branching, so that its loads are issued together as well.
 //   * A row longer than `longest` elements is shared by all waves of a workgroup: by one of those in front of the others,
 //     which look for such rows and queue them in LDS, or, where there are none, by that of its own team.
+//   * Columns are divided into slabs, one to every second, fourth or eighth workgroup (`slabs`).
 //
 // Measured (100 000 rows of 50 non-zeros on average, the longest 15 800, float64): eight lanes per row, one element in
 // flight 547 us, in teams 34 us.  The gathers out of L2 are then what bounds it: 5.5 million lines requested (counted, 87 %
 // of them hits), 158 per nanosecond.  20 000 rows of 24 on average (longest 3400)
 // times a 128-column matrix: one workgroup per row with the sum read and written back in LDS per element 840 us, in
-// teams 42 us, with the long rows in front (below) 34: the longest pulls 1.7 MB through one compute unit, and 165 of the 261 MB
-// that the L2s deliver come from behind them, since the 10 MB matrix does not fit a die's 4 MB.
+// teams 42 us, with the long rows in front (below) 34: the longest pulled 1.7 MB through one compute unit, and 165 of the 261 MB
+// that the L2s deliver came from behind them, since the 10 MB matrix does not fit a die's 4 MB.  In two slabs 26.6 us.
 struct RaggedSum {
   Program& p;
   const Options& opts;
@@ -228,6 +229,35 @@ struct RaggedSum {
 
   static int64_t pow2_at_least(int64_t n) { int64_t q = 1; while (q < n) q *= 2; return q; }
 
+  // Slabs of columns: workgroups b, b + n, b + 2n, ... sum the rows over one n-th of the columns.  Workgroups are dealt to the
+  // eight dies in turn, so with two, four or eight slabs a die's L2 holds its slab of the selected rows only (pieces of 512 / 256
+  // / 128 bytes out of 10 MB: 24.1 us in one slab, 15.8 in two, 12.8 in four; where they end up is a matter of speed alone), and
+  // the longest rows are shared by as many workgroups.  Rows go to as many slabs as leave a wavefront one batch of loads for a
+  // row of average length, 64 lanes with four times 16 bytes (an eighth less will do).  Rows of uneven length, in one slab and
+  // in 2 / 4 / 8, us: 20 000 of 24 times 128 columns 43.7 (33.8 on 1024 threads) and 26.3 / 27.0 (6 KB and 3 KB a wavefront);
+  // 16 000 of 24 times 256: 77.9 (61.3) and 47.5 / 35.0 / 46.9; 8192 of 20 times 128: 19.1 and 11.9 / 13.7 / 22.0; 40 000 of 16
+  // times 128: 50.1 (45.7) and 39.3 / 53.5; 60 000 of 20 times 64: 41.8 and 45.6; 100 000 of 4 times 256: 73.7 and 86.3.
+  static int64_t slabs(const Rows& r, int64_t V, int64_t avg) {
+    if (!r.has_col) return 1;
+    const int64_t slots = r.cols / V;
+    int64_t row = 0;   // bytes of a selected row
+    auto scan = [&](const E& e) {
+      visit_exprs(e, [&](const E& x) { if (x->k == Expr::Index && mentions(x->args[1], r.col)) row = std::max(row, r.cols * elem_bytes(x->ty.sz)); });
+    };
+    scan(r.term);
+    for (auto& d : r.defs) scan(d->expr);
+    // thousandths of the lanes along the columns that have none: no more than in one slab, or than 420 (65 columns on 128 lanes,
+    // two slabs of 13 895 rows of 21 times 129: 33.3 us instead of 28.8; 77 on 128, 3616 of 21 times 153: 13.8 instead of 15.7)
+    auto idle = [&](int64_t n) {
+      const int64_t own = (slots + n - 1) / n, lanes = std::min<int64_t>(WAVE_SIZE, pow2_at_least(own)), taken = (own + lanes - 1) / lanes * lanes;
+      return 1000 - 1000 * own / taken;
+    };
+    int64_t best = 1;
+    for (int64_t n = 2; n <= 8 && r.cols >= 16 * n && slots >= n && r.n * WAVE_SIZE * n <= (int64_t(1) << 30) && avg * row >= 3584 * n; n *= 2)
+      if (idle(n) <= std::max<int64_t>(idle(1), 420)) best = n;
+    return best;
+  }
+
   // a[v + c] and a[v + c + 1]
   static bool adjacent(E a, E b, const Name& v) {
     while (a->k == Expr::Convert) a = a->args[0];
@@ -268,55 +298,64 @@ struct RaggedSum {
     Rows r;
     if (!match(k, r)) return false;
     const int64_t V = column_vector(k, r);
-    const int64_t slots = r.cols / V;                       // vectors along the columns
+    const int64_t words = elem_bytes(r.acc->ty.sz) / 4;
+    const int64_t avg = r.elements > 0 ? std::max<int64_t>(1, r.elements / r.n) : 32;
+    const int64_t SL = slabs(r, V, avg);
+    const int64_t all_slots = r.cols / V, slots = (all_slots + SL - 1) / SL;   // vectors along the columns: all, of a slab
+    const int64_t wide = slots * V;                                            // columns of a slab
     const int64_t L = std::min<int64_t>(WAVE_SIZE, pow2_at_least(slots));
     const int64_t chunks = (slots + L - 1) / L;
     const int64_t K = chunks * V;                           // sums a lane holds
-    const int64_t words = elem_bytes(r.acc->ty.sz) / 4;
     if (K * words > 16) return false;
     // elements in flight per lane: up to sixteen registers of what they select
     const int64_t U = r.has_col ? std::max<int64_t>(2, std::min<int64_t>(8, 16 / (K * words))) : 4;
-    const int64_t avg = r.elements > 0 ? std::max<int64_t>(1, r.elements / r.n) : 32;
     // Subteams: two elements of an average row per lane, at least four lanes so that they share cache lines.  (100 000
     // rows of 50 non-zeros, float64: 4 / 8 / 16 / 32 / 64 lanes 53 / 47 / 40 / 38 / 45 us; 300 000 rows of 16: 41.7 us
     // on four lanes, 36.0 on eight and sixteen; 50 000 rows of 200: 110 us on 16, 94 on 64; 50 000 rows of 8 times 32
     // columns: 22.4 / 17.7 / 17.4 / 20.9 us for 1 / 2 / 4 / 8 subteams.)  Rows that were the threads of one workgroup
     // are too few to fill the chip in any case: 10.3 us on 16 lanes, 11.0 on eight.
-    const int64_t P = r.one_group ? 8 : std::min<int64_t>(WAVE_SIZE / L, std::max<int64_t>(pow2_at_least((avg + 1) / 2), r.has_col ? 1 : 4));
-    const int64_t T = L * P;
+    auto subteams = [&](int64_t lanes) {
+      return r.one_group ? 8 : std::min<int64_t>(WAVE_SIZE / lanes, std::max<int64_t>(pow2_at_least((avg + 1) / 2), r.has_col ? 1 : 4));
+    };
+    const int64_t P = subteams(L), T = L * P;
     // more wavefronts than run at once
     constexpr int64_t RESIDENT = 256 * 2048;
-    const bool queues = r.n * T > RESIDENT;
+    const int64_t lanes0 = std::min<int64_t>(WAVE_SIZE, pow2_at_least(all_slots)), T0 = lanes0 * subteams(lanes0);   // a team of the whole row
+    if ((all_slots + lanes0 - 1) / lanes0 * V * words > 16 || (r.has_col && r.tpb < r.cols)) return false;
+    const bool queues = r.n * T0 > RESIDENT;
     // (single sums: a workgroup is over with its slowest wavefront; 1024 / 512 / 256 threads 36.6 / 34.2 / 34.2 us for the 50
     // non-zeros above, 29.9 / 28.2 / 30.2 in floats, 99.8 / 91.2 / 91.9 for 10^6 rows of 10 floats)
-    const int64_t tpb = !r.has_col && queues ? std::min<int64_t>(r.tpb, 512) : r.tpb;
-    if (tpb % WAVE_SIZE != 0 || tpb < L * V || r.n * T > (int64_t(1) << 30)) return false;
+    // Rows of columns: 512 threads, unless a row of average length is more than one batch of its team and cannot be divided into
+    // slabs, whose longest rows take 1024 (7794 rows of 45 times 32 columns: 13.5 us and 12.6; 3000 of 200 times 20: 25.8 and
+    // 20.2; but 100 000 of 20 times 32: 39.7 and 50.9, 58 973 of 27 times 32: 29.7 and 38.1).
+    const bool fewer = r.has_col ? wide <= 512 && (SL > 1 || 8 * avg < 7 * P * U || r.n * T0 > 4 * RESIDENT) : queues;
+    const int64_t tpb = fewer ? std::min<int64_t>(r.tpb, 512) : r.tpb;
+    if (tpb % WAVE_SIZE != 0 || tpb < L * V || r.n * T * SL > (int64_t(1) << 30)) return false;
     const int64_t teams = tpb / T, waves = tpb / WAVE_SIZE;
-    if (r.has_col && (tpb < r.cols || waves * L * K * elem_bytes(r.acc->ty.sz) > 64 * 1024)) return false;
+    if (r.has_col && (tpb < wide || waves * L * K * elem_bytes(r.acc->ty.sz) > 64 * 1024)) return false;
     // Rows longer than this are shared by the workgroup.  A shared row costs two barriers and a round trip of its own,
     // and the waves that have no such row wait for it: 256 elements for single sums (128 costs 5 to 20 %), fewer when
     // every element moves a row of columns (64 against 256 elements: 17.4 and 20.1 us for the 32-column product above).
     const int64_t longest = r.has_col ? std::max<int64_t>(64, 2 * avg) : std::max<int64_t>(256, 4 * avg);
     // The rows longer than that go to workgroups in front of the others, which look for them and share each as above: started
     // in order, the longest may start last, and in the others' workgroups sixteen wavefronts would wait for them.  Where more
-    // wavefronts are launched than run at once, 1024 such workgroups for rows of columns (20 000 rows of 24 on average times
-    // 128 columns: 34.1 us, 35.1 with 512, 33.8 with 2048, 37.9 with 256; 20 000 of 24 times 64: 20.7, 20.9, 21.0, 23.3) and
-    // 512 for single sums (100 000 rows of 50, doubles: 36.3, 37.5 with 1024; 39.5 us with every long row shared where it is).
-    // Before, rows of columns had 256, for the rows that stand out by another factor of four: 34.7 us for the first and 21.3
-    // for the second, 100 000 of 4 times 256: 85.4 -> 79.5, 50 000 of 20 times 37: 50.4 -> 45.6; 9529 of 41 times 101 loses
-    // by it, 31.0 -> 33.6 (40.8 before the elements of a shared row stood in LDS, below).  Otherwise there is room beside the teams' workgroups: one for eight rows as long as they run at once
-    // (1021 rows of 35 times 256 columns 20.3 -> 13.0 us, 1000 of 64 times 64: 12.9 -> 8.6, 5000 of 64 times 256: 70.4 -> 59.2;
-    // one for 4 / 16 / 32 rows: 13.1 / 13.6 / 15.0, 7.6 / 8.5 / 10.5, 59.4 / 59.2 / 65.5, but 2000 of 64 times 256: 34.8 / 26.2 /
-    // 27.3 and 26.2 with eight), one for sixteen rows for single sums (3000 rows of 60, doubles 6.3 -> 4.9 us, 5.5 with one for
-    // four; 20 000 of 30: 9.8 -> 9.0).  Where the teams leave no room, single sums keep the queues (8000 rows of 150: 18.0 us,
-    // 20.0 with 64 in front) and rows of columns have 512 in front (7500 of 30 times 200: 43.5 -> 32.4, 8000 of 10 times 64:
-    // 8.1 -> 7.3; 256 of them 35.4 and 7.3, 1024 31.5 and 8.1), but for a launch that fills the device exactly.
-    const int64_t groups = (r.n + teams - 1) / teams, room = RESIDENT / tpb - groups;
-    const int64_t scouts = queues ? std::max<int64_t>(r.has_col ? 1024 : 512, (r.n + 1023) / 1024)
+    // wavefronts are launched than run at once (slabs not counted), 1024 such workgroups for rows of columns (30 978 rows of 19
+    // on average times 32 columns: 14.5 us, 15.9 with 512, 17.5 with 256; 20 000 of 24 times 128 in two slabs: 26.9, 30.1, 33.8;
+    // 100 000 of 4 times 256: 74.6, 74.4) and 512 for single sums (100 000 rows of 50, doubles: 36.3, 37.5 with 1024; 39.5 us
+    // with every long row shared where it is).  Fewer rows of columns: one for 160 elements, up to 512 (5835 of 40 times 128:
+    // 29.8 us with 148 in front, 20.0 / 15.9 / 15.3 with 256 / 512 / 1024; 1000 of 64 times 256: 12.4 / 9.1 / 8.8 with 125 / 256
+    // / 512; 1045 of 10 times 256: 4.4 / 4.5 / 5.3 with 130 / 256 / 1024), but for a launch whose undivided rows fill the device
+    // exactly.  Fewer single sums: one for sixteen rows where there is room beside the others (3000 rows of 60, doubles 6.3 ->
+    // 4.9 us, 5.5 with one for four; 20 000 of 30: 9.8 -> 9.0), else the queues (8000 rows of 150: 18.0 us, 20.0 with 64 in front).
+    const int64_t room = RESIDENT / r.tpb - (r.n * T0 + r.tpb - 1) / r.tpb;
+    const int64_t scouts = queues ? std::max<int64_t>(r.has_col ? 1024 : 512, (r.n * SL + 1023) / 1024)
                            : r.one_group ? 0
-                           : room >= 64 ? std::max<int64_t>(1, std::min<int64_t>(room, r.n / (r.has_col ? 8 : 16)))
-                                        : r.has_col && room > 0 ? 512 : 0;
-    const int64_t looked = scouts ? (r.n + scouts - 1) / scouts : 0;   // rows for each of them
+                           : r.has_col ? (room > 0 ? std::max(SL, std::min<int64_t>(512, r.n * avg / 160)) : 0)
+                           : room >= 64 ? std::max<int64_t>(1, std::min<int64_t>(room, r.n / 16))
+                                        : 0;
+    const int64_t slices = scouts / SL;
+    const int64_t looked = scouts ? (r.n + slices - 1) / slices : 0;   // rows for each of them
+    const int64_t groups = (r.n + teams - 1) / teams;                  // workgroups of the others, per slab
     // element numbers in 32 bits when the array they walk is known to be small enough
     const bool small = r.bounded && r.elements < (int64_t(1) << 29);
     const ElemSize esz = small && isz == ElemSize::I64 ? ElemSize::I32 : isz;
@@ -343,14 +382,33 @@ struct RaggedSum {
       loop->unroll = true;
       return S(loop);
     };
-    // the column of slot c of lane l; `inside`: the last vector of columns instead of one past it
-    auto column = [&](const E& c, const E& l, bool inside) {
+    // the column of slot c of lane l, counted from the start of the slab
+    const Name slab = SL > 1 ? gen.fresh("slab") : Name();
+    E sv = mk_var(slab, ity);
+    auto slab_column = [&](const E& c, const E& l) {
       E chunk = mk_binop(BinOp::FloorDiv, c, iint(V), ity), v = mk_binop(BinOp::Rem, c, iint(V), ity);
       E base = chunks == 1 ? l : add(mk_binop(BinOp::Mul, chunk, iint(L), ity), l);
-      if (inside && L * chunks != slots) base = mk_binop(BinOp::Min, base, iint(slots - 1), ity);
       return V == 1 ? base : add(mk_binop(BinOp::Mul, base, iint(V), ity), v);
     };
-    const bool partial = L * K != r.cols;   // lanes or slots past the last column exist
+    // the column itself; past the slab's last vector of columns that vector again
+    auto column = [&](const E& c, const E& l) {
+      E chunk = mk_binop(BinOp::FloorDiv, c, iint(V), ity), v = mk_binop(BinOp::Rem, c, iint(V), ity);
+      E base = chunks == 1 ? l : add(mk_binop(BinOp::Mul, chunk, iint(L), ity), l);
+      if (L * chunks != slots) base = mk_binop(BinOp::Min, base, iint(slots - 1), ity);
+      if (SL > 1) base = add(mk_binop(BinOp::Mul, sv, iint(slots), ity), base);
+      if (slots * SL != all_slots) base = mk_binop(BinOp::Min, base, iint(all_slots - 1), ity);
+      return V == 1 ? base : add(mk_binop(BinOp::Mul, base, iint(V), ity), v);
+    };
+    // is column `at` of the slab (a number below `upto`) one, and one of the array
+    auto in_slab = [&](const E& at, int64_t upto) {
+      E c;
+      if (upto > wide) c = mk_binop(BinOp::Lt, at, iint(wide), bty);
+      if (wide * SL != r.cols) {
+        E whole = mk_binop(BinOp::Lt, add(mk_binop(BinOp::Mul, sv, iint(wide), ity), at), iint(r.cols), bty);
+        c = c ? mk_binop(BinOp::And, c, whole, bty) : whole;
+      }
+      return c;
+    };
     // statements that add the elements first, first + stride, ... of the row to the lane's sums
     // (staged: loads of the elements that stand in LDS, from element `lo` on)
     struct Staged { E load; Name lds; };
@@ -400,7 +458,7 @@ struct RaggedSum {
         Stmts ss;
         named.clear();
         if (r.has_col) {
-          ss.push_back(mk_def(r.col, ity, fold_expr(column(c, l, true)), r.loop->i));
+          ss.push_back(mk_def(r.col, ity, fold_expr(column(c, l)), r.loop->i));
         }
         for (auto& d : r.defs) { E e = bind(d->expr, ss); ss.push_back(mk_def(d->id, d->ty, e, d->i)); }
         Name tv = gen.fresh("term");
@@ -438,11 +496,14 @@ struct RaggedSum {
     auto finish_slots = [&](const E& l) {
       if (!r.has_col) return finish(part(iint(0)));
       return Stmts{per_slot([&](const E& c) {
-        Stmts ss{mk_def(r.col, ity, fold_expr(column(c, l, false)), r.loop->i)};
-        Stmts f = finish(part(c));
-        if (partial) ss.push_back(mk_if(mk_binop(BinOp::Lt, mk_var(r.col, ity), iint(r.cols), bty), f, {}));
-        else ss.insert(ss.end(), f.begin(), f.end());
-        return ss;
+        // (lanes and slots past the slab's last column, or past the array's, store nothing)
+        Stmts f{mk_def(r.col, ity, fold_expr(SL == 1 ? slab_column(c, l) : add(mk_binop(BinOp::Mul, sv, iint(wide), ity), slab_column(c, l))), r.loop->i)};
+        Stmts g = finish(part(c));
+        E some = in_slab(fold_expr(slab_column(c, l)), L * K);
+        if (!some) { f.insert(f.end(), g.begin(), g.end()); return f; }
+        if (SL == 1) { f.push_back(mk_if(mk_binop(BinOp::Lt, mk_var(r.col, ity), iint(r.cols), bty), g, {})); return f; }
+        f.insert(f.end(), g.begin(), g.end());
+        return Stmts{mk_if(some, f, {})};
       })};
     };
     auto limits = [&](Stmts& ss, E* lo, E* hi) {
@@ -493,9 +554,21 @@ struct RaggedSum {
     {
       Stmts body;
       E team = mk_binop(BinOp::FloorDiv, lv, iint(T), ity);
-      if (scouts) team = mk_binop(BinOp::Max, mk_binop(BinOp::Sub, team, iint(scouts * teams), ity), iint(0), ity);   // (known not to be negative)
+      E behind = lv;
+      if (scouts && SL == 1) team = mk_binop(BinOp::Max, mk_binop(BinOp::Sub, team, iint(scouts * teams), ity), iint(0), ity);   // (known not to be negative)
+      if (SL > 1) {
+        if (scouts) {
+          Name at = gen.fresh("behind");
+          behind = mk_var(at, ity);
+          body.push_back(mk_def(at, ity, mk_binop(BinOp::Max, mk_binop(BinOp::Sub, lv, iint(scouts * tpb), ity), iint(0), ity), r.loop->i));
+        }
+        // (every SL-th workgroup is one of the same slab)
+        team = mk_binop(BinOp::FloorDiv, add(mk_binop(BinOp::Mul, mk_binop(BinOp::FloorDiv, behind, iint(SL * tpb), ity), iint(tpb), ity), mk_binop(BinOp::Rem, behind, iint(tpb), ity)), iint(T), ity);
+      }
       body.push_back(mk_def(r.row, ity, team, r.loop->i));
       body.push_back(mk_def(q, ity, mk_binop(BinOp::Rem, lv, iint(T), ity), r.loop->i));
+      if (SL > 1) body.push_back(mk_def(slab, ity, mk_binop(BinOp::Rem, mk_binop(BinOp::FloorDiv, behind, iint(tpb), ity), iint(SL), ity), r.loop->i));
+      const size_t placed = body.size();
       E lo, hi;
       bounds(body, &lo, &hi);
       Stmts own;
@@ -515,9 +588,16 @@ struct RaggedSum {
       Stmts defer;
       if (!scouts) defer = {mk_if(mk_binop(BinOp::Eq, qv, iint(0), bty), {enqueue}, {})};
       body.push_back(mk_if(mk_binop(BinOp::Leq, mk_binop(BinOp::Sub, hi, lo, ety), eint(longest), bty), own, defer));
+      if (SL > 1 && groups * teams != r.n) {
+        // (the last workgroup of every slab may hold teams without a row)
+        Stmts rest(body.begin() + placed, body.end());
+        body.resize(placed);
+        body.push_back(mk_if(mk_binop(BinOp::Lt, mk_var(r.row, ity), iint(r.n), bty), rest, {}));
+      }
       auto nr = clone(k.body[0]);
       nr->id = lane;
-      nr->hi = iint(r.n * T + scouts * tpb);
+      const int64_t lanes = SL == 1 ? r.n * T + scouts * tpb : (groups * SL + scouts) * tpb;
+      nr->hi = iint(lanes);
       nr->body = body;
       if (scouts) {
         Name at = gen.fresh(r.row.s + "_at"), slice = gen.fresh("slice");
@@ -529,7 +609,7 @@ struct RaggedSum {
         const E more = mk_binop(BinOp::Gt, mk_binop(BinOp::Sub, b, a, ity), iint(longest), bty);
         look.push_back(mk_if(mk_binop(BinOp::And, mk_binop(BinOp::Lt, a, b, bty), more, bty), {enqueue}, {}));
         nr->body = {mk_if(mk_binop(BinOp::Lt, lv, iint(scouts * tpb), bty),
-                          {mk_def(slice, ity, mk_binop(BinOp::FloorDiv, lv, iint(tpb), ity)),
+                          {mk_def(slice, ity, mk_binop(BinOp::FloorDiv, lv, iint(SL * tpb), ity)),
                            mk_for(at, add(first, mk_binop(BinOp::Rem, lv, iint(tpb), ity)), mk_binop(BinOp::Min, add(first, iint(looked)), iint(r.n), ity), tpb, look, LoopPar(), r.loop->i)},
                           body)};
       }
@@ -537,7 +617,7 @@ struct RaggedSum {
       nr->map = GpuMap();
       nr->map.k = GpuMap::ThreadBlock;
       nr->map.tpb = tpb;
-      nr->map.n = (r.n * T + scouts * tpb + WAVE_SIZE - 1) / WAVE_SIZE * WAVE_SIZE;
+      nr->map.n = (lanes + WAVE_SIZE - 1) / WAVE_SIZE * WAVE_SIZE;
       top.push_back(nr);
     }
     if (scouts) top.push_back(mk_rawstmt("if (blockIdx.x >= " + std::to_string(scouts) + ") return;"));
@@ -554,6 +634,11 @@ struct RaggedSum {
       Stmts body;
       body.push_back(mk_def(r.row, ity, mk_raw("((int64_t)" + queue.str() + "[" + h.str() + "])", ity), r.loop->i));
       body.push_back(mk_def(tid, ity, tx));
+      if (SL > 1) {
+        auto bx = std::make_shared<Expr>(*tx);
+        bx->k = Expr::BlockIdx;
+        body.push_back(mk_def(slab, ity, mk_binop(BinOp::Rem, E(bx), iint(SL), ity)));
+      }
       E lo, hi;
       bounds(body, &lo, &hi);
       E l = L == 1 ? iint(0) : mk_binop(BinOp::Rem, tv, iint(L), ity), sub = L == 1 ? tv : mk_binop(BinOp::FloorDiv, tv, iint(L), ity);
@@ -628,13 +713,13 @@ struct RaggedSum {
         E base = mk_var(shared, Type::pointer(sty.sz, Mem::LDS));
         E wave = mk_binop(BinOp::FloorDiv, tv, iint(WAVE_SIZE), ity);
         Stmts put{per_slot([&](const E& c) {
-          E at = add(mk_binop(BinOp::Mul, wave, iint(L * K), ity), column(c, l, false));
+          E at = add(mk_binop(BinOp::Mul, wave, iint(L * K), ity), slab_column(c, l));
           return Stmts{mk_assign(mk_index(base, fold_expr(at), sty), part(c))};
         })};
         body.push_back(mk_if(mk_binop(BinOp::Lt, mk_binop(BinOp::Rem, tv, iint(WAVE_SIZE), ity), iint(L), bty), put, {}));
         body.push_back(mk_sync());
         Name s = gen.fresh("whole"), w = gen.fresh("w");
-        Stmts sum{mk_def(r.col, ity, tv), mk_def(s, sty, mk_float(0.0, sty.sz))};
+        Stmts sum{mk_def(r.col, ity, SL == 1 ? tv : add(mk_binop(BinOp::Mul, sv, iint(wide), ity), tv)), mk_def(s, sty, mk_float(0.0, sty.sz))};
         auto over = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(mk_for(
             w, iint(0), iint(waves), 1,
             {mk_assign(mk_var(s, sty), mk_binop(BinOp::Add, mk_var(s, sty),
@@ -644,7 +729,9 @@ struct RaggedSum {
         sum.push_back(over);
         Stmts f = finish(mk_var(s, sty));
         sum.insert(sum.end(), f.begin(), f.end());
-        body.push_back(mk_if(mk_binop(BinOp::Lt, tv, iint(r.cols), bty), sum, {}));
+        E some = in_slab(tv, tpb);
+        if (some) body.push_back(mk_if(some, sum, {}));
+        else body.insert(body.end(), sum.begin(), sum.end());
         body.push_back(mk_sync());
         k.lds_bytes += waves * L * K * elem_bytes(sty.sz);
       }
@@ -653,7 +740,7 @@ struct RaggedSum {
     k.lds_bytes += (std::max(teams, looked) + 1) * 4;
     k.body = top;
     k.block = Dim3{tpb, 1, 1};
-    k.grid = Dim3{groups + scouts, 1, 1};
+    k.grid = Dim3{groups * SL + scouts, 1, 1};
     launch->grid = k.grid;
     launch->block = k.block;
     return true;
