@@ -142,15 +142,24 @@ __device__ __forceinline__ float parpy_fmin3c(float a, float b, float c) { float
 // largest one, which leaves the infinity alone (98 updates of 10^6 doubles: fixup 45.5 us, minimum 41.8).  Results are
 // those of the division bit for bit, except that a quotient below the normal range which lies exactly between two numbers
 // may round to the other one.
-template <int FIX> __device__ __forceinline__ float parpy_div_const(float x, float c, float r) {
+// INF: infinite dividends too, for another instruction (two for floats); without it their quotient is NaN.
+template <int FIX, bool INF = true> __device__ __forceinline__ float parpy_div_const(float x, float c, float r) {
+  const float a = c < 0 ? -c : c, m = c < 0 ? x : -x, k = r < 0 ? r : -r;
   float q = x * r;
-  for (int k = 0; k < FIX; ++k) q = __builtin_fmaf(__builtin_fmaf(-c, q, x), r, q);
+  if (!INF) {
+    for (int j = 0; j < FIX; ++j) q = __builtin_fmaf(__builtin_fmaf(a, q, m), k, q);
+    return q;
+  }
+  for (int j = 0; j < FIX; ++j) q = __builtin_fmaf(__builtin_fmaf(-c, q, x), r, q);
   return __builtin_amdgcn_div_fixupf(q, c, x);
 }
-template <int FIX> __device__ __forceinline__ double parpy_div_const(double x, double c, double r) {
+template <int FIX, bool INF = true> __device__ __forceinline__ double parpy_div_const(double x, double c, double r) {
   const double a = c < 0 ? -c : c, m = c < 0 ? x : -x, k = r < 0 ? r : -r;
   double q = x * r;
-  for (int j = 0; j < FIX; ++j) q = __builtin_fma(__builtin_fmin(__builtin_fma(a, q, m), 1.7976931348623157e+308), k, q);
+  for (int j = 0; j < FIX; ++j) {
+    const double left = __builtin_fma(a, q, m);
+    q = __builtin_fma(INF ? __builtin_fmin(left, 1.7976931348623157e+308) : left, k, q);
+  }
   return q;
 }
 // Quotient of halves, correctly rounded: a quotient in single precision after one correction by the remainder is off by
@@ -667,7 +676,7 @@ struct DevicePrinter {
               if (mag > 1.0 && mag <= 16777216.0 && c == std::trunc(c) && std::frexp(mag, &ex) != 0.5) {
                 const double r = f32 ? (double)(float)(1.0 / c) : 1.0 / c;
                 const bool one = std::fabs(std::fma(r, c, -1.0)) <= (f32 ? std::ldexp(1.0, -25) : std::ldexp(1.0, -54));
-                return std::string("parpy_div_const<") + (one ? "1" : "2") + ">(" + a + ", " + (f32 ? fmt_f32(c) : fmt_f64(c)) + ", " + (f32 ? fmt_f32(r) : fmt_f64(r)) + ")";
+                return std::string("parpy_div_const<") + (one ? "1" : "2") + (no_infinities ? ", false" : "") + ">(" + a + ", " + (f32 ? fmt_f32(c) : fmt_f64(c)) + ", " + (f32 ? fmt_f32(r) : fmt_f64(r)) + ")";
               }
             }
             // A quotient or remainder of 64-bit integers whose operands provably fit 31 bits is computed in 32
@@ -779,6 +788,13 @@ struct DevicePrinter {
       case Expr::RegElem: return e->name.str() + "[" + pexpr(e->args[0]) + "]";
       case Expr::Raw: return e->sval;
       case Expr::Call: {
+        if (!e->ext && e->sval == "parpy_no_infinities") {
+          const bool outer = no_infinities;
+          no_infinities = true;
+          std::string out = pexpr(e->args[0]);
+          no_infinities = outer;
+          return out;
+        }
         std::string out = (e->ext ? e->ext->name : e->sval) + "(";
         for (size_t a = 0; a < e->args.size(); ++a) out += (a ? ", " : "") + pexpr(e->args[a]);
         return out + ")";
@@ -797,6 +813,7 @@ struct DevicePrinter {
     }
   }
 
+  bool no_infinities = false;     // in an expression whose divisions may give NaN for infinite dividends
   std::vector<S> kept_alive;
   int in_unrolled = 0;            // unrolled loops over the elements of a vector around the statement being printed
   std::map<const Expr*, std::string> tail_loads;   // elements of vectors loaded in front of the loop over them
