@@ -23,7 +23,7 @@ LIB_PATH = pathlib.Path(__file__).parent / "libparpy_hipc.so"
 SOURCES = ["ast.cpp", "front.cpp", "constfold.cpp", "specialize.cpp", "lower.cpp",
            "gpu.cpp", "hipopt.cpp", "hipopt_util.cpp", "hipopt_control.cpp", "hipopt_prefetch.cpp", "hipopt_lds.cpp",
            "hipopt_vector.cpp", "hipopt_regs.cpp", "hipopt_keep.cpp", "hipopt_alias.cpp", "hipopt_launch.cpp",
-           "hipopt_ragged.cpp", "hipopt_timetile.cpp", "hipopt_stages.cpp", "hipopt_persist.cpp", "hipprint.cpp", "capi.cpp"]
+           "hipopt_ragged.cpp", "hipopt_timetile.cpp", "hipopt_twosteps.cpp", "hipopt_stages.cpp", "hipopt_persist.cpp", "hipprint.cpp", "capi.cpp"]
 
 _lib = None
 

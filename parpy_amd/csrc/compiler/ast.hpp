@@ -435,6 +435,7 @@ struct Kernel {
   std::set<Name> read_once;     // large inputs of which the launch reads every element once: non-temporal loads
   bool cached_stores = false;   // what this kernel writes is read by the next one: no non-temporal stores
   bool opaque_body = false;     // the body is a call of a device helper: parameters are described by the creator
+  bool finished = false;        // written out by the rewrite that made it, which the passes over single kernels leave as it is; what it writes it does not read
   bool no_restrict = false;     // workgroups exchange data through the parameters during the kernel: no no-alias promise
   bool wave_rows = false;       // every wavefront of a workgroup has an iteration of its own: barriers only order its own accesses
   bool fence_lds_iterations = false;  // keep a thread's LDS load / compute / store groups apart when the code is scheduled

@@ -45,7 +45,8 @@
 // branches, aliases), hipopt_prefetch.cpp, hipopt_lds.cpp, hipopt_vector.cpp,
 // hipopt_regs.cpp (budget, hoisting, register caching), hipopt_keep.cpp and
 // hipopt_alias.cpp; the whole-program rewrites are in hipopt_launch.cpp,
-// hipopt_ragged.cpp, hipopt_timetile.cpp, hipopt_stages.cpp and hipopt_persist.cpp.
+// hipopt_ragged.cpp, hipopt_timetile.cpp, hipopt_twosteps.cpp, hipopt_stages.cpp and
+// hipopt_persist.cpp.
 #include "hipopt_pass.hpp"
 
 namespace parpy {
@@ -56,6 +57,7 @@ void hip_optimize(Program& p, const Options& opts, NameGen& gen) {
     for (auto& k : p.kernels)
       if (!k.opaque_body) hipopt::Pass(k, opts, gen).mark_read_once();
   if (opts.opt_tile_steps && !opts.persistent_loops) hipopt::time_tile(p, opts, gen);
+  if (opts.opt_tile_steps && opts.opt_share_iterations && !opts.persistent_loops) hipopt::two_steps(p, opts, gen);
   if (opts.opt_vectorize) hipopt::reduction_stages(p, opts, gen);
   if (opts.opt_lane_split) hipopt::ragged_sum(p, opts, gen);
   if (opts.opt_lane_split && !opts.opt_mfma_sddmm) hipopt::lane_split(p, opts, gen);
@@ -64,6 +66,11 @@ void hip_optimize(Program& p, const Options& opts, NameGen& gen) {
   for (auto& k : p.kernels) {
     if (k.opaque_body) { k.aligned_params = opts.assume_aligned; continue; }
     hipopt::Pass pass(k, opts, gen);
+    if (k.finished) {
+      pass.mark_read_only();
+      k.aligned_params = opts.assume_aligned;
+      continue;
+    }
     if (opts.opt_unswitch) pass.unswitch_aliases();
     if (opts.opt_mfma_sddmm) k.body = pass.mfma_dot(k.body);
     k.body = pass.propagate_constants(k.body);

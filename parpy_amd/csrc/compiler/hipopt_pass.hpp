@@ -1,7 +1,7 @@
 // What the gfx950 memory passes share: helpers over the kernel IR and the per-kernel pass object.  The methods of
 // `Pass` are defined by concern in hipopt_control.cpp, hipopt_prefetch.cpp, hipopt_lds.cpp, hipopt_vector.cpp,
 // hipopt_regs.cpp, hipopt_keep.cpp and hipopt_alias.cpp; the rewrites that change a launch are in hipopt_launch.cpp,
-// hipopt_ragged.cpp, hipopt_timetile.cpp, hipopt_stages.cpp and hipopt_persist.cpp; hipopt.cpp holds the order in which they run.
+// hipopt_ragged.cpp, hipopt_timetile.cpp, hipopt_twosteps.cpp, hipopt_stages.cpp and hipopt_persist.cpp; hipopt.cpp holds the order in which they run.
 #pragma once
 #include <algorithm>
 #include <functional>
@@ -151,6 +151,7 @@ struct Pass {
 // ---- rewrites of the whole program (they change a launch)
 void gather_transpose(Program& p, const Options& opts, NameGen& gen);   // hipopt_launch.cpp
 void time_tile(Program& p, const Options& opts, NameGen& gen);          // hipopt_timetile.cpp
+void two_steps(Program& p, const Options& opts, NameGen& gen);          // hipopt_twosteps.cpp
 void ragged_sum(Program& p, const Options& opts, NameGen& gen);         // hipopt_ragged.cpp
 void reduction_stages(Program& p, const Options& opts, NameGen& gen);   // hipopt_stages.cpp
 void row_threads(Program& p, const Options& opts, NameGen& gen);        // hipopt_launch.cpp

@@ -749,7 +749,7 @@ struct DevicePrinter {
           ranges[x->name] = r;
         }
         std::string out = pexpr(e->args[0]) + "[" + pexpr(e->args[1]) + "]";
-        if (opts.opt_offset32 && e->args[0]->ty.mem != Mem::LDS && read_only_param(e->args[0]) && !walks_sequentially(e->args[1]) &&
+        if (opts.opt_offset32 && e->args[0]->ty.mem != Mem::LDS && (read_only_param(e->args[0]) || kernel->finished) && !walks_sequentially(e->args[1]) &&
             !(in_unrolled > 0 && (elem_bytes(e->ty.sz) < 4 || in_unaligned > 0))) {
           // An element whose byte offset provably fits 32 bits is addressed as base + 32-bit offset, the
           // form the global memory instructions take (64-bit scalar base, 32-bit per-lane offset): no
@@ -762,7 +762,9 @@ struct DevicePrinter {
           // compiler's own strength reduction and wide loads are worth more (one thread summing a row of
           // 10^5 floats: 0.7 ms against 1.1 ms).  And the elements of a vector keep it when they are one or two
           // bytes wide or the vector may start anywhere: with offsets that wrap they are only joined to one access
-          // when the vector is known to be aligned.
+          // when the vector is known to be aligned.  Kernels that store each element once, to arrays
+          // which they do not read (`finished`), have it for their stores: three to four vector instructions fewer for each
+          // (1500 steps of 16 layers of 7-mers, 16 stores in 1350 instructions: 29.5 -> 28.6 ms).
           Interval r = expr_range(e->args[1], ranges);
           int64_t eb = elem_bytes(e->ty.sz);
           if (r.known && r.lo >= 0 && r.hi * eb + eb <= (int64_t)UINT32_MAX) {
