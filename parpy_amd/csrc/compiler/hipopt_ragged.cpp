@@ -307,8 +307,6 @@ struct RaggedSum {
     const int64_t chunks = (slots + L - 1) / L;
     const int64_t K = chunks * V;                           // sums a lane holds
     if (K * words > 16) return false;
-    // elements in flight per lane: up to sixteen registers of what they select
-    const int64_t U = r.has_col ? std::max<int64_t>(2, std::min<int64_t>(8, 16 / (K * words))) : 4;
     // Subteams: two elements of an average row per lane, at least four lanes so that they share cache lines.  (100 000
     // rows of 50 non-zeros, float64: 4 / 8 / 16 / 32 / 64 lanes 53 / 47 / 40 / 38 / 45 us; 300 000 rows of 16: 41.7 us
     // on four lanes, 36.0 on eight and sixteen; 50 000 rows of 200: 110 us on 16, 94 on 64; 50 000 rows of 8 times 32
@@ -317,18 +315,29 @@ struct RaggedSum {
     auto subteams = [&](int64_t lanes) {
       return r.one_group ? 8 : std::min<int64_t>(WAVE_SIZE / lanes, std::max<int64_t>(pow2_at_least((avg + 1) / 2), r.has_col ? 1 : 4));
     };
-    const int64_t P = subteams(L), T = L * P;
     // more wavefronts than run at once
     constexpr int64_t RESIDENT = 256 * 2048;
+    // Elements in flight per lane: up to sixteen registers of what they select; four for single sums, but where many wavefronts
+    // follow each other, as many as an average row has for 32 lanes: every load of a batch is issued for all of its lanes.
+    // (100 000 rows of 33 / 40 / 50 / 64 doubles on 32 lanes, two and four: 23.5 and 27.1 us, 26.7 and 30.1, 32.5 and 34.0, 50.4
+    // and 53.6, but 40 000 of 64 20.9 and 19.4, and floats 20.1 and 20.5, 23.2 and 23.2, 29.8 and 28.1, 36.1 and 34.6.  40 000
+    // rows of 200 doubles with eight on 32 lanes 63.0, four on 64 72.7, as many floats 56.1 and 63.4, 50 000 of 200 doubles 74.9 and
+    // 83.5, of 150 61.5 and 61.7, of 150 floats 44.3 and 46.4; 60 000 of 130 doubles 65.8 and 64.4.)
+    const bool two = !r.has_col && words == 2 && subteams(L) == 32 && r.n * 32 > 7 * RESIDENT / 2, eight = !r.has_col && avg >= (words == 2 ? 160 : 128) && r.n * 64 > 4 * RESIDENT;
+    const int64_t U = r.has_col ? std::max<int64_t>(2, std::min<int64_t>(8, 16 / (K * words))) : two ? 2 : eight ? 8 : 4;
+    const int64_t P = eight ? 32 : subteams(L), T = L * P;
     const int64_t lanes0 = std::min<int64_t>(WAVE_SIZE, pow2_at_least(all_slots)), T0 = lanes0 * subteams(lanes0);   // a team of the whole row
     if ((all_slots + lanes0 - 1) / lanes0 * V * words > 16 || (r.has_col && r.tpb < r.cols)) return false;
     const bool queues = r.n * T0 > RESIDENT;
-    // (single sums: a workgroup is over with its slowest wavefront; 1024 / 512 / 256 threads 36.6 / 34.2 / 34.2 us for the 50
-    // non-zeros above, 29.9 / 28.2 / 30.2 in floats, 99.8 / 91.2 / 91.9 for 10^6 rows of 10 floats)
+    // Single sums: a workgroup is over with its slowest wavefront; 1024 / 512 / 256 threads 36.6 / 34.2 / 34.2 us for the 50
+    // non-zeros above, 29.9 / 28.2 / 30.2 in floats, 99.8 / 91.2 / 91.9 for 10^6 rows of 10 floats.  Where all wavefronts run at
+    // once: 16 000 rows of 60 floats 12.5 / 10.6 / 10.4, doubles 15.2 / 14.0 / 13.0, 20 000 of 7 floats 6.6 / 5.8 / 5.6, 10 000 of
+    // 100 10.5 / 10.5 / 10.2, 12 000 of 200 doubles 26.2 / 26.1 / 26.5; with fewer rows the shared ones count: 5000 of 100 floats
+    // 5.7 / 5.6 / 5.8, 3000 of 200 7.3 / 6.9 / 7.7, 3000 of 60 doubles 5.0 / 4.7 / 4.3.
     // Rows of columns: 512 threads, unless a row of average length is more than one batch of its team and cannot be divided into
     // slabs, whose longest rows take 1024 (7794 rows of 45 times 32 columns: 13.5 us and 12.6; 3000 of 200 times 20: 25.8 and
     // 20.2; but 100 000 of 20 times 32: 39.7 and 50.9, 58 973 of 27 times 32: 29.7 and 38.1).
-    const bool fewer = r.has_col ? wide <= 512 && (SL > 1 || 8 * avg < 7 * P * U || r.n * T0 > 4 * RESIDENT) : queues;
+    const bool fewer = r.has_col ? wide <= 512 && (SL > 1 || 8 * avg < 7 * P * U || r.n * T0 > 4 * RESIDENT) : queues || r.n > 5000;
     const int64_t tpb = fewer ? std::min<int64_t>(r.tpb, 512) : r.tpb;
     if (tpb % WAVE_SIZE != 0 || tpb < L * V || r.n * T * SL > (int64_t(1) << 30)) return false;
     const int64_t teams = tpb / T, waves = tpb / WAVE_SIZE;
@@ -423,7 +432,7 @@ struct RaggedSum {
       }());
       out.push_back(per_slot([&](const E& c) { return Stmts{mk_assign(part(c), mk_float(0.0, sty.sz))}; }));
     };
-    auto walk = [&](Stmts& out, const E& lo, const E& hi, const E& first, int64_t stride, const E& l, const std::vector<Staged>& staged = {}) {
+    auto walk = [&](Stmts& out, const E& lo, const E& hi, const E& first, int64_t stride, const E& l, int64_t U, const std::vector<Staged>& staged = {}) {
       Name b = gen.fresh(r.loop->id.s + "_b"), at = gen.fresh(r.loop->id.s + "_at");
       E bv = mk_var(b, ety), iv = mk_var(r.loop->id, ety), atv = mk_var(at, ety);
       Stmts batch;
@@ -579,7 +588,7 @@ struct RaggedSum {
         l = mk_var(ln, ity);
       }
       sums_from_zero(own);
-      walk(own, lo, hi, narrow(sub), P, l);
+      walk(own, lo, hi, narrow(sub), P, l, U);
       if (P > 1) own.push_back(team_sum(L == 1 && P == 8 ? "parpy_sum8" : "parpy_team_sum<" + std::to_string(L) + ", " + std::to_string(T) + ">"));
       Stmts f = finish_slots(l);
       if (P > 1) own.push_back(mk_if(mk_binop(BinOp::Lt, qv, iint(L), bty), f, {}));
@@ -657,7 +666,7 @@ struct RaggedSum {
           bytes += elem_bytes(e->ty.sz);
         }
       if (staged.empty() || bytes > 16) {
-        walk(body, lo, hi, narrow(sub), tpb / L, l);
+        walk(body, lo, hi, narrow(sub), tpb / L, l, std::max<int64_t>(U, r.has_col ? U : 4));
       } else {
         Name from = gen.fresh("from"), upto = gen.fresh("upto");
         E fv = mk_var(from, ety), uv = mk_var(upto, ety);
@@ -686,7 +695,7 @@ struct RaggedSum {
         piece.insert(piece.end(), put.begin(), put.end());
         piece.push_back(mk_sync());
         piece.insert(piece.end(), fetch_next.begin(), fetch_next.end());
-        walk(piece, fv, uv, narrow(sub), tpb / L, l, staged);
+        walk(piece, fv, uv, narrow(sub), tpb / L, l, U, staged);
         body.push_back(mk_for(from, lo, hi, tpb, piece, LoopPar(), r.loop->i));
       }
       if (!r.has_col) {
