@@ -28,7 +28,7 @@
 //                   transposed copy made by a tiled kernel in front of the launch;
 //   RaggedSum       sums whose bounds are data (a CSR row): teams of lanes take
 //                   the rows, whole workgroups the very long ones;
-//   LaneSplit       eight adjacent lanes share one iteration's sequential sum
+//   LaneSplit       eight adjacent lanes share one iteration's sequential sum, long rows out of large tables in slabs over the dies
 //                   over constant bounds, 16-byte pieces of each line each;
 //   Stages          reductions over several workgroups take vectors and finish in
 //                   one launch;

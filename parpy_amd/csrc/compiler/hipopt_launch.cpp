@@ -228,6 +228,10 @@ struct LaneSplit {
   NameGen& gen;
   ElemSize isz;
   static constexpr int64_t G = 8;
+  Stmts in_slabs;              // what takes the place of the launch at hand where `room` says so
+  E room;
+  std::vector<Kernel> extra;
+  std::vector<StmtP> wholes;   // their launches that add parts up
 
   LaneSplit(Program& prog, const Options& o, NameGen& g) : p(prog), opts(o), gen(g), isz(o.int_size()) {}
 
@@ -419,6 +423,221 @@ struct LaneSplit {
     return true;
   }
 
+  // `t += term` for those of the sum's iterations start * vec .. start * vec + len - 1 that lane g of a group has: every G-th vector
+  Stmts share(const S& loop, int vec, const E& term, const E& t, const E& gv, const E& start, int64_t len) {
+    const Type ity = Type::scalar(isz);
+    const Name d0 = gen.fresh(loop->id.s + "_c"), u = gen.fresh(loop->id.s + "_u");
+    // d = (start + d0 * G + g) * V + u
+    E piece = mk_binop(BinOp::Add, mk_binop(BinOp::Mul, mk_var(d0, ity), mk_int(G, isz), ity), gv, ity);
+    auto element = [&](const E& v, const E& u) {
+      return mk_binop(BinOp::Add, mk_binop(BinOp::Mul, start ? mk_binop(BinOp::Add, start, v, ity) : v, mk_int(vec, isz), ity), u, ity);
+    };
+    const S add = mk_assign(t, mk_binop(BinOp::Add, t, term, t->ty), loop->i);
+    auto inner = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(mk_for(
+        u, mk_int(0, isz), mk_int(vec, isz), 1, {mk_def(loop->id, ity, element(piece, mk_var(u, ity)), loop->i), add}, LoopPar(), loop->i)));
+    inner->unroll = true;
+    const bool whole = loop->hi->iv % vec == 0;
+    const int64_t chunk = vec * G, rounds = len / chunk, vectors = len / vec;
+    auto outer = clone(loop);
+    outer->id = d0;
+    auto part_of = [&](int64_t lanes, const Stmts& ss) {
+      return mk_if(mk_binop(BinOp::Lt, gv, mk_int(lanes, isz), Type::scalar(ElemSize::Bool)), ss, {});
+    };
+    if (!whole) inner->iv = 1;   // (rows that start at any element)
+    if (len % chunk == 0 || !whole) {
+      outer->hi = mk_int(rounds, isz);
+      outer->body = {S(inner)};
+    } else {
+      // the last round covers only part of the group: lanes whose vector starts past the end sit it out
+      outer->hi = mk_int(rounds + 1, isz);
+      outer->body = {mk_if(mk_binop(BinOp::Lt, mk_binop(BinOp::Mul, piece, mk_int(vec, isz), ity), mk_int(len, isz), Type::scalar(ElemSize::Bool)), {S(inner)}, {})};
+    }
+    Stmts body{outer};
+    if (!whole && len % chunk != 0) {
+      // whole rounds of the group, then a round that covers part of it, then what is left of a vector, an element per lane
+      if (vectors % G != 0) {
+        auto tail = clone(S(inner));
+        tail->id = gen.fresh(loop->id.s + "_u");
+        tail->body = {mk_def(loop->id, ity, start ? element(mk_binop(BinOp::Add, mk_int(rounds * G, isz), gv, ity), mk_var(tail->id, ity))
+                                                  : mk_binop(BinOp::Add, mk_int(rounds * chunk, isz), element(gv, mk_var(tail->id, ity)), ity), loop->i),
+                      add};
+        body.push_back(part_of(vectors % G, {S(tail)}));
+      }
+      if (len % vec != 0) body.push_back(part_of(len % vec, {mk_def(loop->id, ity, start ? element(mk_int(vectors, isz), gv) : mk_binop(BinOp::Add, mk_int(vectors * vec, isz), gv, ity), loop->i), add}));
+    }
+    return body;
+  }
+
+  // Sums over long rows that memory selects out of large tables, cut into slabs along the rows.  Whole rows come from the memory
+  // side: 270 MB to 2.7 GB of them at 6 to 8 TB/s.  Here a workgroup takes a slab of its rows, and the slabs are dealt out to
+  // the dies (a workgroup's number modulo 8; slabs beyond the eighth follow when all workgroups of the first eight have
+  // started), so that a die's L2 sees an eighth of the table or less: 11 to 14 TB/s.  The parts of a sum go to memory, and a
+  // second launch adds them up and does the rest of the iteration.  In microseconds, the whole call, before and after:
+  //   223 000 products over 1024 floats, 61 MB table     160 -> 113     330 000 over 1024 doubles, 75 MB     394 -> 269
+  //    80 000 over 1024 floats, 36 MB                     67 -> 48.5      46 000 over 1024 doubles, 17 MB    51.8 -> 38.2
+  //   640 000 over 512 floats, 33 MB                     183 -> 134     300 000 over 512 floats, 10 MB      66.6 -> 50.0
+  //    16 000 over 1024 doubles, 32 MB                  34.6 -> 26.2     32 000 over 1024 floats, 66 MB     51.4 -> 50.7
+  // The bounds: tables below 9 MiB gain nothing (8192 x 256 floats 55.6 -> 54.5 without the second table's passes, 1000 x 1024
+  // 26.7 -> 28.5), nor do launches that read less than 96 MiB of rows, which the added launch costs more.  Slabs are halved
+  // while theirs of the table is above 5 MiB, down to 512 bytes: four 16-byte pieces for each of eight lanes (the first product above in
+  // slabs of 1024, 512, 256 and 128 bytes 108, 86, 96 and 156, the main launches alone; 3000 rows of 4 KB, 12 MB: 49, 58, 75 and 122).
+  // Rows next to each other that select neighbouring rows would find them in L2 as they are: the program does not say.
+  static constexpr int64_t DIES = 8, SLAB_ROW = 512, SLAB_TABLE = int64_t(5) << 20, WHOLE_TABLE = int64_t(9) << 20, GATHERED = int64_t(96) << 20;
+  void slabs(const Kernel& k, const StmtP& launch, const S& root, size_t pos, int vec, const E& term) {
+    const S& loop = root->body[pos];
+    const E& acc = loop->body[0]->dst;
+    const int64_t N = root->hi->iv, K = loop->hi->iv, es = elem_bytes(acc->ty.sz), chunk = vec * G, tpb = root->map.tpb;
+    if (acc->k != Expr::Var || tpb % WAVE_SIZE != 0) return;
+    // straight iterations: definitions, the sum, definitions and stores to arrays that the sum does not read
+    std::set<Name> from_memory, read, stored;
+    auto reads = [&](const E& e) { visit_exprs(e, [&](const E& v) { if (v->k == Expr::Var) read.insert(v->name); }); };
+    for (size_t q = 0; q < root->body.size(); ++q) {
+      const S& st = root->body[q];
+      if (q == pos) { reads(term); continue; }
+      if (st->k == Stmt::Def && st->ty.is_scalar()) {
+        if (q < pos) {
+          if (st->id != acc->name && mentions(st->expr, acc->name)) return;
+          bool loads = has_load(st->expr);
+          visit_exprs(st->expr, [&](const E& v) { if (v->k == Expr::Var && from_memory.count(v->name)) loads = true; });
+          if (loads) from_memory.insert(st->id);
+          reads(st->expr);
+        }
+      } else if (q > pos && st->k == Stmt::Assign && st->dst->k == Expr::Index && st->dst->args[0]->k == Expr::Var) {
+        stored.insert(st->dst->args[0]->name);
+      } else {
+        return;
+      }
+    }
+    if (stored.empty()) return;
+    for (auto& n : stored) if (read.count(n)) return;
+    // the smallest of the tables that the rows are selected from
+    int64_t table = 0;
+    bool ok = true;
+    visit_exprs(term, [&](const E& e) {
+      if (e->k != Expr::Index || !mentions(e->args[1], loop->id)) return;
+      bool selected = false;
+      visit_exprs(e->args[1], [&](const E& v) { if (v->k == Expr::Var && from_memory.count(v->name)) selected = true; });
+      if (!selected) return;
+      int64_t bytes = elem_bytes(e->ty.sz);
+      for (int64_t d : e->dim_shape) bytes *= d;
+      if (e->dim_shape.empty() || e->ty.sz != acc->ty.sz) ok = false;
+      table = table == 0 ? bytes : std::min(table, bytes);
+    });
+    if (!ok || table <= WHOLE_TABLE || N * K * es < GATHERED) return;
+    int64_t cut = 1;
+    const int64_t chunks = (K + chunk - 1) / chunk;
+    auto divides = [&](int64_t n) { return (n - 1) * ((chunks + n - 1) / n) < chunks; };
+    while (cut < 64 && chunks * chunk * es / (2 * cut) >= SLAB_ROW && table / cut > SLAB_TABLE && divides(2 * cut)) cut *= 2;
+    if (cut == 1 || cut * N * es > (int64_t(1) << 30) || N * G * cut > (int64_t(1) << 30)) return;
+    const int64_t width = (chunks + cut - 1) / cut * chunk, last = K - (cut - 1) * width;
+
+    const Type ity = Type::scalar(isz), bty = Type::scalar(ElemSize::Bool), ety = Type::scalar(acc->ty.sz), pty = Type::pointer(acc->ty.sz);
+    auto iint = [&](int64_t v) { return mk_int(v, isz); };
+    const Name parts = gen.fresh(acc->name.s + "_parts"), slab = gen.fresh("slab"), place = gen.fresh("place"), g = gen.fresh("g"), tid = gen.fresh("t"), sum = gen.fresh(acc->name.s);
+    auto index = [&](Expr::Kind kind) {
+      auto e = std::make_shared<Expr>();
+      e->k = kind;
+      e->ty = ity;
+      e->iv = 0;
+      return E(e);
+    };
+    const E bx = index(Expr::BlockIdx), tv = mk_var(tid, ity), gv = mk_var(g, ity), sv = mk_var(sum, ety);
+    const int64_t of_group = tpb / G, groups = (N + of_group - 1) / of_group;
+    auto div = [&](const E& a, int64_t b) { return mk_binop(BinOp::FloorDiv, a, iint(b), ity); };
+    auto rem = [&](const E& a, int64_t b) { return mk_binop(BinOp::Rem, a, iint(b), ity); };
+    auto part = [&](const E& i, const E& s) { return mk_index(mk_var(parts, pty), fold_expr(mk_binop(BinOp::Add, mk_binop(BinOp::Mul, s, iint(N), ity), i, ity)), ety); };
+    Stmts top;
+    if (cut <= DIES) {
+      top.push_back(mk_def(slab, ity, rem(bx, cut)));
+      top.push_back(mk_def(place, ity, div(bx, cut)));
+    } else {
+      top.push_back(mk_def(slab, ity, mk_binop(BinOp::Add, mk_binop(BinOp::Mul, div(bx, DIES * groups), iint(DIES), ity), rem(bx, DIES), ity)));
+      top.push_back(mk_def(place, ity, rem(div(bx, DIES), groups)));
+    }
+    top.push_back(mk_def(tid, ity, index(Expr::ThreadIdx)));
+    top.push_back(mk_def(g, ity, rem(tv, G)));
+    top.push_back(mk_def(root->id, ity, mk_binop(BinOp::Add, mk_binop(BinOp::Mul, mk_var(place, ity), iint(of_group), ity), div(tv, G), ity), root->i));
+    Stmts own;
+    for (size_t q = 0; q < pos; ++q)
+      if (root->body[q]->id != acc->name) own.push_back(root->body[q]);
+    own.push_back(mk_def(sum, ety, mk_float(0.0, acc->ty.sz), loop->i));
+    const E start = mk_binop(BinOp::Mul, mk_var(slab, ity), iint(width / vec), ity);
+    const Stmts mine = share(loop, vec, term, sv, gv, start, width);
+    if (last == width) own.insert(own.end(), mine.begin(), mine.end());
+    else own.push_back(mk_if(mk_binop(BinOp::Lt, mk_var(slab, ity), iint(cut - 1), bty), mine, share(loop, vec, term, sv, gv, iint((cut - 1) * width / vec), last)));
+    own.push_back(mk_assign(sv, mk_raw("parpy_sum8(" + sum.str() + ")", ety)));
+    own.push_back(mk_if(mk_binop(BinOp::Eq, gv, iint(0), bty), {mk_assign(part(mk_var(root->id, ity), mk_var(slab, ity)), sv, loop->i)}, {}));
+    if (N % of_group == 0) top.insert(top.end(), own.begin(), own.end());
+    else top.push_back(mk_if(mk_binop(BinOp::Lt, mk_var(root->id, ity), iint(N), bty), own, {}));
+
+    Kernel sums = k;
+    sums.name = k.name + "_slabs_" + std::to_string(gen.next++);
+    sums.body = top;
+    sums.grid.x = groups * cut;
+    sums.cached_stores = true;
+
+    // the iterations once more, a thread each, with the parts in place of the sum
+    Kernel whole = k;
+    whole.name = k.name + "_whole_" + std::to_string(gen.next++);
+    auto nr = clone(root);
+    nr->map.tpb = 256;
+    nr->map.n = (N + WAVE_SIZE - 1) / WAVE_SIZE * WAVE_SIZE;
+    std::set<Name> needed{acc->name};
+    auto uses = [](const E& e, std::set<Name>& names) { if (e) visit_exprs(e, [&](const E& v) { if (v->k == Expr::Var) names.insert(v->name); }); };
+    Stmts from_last;
+    for (size_t q = root->body.size(); q-- > 0;) {
+      const S& st = root->body[q];
+      if (q == pos) {
+        for (int64_t n = cut; n-- > 0;) from_last.push_back(mk_assign(acc, mk_binop(BinOp::Add, acc, part(mk_var(root->id, ity), iint(n)), ety), loop->i));
+      } else if (st->k != Stmt::Def || needed.count(st->id)) {
+        uses(st->expr, needed);
+        uses(st->dst, needed);
+        from_last.push_back(st);
+      }
+    }
+    nr->body = Stmts(from_last.rbegin(), from_last.rend());
+    whole.body = {S(nr)};
+    whole.block.x = 256;
+    whole.grid.x = (nr->map.n + 255) / 256;
+
+    auto launch_of = [&](Kernel& kernel) {
+      auto l = std::make_shared<Stmt>(*launch);
+      l->fname = kernel.name;
+      l->grid = kernel.grid;
+      l->block = kernel.block;
+      l->args.clear();
+      std::set<Name> used;
+      visit_stmts(kernel.body, [&](const S& st) { for (const E& e : {st->dst, st->expr, st->lo, st->hi}) uses(e, used); });
+      std::vector<KernelParam> params;
+      for (size_t i = 0; i < kernel.params.size(); ++i)
+        if (used.count(kernel.params[i].id)) { params.push_back(kernel.params[i]); l->args.push_back(launch->args[i]); }
+      KernelParam q;
+      q.id = parts;
+      q.ty = pty;
+      params.push_back(q);
+      l->args.push_back(mk_var(parts, pty));
+      kernel.params = params;
+      return l;
+    };
+    auto alloc = std::make_shared<Stmt>(), give = std::make_shared<Stmt>();
+    alloc->k = Stmt::Alloc;
+    alloc->id = parts;
+    alloc->ty = ety;
+    alloc->iv = N * cut;
+    give->k = Stmt::Free;
+    give->id = parts;
+    const StmtP a = launch_of(sums), b = launch_of(whole);
+    in_slabs = {S(alloc), S(a), S(b), S(give)};
+    // (the call must not fail for the parts: what the device has left, or the fixed amount of memory of a run that may
+    // allocate nothing, may not hold them)
+    auto fits = std::make_shared<Expr>(*mk_raw("parpy_temporaries_fit(" + std::to_string(N * cut * es) + ")", bty));
+    fits->iv = N * cut * es;
+    room = fits;
+    extra.push_back(sums);
+    extra.push_back(whole);
+    wholes.push_back(b);
+  }
+
   bool apply(Kernel& k, const StmtP& launch) {
     if (k.body.size() != 1) return false;
     const S root = k.body[0];
@@ -468,7 +687,7 @@ struct LaneSplit {
     for (int q = 0; q < pos; ++q)   // other stores in front of the sum would be repeated by every lane of a group: harmless, same value
       if (root->body[q]->k == Stmt::Assign && root->body[q]->dst->k == Expr::Index && !expr_eq(root->body[q]->dst, acc)) return false;
     Type ity = Type::scalar(isz);
-    Name gi = gen.fresh(root->id.s + "_lane"), g = gen.fresh("g"), d0 = gen.fresh(loop->id.s + "_c"), u = gen.fresh(loop->id.s + "_u");
+    Name gi = gen.fresh(root->id.s + "_lane"), g = gen.fresh("g");
     E giv = mk_var(gi, ity), gv = mk_var(g, ity);
     E lane0 = mk_binop(BinOp::Eq, gv, mk_int(0, isz), Type::scalar(ElemSize::Bool));
     Stmts body;
@@ -491,51 +710,7 @@ struct LaneSplit {
       body.push_back(mk_def(tn, acc->ty, mk_float(0.0, acc->ty.sz), loop->i));
       t = mk_var(tn, acc->ty);
     }
-    // d = (d0 * G + g) * V + u
-    E d = mk_binop(BinOp::Add,
-                   mk_binop(BinOp::Mul, mk_binop(BinOp::Add, mk_binop(BinOp::Mul, mk_var(d0, ity), mk_int(G, isz), ity), gv, ity),
-                            mk_int(vec, isz), ity),
-                   mk_var(u, ity), ity);
-    Stmts ib;
-    ib.push_back(mk_def(loop->id, ity, d, loop->i));
-    ib.push_back(mk_assign(t, mk_binop(BinOp::Add, t, term, t->ty), loop->i));
-    auto inner = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(
-        mk_for(u, mk_int(0, isz), mk_int(vec, isz), 1, ib, LoopPar(), loop->i)));
-    inner->unroll = true;
-    const int64_t K = loop->hi->iv, chunk = vec * G, rounds = K / chunk, vectors = K / vec;
-    auto outer = clone(loop);
-    outer->id = d0;
-    auto part_of = [&](int64_t lanes, const Stmts& ss) {
-      return mk_if(mk_binop(BinOp::Lt, gv, mk_int(lanes, isz), Type::scalar(ElemSize::Bool)), ss, {});
-    };
-    if (K % chunk == 0) {
-      outer->hi = mk_int(rounds, isz);
-      outer->body = {S(inner)};
-      body.push_back(outer);
-    } else if (K % vec == 0) {
-      // the last round covers only part of the group: lanes whose vector starts past the end sit it out
-      outer->hi = mk_int(rounds + 1, isz);
-      E base = mk_binop(BinOp::Mul, mk_binop(BinOp::Add, mk_binop(BinOp::Mul, mk_var(d0, ity), mk_int(G, isz), ity), gv, ity),
-                        mk_int(vec, isz), ity);
-      outer->body = {mk_if(mk_binop(BinOp::Lt, base, mk_int(K, isz), Type::scalar(ElemSize::Bool)), {S(inner)}, {})};
-      body.push_back(outer);
-    } else {
-      // rows that start at any element: whole rounds of the group, then a round that covers part of it, then what is left
-      // of a vector, an element per lane
-      inner->iv = 1;
-      outer->hi = mk_int(rounds, isz);
-      outer->body = {S(inner)};
-      body.push_back(outer);
-      if (vectors % G != 0) {
-        auto tail = clone(S(inner));
-        tail->id = gen.fresh(loop->id.s + "_u");
-        tail->body = {mk_def(loop->id, ity, mk_binop(BinOp::Add, mk_int(rounds * chunk, isz),
-                                                     mk_binop(BinOp::Add, mk_binop(BinOp::Mul, gv, mk_int(vec, isz), ity), mk_var(tail->id, ity), ity), ity), loop->i),
-                      ib[1]};
-        body.push_back(part_of(vectors % G, {S(tail)}));
-      }
-      body.push_back(part_of(K % vec, {mk_def(loop->id, ity, mk_binop(BinOp::Add, mk_int(vectors * vec, isz), gv, ity), loop->i), ib[1]}));
-    }
+    for (const S& st : share(loop, vec, term, t, gv, E(), loop->hi->iv)) body.push_back(st);
     body.push_back(mk_assign(t, mk_raw("parpy_sum8(" + t->name.str() + ")", t->ty)));
     if (!elem_acc && !from_zero) body.push_back(mk_assign(acc, mk_binop(BinOp::Add, acc, t, acc->ty), loop->i));
     Stmts stores;
@@ -561,6 +736,7 @@ struct LaneSplit {
     nr->map.k = GpuMap::ThreadBlock;
     nr->map.tpb = tpb;
     nr->map.n = (N * G + WAVE_SIZE - 1) / WAVE_SIZE * WAVE_SIZE;
+    if (!one_group) slabs(k, launch, root, (size_t)pos, vec, term);
     k.body = {S(nr)};
     k.block.x = tpb;
     k.grid.x = (nr->map.n + tpb - 1) / tpb;
@@ -577,9 +753,14 @@ struct LaneSplit {
       for (auto& kk : p.kernels)
         if (kk.name == s->fname) k = &kk;
       auto ns = std::make_shared<Stmt>(*s);
+      in_slabs.clear();
       if (k && !k->opaque_body) apply(*k, ns);
-      host.push_back(ns);
+      if (in_slabs.empty()) { host.push_back(ns); continue; }
+      auto either = clone(mk_if(room, in_slabs, {ns}));
+      either->fname = "whole sums";
+      host.push_back(S(either));
     }
+    for (auto& k : extra) p.kernels.push_back(k);
     p.host = host;
   }
 };
@@ -844,7 +1025,14 @@ struct RowThreads {
 
 void row_threads(Program& p, const Options& opts, NameGen& gen) { RowThreads(p, opts, gen).run(); }
 void gather_transpose(Program& p, const Options& opts, NameGen& gen) { GatherTranspose(p, opts, gen).run(); }
-void lane_split(Program& p, const Options& opts, NameGen& gen) { LaneSplit(p, opts, gen).run(); }
+void lane_split(Program& p, const Options& opts, NameGen& gen) {
+  LaneSplit split(p, opts, gen);
+  split.run();
+  if (!opts.opt_vectorize) return;
+  for (auto& l : split.wholes)
+    for (auto& k : p.kernels)
+      if (k.name == l->fname) Coarsen(p, opts, gen).apply(k, l);
+}
 void coarsen(Program& p, const Options& opts, NameGen& gen) { Coarsen(p, opts, gen).run(); }
 
 }  // namespace hipopt
