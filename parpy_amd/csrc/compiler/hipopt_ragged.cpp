@@ -311,9 +311,12 @@ struct RaggedSum {
     // rows of 50 non-zeros, float64: 4 / 8 / 16 / 32 / 64 lanes 53 / 47 / 40 / 38 / 45 us; 300 000 rows of 16: 41.7 us
     // on four lanes, 36.0 on eight and sixteen; 50 000 rows of 200: 110 us on 16, 94 on 64; 50 000 rows of 8 times 32
     // columns: 22.4 / 17.7 / 17.4 / 20.9 us for 1 / 2 / 4 / 8 subteams.)  Rows that were the threads of one workgroup
-    // are too few to fill the chip in any case: 10.3 us on 16 lanes, 11.0 on eight.
+    // are too few to fill the chip in any case and take eight lanes, but for long ones, of which the others' round trips are what
+    // they wait for (1000 rows of 50 doubles on 8 / 16 / 32 / 64 lanes 5.1 / 4.2 / 4.0 / 4.0 us, of 100 6.9 / 5.3 / 4.5 / 4.2, of 200 11.2 /
+    // 8.0 / 6.3 / 5.6, of 200 floats 9.4 / 6.8 / 5.4 / 5.0, of 20 3.9 on any; sums of columns have lanes enough).
     auto subteams = [&](int64_t lanes) {
-      return r.one_group ? 8 : std::min<int64_t>(WAVE_SIZE / lanes, std::max<int64_t>(pow2_at_least((avg + 1) / 2), r.has_col ? 1 : 4));
+      if (r.one_group && (r.has_col || avg < 48)) return int64_t(8);
+      return std::min<int64_t>(WAVE_SIZE / lanes, std::max<int64_t>(pow2_at_least((avg + 1) / 2), r.has_col ? 1 : 4));
     };
     // more wavefronts than run at once
     constexpr int64_t RESIDENT = 256 * 2048;
@@ -355,12 +358,16 @@ struct RaggedSum {
     // 29.8 us with 148 in front, 20.0 / 15.9 / 15.3 with 256 / 512 / 1024; 1000 of 64 times 256: 12.4 / 9.1 / 8.8 with 125 / 256
     // / 512; 1045 of 10 times 256: 4.4 / 4.5 / 5.3 with 130 / 256 / 1024), but for a launch whose undivided rows fill the device
     // exactly.  Fewer single sums: one for sixteen rows where there is room beside the others (3000 rows of 60, doubles 6.3 ->
-    // 4.9 us, 5.5 with one for four; 20 000 of 30: 9.8 -> 9.0), else the queues (8000 rows of 150: 18.0 us, 20.0 with 64 in front).
+    // 4.9 us, 5.5 with one for four; 20 000 of 30: 9.8 -> 9.0), else 256 for doubles, whose others then start a little later
+    // (none / 64 / 128 / 256 / 512: 16 000 rows of 60 14.1 / 14.4 / 13.1 / 11.6 / 12.4, 15 500 of 40 10.3 / 10.2 / 8.9 / 8.5 / 9.1, 7800
+    // of 80 10.4 / 11.0 / 9.5 / 9.0 / 9.2, 8000 of 150 16.0 / 17.5 / 15.4 / 15.5 / 15.6), and for floats, which gain less, the
+    // queues of the others' workgroups (8000 rows of 150 12.7 us, 14.2 with 64 in front, 12.0 with 256).
     const int64_t room = RESIDENT / r.tpb - (r.n * T0 + r.tpb - 1) / r.tpb;
     const int64_t scouts = queues ? std::max<int64_t>(r.has_col ? 1024 : 512, (r.n * SL + 1023) / 1024)
                            : r.one_group ? 0
                            : r.has_col ? (room > 0 ? std::max(SL, std::min<int64_t>(512, r.n * avg / 160)) : 0)
                            : room >= 64 ? std::max<int64_t>(1, std::min<int64_t>(room, r.n / 16))
+                           : words == 2 ? 256
                                         : 0;
     const int64_t slices = scouts / SL;
     const int64_t looked = scouts ? (r.n + slices - 1) / slices : 0;   // rows for each of them
@@ -665,8 +672,18 @@ struct RaggedSum {
           staged.push_back({e, gen.fresh("staged")});
           bytes += elem_bytes(e->ty.sz);
         }
-      if (staged.empty() || bytes > 16) {
-        walk(body, lo, hi, narrow(sub), tpb / L, l, std::max<int64_t>(U, r.has_col ? U : 4));
+      if (!r.has_col) {
+        // Single sums: eight in flight for each thread while the row fills them (10 468 rows of 185 on average, the longest of 18 900,
+        // doubles 21.1 -> 19.9 us, floats 18.2 -> 16.4, 30 000 of 100 floats 22.0 -> 20.0), then four.  Sixteen take more registers
+        // than leave the other rows their wavefronts.
+        const Name full = gen.fresh("full");
+        const E fv = mk_var(full, ety), piece = eint(8 * tpb);
+        auto minus = [&](const E& a, const E& b) { return mk_binop(BinOp::Sub, a, b, ety); };
+        body.push_back(mk_def(full, ety, mk_binop(BinOp::Add, lo, mk_binop(BinOp::Mul, mk_binop(BinOp::FloorDiv, minus(hi, lo), piece, ety), piece, ety), ety)));
+        walk(body, lo, fv, narrow(sub), tpb, l, 8);
+        walk(body, fv, hi, narrow(sub), tpb, l, 4);
+      } else if (staged.empty() || bytes > 16) {
+        walk(body, lo, hi, narrow(sub), tpb / L, l, U);
       } else {
         Name from = gen.fresh("from"), upto = gen.fresh("upto");
         E fv = mk_var(from, ety), uv = mk_var(upto, ety);
