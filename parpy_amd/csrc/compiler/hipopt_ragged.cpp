@@ -203,8 +203,29 @@ struct RaggedSum {
     return false;
   }
 
-  // columns a lane takes side by side: 16 bytes when every access along the columns is unit-stride through an
-  // aligned parameter and rows are whole vectors
+  static int64_t average(const Rows& r) { return r.elements > 0 ? std::max<int64_t>(1, r.elements / r.n) : 32; }
+
+  // Rows that are no whole number of vectors: the last vector ends with the row, and what it shares with the one in front of it
+  // is summed and stored twice, in the same order.  Not where the end of a row reads memory: the element that one of the two has
+  // stored may be what the other reads.  A quarter of the load instructions, and as many more rows to a wavefront.  Floats, a
+  // column per lane before and four now, us: 20 000 rows of 24 times 33 / 65 / 101 / 162 / 255 columns 26.1 -> 19.7, 33.2 -> 27.7,
+  // 43.0 -> 32.0, 64.8 -> 50.8, 69.4 -> 62.9, 3000 of 40 times 33 / 65 / 101 / 199 14.6 -> 9.1, 18.3 -> 11.8, 15.0 -> 12.1, 20.5 -> 17.1,
+  // 60 000 of 6 times 17 / 65 / 101 20.9 -> 14.5, 34.2 -> 28.5, 36.2 -> 32.2.  Rows of a wavefront each gain less, and lose
+  // where they are short (60 000 of 6 times 162 46.6 -> 47.6, 255 67.5 -> 67.7; 8000 of 10 times 162 15.2 -> 16.4, but times 250
+  // 17.4 -> 15.0) or leave lanes idle (20 000 of 24 times 129 / 145
+  // 43.0 -> 45.4, 45.8 -> 47.3).  Doubles, of which the device compiler makes two loads again, stay a column per lane.
+  static bool whole_vectors_pay(const Rows& r, int64_t v) {
+    const int64_t slots = (r.cols + v - 1) / v, lanes = (slots + WAVE_SIZE - 1) / WAVE_SIZE * WAVE_SIZE;
+    if (v != 4 || r.cols < 4 * v || has_load(r.start)) return false;
+    if (slots > WAVE_SIZE / 2 && (average(r) < 8 || 1000 - 1000 * slots / lanes > (average(r) < 24 ? 130 : 420))) return false;
+    for (auto& st : r.post) {
+      if (has_load(st->expr)) return false;
+      if (st->dst && st->dst->k == Expr::Index && has_load(st->dst->args[1])) return false;
+    }
+    return true;
+  }
+
+  // columns a lane takes side by side: 16 bytes when every access along the columns is unit-stride through an aligned parameter
   int64_t column_vector(const Kernel& k, const Rows& r) {
     if (!r.has_col || !opts.assume_aligned) return 1;
     int64_t v = 0;
@@ -224,7 +245,8 @@ struct RaggedSum {
     scan(r.term);
     scan(r.acc);
     for (auto& d : r.defs) scan(d->expr);
-    return ok && v > 0 && r.cols % v == 0 ? v : 1;
+    if (!ok || v <= 0) return 1;
+    return r.cols % v == 0 || whole_vectors_pay(r, v) ? v : 1;
   }
 
   static int64_t pow2_at_least(int64_t n) { int64_t q = 1; while (q < n) q *= 2; return q; }
@@ -239,7 +261,7 @@ struct RaggedSum {
   // times 128: 50.1 (45.7) and 39.3 / 53.5; 60 000 of 20 times 64: 41.8 and 45.6; 100 000 of 4 times 256: 73.7 and 86.3.
   static int64_t slabs(const Rows& r, int64_t V, int64_t avg) {
     if (!r.has_col) return 1;
-    const int64_t slots = r.cols / V;
+    const int64_t slots = (r.cols + V - 1) / V;
     int64_t row = 0;   // bytes of a selected row
     auto scan = [&](const E& e) {
       visit_exprs(e, [&](const E& x) { if (x->k == Expr::Index && mentions(x->args[1], r.col)) row = std::max(row, r.cols * elem_bytes(x->ty.sz)); });
@@ -299,9 +321,10 @@ struct RaggedSum {
     if (!match(k, r)) return false;
     const int64_t V = column_vector(k, r);
     const int64_t words = elem_bytes(r.acc->ty.sz) / 4;
-    const int64_t avg = r.elements > 0 ? std::max<int64_t>(1, r.elements / r.n) : 32;
+    const int64_t avg = average(r);
     const int64_t SL = slabs(r, V, avg);
-    const int64_t all_slots = r.cols / V, slots = (all_slots + SL - 1) / SL;   // vectors along the columns: all, of a slab
+    const bool moved = r.cols % V != 0;                     // the last vector of columns, to end with the row
+    const int64_t all_slots = (r.cols + V - 1) / V, slots = (all_slots + SL - 1) / SL;   // vectors along the columns: all, of a slab
     const int64_t wide = slots * V;                                            // columns of a slab
     const int64_t L = std::min<int64_t>(WAVE_SIZE, pow2_at_least(slots));
     const int64_t chunks = (slots + L - 1) / L;
@@ -396,8 +419,10 @@ struct RaggedSum {
       auto loop = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(
           mk_for(c, iint(0), iint(K), 1, f(mk_var(c, ity)), LoopPar())));
       loop->unroll = true;
+      if (moved) loop->iv = 1;   // (rows that start at any element)
       return S(loop);
     };
+    auto to_end = [&](const E& first) { return moved ? mk_binop(BinOp::Min, first, iint(r.cols - V), ity) : first; };
     // the column of slot c of lane l, counted from the start of the slab
     const Name slab = SL > 1 ? gen.fresh("slab") : Name();
     E sv = mk_var(slab, ity);
@@ -413,14 +438,14 @@ struct RaggedSum {
       if (L * chunks != slots) base = mk_binop(BinOp::Min, base, iint(slots - 1), ity);
       if (SL > 1) base = add(mk_binop(BinOp::Mul, sv, iint(slots), ity), base);
       if (slots * SL != all_slots) base = mk_binop(BinOp::Min, base, iint(all_slots - 1), ity);
-      return V == 1 ? base : add(mk_binop(BinOp::Mul, base, iint(V), ity), v);
+      return V == 1 ? base : add(to_end(mk_binop(BinOp::Mul, base, iint(V), ity)), v);
     };
     // is column `at` of the slab (a number below `upto`) one, and one of the array
     auto in_slab = [&](const E& at, int64_t upto) {
       E c;
       if (upto > wide) c = mk_binop(BinOp::Lt, at, iint(wide), bty);
       if (wide * SL != r.cols) {
-        E whole = mk_binop(BinOp::Lt, add(mk_binop(BinOp::Mul, sv, iint(wide), ity), at), iint(r.cols), bty);
+        E whole = mk_binop(BinOp::Lt, SL == 1 ? at : add(mk_binop(BinOp::Mul, sv, iint(wide), ity), at), iint(r.cols), bty);
         c = c ? mk_binop(BinOp::And, c, whole, bty) : whole;
       }
       return c;
@@ -513,9 +538,16 @@ struct RaggedSum {
       if (!r.has_col) return finish(part(iint(0)));
       return Stmts{per_slot([&](const E& c) {
         // (lanes and slots past the slab's last column, or past the array's, store nothing)
-        Stmts f{mk_def(r.col, ity, fold_expr(SL == 1 ? slab_column(c, l) : add(mk_binop(BinOp::Mul, sv, iint(wide), ity), slab_column(c, l))), r.loop->i)};
+        // (of vectors that may be moved the first column tells)
+        auto of_row = [&](const E& at) { return SL == 1 ? at : add(mk_binop(BinOp::Mul, sv, iint(wide), ity), at); };
+        const E v = mk_binop(BinOp::Rem, c, iint(V), ity), own = slab_column(c, l), head = moved ? slab_column(mk_binop(BinOp::Sub, c, v, ity), l) : own;
+        Stmts f{mk_def(r.col, ity, fold_expr(moved ? add(to_end(of_row(head)), v) : of_row(own)), r.loop->i)};
         Stmts g = finish(part(c));
-        E some = in_slab(fold_expr(slab_column(c, l)), L * K);
+        E some = in_slab(fold_expr(head), L * K);
+        if (some && moved) {
+          f.insert(f.end(), g.begin(), g.end());
+          return Stmts{mk_if(some, f, {})};
+        }
         if (!some) { f.insert(f.end(), g.begin(), g.end()); return f; }
         if (SL == 1) { f.push_back(mk_if(mk_binop(BinOp::Lt, mk_var(r.col, ity), iint(r.cols), bty), g, {})); return f; }
         f.insert(f.end(), g.begin(), g.end());
@@ -746,10 +778,17 @@ struct RaggedSum {
         body.push_back(mk_sync());
         Name s = gen.fresh("whole"), w = gen.fresh("w");
         Stmts sum{mk_def(r.col, ity, SL == 1 ? tv : add(mk_binop(BinOp::Mul, sv, iint(wide), ity), tv)), mk_def(s, sty, mk_float(0.0, sty.sz))};
+        // (columns of the last vector lie where it would without having been moved)
+        E place = tv;
+        if (moved) {
+          Name at = gen.fresh("place");
+          sum.push_back(mk_def(at, ity, mk_ifexpr(mk_binop(BinOp::Lt, mk_var(r.col, ity), iint((all_slots - 1) * V), bty), tv, add(tv, iint(all_slots * V - r.cols)), ity)));
+          place = mk_var(at, ity);
+        }
         auto over = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(mk_for(
             w, iint(0), iint(waves), 1,
             {mk_assign(mk_var(s, sty), mk_binop(BinOp::Add, mk_var(s, sty),
-                                                mk_index(base, add(mk_binop(BinOp::Mul, mk_var(w, ity), iint(L * K), ity), tv), sty), sty))},
+                                                mk_index(base, add(mk_binop(BinOp::Mul, mk_var(w, ity), iint(L * K), ity), place), sty), sty))},
             LoopPar())));
         over->unroll = true;
         sum.push_back(over);
