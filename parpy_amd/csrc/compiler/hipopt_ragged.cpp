@@ -206,7 +206,8 @@ struct RaggedSum {
   static int64_t average(const Rows& r) { return r.elements > 0 ? std::max<int64_t>(1, r.elements / r.n) : 32; }
 
   // Rows that are no whole number of vectors: the last vector ends with the row, and what it shares with the one in front of it
-  // is summed and stored twice, in the same order.  Not where the end of a row reads memory: the element that one of the two has
+  // is summed and stored twice, in the same order, by lanes of one wavefront, which has read what a sum reads before it stores
+  // any.  Not where the end of a row reads memory: the element that one of the two has
   // stored may be what the other reads.  A quarter of the load instructions, and as many more rows to a wavefront.  Floats, a
   // column per lane before and four now, us: 20 000 rows of 24 times 33 / 65 / 101 / 162 / 255 columns 26.1 -> 19.7, 33.2 -> 27.7,
   // 43.0 -> 32.0, 64.8 -> 50.8, 69.4 -> 62.9, 3000 of 40 times 33 / 65 / 101 / 199 14.6 -> 9.1, 18.3 -> 11.8, 15.0 -> 12.1, 20.5 -> 17.1,
@@ -259,6 +260,8 @@ struct RaggedSum {
   // in 2 / 4 / 8, us: 20 000 of 24 times 128 columns 43.7 (33.8 on 1024 threads) and 26.3 / 27.0 (6 KB and 3 KB a wavefront);
   // 16 000 of 24 times 256: 77.9 (61.3) and 47.5 / 35.0 / 46.9; 8192 of 20 times 128: 19.1 and 11.9 / 13.7 / 22.0; 40 000 of 16
   // times 128: 50.1 (45.7) and 39.3 / 53.5; 60 000 of 20 times 64: 41.8 and 45.6; 100 000 of 4 times 256: 73.7 and 86.3.
+  // A last vector that is moved is not the first of its slab: what it shares with the one in front of it would be columns of two
+  // workgroups, and one of them may read what the other has stored (`t += A[k] * (B[cols[k], j] - E[i, j])`, `E[i, j] = t`).
   static int64_t slabs(const Rows& r, int64_t V, int64_t avg) {
     if (!r.has_col) return 1;
     const int64_t slots = (r.cols + V - 1) / V;
@@ -276,7 +279,7 @@ struct RaggedSum {
     };
     int64_t best = 1;
     for (int64_t n = 2; n <= 8 && r.cols >= 16 * n && slots >= n && r.n * WAVE_SIZE * n <= (int64_t(1) << 30) && avg * row >= 3584 * n; n *= 2)
-      if (idle(n) <= std::max<int64_t>(idle(1), 420)) best = n;
+      if (idle(n) <= std::max<int64_t>(idle(1), 420) && !(r.cols % V != 0 && (slots - 1) % ((slots + n - 1) / n) == 0)) best = n;
     return best;
   }
 

@@ -1,9 +1,10 @@
 """Sums over sparse rows times a matrix whose rows are no whole number of vectors: the last vector of a row of columns is moved to
-end with the row, alone in its slab, beside others, in the second vector of a lane; rows at the bound of the shared ones."""
+end with the row, beside others in its slab, in the second vector of a lane; rows at the bound of the shared ones."""
 import re
 
 import numpy as np
 import pytest
+import torch
 
 import parpy_amd as parpy
 from parpy_amd.compile import hiprtc_compile
@@ -24,7 +25,33 @@ def spmm_twice(A, B, C, D):
             D[i, j] = t * 2.0
 
 
-# columns: the fewest, one and three past whole vectors, one vector for the last of four and of eight slabs, two vectors a lane
+@parpy.jit
+def apart(A, B, E):
+    parpy.label('i')
+    for i in range(A["nrows"]):
+        parpy.label('j')
+        for j in range(B["ncols"]):
+            t = 0.0
+            parpy.label('k')
+            for k in range(A["rows"][i], A["rows"][i + 1]):
+                t += A["values"][k] * (B["values"][A["cols"][k], j] - E[i, j])
+            E[i, j] = t
+
+
+@parpy.jit
+def apart_into(A, B, E, F):
+    parpy.label('i')
+    for i in range(A["nrows"]):
+        parpy.label('j')
+        for j in range(B["ncols"]):
+            t = 0.0
+            parpy.label('k')
+            for k in range(A["rows"][i], A["rows"][i + 1]):
+                t += A["values"][k] * (B["values"][A["cols"][k], j] - E[i, j])
+            F[i, j] = t
+
+
+# columns: the fewest, one and three past whole vectors, last slabs of few vectors, two vectors a lane
 MOVED = [(900, 20, 17), (900, 12, 33), (2100, 60, 35), (515, 70, 101), (640, 24, 65), (700, 40, 199), (700, 40, 227), (1001, 24, 162),
          (20011, 9, 255), (640, 30, 311), (70, 3, 101)]
 # a wavefront to a row of columns and lanes or elements too few, fewer than four vectors, doubles
@@ -56,9 +83,17 @@ def test_columns_that_stay_single(n, avg, cols, dtype):
     assert not moved(text_of(spmm, n, avg, cols, dtype, 1), cols)
 
 
-def test_last_slab_of_one_vector():
-    assert slabs_in(text_of(spmm, 700, 40, 199, np.float32, 1)) == 8
-    assert slabs_in(text_of(spmm, 700, 40, 227, np.float32, 1)) == 8
+# vectors of columns that, cut into as many slabs as the row length asks for, would leave the moved one alone in the last slab
+ALONE = [(700, 45, 171), (700, 40, 199), (700, 40, 227)]
+
+
+@pytest.mark.parametrize("n,avg,cols", ALONE)
+def test_shared_columns_are_of_one_slab(n, avg, cols):
+    for fun, results in ((spmm, 1), (apart, 1), (apart_into, 2)):
+        s = text_of(fun, n, avg, cols, np.float32, results)
+        vectors = min([int(v) for v in re.findall(r"slab_\d+ \* (\d+)", s)] or [cols])   # of a slab
+        assert moved(s, cols) and slabs_in(s) > 1
+        assert (cols - 4) // (4 * vectors) == (cols - 1) // (4 * vectors)
 
 
 @pytest.mark.gpu
@@ -96,3 +131,22 @@ def test_infinities_beside_the_moved_vector():
     assert np.array_equal(np.isnan(C), np.isnan(want)) and np.array_equal(np.isinf(C), np.isinf(want))
     at = np.isfinite(want)
     assert np.abs(C[at] - want[at]).max() < 2e-6 * 60 * 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,avg,cols", ALONE)
+def test_sums_that_read_what_the_row_stores(n, avg, cols):
+    A, B = operands(n, avg, cols, np.float32)
+    E = np.random.default_rng(9).standard_normal((n, cols)).astype(np.float32)
+    weight = np.zeros(n)
+    np.add.at(weight, np.repeat(np.arange(n), np.diff(A["rows"])), A["values"].astype(np.float64))
+    want = expected(A, B) - weight[:, None] * E
+    on_gpu = lambda x: torch.from_numpy(x.copy()).cuda()
+    A, B = ({k: on_gpu(v) if isinstance(v, np.ndarray) else v for k, v in d.items()} for d in (A, B))
+    tol = 2 * 2e-6 * 60 * 8   # as above, of products up to twice the size
+    out = on_gpu(E)
+    apart(A, B, out, opts=options(n, cols))
+    assert np.abs(out.cpu().numpy() - want).max() < tol
+    out = on_gpu(E)
+    apart_into(A, B, out, out, opts=options(n, cols))
+    assert np.abs(out.cpu().numpy() - want).max() < tol
