@@ -250,6 +250,24 @@ struct RaggedSum {
     return r.cols % v == 0 || whole_vectors_pay(r, v) ? v : 1;
   }
 
+  // does a row read, in front of its columns, an array that they store, or one that may be the same memory
+  static bool reads_first(const Rows& r) {
+    std::vector<E> stored;
+    if (r.acc->k == Expr::Index) stored.push_back(r.acc);
+    for (auto& st : r.post) if (st->dst && st->dst->k == Expr::Index) stored.push_back(st->dst);
+    bool found = false;
+    auto scan = [&](const E& e) {
+      visit_exprs(e, [&](const E& x) {
+        if (x->k != Expr::Index) return;
+        for (auto& q : stored) found = found || expr_eq(x->args[0], q->args[0]) || (x->ty.sz == q->ty.sz && x->dim_shape == q->dim_shape);
+      });
+    };
+    for (auto& st : r.pre) scan(st->expr);
+    scan(r.loop->lo);
+    scan(r.loop->hi);
+    return found;
+  }
+
   static int64_t pow2_at_least(int64_t n) { int64_t q = 1; while (q < n) q *= 2; return q; }
 
   // Slabs of columns: workgroups b, b + n, b + 2n, ... sum the rows over one n-th of the columns.  Workgroups are dealt to the
@@ -261,9 +279,10 @@ struct RaggedSum {
   // 16 000 of 24 times 256: 77.9 (61.3) and 47.5 / 35.0 / 46.9; 8192 of 20 times 128: 19.1 and 11.9 / 13.7 / 22.0; 40 000 of 16
   // times 128: 50.1 (45.7) and 39.3 / 53.5; 60 000 of 20 times 64: 41.8 and 45.6; 100 000 of 4 times 256: 73.7 and 86.3.
   // A last vector that is moved is not the first of its slab: what it shares with the one in front of it would be columns of two
-  // workgroups, and one of them may read what the other has stored (`t += A[k] * (B[cols[k], j] - E[i, j])`, `E[i, j] = t`).
+  // workgroups, and one of them may read what the other has stored (`t += A[k] * (B[cols[k], j] - E[i, j])`, `E[i, j] = t`).  Nor
+  // is a row divided that reads in front of its columns what they store (`x = E[i, 0]`), under whatever name.
   static int64_t slabs(const Rows& r, int64_t V, int64_t avg) {
-    if (!r.has_col) return 1;
+    if (!r.has_col || reads_first(r)) return 1;
     const int64_t slots = (r.cols + V - 1) / V;
     int64_t row = 0;   // bytes of a selected row
     auto scan = [&](const E& e) {

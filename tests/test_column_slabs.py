@@ -4,6 +4,7 @@ import re
 
 import numpy as np
 import pytest
+import torch
 
 import parpy_amd as parpy
 from parpy_amd.compile import hiprtc_compile
@@ -35,6 +36,47 @@ def spmm_onto(A, B, C, D):
                 t += A["values"][k] * B["values"][A["cols"][k], j]
             C[i, j] = t
             D[i, j] = t * 2.0
+
+
+@parpy.jit
+def spmm_less(A, B, C, D):
+    parpy.label('i')
+    for i in range(A["nrows"]):
+        x = C[i, 0]
+        parpy.label('j')
+        for j in range(B["ncols"]):
+            t = 0.0
+            parpy.label('k')
+            for k in range(A["rows"][i], A["rows"][i + 1]):
+                t += A["values"][k] * B["values"][A["cols"][k], j]
+            D[i, j] = t - x
+
+
+@parpy.jit
+def spmm_less_kept(A, B, C):
+    parpy.label('i')
+    for i in range(A["nrows"]):
+        x = C[i, 0]
+        parpy.label('j')
+        for j in range(B["ncols"]):
+            t = 0.0
+            parpy.label('k')
+            for k in range(A["rows"][i], A["rows"][i + 1]):
+                t += A["values"][k] * B["values"][A["cols"][k], j]
+            C[i, j] = t - x
+
+
+@parpy.jit
+def spmm_scaled(A, B, w, C):
+    parpy.label('i')
+    for i in range(A["nrows"]):
+        x = w[i]
+        parpy.label('j')
+        for j in range(B["ncols"]):
+            C[i, j] = 0.0
+            parpy.label('k')
+            for k in range(A["rows"][i], A["rows"][i + 1]):
+                C[i, j] += A["values"][k] * B["values"][A["cols"][k], j] * x
 
 
 def options(n, cols):
@@ -95,3 +137,30 @@ def test_sums_in_slabs(n, avg, cols, slabs, dtype, tol):
     spmm_onto(A, B, C, D, opts=options(n, cols))
     assert np.abs(C - (want + C0)).max() < tol * 60 * 8
     assert np.array_equal(D, C * dtype(2.0))
+
+
+@pytest.mark.parametrize("n,avg,cols,slabs", SHAPES[:3])
+def test_rows_that_read_first_what_they_store(n, avg, cols, slabs):
+    A = {"values": np.zeros(n * avg, np.float32), "rows": np.arange(n + 1) * avg, "cols": np.zeros(n * avg, np.int64), "nrows": n}
+    B, C = {"values": np.zeros((99, cols), np.float32), "ncols": cols}, np.zeros((n, cols), np.float32)
+    listing = lambda fun, *args: parpy.print_compiled(fun, [A, B, *args], options(n, cols))
+    for s in (listing(spmm_less_kept, C), listing(spmm_less, C, C.copy())):
+        hiprtc_compile(s[:s.index("// host side")], options(n, cols))
+        assert slabs_in(s) == 1
+    assert slabs_in(listing(spmm_scaled, np.zeros(n, np.float32), C)) == slabs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,avg,cols,slabs", SHAPES[:3])
+def test_sums_of_rows_that_read_first(n, avg, cols, slabs):
+    A, B = operands(n, avg, cols, np.float32)
+    C0 = np.random.default_rng(9).standard_normal((n, cols)).astype(np.float32)
+    want = expected(A, B) - C0[:, :1]
+    on_gpu = lambda x: torch.from_numpy(x.copy()).cuda()
+    A, B = ({k: on_gpu(v) if isinstance(v, np.ndarray) else v for k, v in d.items()} for d in (A, B))
+    C = on_gpu(C0)
+    spmm_less_kept(A, B, C, opts=options(n, cols))
+    assert np.abs(C.cpu().numpy() - want).max() < 2e-6 * 60 * 8   # (as above)
+    C = on_gpu(C0)
+    spmm_less(A, B, C, C, opts=options(n, cols))
+    assert np.abs(C.cpu().numpy() - want).max() < 2e-6 * 60 * 8
