@@ -24,7 +24,8 @@ namespace {
 //     the launch's first or in that one; a launch of copies behind the last of them makes up for the rows that end there.
 //   * Launches come in pairs, so that the arrays are where the loop of single steps has them, and the last one to four steps
 //     run as single steps: both arrays end as they would.
-//   * The arithmetic of an element is that of the statements as written: same operations, same order.
+//   * The arithmetic of an element is that of the statements as written: same operations, same order, and the value of the step
+//     between is rounded as the store of it would.
 //
 // The step of a model of 16 layers of 16 384 states (`forward_kernel`, one thread per state of a layer, 100 rows of 1 MB that
 // fit the memory-side cache): 31 us as a launch of its own, of which a copy of the arrays takes 25.6 and the vector ALU 24; two
@@ -371,6 +372,15 @@ struct TwoSteps {
     second(false);
     if (!ok) return {};
 
+    // (a product of the first step must not become part of a sum of the second)
+    auto rounded = [&](const E& v) {
+      auto call = std::make_shared<Expr>();
+      call->k = Expr::Call;
+      call->ty = vty;
+      call->sval = "parpy_rounded";
+      call->args = {v->ty.sz == st.sz ? v : mk_convert(v, st.sz)};
+      return E(call);
+    };
     // the first step: own elements, then those of others that the second one takes
     Stmts body;
     std::map<int64_t, E> loaded;   // own elements of `from`, all of them in front
@@ -394,7 +404,7 @@ struct TwoSteps {
       set_slot(own, s);
       copy_of(own, st, st.loop->body);
       const Name n = gen.fresh("between");
-      own.out.push_back(mk_def(n, vty, own.stored));
+      own.out.push_back(mk_def(n, vty, rounded(own.stored)));
       mids.push_back(mk_var(n, vty));
       sooner.push_back(own.out);
     }
@@ -410,7 +420,7 @@ struct TwoSteps {
       copy_of(c, st, st.loop->body);
       body.insert(body.end(), c.out.begin(), c.out.end());
       const Name n = gen.fresh("between");
-      body.push_back(mk_def(n, vty, c.stored));
+      body.push_back(mk_def(n, vty, rounded(c.stored)));
       return mk_var(n, vty);
     };
     // four values, the same for four neighbouring threads and evenly apart: one for each of them

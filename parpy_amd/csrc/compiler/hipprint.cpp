@@ -319,6 +319,8 @@ __device__ __forceinline__ int parpy_mask(bool c) {
   asm("" : "+v"(m));   // (not to be turned back into a test)
   return m;
 }
+// a value as memory would hold it: a product does not become part of the sum that it goes into
+template <class T> __device__ __forceinline__ T parpy_rounded(T v) { asm("" : "+v"(v)); return v; }
 __device__ __forceinline__ int parpy_blend_bits(int m, int a, int b) { int r; asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(a), "v"(b)); return r; }
 template <class T> __device__ __forceinline__ T parpy_blend(int m, T a, T b) {
   if constexpr (sizeof(T) == 8) {

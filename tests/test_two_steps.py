@@ -57,6 +57,25 @@ def one_other(x, a, b, p, q, lens, n, steps):
 
 
 @parpy.jit
+def product_last(x, a, b, p, q, lens, n, steps):
+    """An update that ends in a product, which the next step adds to another: rounded in between."""
+    parpy.label('r')
+    for r in range(n):
+        for t in range(1, steps):
+            src = b
+            dst = a
+            if t & 1:
+                src = a
+                dst = b
+            parpy.label('s')
+            for s in range(1024):
+                if t < lens[r]:
+                    dst[r, s] = (src[r, s] + src[r, (s // 4) % 32]) * p[s // 128]
+                elif t == lens[r]:
+                    dst[r, s] = src[r, s]
+
+
+@parpy.jit
 def four_others(x, a, b, p, q, lens, n, steps):
     """Four elements of others, not evenly apart: half of a thread's own, too many to compute again."""
     parpy.label('r')
@@ -137,7 +156,7 @@ def arguments(steps, lens, dtype, seed=1):
             rng.standard_normal(8).astype(dtype), rng.standard_normal((6, 128)).astype(dtype), np.array(lens, np.int64), R, steps]
 
 
-@pytest.mark.parametrize("fn,joined", [(quads, True), (one_other, True), (four_others, False), (looked_up, False), (cut_short, False), (goes_on, False)])
+@pytest.mark.parametrize("fn,joined", [(quads, True), (one_other, True), (product_last, True), (four_others, False), (looked_up, False), (cut_short, False), (goes_on, False)])
 def test_which_loops(fn, joined):
     s = parpy.print_compiled(fn, arguments(40, [40] * R, np.float32), options())
     hiprtc_compile(s[:s.index("// host side")], options())
@@ -147,6 +166,13 @@ def test_which_loops(fn, joined):
         s = parpy.print_compiled(fn, arguments(steps, [steps] * R, np.float32), options())
         assert "_two_steps_" not in s
     assert "_two_steps_" not in parpy.print_compiled(fn, arguments(40, [40] * R, np.float32), options(opt_tile_steps=False))
+
+
+@pytest.mark.parametrize("fn", [quads, one_other, product_last])
+def test_values_between_are_rounded(fn):
+    s = parpy.print_compiled(fn, arguments(40, [40] * R, np.float32), options())
+    between = re.findall(r"float between_\d+ = (\w+)", s)
+    assert len(between) > 8 and set(between) <= {"parpy_rounded", "parpy_dpp"}
 
 
 def test_arrays_that_overlap_run_as_single_steps():
@@ -167,9 +193,10 @@ def test_rows_end_everywhere(steps, dtype):
     ends += [steps] * (-len(ends) % R)
     for q in range(0, len(ends), R):
         got, want = arguments(steps, ends[q:q + R], dtype), arguments(steps, ends[q:q + R], dtype)
-        quads(*got, opts=options())
-        quads(*want, opts=options(opt_tile_steps=False))
-        assert np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2]), (steps, ends[q:q + R])
+        for fn in (quads, product_last):
+            fn(*got, opts=options())
+            fn(*want, opts=options(opt_tile_steps=False))
+            assert np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2]), (steps, ends[q:q + R])
 
 
 @pytest.mark.gpu
