@@ -372,8 +372,10 @@ struct TwoSteps {
     second(false);
     if (!ok) return {};
 
-    // (a product of the first step must not become part of a sum of the second)
+    // (A product of the first step must not become part of a sum of the second.  What ends in a sum is left alone, since no
+    // operation takes one in: kept apart all the same, 1500 steps of 16 layers of 7-mers take 29.6 ms instead of 29.1.)
     auto rounded = [&](const E& v) {
+      if (v->k == Expr::BinOpE && (v->bop == BinOp::Add || v->bop == BinOp::Sub) && v->ty.sz == st.sz) return v;
       auto call = std::make_shared<Expr>();
       call->k = Expr::Call;
       call->ty = vty;

@@ -168,11 +168,13 @@ def test_which_loops(fn, joined):
     assert "_two_steps_" not in parpy.print_compiled(fn, arguments(40, [40] * R, np.float32), options(opt_tile_steps=False))
 
 
-@pytest.mark.parametrize("fn", [quads, one_other, product_last])
-def test_values_between_are_rounded(fn):
+@pytest.mark.parametrize("fn,product", [(quads, False), (product_last, True)])
+def test_products_between_are_rounded(fn, product):
     s = parpy.print_compiled(fn, arguments(40, [40] * R, np.float32), options())
-    between = re.findall(r"float between_\d+ = (\w+)", s)
-    assert len(between) > 8 and set(between) <= {"parpy_rounded", "parpy_dpp"}
+    between = re.findall(r"float between_\d+ = (.*);", s)
+    assert len(between) > 8
+    for value in between:
+        assert value.startswith("parpy_dpp<") or value.startswith("parpy_rounded(") == product
 
 
 def test_arrays_that_overlap_run_as_single_steps():
