@@ -526,10 +526,13 @@ struct TimeTile {
       ss.push_back(mk_for(s, mk_int(0, ElemSize::I32), mk_var(count.id, Type::scalar(ElemSize::I32)), 1, step, LoopPar()));
       const int64_t outer = margin / Es;
       if (!any) {
-        const std::string l = lost.str();
+        // (elements outside the arrays may be NaN, quotients of the zeros that stand there)
+        const std::string l = lost.str(), place = at.str() + " + e";
         ss.push_back(mk_rawstmt("bool " + l + " = false;"));
         for (auto& a : arrays)
-          if (a.written) ss.push_back(mk_rawstmt("for (int e = 0; e < " + std::to_string(Es) + "; ++e) " + l + " = " + l + " || " + reg[a.host].str() + "[e] != " + reg[a.host].str() + "[e];"));
+          if (a.written)
+            ss.push_back(mk_rawstmt("for (int e = 0; e < " + std::to_string(Es) + "; ++e) " + l + " = " + l + " || (" + reg[a.host].str() + "[e] != " + reg[a.host].str() + "[e]" +
+                                    (edge ? " && " + place + " >= 0 && " + place + " < " + std::to_string(a.n) : "") + ");"));
         ss.push_back(mk_rawstmt("if (__builtin_amdgcn_ballot_w64(" + l + " && " + lane.str() + " >= " + std::to_string(outer) + " && " + lane.str() + " < " + std::to_string(WAVE_SIZE - outer) + ") == 0) {"));
       }
       Stmts put, put_kept;

@@ -1,5 +1,7 @@
 """Stretches of time loops whose divisions by constants leave infinite dividends out: what would have been infinite is NaN at
 the end and the stretch is computed again, so the results are those of one launch per update, bit for bit."""
+import re
+
 import numpy as np
 import pytest
 
@@ -28,6 +30,15 @@ def coefficients(A, B, K, n, steps):
         parpy.label('N')
         for i in range(n - 1):
             A[i] = B[i + 1] / 6.0
+
+
+def weighted(A, B, K, n, steps):
+    """A division by an element, which is 0 / 0 outside the arrays."""
+    for t in range(steps):
+        parpy.label('N')
+        B[1:-1] = (A[:-2] + A[2:]) / 3.0 / K[1:-1]
+        parpy.label('N')
+        A[1:-1] = (B[:-2] + B[2:]) / 3.0 / K[1:-1]
 
 
 def largest(A, B, K, n, steps):
@@ -69,9 +80,17 @@ def test_which_updates_leave_infinities_out(fn, left_out):
     assert (", false>(" in s[s.index('extern "C"'):]) == left_out
 
 
+def test_nan_outside_the_arrays_does_not_count():
+    n = 5003
+    s = parpy.print_compiled(parpy.jit(weighted), [np.zeros(n, np.float32) for _ in range(3)] + [n, 20], options(n))
+    tests = re.findall(r"(\w+_r_\d+)\[e\] != \1\[e\](.*)\);", s)   # of A and B, in the stretches inside and in those at the ends
+    bounds = re.compile(rf" && at_\d+ \+ e >= 0 && at_\d+ \+ e < {n}")
+    assert [t[1] == "" for t in tests] == [True, True, False, False] and all(bounds.fullmatch(t[1]) for t in tests[2:])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
-@pytest.mark.parametrize("fn", [averages, coefficients, largest, chosen])
+@pytest.mark.parametrize("fn", [averages, coefficients, weighted, largest, chosen])
 def test_infinities_and_nan(fn, dtype):
     f = parpy.jit(fn)
     rng = np.random.default_rng(17)
