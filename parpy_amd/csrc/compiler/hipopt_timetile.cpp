@@ -28,7 +28,8 @@ namespace {
 //     written in whole lines; a wavefront's part of LDS is its own, without barriers.
 //   * At the ends of the arrays an update covers a part of a stretch: there the new value is blended with the old one under
 //     a mask kept in a register, for the elements of a lane that may be such.
-//   * Divisions by constants leave infinite dividends out where a NaN at the end shows them; such a stretch is computed again.
+//   * Divisions by constants leave infinite dividends out where a NaN at the end shows them; such a stretch is computed again,
+//     one that loads infinities or NaN without them from the start.
 //
 // A three-point average back and forth over 10^6 float64 elements, 98 updates, two launches of 25 steps: 447 us as launches
 // of 4.5 us each, 45.6 on eight elements per lane with their own accesses and a division of four instructions one of which
@@ -391,10 +392,14 @@ struct TimeTile {
       return both(le(iint(from), g), lt(g, iint(to)));
     };
 
-    // Stretches whose results hold no NaN keep them, the others are computed again with the tests of the ends and divisions of
-    // any dividend.  Steps of two three-point averages before this and the masks for some elements only, with this, and with
-    // both: 98 updates of 10^6 doubles 39.1, 32.7 and 31.6 us, 198 of 4 * 10^6 doubles 228, 190 and 183, of as many floats 153,
-    // 114 and 109, 118 of 1500 doubles 13.5, 11.7 and 10.6.
+    // Stretches whose results hold no NaN keep them, the others are computed again with divisions of any dividend; those that
+    // load a NaN or an infinity are computed with these from the start.  98 updates of 10^6 doubles that are all NaN: 39.6 us
+    // with divisions of any dividend alone, 63.0 with one attempt for all and the tests of the ends when it was in vain, 36.4 as
+    // it is; with a NaN in every 10 000 40.0, 47.7 and 35.0, of 300 000 doubles, 58 updates, 11.8, 14.4 and 12.4; with none 41.8,
+    // 30.6 and 30.3.  Short launches pay up to 0.1 us each for the look at what they load.
+    // Steps of two three-point averages before this and the masks for some elements only, with this, and with both: 98 updates of
+    // 10^6 doubles 39.1, 32.7 and 31.6 us, 198 of 4 * 10^6 doubles 228, 190 and 183, of as many floats 153, 114 and 109, 118 of
+    // 1500 doubles 13.5, 11.7 and 10.6.
     bool divides = false, nan_stays = true;
     for (auto& u : ups)
       for (auto& st : u.body) nan_stays = nan_stays && is_float(st->k == Stmt::Def ? st->ty.sz : st->dst->ty.sz) && carries_nan(st->expr, &divides);
@@ -426,6 +431,8 @@ struct TimeTile {
     // is one of the elements from .. to - 1 element e of its lane
     auto some_of = [&](int64_t from, int64_t to, int64_t e) { return from < to && (e - from % Es + Es) % Es < to - from; };
 
+    auto no_number = [&](const Arr& a) { return "parpy_no_number<" + std::to_string(Es) + ">(" + reg[a.host].str() + ")"; };
+
     // the path of a stretch: `edge` tests every element against the bounds of the arrays and of the updates
     // (`any`: with divisions of any dividend)
     auto path = [&](bool edge, bool any) {
@@ -440,6 +447,12 @@ struct TimeTile {
           S ld = mk_assign(slot(a, e), elem(a.host, a, e));
           ss.push_back(!edge ? ld : mk_if(within(e, 0, a.n), {ld}, {mk_assign(slot(a, e), is_float(a.sz) ? mk_float(0.0, a.sz) : mk_int(0, a.sz))}));
         }
+      }
+      if (!any) {
+        // (not for values that are no numbers to begin with)
+        std::string some = "false";
+        for (auto& a : arrays) if (is_float(a.sz) && !scratch.count(a.host)) some += " || " + no_number(a);
+        ss.push_back(mk_rawstmt("if (__builtin_amdgcn_ballot_w64(" + some + ") == 0) {"));
       }
       Stmts step, masks;
       std::vector<std::pair<std::vector<int64_t>, E>> known;
@@ -531,8 +544,9 @@ struct TimeTile {
         ss.push_back(mk_rawstmt("bool " + l + " = false;"));
         for (auto& a : arrays)
           if (a.written)
-            ss.push_back(mk_rawstmt("for (int e = 0; e < " + std::to_string(Es) + "; ++e) " + l + " = " + l + " || (" + reg[a.host].str() + "[e] != " + reg[a.host].str() + "[e]" +
-                                    (edge ? " && " + place + " >= 0 && " + place + " < " + std::to_string(a.n) : "") + ");"));
+            ss.push_back(mk_rawstmt(!edge ? l + " = " + l + " || " + no_number(a) + ";" :
+                                    "for (int e = 0; e < " + std::to_string(Es) + "; ++e) " + l + " = " + l + " || (" + reg[a.host].str() + "[e] != " + reg[a.host].str() + "[e] && " +
+                                    place + " >= 0 && " + place + " < " + std::to_string(a.n) + ");"));
         ss.push_back(mk_rawstmt("if (__builtin_amdgcn_ballot_w64(" + l + " && " + lane.str() + " >= " + std::to_string(outer) + " && " + lane.str() + " < " + std::to_string(WAVE_SIZE - outer) + ") == 0) {"));
       }
       Stmts put, put_kept;
@@ -550,17 +564,14 @@ struct TimeTile {
       }
       if (!put_kept.empty()) put.push_back(mk_if(mk_raw(keep.id.str(), bty), put_kept, {}));
       if (!put.empty()) ss.push_back(mk_if(both(le(iint(outer), lv), lt(lv, iint(WAVE_SIZE - outer))), put, {}));
-      if (!any) ss.push_back(mk_rawstmt("return; }"));
+      if (!any) ss.push_back(mk_rawstmt("return; } }"));
       return ss;
     };
     // A stretch that lies inside all bounds takes the plain path.  Values next to the bounds of a stretch are wrong (its
     // outermost lanes have no neighbour) and stay within the margin.
     E inside = both(le(iint(lo), start), le(add(start, iint(width)), iint(hi)));
     top.push_back(mk_if(inside, path(false, !hopeful), path(true, !hopeful)));
-    if (hopeful) {
-      const Stmts again = path(true, true);
-      top.insert(top.end(), again.begin(), again.end());
-    }
+    if (hopeful) top.push_back(mk_if(inside, path(false, true), path(true, true)));
     f.body = top;
     p.kernels.push_back(f);
 

@@ -319,6 +319,16 @@ __device__ __forceinline__ int parpy_mask(bool c) {
   asm("" : "+v"(m));   // (not to be turned back into a test)
   return m;
 }
+// is one of the values an infinity or NaN: zero times such a one is NaN
+template <int N, class T> __device__ __forceinline__ bool parpy_no_number(const T* v) {
+  T z[2] = {0, 0};
+  #pragma unroll
+  for (int e = 0; e < N; ++e) {
+    if constexpr (sizeof(T) == 8) z[e % 2] = __builtin_fma(v[e], 0.0, z[e % 2]);
+    else z[e % 2] = __builtin_fmaf(v[e], 0.0f, z[e % 2]);
+  }
+  return !(z[0] + z[1] == 0);
+}
 // a value as memory would hold it: a product does not become part of the sum that it goes into
 template <class T> __device__ __forceinline__ T parpy_rounded(T v) { asm("" : "+v"(v)); return v; }
 __device__ __forceinline__ int parpy_blend_bits(int m, int a, int b) { int r; asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(a), "v"(b)); return r; }

@@ -83,9 +83,21 @@ def test_which_updates_leave_infinities_out(fn, left_out):
 def test_nan_outside_the_arrays_does_not_count():
     n = 5003
     s = parpy.print_compiled(parpy.jit(weighted), [np.zeros(n, np.float32) for _ in range(3)] + [n, 20], options(n))
-    tests = re.findall(r"(\w+_r_\d+)\[e\] != \1\[e\](.*)\);", s)   # of A and B, in the stretches inside and in those at the ends
+    tests = re.findall(r"(\w)_r_\d+\[e\] != \1_r_\d+\[e\](.*)\);", s)   # in the stretches at the ends
     bounds = re.compile(rf" && at_\d+ \+ e >= 0 && at_\d+ \+ e < {n}")
-    assert [t[1] == "" for t in tests] == [True, True, False, False] and all(bounds.fullmatch(t[1]) for t in tests[2:])
+    assert sorted(t[0] for t in tests) == ["A", "B"] and all(bounds.fullmatch(t[1]) for t in tests)
+
+
+def test_what_is_no_number_from_the_start():
+    n = 200000
+    s = parpy.print_compiled(parpy.jit(averages), [np.zeros(n) for _ in range(3)] + [n, 40], options(n))
+    # the array that is loaded is looked at, B is not, inside and at the ends
+    assert re.findall(r"ballot_w64\(false(?: \|\| parpy_no_number<\d>\((\w)_r_\d+\))*\) == 0", s) == ["A", "A"]
+    # then divisions of any dividend, inside without the tests of the ends
+    parts = s[s.index('extern "C"'):s.index("// host side")].split("return; }")
+    assert len(parts) == 3 and all(", false>(" in p for p in parts[:2]) and ", false>(" not in parts[2]
+    inside, ends = re.split(r"\n  \} else \{", parts[2])
+    assert "parpy_div_const<" in inside and "parpy_blend" not in inside and "parpy_blend" in ends
 
 
 @pytest.mark.gpu
