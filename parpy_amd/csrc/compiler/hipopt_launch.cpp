@@ -121,43 +121,73 @@ struct GatherTranspose {
     return k;
   }
 
+  // the matrices that a launch reads in this way, rows of their copies on cache lines where `pitch` says so
+  std::map<Name, Cand> candidates(const Kernel& k) {
+    std::map<Name, Cand> cands;
+    std::set<Name> written;
+    visit_stmts(k.body, [&](const S& st) {
+      if (st->k == Stmt::Assign && st->dst->k == Expr::Index)
+        visit_exprs(st->dst->args[0], [&](const E& x) { if (x->k == Expr::Var) written.insert(x->name); });
+      if ((st->k == Stmt::Def && !st->ty.is_scalar()) || (st->k == Stmt::Assign && st->dst->k == Expr::Var && !st->dst->ty.is_scalar()))
+        visit_exprs(st->expr, [&](const E& x) { if (x->k == Expr::Var) written.insert(x->name); });  // aliased: leave alone
+    });
+    for (auto& q : k.params)
+      if (q.ty.is_pointer() && !written.count(q.id)) { Cand c; c.arr = q.id; cands[q.id] = c; }
+    std::vector<std::pair<Name, int64_t>> seq_loops;
+    scan(k.body, seq_loops, cands);
+    std::map<Name, Cand> out;
+    for (auto& kv : cands) {
+      Cand c = kv.second;
+      // worth it when the stride is at least a cache line and the matrix is re-read many times
+      if (!c.ok || !c.seen || c.N < 32 || c.K < 8 || c.K * c.N * elem_bytes(c.sz) > (int64_t(1) << 30)) continue;
+      const int64_t line = CACHE_LINE / elem_bytes(c.sz);
+      c.pitch = tiles(c) && c.K >= 8 * line ? (c.K + line - 1) / line * line : c.K;
+      out[kv.first] = c;
+    }
+    return out;
+  }
+
+  // Rows of the copies start on cache lines where they are longer than eight of them: eight lanes that read 128 bytes of a row
+  // then ask for one line, not for two (2500 rows of 1000 doubles, 50 000 products 51.7 -> 42.5 us, 9000 of 780 floats, 270 000:
+  // 119 -> 107, 12 000 of 331 doubles, 720 000: 262 -> 253; shorter rows do not repay the lines that are added: 8192 of 97
+  // floats 30.6 -> 31.4).
+  // A run that may allocate nothing has a fixed amount of memory for the program's temporaries at a time, and a captured one
+  // what the plan keeps for all of them: where they fit without the lines they fit with them.
+  static bool lines_fit(int64_t plain, int64_t lined, int64_t others, int64_t of_program) {
+    return of_program <= KEPT_MEMORY && (plain > FIXED_MEMORY || others + lined <= FIXED_MEMORY / 8 * 7);
+  }
+
   void run() {
     Stmts host;
     std::vector<Kernel> extra;
-    for (auto& s : p.host) {
-      if (s->k != Stmt::Launch) { host.push_back(s); continue; }
+    auto kernel_of = [&](const S& s) -> Kernel* {
+      if (s->k != Stmt::Launch) return nullptr;
       Kernel* k = nullptr;
       for (auto& kk : p.kernels)
         if (kk.name == s->fname) k = &kk;
+      return k;
+    };
+    const int64_t others = temporaries(p.host);
+    auto bytes_of = [](const Cand& c, int64_t pitch) { return (pitch * c.N * elem_bytes(c.sz) + 255) / 256 * 256; };
+    int64_t of_program = others;
+    for (auto& s : p.host)
+      if (const Kernel* k = kernel_of(s))
+        for (auto& kv : candidates(*k)) of_program += bytes_of(kv.second, kv.second.pitch);
+    for (auto& s : p.host) {
+      Kernel* k = kernel_of(s);
       if (!k) { host.push_back(s); continue; }
-      std::map<Name, Cand> cands;
-      std::set<Name> written;
-      visit_stmts(k->body, [&](const S& st) {
-        if (st->k == Stmt::Assign && st->dst->k == Expr::Index)
-          visit_exprs(st->dst->args[0], [&](const E& x) { if (x->k == Expr::Var) written.insert(x->name); });
-        if ((st->k == Stmt::Def && !st->ty.is_scalar()) || (st->k == Stmt::Assign && st->dst->k == Expr::Var && !st->dst->ty.is_scalar()))
-          visit_exprs(st->expr, [&](const E& x) { if (x->k == Expr::Var) written.insert(x->name); });  // aliased: leave alone
-      });
-      for (auto& q : k->params)
-        if (q.ty.is_pointer() && !written.count(q.id)) { Cand c; c.arr = q.id; cands[q.id] = c; }
-      std::vector<std::pair<Name, int64_t>> seq_loops;
-      scan(k->body, seq_loops, cands);
+      std::map<Name, Cand> cands = candidates(*k);
       std::map<Name, Name> staged;
       Stmts pre, post;
-      int64_t copied = 0;
+      int64_t plain = 0, lined = 0;
+      for (auto& kv : cands) {
+        plain += bytes_of(kv.second, kv.second.K);
+        lined += bytes_of(kv.second, kv.second.pitch);
+      }
+      const bool lines = lines_fit(plain, lined, others, of_program);
       for (auto& kv : cands) {
         Cand& c = kv.second;
-        // worth it when the stride is at least a cache line and the matrix is re-read many times
-        if (!c.ok || !c.seen || c.N < 32 || c.K < 8 || c.K * c.N * elem_bytes(c.sz) > (int64_t(1) << 30)) continue;
-        // Rows of the copy start on cache lines where they are longer than eight of them: eight lanes that read 128 bytes of a
-        // row then ask for one line, not for two (2500 rows of 1000 doubles, 50 000 products 51.7 -> 42.5 us, 9000 of 780 floats,
-        // 270 000: 119 -> 107, 12 000 of 331 doubles, 720 000: 262 -> 253; shorter rows do not repay the lines that are added:
-        // 8192 of 97 floats 30.6 -> 31.4).
-        // (A run that may allocate nothing has a fixed amount of memory: what fits there without the lines fits with them.)
-        const int64_t es = elem_bytes(c.sz), line = CACHE_LINE / es, padded = (c.K + line - 1) / line * line;
-        const bool pad = tiles(c) && c.K >= 8 * line && (c.K * c.N * es > FIXED_MEMORY || copied + padded * c.N * es <= FIXED_MEMORY / 8 * 7);
-        c.pitch = pad ? padded : c.K;
-        copied += c.pitch * c.N * es;
+        if (!lines) c.pitch = c.K;
         Name xt = gen.fresh(c.arr.s + "_T");
         staged[c.arr] = xt;
         auto a = std::make_shared<Stmt>();
@@ -182,7 +212,7 @@ struct GatherTranspose {
         auto f = std::make_shared<Stmt>();
         f->k = Stmt::Free;
         f->id = xt;
-        post.push_back(f);
+        post.insert(post.begin(), f);   // (the last one first, as fixed memory is given back)
       }
       if (staged.empty()) { host.push_back(s); continue; }
       Type ity = Type::scalar(isz);

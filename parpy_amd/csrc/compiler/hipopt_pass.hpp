@@ -33,6 +33,10 @@ E subst_vars(const E& e, const std::map<Name, E>& m);
 // no array which is written can be reached under another name: address ranges of every such pair; null when there is none.
 struct HostArray { Name name; int64_t bytes = 0; bool written = false; };
 E arrays_disjoint(const Program& p, const std::vector<HostArray>& arrays);
+// Bytes of all temporaries that a program makes, and what a plan keeps of them from one run to the next: what it does not keep
+// cannot be had inside a graph capture.
+int64_t temporaries(const Stmts& host);
+constexpr int64_t KEPT_MEMORY = int64_t(1) << 30;
 
 template <class F> E rewrite_expr(const E& e, F f) {  // bottom-up rewrite
   if (!e) return e;

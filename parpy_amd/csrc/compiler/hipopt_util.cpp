@@ -77,5 +77,11 @@ E arrays_disjoint(const Program& p, const std::vector<HostArray>& arrays) {
   return all;
 }
 
+int64_t temporaries(const Stmts& host) {
+  int64_t bytes = 0;
+  visit_stmts(host, [&](const S& s) { if (s->k == Stmt::Alloc) bytes += (s->iv * elem_bytes(s->ty.sz) + 255) / 256 * 256; });
+  return bytes;
+}
+
 }  // namespace hipopt
 }  // namespace parpy

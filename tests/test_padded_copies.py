@@ -44,6 +44,56 @@ def test_copies_that_fit_stay_so():
         assert bytes_copied(listing(n, k, 900, "float32")) == n * pitch * 4
 
 
+@parpy.jit
+def gathered(X, Y, Z, cols, out, n, k):
+    parpy.label('nnz')
+    for i in range(n):
+        c = cols[i]
+        t = 0.0
+        for d in range(k):
+            t += X[d, c] * Y[d, c]
+        out[i] = t
+    parpy.label('nnz')
+    for i in range(n):
+        c = cols[i]
+        t = 0.0
+        for d in range(k):
+            t += Z[d, c]
+        out[i] += t
+
+
+def plan_of(k, x, y, z):
+    f = lambda n: np.zeros((k, n), np.float32)
+    return parpy.print_compiled(gathered, [f(x), f(y), f(z), np.zeros(900, np.int64), np.zeros(900, np.float32), 900, k], options(900))
+
+
+def most_at_once(s):
+    """Bytes in use at most where only the last temporary gives its place back before the run ends, and all bytes."""
+    live, top, most, total = [], 0, 0, 0
+    for name, size, freed in re.findall(r"(\w+) = \(\w+\*\)parpy_alloc_buffer\((\d+)\)|parpy_free_buffer\((\w+)\)", s):
+        if freed and live[-1][0] == freed:
+            top = live.pop()[1]
+        elif not freed:
+            live.append((name, top))
+            top = -(-top // 256) * 256 + int(size)
+            most, total = max(most, top), total + int(size)
+    return most, total
+
+
+# columns of two tables that one launch copies and of the next launch's; what is added to their rows of 260 elements
+@pytest.mark.parametrize("x,y,z,added", [(5000, 5000, 9900, 28), (7800, 7700, 5000, (0, 28)), (5000, 5000, 5000, 28), (420000, 420000, 150000, 0)])
+def test_copies_of_several_tables(x, y, z, added):
+    s, k = plan_of(260, x, y, z), 260
+    sizes = {m[0]: int(m[1]) for m in re.findall(r"([XYZ])_T_\d+ = \(float\*\)parpy_alloc_buffer\((\d+)\)", s)}
+    first, second = added if isinstance(added, tuple) else (added, added)
+    assert sizes == {"X": 4 * x * (k + first), "Y": 4 * y * (k + first), "Z": 4 * z * (k + second)}
+    most, total = most_at_once(s)
+    if 4 * k * (x + y) + 512 <= 16 << 20 and 4 * k * z <= 16 << 20:
+        assert most <= 16 << 20     # what a run that allocates nothing has
+    if 4 * k * (x + y + z) <= 1 << 30:
+        assert total <= 1 << 30     # what a plan keeps for captured runs
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("k,n,dtype,pitch", SHAPES)
 def test_products_out_of_a_copy(k, n, dtype, pitch):
