@@ -262,6 +262,7 @@ struct LaneSplit {
   E room;
   std::vector<Kernel> extra;
   std::vector<StmtP> wholes;   // their launches that add parts up
+  int64_t taken = 0;           // bytes of the program's temporaries
 
   LaneSplit(Program& prog, const Options& o, NameGen& g) : p(prog), opts(o), gen(g), isz(o.int_size()) {}
 
@@ -558,7 +559,8 @@ struct LaneSplit {
     const int64_t chunks = (K + chunk - 1) / chunk;
     auto divides = [&](int64_t n) { return (n - 1) * ((chunks + n - 1) / n) < chunks; };
     while (cut < 64 && chunks * chunk * es / (2 * cut) >= SLAB_ROW && table / cut > SLAB_TABLE && divides(2 * cut)) cut *= 2;
-    if (cut == 1 || cut * N * es > (int64_t(1) << 30) || N * G * cut > (int64_t(1) << 30)) return;
+    if (cut == 1 || taken + cut * N * es > KEPT_MEMORY || N * G * cut > (int64_t(1) << 30)) return;
+    taken += cut * N * es;
     const int64_t width = (chunks + cut - 1) / cut * chunk, last = K - (cut - 1) * width;
 
     const Type ity = Type::scalar(isz), bty = Type::scalar(ElemSize::Bool), ety = Type::scalar(acc->ty.sz), pty = Type::pointer(acc->ty.sz);
@@ -777,6 +779,7 @@ struct LaneSplit {
 
   void run() {
     Stmts host;
+    taken = temporaries(p.host);
     for (auto& s : p.host) {
       if (s->k != Stmt::Launch) { host.push_back(s); continue; }
       Kernel* k = nullptr;

@@ -57,6 +57,12 @@ def test_slabs_of_a_shape(n, k, nnz, dtype, slabs):
         assert re.search(rf"\(slab_\d+ \* {width}\)", s) and (slabs - 1) * width * vec < k
 
 
+def test_parts_beyond_what_a_plan_keeps():
+    # 16 * 10^6 products in eight slabs: parts of 488 MiB, beside a copy of 391 MiB and one of 781 (zeros that are never touched)
+    assert slabs_in(listing(100000, 1024, 16000000, "float32")) == 8
+    assert slabs_in(listing(200000, 1024, 16000000, "float32")) == 1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tpb", [256, 64])
 @pytest.mark.parametrize("n,k,nnz,dtype,slabs", SHAPES)
