@@ -1,8 +1,8 @@
 // Options of a call, built without the interpreter: `threads(n)` and `par({...})`.
 //
 // Programs write `opts=parpy.par({'i': parpy.threads(n), ...})` where the call stands, so two or three small objects are
-// made per call.  The Python statements of it take 0.5 us of the 3.9 us that a call on 10 x 1000 floats takes, 2.6 of which are
-// the launch; these take 0.2 (3.92 -> 3.58 us).  What is not plainly an int, or a dict of strings and LoopPar, goes to the Python
+// made per call.  The Python statements of it take 0.52 us of the 4.06 us that a call on 10 x 1000 floats takes, 2.6 of which are
+// the launch; these take 0.23 (the call 3.74 us: medians of 25 times 4000 calls of each kind in turn, half of them within 0.02).  What is not plainly an int, or a dict of strings and LoopPar, goes to the Python
 // functions, which decide and report everything.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>

@@ -74,3 +74,13 @@ def test_without_the_extension_the_python_functions_stay(monkeypatch):
     monkeypatch.setattr(fastopts._buildstamp, "ensure_current", missing)
     threads, par = object(), object()
     assert fastopts.faster(LoopPar, 1024, CompileOptions, threads, par) == (threads, par)
+
+
+def test_without_the_extension(monkeypatch):
+    """A folder that cannot be written: no compiler is started, the functions stay as they are and a warning says so."""
+    functions = object(), object()
+    monkeypatch.setattr(fastopts.os, "access", lambda path, mode: False)
+    monkeypatch.setattr(fastopts._buildstamp, "is_current", lambda *args: False)
+    monkeypatch.setattr(fastopts.subprocess, "run", lambda *args, **kw: pytest.fail("a compiler was started"))
+    with pytest.warns(RuntimeWarning, match="cannot be written"):
+        assert fastopts.faster(LoopPar, 1024, CompileOptions, *functions) == functions
