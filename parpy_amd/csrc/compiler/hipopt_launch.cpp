@@ -308,6 +308,138 @@ struct LaneSplit {
     return true;
   }
 
+  static constexpr int64_t ROW_REGISTERS = 48, L2_OF_A_DIE = int64_t(4) << 20;   // (registers for 16 bytes per lane and round of three rows)
+
+  // the two rows of a product: the one that neighbouring iterations may have in common, and the other
+  bool rows_of(const S& loop, const E& term, E* common, E* other, bool* swapped) {
+    const E& acc = loop->body[0]->dst;
+    if (!(term->k == Expr::BinOpE && term->bop == BinOp::Mul)) return false;
+    E x = term->args[0], y = term->args[1];
+    for (const E& e : {x, y})
+      if (e->k != Expr::Index || e->args[0]->k != Expr::Var || e->ty.sz != acc->ty.sz || !mentions(e->args[1], loop->id) || has_load(e->args[1])) return false;
+    // (in common: of the array that the program passes, where the other is a copy made for this launch)
+    auto passed = [&](const E& e) {
+      for (auto& q : p.entry_params) if (q.id == e->args[0]->name) return true;
+      return false;
+    };
+    *swapped = !passed(x) && passed(y);
+    *common = *swapped ? y : x;
+    *other = *swapped ? x : y;
+    return true;
+  }
+
+  // The products of iterations `fv` and the one behind it over `len` elements of two rows, from vector `start` of them on (from the
+  // first where it is null): `names` of each iteration's values, `sum` of its products in all lanes.  Where that is no whole
+  // number of rounds of the group, it ends with the rows: their last vector is moved to end there, and what it has of the one in
+  // front of it and what lies behind counts as zero.
+  Stmts two_sums(const S& root, size_t pos, int vec, const E& x, const E& y, bool swapped, const E& fv, const E& gv, const E& start, int64_t len,
+                 std::map<Name, E>* names, Name* sum) {
+    const S& loop = root->body[pos];
+    const E& acc = loop->body[0]->dst;
+    const int64_t N = root->hi->iv, K = loop->hi->iv;
+    const Type ity = Type::scalar(isz), bty = Type::scalar(ElemSize::Bool), ety = Type::scalar(acc->ty.sz);
+    auto iint = [&](int64_t v) { return mk_int(v, isz); };
+    auto add = [&](const E& a, const E& b) { return mk_binop(BinOp::Add, a, b, ity); };
+    auto mul = [&](const E& a, int64_t b) { return mk_binop(BinOp::Mul, a, iint(b), ity); };
+    Stmts body;
+    auto reg = [&](const Name& name, const E& c) {
+      auto e = std::make_shared<Expr>();
+      e->k = Expr::RegElem;
+      e->ty = ety;
+      e->name = name;
+      e->args = {c};
+      return E(e);
+    };
+    auto unrolled = [&](const Name& id, int64_t n, const Stmts& ss) {
+      auto l = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(mk_for(id, iint(0), iint(n), 1, ss, LoopPar(), loop->i)));
+      l->unroll = true;
+      return l;
+    };
+    // Pieces of as many rounds as registers hold of three rows.  The place of each follows from the sums of the one in front of it
+    // as far as the device compiler can tell, which would load them all in front otherwise (eight rounds of doubles in 135 registers,
+    // 83 so) and in a loop lose track of which elements are one vector.  Two rounds of doubles, which leave a SIMD more
+    // wavefronts (300 000 products over 900 doubles 193 us, 214 with four, over 1024 114.5 and 115.8).
+    const int64_t chunk = vec * G, rounds = (len + chunk - 1) / chunk, most = ROW_REGISTERS / 12, of_piece = rounds <= most ? rounds : vec == 2 ? 2 : most;
+    const bool single = rounds <= of_piece;
+    auto declare = [&](const Name& name) {
+      auto d = std::make_shared<Stmt>();
+      d->k = Stmt::RegDecl;
+      d->id = name;
+      d->ty = ety;
+      d->iv = of_piece * vec;
+      body.push_back(S(d));
+    };
+    for (int u = 0; u < 2; ++u) {
+      Name i = gen.fresh(root->id.s);
+      E at = u == 0 ? fv : add(fv, iint(1));
+      if (u == 1 && N % 2 != 0) at = mk_binop(BinOp::Min, at, iint(N - 1), ity);   // (the last one again, not stored)
+      body.push_back(mk_def(i, ity, at, root->i));
+      names[u][root->id] = mk_var(i, ity);
+      sum[u] = gen.fresh(acc->name.s);
+      for (size_t q = 0; q < pos; ++q) {
+        const S& st = root->body[q];
+        const bool total = st->id == acc->name;
+        Name n = total ? sum[u] : gen.fresh(st->id.s);
+        E e = total ? mk_float(0.0, acc->ty.sz) : subst_vars(st->expr, names[u]);
+        names[u][st->id] = mk_var(n, st->ty);
+        body.push_back(mk_def(n, st->ty, e, st->i));
+      }
+    }
+    Name xs = gen.fresh("row"), ys[2] = {gen.fresh("other"), gen.fresh("other")};
+    declare(xs);
+    declare(ys[0]);
+    declare(ys[1]);
+    auto total = [&](int u) { return mk_assign(mk_var(sum[u], ety), mk_raw("parpy_sum8(" + sum[u].str() + ")", ety)); };
+    // `n` rounds behind the first `from`; `ends`: the rows end in the last of them
+    auto piece = [&](const E& from, int64_t n, bool ends) {
+      Stmts ss;
+      // the first element of round c's vector, and where it stands
+      auto vector = [&](const E& c) {
+        E v = add(mul(c, G), gv);
+        if (from) v = add(mul(from, G), v);
+        return mul(start ? add(start, v) : v, vec);
+      };
+      auto place = [&](const E& c) { return ends ? mk_binop(BinOp::Min, vector(c), iint(K - vec), ity) : vector(c); };
+      // the group's pieces of a row into registers
+      auto load = [&](const Name& name, const E& e) {
+        Name c = gen.fresh("c"), u = gen.fresh(loop->id.s + "_u"), d = gen.fresh(loop->id.s);
+        auto each = unrolled(u, vec, {mk_def(d, ity, add(place(mk_var(c, ity)), mk_var(u, ity)), loop->i),
+                                      mk_assign(reg(name, add(mul(mk_var(c, ity), vec), mk_var(u, ity))), subst_vars(e, {{loop->id, mk_var(d, ity)}}))});
+        if (K % vec != 0) each->iv = 1;   // (rows that start at any element)
+        return S(unrolled(c, n, {S(each)}));
+      };
+      ss.push_back(load(xs, subst_vars(x, names[0])));
+      for (int u = 0; u < 2; ++u) ss.push_back(load(ys[u], subst_vars(y, names[u])));
+      for (int u = 0; u < 2; ++u) {
+        if (u == 1) {
+          E a = subst_vars(subst_vars(x, names[0])->args[1], {{loop->id, iint(0)}}), b = subst_vars(subst_vars(x, names[1])->args[1], {{loop->id, iint(0)}});
+          ss.push_back(mk_if(mk_binop(BinOp::Neq, fold_expr(a), fold_expr(b), bty), {load(xs, subst_vars(x, names[1]))}, {}));
+        }
+        Name c = gen.fresh("c");
+        const E cv = mk_var(c, ity), sv = mk_var(sum[u], ety);
+        E l = reg(xs, cv), r = reg(ys[u], cv);
+        if (swapped) std::swap(l, r);
+        E product = mk_binop(BinOp::Mul, l, r, ety);
+        if (ends) {
+          const E round = mk_binop(BinOp::FloorDiv, cv, iint(vec), ity);
+          const E own = mk_binop(BinOp::Geq, add(place(round), mk_binop(BinOp::Rem, cv, iint(vec), ity)), vector(round), bty);
+          product = mk_ifexpr(own, product, mk_float(0.0, acc->ty.sz), ety);
+        }
+        ss.push_back(S(unrolled(c, n * vec, {mk_assign(sv, mk_binop(BinOp::Add, sv, product, ety), loop->i)})));
+        if (single) ss.push_back(total(u));
+      }
+      return ss;
+    };
+    for (int64_t from = 0; from < rounds; from += of_piece) {
+      const int64_t n = std::min(of_piece, rounds - from);
+      if (from > 0) body.push_back(mk_rawstmt("asm(\"\" : \"+v\"(" + gv->name.str() + "), \"+v\"(" + sum[0].str() + "), \"+v\"(" + sum[1].str() + "));"));
+      const Stmts ss = piece(from > 0 ? iint(from) : E(), n, len % chunk != 0 && from + n == rounds);
+      body.insert(body.end(), ss.begin(), ss.end());
+    }
+    if (!single) for (int u = 0; u < 2; ++u) body.push_back(total(u));
+    return body;
+  }
+
   // Two neighbouring iterations per group for products of two short rows, `t += X[a*K + d] * Y[b*K + d]` with a and b from
   // memory.  Neighbours mostly have one row in common (non-zeros sorted by rows or columns): the group loads it once and
   // tests whether the second iteration's is another one; a quarter of the 16-byte pieces that pass through L1 go away.
@@ -316,23 +448,14 @@ struct LaneSplit {
   // round, and 48 registers of them leave a SIMD its wavefronts: not for rows of more than 512 bytes (256 floats: 37.4 ->
   // 43.1).  Nor for tables that the 4 MiB L2 of a die does not hold, where the pieces come from farther than L1 anyway (8 MiB:
   // 43.9 -> 45.7), nor for launches that run at once as they are.
-  static constexpr int64_t ROW_REGISTERS = 48, L2_OF_A_DIE = int64_t(4) << 20;
   bool pair(Kernel& k, const StmtP& launch, const S& root, size_t pos, int vec, const E& term) {
     const S& loop = root->body[pos];
     const E& acc = loop->body[0]->dst;
     const int64_t N = root->hi->iv, K = loop->hi->iv, rounds = K / (vec * G);
     if (acc->k != Expr::Var || K % (vec * G) != 0 || 3 * rounds * 4 > ROW_REGISTERS || N * G <= 2 * 256 * 2048) return false;
-    if (!(term->k == Expr::BinOpE && term->bop == BinOp::Mul)) return false;
-    E x = term->args[0], y = term->args[1];
-    for (const E& e : {x, y})
-      if (e->k != Expr::Index || e->args[0]->k != Expr::Var || e->ty.sz != acc->ty.sz || !mentions(e->args[1], loop->id) || has_load(e->args[1])) return false;
-    // the row in common: of the array that the program passes, where the other is a copy made for this launch
-    auto passed = [&](const E& e) {
-      for (auto& q : p.entry_params) if (q.id == e->args[0]->name) return true;
-      return false;
-    };
-    const bool swapped = !passed(x) && passed(y);
-    if (swapped) std::swap(x, y);
+    E x, y;
+    bool swapped = false;
+    if (!rows_of(loop, term, &x, &y, &swapped)) return false;
     int64_t table = elem_bytes(y->ty.sz);
     for (int64_t d : y->dim_shape) table *= d;
     if (y->dim_shape.empty() || table > L2_OF_A_DIE) return false;
@@ -354,77 +477,16 @@ struct LaneSplit {
     auto selected = [&](const E& e) { bool f = false; visit_exprs(e->args[1], [&](const E& v) { if (v->k == Expr::Var && from_memory.count(v->name)) f = true; }); return f; };
     if (!zero || !stores || !selected(x) || !selected(y)) return false;
 
-    const Type ity = Type::scalar(isz), bty = Type::scalar(ElemSize::Bool), ety = Type::scalar(acc->ty.sz);
+    const Type ity = Type::scalar(isz), bty = Type::scalar(ElemSize::Bool);
     Name lane = gen.fresh(root->id.s + "_lane"), g = gen.fresh("g"), first = gen.fresh(root->id.s + "_pair");
     E gv = mk_var(g, ity), fv = mk_var(first, ity);
     Stmts body;
     body.push_back(mk_def(first, ity, mk_binop(BinOp::Mul, mk_binop(BinOp::FloorDiv, mk_var(lane, ity), mk_int(G, isz), ity), mk_int(2, isz), ity), root->i));
     body.push_back(mk_def(g, ity, mk_binop(BinOp::Rem, mk_var(lane, ity), mk_int(G, isz), ity), root->i));
-    auto reg = [&](const Name& name, const E& c) {
-      auto e = std::make_shared<Expr>();
-      e->k = Expr::RegElem;
-      e->ty = ety;
-      e->name = name;
-      e->args = {c};
-      return E(e);
-    };
-    // the group's pieces of a row into registers
-    auto load = [&](const Name& name, const E& e) {
-      Name c = gen.fresh("c"), u = gen.fresh(loop->id.s + "_u"), d = gen.fresh(loop->id.s);
-      E at = mk_binop(BinOp::Add, mk_binop(BinOp::Mul, mk_binop(BinOp::Add, mk_binop(BinOp::Mul, mk_var(c, ity), mk_int(G, isz), ity), gv, ity), mk_int(vec, isz), ity), mk_var(u, ity), ity);
-      E slot = mk_binop(BinOp::Add, mk_binop(BinOp::Mul, mk_var(c, ity), mk_int(vec, isz), ity), mk_var(u, ity), ity);
-      auto unrolled = [&](const Name& id, int64_t n, const Stmts& ss) {
-        auto l = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(mk_for(id, mk_int(0, isz), mk_int(n, isz), 1, ss, LoopPar(), loop->i)));
-        l->unroll = true;
-        return S(l);
-      };
-      return unrolled(c, rounds, {unrolled(u, vec, {mk_def(d, ity, at, loop->i), mk_assign(reg(name, slot), subst_vars(e, {{loop->id, mk_var(d, ity)}}))})});
-    };
-    auto declare = [&](const Name& name) {
-      auto d = std::make_shared<Stmt>();
-      d->k = Stmt::RegDecl;
-      d->id = name;
-      d->ty = ety;
-      d->iv = rounds * vec;
-      body.push_back(S(d));
-    };
     std::map<Name, E> names[2];
     Name sum[2];
-    for (int u = 0; u < 2; ++u) {
-      Name i = gen.fresh(root->id.s);
-      E at = u == 0 ? fv : mk_binop(BinOp::Add, fv, mk_int(1, isz), ity);
-      if (u == 1 && N % 2 != 0) at = mk_binop(BinOp::Min, at, mk_int(N - 1, isz), ity);   // (the last one again, not stored)
-      body.push_back(mk_def(i, ity, at, root->i));
-      names[u][root->id] = mk_var(i, ity);
-      sum[u] = gen.fresh(acc->name.s);
-      for (size_t q = 0; q < pos; ++q) {
-        const S& st = root->body[q];
-        Name n = st->id == acc->name ? sum[u] : gen.fresh(st->id.s);
-        E e = subst_vars(st->expr, names[u]);
-        names[u][st->id] = mk_var(n, st->ty);
-        body.push_back(mk_def(n, st->ty, e, st->i));
-      }
-    }
-    Name xs = gen.fresh("row"), ys[2] = {gen.fresh("other"), gen.fresh("other")};
-    declare(xs);
-    declare(ys[0]);
-    declare(ys[1]);
-    body.push_back(load(xs, subst_vars(x, names[0])));
-    for (int u = 0; u < 2; ++u) body.push_back(load(ys[u], subst_vars(y, names[u])));
-    for (int u = 0; u < 2; ++u) {
-      if (u == 1) {
-        E a = subst_vars(subst_vars(x, names[0])->args[1], {{loop->id, mk_int(0, isz)}}), b = subst_vars(subst_vars(x, names[1])->args[1], {{loop->id, mk_int(0, isz)}});
-        body.push_back(mk_if(mk_binop(BinOp::Neq, fold_expr(a), fold_expr(b), bty), {load(xs, subst_vars(x, names[1]))}, {}));
-      }
-      Name c = gen.fresh("c");
-      E sv = mk_var(sum[u], ety), l = reg(xs, mk_var(c, ity)), r = reg(ys[u], mk_var(c, ity));
-      if (swapped) std::swap(l, r);
-      auto add = std::const_pointer_cast<Stmt>(std::static_pointer_cast<const Stmt>(mk_for(
-          c, mk_int(0, isz), mk_int(rounds * vec, isz), 1, {mk_assign(sv, mk_binop(BinOp::Add, sv, mk_binop(BinOp::Mul, l, r, ety), ety), loop->i)}, LoopPar(), loop->i)));
-      add->unroll = true;
-      body.push_back(S(add));
-      body.push_back(mk_assign(sv, mk_raw("parpy_sum8(" + sum[u].str() + ")", ety)));
-    }
+    const Stmts sums = two_sums(root, pos, vec, x, y, swapped, fv, gv, E(), K, names, sum);
+    body.insert(body.end(), sums.begin(), sums.end());
     for (int u = 0; u < 2; ++u) {
       Stmts ss;
       for (size_t q = pos + 1; q < root->body.size(); ++q) {
@@ -503,16 +565,26 @@ struct LaneSplit {
   // side: 270 MB to 2.7 GB of them at 6 to 8 TB/s.  Here a workgroup takes a slab of its rows, and the slabs are dealt out to
   // the dies (a workgroup's number modulo 8; slabs beyond the eighth follow when all workgroups of the first eight have
   // started), so that a die's L2 sees an eighth of the table or less: 11 to 14 TB/s.  The parts of a sum go to memory, and a
-  // second launch adds them up and does the rest of the iteration.  In microseconds, the whole call, before and after:
-  //   223 000 products over 1024 floats, 61 MB table     160 -> 113     330 000 over 1024 doubles, 75 MB     394 -> 269
-  //    80 000 over 1024 floats, 36 MB                     67 -> 48.5      46 000 over 1024 doubles, 17 MB    51.8 -> 38.2
-  //   640 000 over 512 floats, 33 MB                     183 -> 134     300 000 over 512 floats, 10 MB      66.6 -> 50.0
-  //    16 000 over 1024 doubles, 32 MB                  34.6 -> 26.2     32 000 over 1024 floats, 66 MB     51.4 -> 50.7
+  // second launch adds them up and does the rest of the iteration.  A group of lanes takes two iterations, which mostly have a row
+  // in common, as above.  Microseconds of the whole call, in one piece, in slabs an iteration at a time, and so; masks whose
+  // columns lie anywhere, and within 32 of the row:
+  //   225 000 products over 1024 floats, 61 MB table     157, 104, 104       94,  80,  74
+  //    81 000 over 1024 floats, 37 MB                     62,  41,  41       51,  37,  36
+  //   640 000 over 512 floats, 33 MB                     178, 127, 125       85,  95,  78
+  //   300 000 over 512 floats, 10 MB                      66,  52,  48       43,  46,  39
+  //   300 000 over 1024 floats, 12 MB                    122,  86,  73       76,  80,  65
+  //   300 000 over 777 floats, 16 MB                     114,  89,  83       64,  79,  66
+  //   324 000 over 1024 doubles, 74 MB                   383, 244, 202      170, 232, 178
+  //   324 000 over 1000 doubles, 72 MB                   386, 256, 190      177, 192, 173
+  //   300 000 over 900 doubles, 43 MB                    293, 191, 163      145, 189, 139
+  //    16 000 over 1024 doubles, 131 MB                   94,  81,  82       99,  78,  79
+  // Rows next to each other that select neighbouring rows find them in L2 as they are, which the program does not say: there the
+  // requests to L1 are what bounds it (77 % of its cycles, counted), and a row in common is a quarter of them.
   // The bounds: tables below 9 MiB gain nothing (8192 x 256 floats 55.6 -> 54.5 without the second table's passes, 1000 x 1024
   // 26.7 -> 28.5), nor do launches that read less than 96 MiB of rows, which the added launch costs more.  Slabs are halved
-  // while theirs of the table is above 5 MiB, down to 512 bytes: four 16-byte pieces for each of eight lanes (the first product above in
-  // slabs of 1024, 512, 256 and 128 bytes 108, 86, 96 and 156, the main launches alone; 3000 rows of 4 KB, 12 MB: 49, 58, 75 and 122).
-  // Rows next to each other that select neighbouring rows would find them in L2 as they are: the program does not say.
+  // while theirs of the table is above 5 MiB, down to 512 bytes on average, a sixteenth less will do: four 16-byte pieces for each of
+  // eight lanes (the first product above in slabs of 1024, 512, 256 and 128 bytes 108, 86, 96 and 156, the main launches alone; 3000 rows
+  // of 4 KB, 12 MB: 49, 58, 75 and 122).
   static constexpr int64_t DIES = 8, SLAB_ROW = 512, SLAB_TABLE = int64_t(5) << 20, WHOLE_TABLE = int64_t(9) << 20, GATHERED = int64_t(96) << 20;
   void slabs(const Kernel& k, const StmtP& launch, const S& root, size_t pos, int vec, const E& term) {
     const S& loop = root->body[pos];
@@ -558,14 +630,14 @@ struct LaneSplit {
     int64_t cut = 1;
     const int64_t chunks = (K + chunk - 1) / chunk;
     auto divides = [&](int64_t n) { return (n - 1) * ((chunks + n - 1) / n) < chunks; };
-    while (cut < 64 && chunks * chunk * es / (2 * cut) >= SLAB_ROW && table / cut > SLAB_TABLE && divides(2 * cut)) cut *= 2;
+    while (cut < 64 && chunks * chunk * es / (2 * cut) >= SLAB_ROW / 16 * 15 && table / cut > SLAB_TABLE && divides(2 * cut)) cut *= 2;
     if (cut == 1 || taken + cut * N * es > KEPT_MEMORY || N * G * cut > (int64_t(1) << 30)) return;
     taken += cut * N * es;
     const int64_t width = (chunks + cut - 1) / cut * chunk, last = K - (cut - 1) * width;
 
     const Type ity = Type::scalar(isz), bty = Type::scalar(ElemSize::Bool), ety = Type::scalar(acc->ty.sz), pty = Type::pointer(acc->ty.sz);
     auto iint = [&](int64_t v) { return mk_int(v, isz); };
-    const Name parts = gen.fresh(acc->name.s + "_parts"), slab = gen.fresh("slab"), place = gen.fresh("place"), g = gen.fresh("g"), tid = gen.fresh("t"), sum = gen.fresh(acc->name.s);
+    const Name parts = gen.fresh(acc->name.s + "_parts"), slab = gen.fresh("slab"), place = gen.fresh("place"), g = gen.fresh("g"), tid = gen.fresh("t");
     auto index = [&](Expr::Kind kind) {
       auto e = std::make_shared<Expr>();
       e->k = kind;
@@ -573,8 +645,12 @@ struct LaneSplit {
       e->iv = 0;
       return E(e);
     };
-    const E bx = index(Expr::BlockIdx), tv = mk_var(tid, ity), gv = mk_var(g, ity), sv = mk_var(sum, ety);
-    const int64_t of_group = tpb / G, groups = (N + of_group - 1) / of_group;
+    const E bx = index(Expr::BlockIdx), tv = mk_var(tid, ity), gv = mk_var(g, ity);
+    // two products to a group of lanes, as above
+    E x, y;
+    bool swapped = false;
+    const bool twice = width / chunk <= 32 && rows_of(loop, term, &x, &y, &swapped);   // (written out)
+    const int64_t of_group = tpb / G * (twice ? 2 : 1), groups = (N + of_group - 1) / of_group;
     auto div = [&](const E& a, int64_t b) { return mk_binop(BinOp::FloorDiv, a, iint(b), ity); };
     auto rem = [&](const E& a, int64_t b) { return mk_binop(BinOp::Rem, a, iint(b), ity); };
     auto part = [&](const E& i, const E& s) { return mk_index(mk_var(parts, pty), fold_expr(mk_binop(BinOp::Add, mk_binop(BinOp::Mul, s, iint(N), ity), i, ity)), ety); };
@@ -588,17 +664,35 @@ struct LaneSplit {
     }
     top.push_back(mk_def(tid, ity, index(Expr::ThreadIdx)));
     top.push_back(mk_def(g, ity, rem(tv, G)));
-    top.push_back(mk_def(root->id, ity, mk_binop(BinOp::Add, mk_binop(BinOp::Mul, mk_var(place, ity), iint(of_group), ity), div(tv, G), ity), root->i));
-    Stmts own;
-    for (size_t q = 0; q < pos; ++q)
-      if (root->body[q]->id != acc->name) own.push_back(root->body[q]);
-    own.push_back(mk_def(sum, ety, mk_float(0.0, acc->ty.sz), loop->i));
-    const E start = mk_binop(BinOp::Mul, mk_var(slab, ity), iint(width / vec), ity);
-    const Stmts mine = share(loop, vec, term, sv, gv, start, width);
-    if (last == width) own.insert(own.end(), mine.begin(), mine.end());
-    else own.push_back(mk_if(mk_binop(BinOp::Lt, mk_var(slab, ity), iint(cut - 1), bty), mine, share(loop, vec, term, sv, gv, iint((cut - 1) * width / vec), last)));
-    own.push_back(mk_assign(sv, mk_raw("parpy_sum8(" + sum.str() + ")", ety)));
-    own.push_back(mk_if(mk_binop(BinOp::Eq, gv, iint(0), bty), {mk_assign(part(mk_var(root->id, ity), mk_var(slab, ity)), sv, loop->i)}, {}));
+    const E team = div(tv, G);
+    top.push_back(mk_def(root->id, ity, mk_binop(BinOp::Add, mk_binop(BinOp::Mul, mk_var(place, ity), iint(of_group), ity), twice ? mk_binop(BinOp::Mul, team, iint(2), ity) : team, ity), root->i));
+    const E first = mk_var(root->id, ity);
+    // the slab that starts with vector `from`, `len` elements of it
+    auto sum_of = [&](const E& from, int64_t len) {
+      Stmts ss;
+      if (twice) {
+        std::map<Name, E> names[2];
+        Name sums[2];
+        ss = two_sums(root, pos, vec, x, y, swapped, first, gv, from, len, names, sums);
+        for (int u = 0; u < 2; ++u) {
+          E mine = mk_binop(BinOp::Eq, gv, iint(u), bty);
+          if (u == 1 && N % 2 != 0) mine = mk_binop(BinOp::And, mine, mk_binop(BinOp::Lt, first, iint(N - 1), bty), bty);
+          ss.push_back(mk_if(mine, {mk_assign(part(u == 0 ? first : mk_binop(BinOp::Add, first, iint(1), ity), mk_var(slab, ity)), mk_var(sums[u], ety), loop->i)}, {}));
+        }
+        return ss;
+      }
+      const Name sum = gen.fresh(acc->name.s);
+      const E sv = mk_var(sum, ety);
+      for (size_t q = 0; q < pos; ++q)
+        if (root->body[q]->id != acc->name) ss.push_back(root->body[q]);
+      ss.push_back(mk_def(sum, ety, mk_float(0.0, acc->ty.sz), loop->i));
+      for (const S& st : share(loop, vec, term, sv, gv, from, len)) ss.push_back(st);
+      ss.push_back(mk_assign(sv, mk_raw("parpy_sum8(" + sum.str() + ")", ety)));
+      ss.push_back(mk_if(mk_binop(BinOp::Eq, gv, iint(0), bty), {mk_assign(part(first, mk_var(slab, ity)), sv, loop->i)}, {}));
+      return ss;
+    };
+    Stmts own = sum_of(mk_binop(BinOp::Mul, mk_var(slab, ity), iint(width / vec), ity), width);
+    if (last != width) own = {mk_if(mk_binop(BinOp::Lt, mk_var(slab, ity), iint(cut - 1), bty), own, sum_of(iint((cut - 1) * width / vec), last))};
     if (N % of_group == 0) top.insert(top.end(), own.begin(), own.end());
     else top.push_back(mk_if(mk_binop(BinOp::Lt, mk_var(root->id, ity), iint(N), bty), own, {}));
 
@@ -607,6 +701,7 @@ struct LaneSplit {
     sums.body = top;
     sums.grid.x = groups * cut;
     sums.cached_stores = true;
+    sums.read_once.clear();   // (by every slab)
 
     // the iterations once more, a thread each, with the parts in place of the sum
     Kernel whole = k;

@@ -39,9 +39,9 @@ def listing(n, k, nnz, dtype, to=lambda x: x, **flags):
 
 
 def slabs_in(text):
-    sums = re.search(r"_slabs_\d+<<<dim3\((\d+), 1, 1\), dim3\((\d+)", text)
+    parts = re.search(r"(float|double)\* t_parts_\d+ = \(\w+\*\)parpy_alloc_buffer\((\d+)\)", text)
     products = re.search(r"t_parts_\d+\[\(\(slab_\d+ \* (\d+)\)", text)
-    return int(sums.group(1)) // -(-int(products.group(1)) * 8 // int(sums.group(2))) if sums else 1
+    return int(parts.group(2)) // ((4 if parts.group(1) == "float" else 8) * int(products.group(1))) if parts else 1
 
 
 @pytest.mark.parametrize("n,k,nnz,dtype,slabs", SHAPES)
@@ -89,6 +89,26 @@ def test_products_in_slabs(n, k, nnz, dtype, slabs, tpb):
     assert (err[0] <= bound).all()
     # and no less exact than one thread's sum over the whole row
     assert np.sqrt((err[0] ** 2).mean()) <= np.sqrt((err[1] ** 2).mean())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k,nnz,dtype", [(5300, 1024, 25011, "float32"), (6000, 777, 33003, "float32"), (9000, 331, 39001, "float64"), (5300, 1021, 25011, "float32")])
+def test_infinities_where_slabs_meet(n, k, nnz, dtype):
+    """Elements that another slab's last vector holds as well, or that stand in front of a moved one, count once and in their own row."""
+    A, B, rows, cols, vals = operands(n, k, nnz, dtype)
+    A[:] = B[:] = 1.0
+    at = [0, 1, k // 8, k // 4 - 1, k // 4, k // 2, k - 5, k - 4, k - 3, k - 2, k - 1]
+    for q, d in enumerate(at):
+        A[10 * q, d], A[10 * q + 1, d], B[d, 10 * q] = np.inf, np.nan, 3.0
+    dev = [torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (A, B, rows, cols, vals)]
+    D = torch.full((nnz,), -7.0, dtype=dev[0].dtype, device="cuda")
+    one = np.dtype(dtype).type
+    W.sddmm_coo(dev[0], dev[1], {"rows": dev[2], "cols": dev[3], "values": torch.zeros_like(dev[4]), "nnz": nnz}, D, one(1.0), one(0.0), opts=options(nnz))
+    clean = np.where(np.isfinite(A), A, 0.0).sum(1)
+    want = np.where(np.isnan(A).any(1)[rows], np.nan, np.where(np.isinf(A).any(1)[rows], np.inf, clean[rows]))
+    for q, d in enumerate(at):
+        want = want + np.where((cols == 10 * q) & np.isfinite(want), 2.0 * A[rows, d], 0.0)
+    assert np.array_equal(D.cpu().numpy(), want, equal_nan=True)    # (whole numbers below 2^11)
 
 
 @pytest.mark.gpu
