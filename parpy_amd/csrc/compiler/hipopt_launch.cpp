@@ -581,11 +581,14 @@ struct LaneSplit {
   // Rows next to each other that select neighbouring rows find them in L2 as they are, which the program does not say: there the
   // requests to L1 are what bounds it (77 % of its cycles, counted), and a row in common is a quarter of them.
   // The bounds: tables below 9 MiB gain nothing (8192 x 256 floats 55.6 -> 54.5 without the second table's passes, 1000 x 1024
-  // 26.7 -> 28.5), nor do launches that read less than 96 MiB of rows, which the added launch costs more.  Slabs are halved
+  // 26.7 -> 28.5), nor do launches that read less than 96 MiB of rows, which the added launch costs more, or less than half as much again
+  // of 4 KB and more out of tables below 16 MiB (26 400 products over 1024 floats, 10 MB: 19.7 in one piece, 22.9; 48 000: 27.5 and 26.3;
+  // 27 000 and 60 000 of 12 MB: 21.8 and 23.3, 32.6 and 29.1; 15 600 and 52 000 over 1024 doubles, 11 MB: 21.2 and 22.1, 45.5 and
+  // 36.6; but 60 000 over 512 floats, 10 MB: 24.1 and 23.4).  Slabs are halved
   // while theirs of the table is above 5 MiB, down to 512 bytes on average, a sixteenth less will do: four 16-byte pieces for each of
   // eight lanes (the first product above in slabs of 1024, 512, 256 and 128 bytes 108, 86, 96 and 156, the main launches alone; 3000 rows
   // of 4 KB, 12 MB: 49, 58, 75 and 122).
-  static constexpr int64_t DIES = 8, SLAB_ROW = 512, SLAB_TABLE = int64_t(5) << 20, WHOLE_TABLE = int64_t(9) << 20, GATHERED = int64_t(96) << 20;
+  static constexpr int64_t DIES = 8, SLAB_ROW = 512, SLAB_TABLE = int64_t(5) << 20, WHOLE_TABLE = int64_t(9) << 20, LARGE_TABLE = int64_t(16) << 20, LONG_ROW = 4096, GATHERED = int64_t(96) << 20;
   void slabs(const Kernel& k, const StmtP& launch, const S& root, size_t pos, int vec, const E& term) {
     const S& loop = root->body[pos];
     const E& acc = loop->body[0]->dst;
@@ -626,7 +629,7 @@ struct LaneSplit {
       if (e->dim_shape.empty() || e->ty.sz != acc->ty.sz) ok = false;
       table = table == 0 ? bytes : std::min(table, bytes);
     });
-    if (!ok || table <= WHOLE_TABLE || N * K * es < GATHERED) return;
+    if (!ok || table <= WHOLE_TABLE || N * K * es < (table < LARGE_TABLE && K * es >= LONG_ROW ? GATHERED / 2 * 3 : GATHERED)) return;
     int64_t cut = 1;
     const int64_t chunks = (K + chunk - 1) / chunk;
     auto divides = [&](int64_t n) { return (n - 1) * ((chunks + n - 1) / n) < chunks; };
