@@ -380,12 +380,13 @@ struct RaggedSum {
     // Single sums: a workgroup is over with its slowest wavefront; 1024 / 512 / 256 threads 36.6 / 34.2 / 34.2 us for the 50
     // non-zeros above, 29.9 / 28.2 / 30.2 in floats, 99.8 / 91.2 / 91.9 for 10^6 rows of 10 floats.  Where all wavefronts run at
     // once: 16 000 rows of 60 floats 12.5 / 10.6 / 10.4, doubles 15.2 / 14.0 / 13.0, 20 000 of 7 floats 6.6 / 5.8 / 5.6, 10 000 of
-    // 100 10.5 / 10.5 / 10.2, 12 000 of 200 doubles 26.2 / 26.1 / 26.5; with fewer rows the shared ones count: 5000 of 100 floats
-    // 5.7 / 5.6 / 5.8, 3000 of 200 7.3 / 6.9 / 7.7, 3000 of 60 doubles 5.0 / 4.7 / 4.3.
+    // 100 10.5 / 10.5 / 10.2, 12 000 of 200 doubles 26.2 / 26.1 / 26.5.  Up to 5000 rows doubles gain (1100 of 100 4.6 / 4.0, 2500
+    // of 150 7.0 / 6.4, 3000 of 200 12.1 / 11.0, 4000 of 100 7.8 / 6.9, 4900 of 60 5.9 / 5.4; where the time is that of one longest row
+    // it depends on the matrix: 4500 of 180 12.0 / 11.5 and 11.9 / 12.2, 2000 of 100 5.1 / 5.1), and floats gain or lose (2000 of 100 3.8 / 4.0, 4000 of 199 7.7 / 8.1, 5000 of 150 8.3 / 8.5; 3000 of 200 8.7 / 8.2, 4500 of 180 8.6 / 8.2).
     // Rows of columns: 512 threads, unless a row of average length is more than one batch of its team and cannot be divided into
     // slabs, whose longest rows take 1024 (7794 rows of 45 times 32 columns: 13.5 us and 12.6; 3000 of 200 times 20: 25.8 and
     // 20.2; but 100 000 of 20 times 32: 39.7 and 50.9, 58 973 of 27 times 32: 29.7 and 38.1).
-    const bool fewer = r.has_col ? wide <= 512 && (SL > 1 || 8 * avg < 7 * P * U || r.n * T0 > 4 * RESIDENT) : queues || r.n > 5000;
+    const bool fewer = r.has_col ? wide <= 512 && (SL > 1 || 8 * avg < 7 * P * U || r.n * T0 > 4 * RESIDENT) : queues || words == 2 || r.n > 5000;
     const int64_t tpb = fewer ? std::min<int64_t>(r.tpb, 512) : r.tpb;
     if (tpb % WAVE_SIZE != 0 || tpb < L * V || r.n * T * SL > (int64_t(1) << 30)) return false;
     const int64_t teams = tpb / T, waves = tpb / WAVE_SIZE;
