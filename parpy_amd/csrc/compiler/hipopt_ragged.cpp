@@ -250,16 +250,23 @@ struct RaggedSum {
     return r.cols % v == 0 || whole_vectors_pay(r, v) ? v : 1;
   }
 
-  // does a row read, in front of its columns, an array that they store, or one that may be the same memory
+  // does a row read, in front of its columns, an array that they store, or one that may be the same memory: of the same type,
+  // and large enough to have an element in every row
   static bool reads_first(const Rows& r) {
     std::vector<E> stored;
     if (r.acc->k == Expr::Index) stored.push_back(r.acc);
     for (auto& st : r.post) if (st->dst && st->dst->k == Expr::Index) stored.push_back(st->dst);
+    auto elements = [](const E& x) {
+      if (x->dim_shape.empty()) return INT64_MAX;
+      int64_t n = 1;
+      for (int64_t d : x->dim_shape) n *= d;
+      return n;
+    };
     bool found = false;
     auto scan = [&](const E& e) {
       visit_exprs(e, [&](const E& x) {
         if (x->k != Expr::Index) return;
-        for (auto& q : stored) found = found || expr_eq(x->args[0], q->args[0]) || (x->ty.sz == q->ty.sz && x->dim_shape == q->dim_shape);
+        for (auto& q : stored) found = found || expr_eq(x->args[0], q->args[0]) || (x->ty.sz == q->ty.sz && elements(x) > (r.n - 1) * r.cols);
       });
     };
     for (auto& st : r.pre) scan(st->expr);

@@ -67,6 +67,20 @@ def spmm_less_kept(A, B, C):
 
 
 @parpy.jit
+def spmm_less_flat(A, B, C, D):
+    parpy.label('i')
+    for i in range(A["nrows"]):
+        x = C[i * B["ncols"]]
+        parpy.label('j')
+        for j in range(B["ncols"]):
+            t = 0.0
+            parpy.label('k')
+            for k in range(A["rows"][i], A["rows"][i + 1]):
+                t += A["values"][k] * B["values"][A["cols"][k], j]
+            D[i, j] = t - x
+
+
+@parpy.jit
 def spmm_scaled(A, B, w, C):
     parpy.label('i')
     for i in range(A["nrows"]):
@@ -144,7 +158,7 @@ def test_rows_that_read_first_what_they_store(n, avg, cols, slabs):
     A = {"values": np.zeros(n * avg, np.float32), "rows": np.arange(n + 1) * avg, "cols": np.zeros(n * avg, np.int64), "nrows": n}
     B, C = {"values": np.zeros((99, cols), np.float32), "ncols": cols}, np.zeros((n, cols), np.float32)
     listing = lambda fun, *args: parpy.print_compiled(fun, [A, B, *args], options(n, cols))
-    for s in (listing(spmm_less_kept, C), listing(spmm_less, C, C.copy())):
+    for s in (listing(spmm_less_kept, C), listing(spmm_less, C, C.copy()), listing(spmm_less_flat, C.reshape(-1).copy(), C)):
         hiprtc_compile(s[:s.index("// host side")], options(n, cols))
         assert slabs_in(s) == 1
     assert slabs_in(listing(spmm_scaled, np.zeros(n, np.float32), C)) == slabs
@@ -163,4 +177,7 @@ def test_sums_of_rows_that_read_first(n, avg, cols, slabs):
     assert np.abs(C.cpu().numpy() - want).max() < 2e-6 * 60 * 8   # (as above)
     C = on_gpu(C0)
     spmm_less(A, B, C, C, opts=options(n, cols))
+    assert np.abs(C.cpu().numpy() - want).max() < 2e-6 * 60 * 8
+    C = on_gpu(C0)
+    spmm_less_flat(A, B, C.view(-1), C, opts=options(n, cols))
     assert np.abs(C.cpu().numpy() - want).max() < 2e-6 * 60 * 8
