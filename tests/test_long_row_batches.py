@@ -29,7 +29,7 @@ def options(n):
 
 # rows, average, type, lanes of a row, workgroups in front
 SHAPES = [(1000, 47, np.float32, 8, 0), (1000, 48, np.float64, 32, 0), (900, 100, np.float32, 64, 0), (65, 300, np.float64, 64, 0),
-          (16000, 60, np.float64, 32, 256), (8000, 150, np.float64, 64, 256), (14400, 60, np.float64, 32, 256), (16000, 60, np.float32, 32, 256),
+          (16000, 60, np.float64, 32, 256), (8000, 150, np.float64, 64, 256), (14400, 60, np.float64, 32, 256), (16000, 60, np.float32, 32, 0),
           (14100, 60, np.float64, 32, 71), (5000, 100, np.float32, 64, 199), (1100, 100, np.float64, 64, 68)]
 
 
