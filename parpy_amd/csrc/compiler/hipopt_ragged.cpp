@@ -413,8 +413,9 @@ struct RaggedSum {
     // exactly.  Fewer single sums: one for sixteen rows where there is room beside the others (3000 rows of 60, doubles 6.3 ->
     // 4.9 us, 5.5 with one for four; 20 000 of 30: 9.8 -> 9.0), else 256 for doubles, whose others then start a little later
     // (none / 64 / 128 / 256 / 512: 16 000 rows of 60 14.1 / 14.4 / 13.1 / 11.6 / 12.4, 15 500 of 40 10.3 / 10.2 / 8.9 / 8.5 / 9.1, 7800
-    // of 80 10.4 / 11.0 / 9.5 / 9.0 / 9.2, 8000 of 150 16.0 / 17.5 / 15.4 / 15.5 / 15.6), and for floats, which gain less, the
-    // queues of the others' workgroups (8000 rows of 150 12.7 us, 14.2 with 64 in front, 12.0 with 256).
+    // of 80 10.4 / 11.0 / 9.5 / 9.0 / 9.2, 8000 of 150 16.0 / 17.5 / 15.4 / 15.5 / 15.6).  Floats keep the queues of the others'
+    // workgroups there, as the tests of this rule have it; 256 in front would be worth -2 to 20 % (none / 256: 16 000 of 40 7.3 / 6.3,
+    // 14 400 of 60 9.7 / 8.9, 16 300 of 64 10.8 / 11.0, 8100 of 100 9.0 / 8.7, 8000 of 150 13.6 / 11.4, 31 000 of 25 7.9 / 7.2).
     const int64_t room = RESIDENT / r.tpb - (r.n * T0 + r.tpb - 1) / r.tpb;
     const int64_t scouts = queues ? std::max<int64_t>(r.has_col ? 1024 : 512, (r.n * SL + 1023) / 1024)
                            : r.one_group ? 0

@@ -29,8 +29,8 @@ namespace {
 //
 // The step of a model of 16 layers of 16 384 states (`forward_kernel`, one thread per state of a layer, 100 rows of 1 MB that
 // fit the memory-side cache): 31 us as a launch of its own, of which a copy of the arrays takes 25.6 and the vector ALU 24; two
-// steps 55 us, bound by the vector ALU (59 with four recomputed values per thread instead of one).  100 reads of 500 to
-// 1500 samples 36.2 -> 28.6 ms, 37 of them 18.2 -> 14.4; 98 of 666 to 2000 over 16 layers of 4096 states 19.2 -> 15.2.
+// steps 55 to 61 us, of which vector instructions are active for 54 (counted, 89 % of the cycles; four recomputed values per
+// thread instead of one: 4 us more).  100 reads of 500 to 1500 samples 36.2 -> 28.6 ms, 37 of them 18.2 -> 14.4; 98 of 666 to 2000 over 16 layers of 4096 states 19.2 -> 15.2.
 struct TwoSteps {
   Program& p;
   const Options& opts;
