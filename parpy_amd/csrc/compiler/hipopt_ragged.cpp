@@ -389,7 +389,9 @@ struct RaggedSum {
     // once: 16 000 rows of 60 floats 12.5 / 10.6 / 10.4, doubles 15.2 / 14.0 / 13.0, 20 000 of 7 floats 6.6 / 5.8 / 5.6, 10 000 of
     // 100 10.5 / 10.5 / 10.2, 12 000 of 200 doubles 26.2 / 26.1 / 26.5.  Up to 5000 rows doubles gain (1100 of 100 4.6 / 4.0, 2500
     // of 150 7.0 / 6.4, 3000 of 200 12.1 / 11.0, 4000 of 100 7.8 / 6.9, 4900 of 60 5.9 / 5.4; where the time is that of one longest row
-    // it depends on the matrix: 4500 of 180 12.0 / 11.5 and 11.9 / 12.2, 2000 of 100 5.1 / 5.1), and floats gain or lose (2000 of 100 3.8 / 4.0, 4000 of 199 7.7 / 8.1, 5000 of 150 8.3 / 8.5; 3000 of 200 8.7 / 8.2, 4500 of 180 8.6 / 8.2).
+    // it depends on the matrix: 4500 of 180 12.0 / 11.5 and 11.9 / 12.2, 2000 of 100 5.1 / 5.1), and floats, which gain or lose,
+    // keep the threads they have (2000 of 100 3.8 / 4.0, 4000 of 199 7.7 / 8.1, 5000 of 150 8.3 / 8.5; 3000 of 200 8.7 / 8.2, 4500 of
+    // 180 8.6 / 8.2).
     // Rows of columns: 512 threads, unless a row of average length is more than one batch of its team and cannot be divided into
     // slabs, whose longest rows take 1024 (7794 rows of 45 times 32 columns: 13.5 us and 12.6; 3000 of 200 times 20: 25.8 and
     // 20.2; but 100 000 of 20 times 32: 39.7 and 50.9, 58 973 of 27 times 32: 29.7 and 38.1).
